@@ -80,6 +80,43 @@ def test_gemm_forms_exact(form, M_, N, K):
     np.testing.assert_array_equal(c, ref.astype(np.float32))
 
 
+@pytest.mark.parametrize("M_,N,K", [(65, 128, 1024), (256, 256, 1344), (257, 768, 2112), (391, 512, 4096),
+                                    (1001, 384, 1088), (17, 192 * 6, 16384)])
+def test_gemm_k_slices_exact(M_, N, K):
+    """Few tiles and a deep sum: K is cut into slices (uneven ones too, 21 and 33 K tiles) whose f32
+    partials a second launch sums. Small integers, so every order of the sums is exact."""
+    rng = np.random.default_rng(M_ + N + K)
+    a = rng.integers(-4, 5, size=(M_, K)).astype(np.float16)
+    w = rng.integers(-4, 5, size=(N, K)).astype(np.float16)
+    w[:, 0] += np.arange(N, dtype=np.float16) % 7
+    ref = a.astype(np.float64) @ w.astype(np.float64).T
+    np.testing.assert_array_equal(rt().gemm_f16(a, w), ref.astype(np.float32))
+
+
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("T", [5, 64, 65, 200, 300])
+def test_prefill_k_slices_match_whole(T, split):
+    """The whole prefill with K slices (two-depth QKV, gated pair, residual sums with the next norm)
+    against the same with whole tiles: sums in another order, then the same f16 roundings."""
+    R = rt()
+    cfg = M.ModelConfig(dim=1536, hidden_dim=4096, head_dim=128, n_layers=2, n_heads=12, n_kv_heads=4, vocab_size=1024,
+                        max_seq_len=320, rope_theta=1e6, act=M.SILU, weight_dtype=M.F16)
+    dm = R.DeviceModel.from_arrays(cfg, M.synth_host_tensors(cfg, seed=3))
+    dec = R.Decoder(dm)
+    try:
+        tok = (np.arange(T) * 37 + 5) % cfg.vocab_size
+        got = {}
+        for form in ("", "ksplit:0,wnorm:0,skinny:0"):
+            dec.set_prefill_forms(form)
+            dec.set_prefill_precision(R.PREFILL_SPLIT if split else R.PREFILL_FAST)
+            got[form] = dec.prefill(tok)
+        a, b = got.values()
+        assert np.max(np.abs(a - b)) < (2e-4 if split else LP_ATOL / 2)
+    finally:
+        dec.close()
+        dm.close()
+
+
 @pytest.mark.parametrize("M_,N,K", [(300, 384, 512), (4096, 128, 3072)])
 def test_gemm_random(M_, N, K):
     rng = np.random.default_rng(7)

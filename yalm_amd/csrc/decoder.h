@@ -76,7 +76,7 @@ struct PrefillBufs {
 	float *pmax = nullptr, *psum = nullptr; // [cap][vocab / 128] logits partials
 	float *tgt_logit = nullptr, *lp = nullptr; // [cap]
 	float *rope = nullptr;                     // [cap][head_dim / 2][2]
-	float *skp = nullptr;                      // split-K partials of the short-prompt GEMMs (prefill_skinny.h)
+	float *skp = nullptr;                      // split-K partials (prefill_skinny.h; gemm8p_kernel's slices)
 	size_t skp_floats = 0;
 	unsigned *range = nullptr;                 // [n_layers + 1][4] f16-operand range guard (prefill.h range_note)
 	uint16_t *wdq = nullptr;                   // fp8 models: one layer's (or the classifier's) weights as f16
@@ -95,6 +95,7 @@ struct PfForms {
 	bool skl = true;        // skinny GEMMs: weight rows staged by LDS-DMA (prefill_skinny.h)
 	bool split = false;     // split-operand precision form (yalm_set_prefill_precision): every f16
 							// activation operand as [hi | lo], the large-tile GEMMs at every T
+	bool ksplit = true;     // large tiles: K split over workgroups where the tiles leave CUs idle (gemm8p_kernel)
 	bool wnorm = true;      // row norms: one wave per row, the row in registers (rmsnorm_rows_wave_kernel)
 };
 PfForms pf_forms_default(); // prefill.hip: the production forms (A/B build: YALM_PF_FORMS)

@@ -26,7 +26,7 @@
 // the 2-phase kernel, persist:0 one workgroup per tile, skinny:0 the large tiles at
 // T <= 64 too (prefill_skinny.h otherwise), qkv1:0 the q and k | v GEMMs as two
 // launches, skl:0 the skinny GEMMs' weights as register loads instead of LDS-DMA stages,
-// wnorm:0 the workgroup-per-row norm kernel instead of one wave per row.
+// ksplit:0 no K slices (plan_split), wnorm:0 the workgroup-per-row norm kernel instead of one wave per row.
 // The production library reads no environment for them; the A/B build (-DYALM_AB)
 // takes a decoder's initial forms from YALM_PF_FORMS (same syntax).
 static int parse_pf_forms(const char *spec, PfForms &f) {
@@ -62,6 +62,8 @@ static int parse_pf_forms(const char *spec, PfForms &f) {
 			f.skl = val != 0, known = true;
 		else if (!strcmp(key, "split"))
 			f.split = val != 0, known = true;
+		else if (!strcmp(key, "ksplit"))
+			f.ksplit = val != 0, known = true;
 		else if (!strcmp(key, "wnorm"))
 			f.wnorm = val != 0, known = true;
 		if (!known) {
@@ -142,10 +144,88 @@ int pick_bn(const PfForms &f, int kind, int M, int n_eff, bool glu, bool ragged 
 	return best;
 }
 
+// A GEMM of few rows on the large tiles: tile width bn, K in slices of nkc K tiles (ks of them; ks2 of
+// the deeper columns). ks = 1: not split.
+struct SplitPlan {
+	int bn = 0, nkc = 1 << 24, ks = 1, ks2 = 1;
+};
+int slices(int K, int nkc) { return (K / pf::BK + nkc - 1) / nkc; }
+
+// Time of one round of 256-row tiles, in us per K tile of 64 and per tile (pipeline fill, epilogue), as
+// measured with the chip full (Mistral-7B: 391 rows, W1 | W3, 64 K tiles at width 256, 93-100 us; the 104
+// K tiles of its QKV, Wo and W2 slices at width 128, 129 us; 1001 rows, QKV slices of 32 at 256, 58 us), and
+// a slot's f32 traffic (written, and read back from L2 and the Infinity Cache at about 5 TB/s: 45 MB in the
+// 10 us of a 391-row reduce + norm). The whole is the rounds that the busiest CU walks; the deeper columns
+// (Nd of depth Kd) count by their own slices. Split only where that model gains a tenth: the partials are
+// extra bytes. Mistral-7B, 391 rows, QKV + Wo + W2 of a layer: 425 us whole, 129 us + 28 us of sums in slices.
+constexpr float T8P_KT[3] = {1.05f, 1.3f, 1.55f}, T8P_TILE = 5.0f; // widths 128, 192, 256
+SplitPlan plan_split(const PfForms &f, int kind, int M, int N, int K, int Nd, int Kd, bool glu, size_t cap) {
+	SplitPlan best;
+	if (!f.ksplit || !f.p8 || f.g16[kind] > 0)
+		return best;
+	const long ncu = device_cu_count(), tm = (M + pf::G_BM - 1) / pf::G_BM, TP = (M + 15) / 16 * 16;
+	const int nk = K / pf::BK, nkd = Nd ? Kd / pf::BK : 0;
+	float whole = 0.0f, least = 0.0f;
+	for (int w = 0; w < 3; ++w) {
+		const int bn = 128 + 64 * w;
+		if (N % bn || Nd % bn || (glu && bn != 256))
+			continue;
+		for (int ks = 1; ks <= 16; ++ks) {
+			const int nkc = (nk + ks - 1) / ks;
+			if (ks > 1 && (nkc < 8 || nkc == (nk + ks - 2) / (ks - 1)))
+				continue;
+			const int k1 = (nk + nkc - 1) / nkc, k2 = Nd ? (nkd + nkc - 1) / nkc : 1;
+			if (ks > 1 && (size_t)std::max(k1, k2) * TP * (N + Nd) > cap)
+				break;
+			// (not split, two depths: the deep tiles alone, or the mean over the CUs)
+			const long items = tm * (N / bn * k1 + Nd / bn * k2);
+			float t = (float)((items + ncu - 1) / ncu) * (nkc * T8P_KT[w] + T8P_TILE);
+			if (ks == 1 && Nd)
+				t = std::max((float)nkd, (float)(tm * (N / bn * nk + Nd / bn * nkd)) / ncu) * T8P_KT[w] + T8P_TILE;
+			if (ks == 1) {
+				whole = whole == 0.0f ? t : std::min(whole, t);
+				continue;
+			}
+			t += 3.0f + (float)((long)k1 * N + (long)k2 * Nd) * M * 8.0f / 5e6f;
+			if (least == 0.0f || t < least) {
+				least = t;
+				best = {bn, nkc, k1, k2};
+			}
+		}
+	}
+	return best.ks > 1 && least < 0.9f * whole ? best : SplitPlan{};
+}
+
+template <class EPI, class BMAP, int FJ0, int FJ1>
+int launch_g8p(const PfForms &f, const uint16_t *A, int lda, int M, int K, int kb, const BMAP &bm, int N,
+               const EPI &epi, hipStream_t st, int c0, int c_split = -1, int K2 = 0, int nkc = 1 << 24);
+
+// The K slices' partials of C = A B^T into `part` ([slot][16-row-rounded M][N + Nd]); columns [N, N + Nd)
+// (Nd > 0: width 256) run depth Kd
+template <class BMAP, bool BF = false>
+int launch_split(const PfForms &f, const SplitPlan &s, const uint16_t *A, int lda, int M, int K, int kb, const BMAP &bm,
+                 int N, int Nd, int Kd, float *part, hipStream_t st) {
+	pf::E16Part<BF> e;
+	e.part = part;
+	e.ld = N + Nd;
+	e.kstride = (size_t)((M + 15) / 16 * 16) * (N + Nd);
+	e.M = M;
+	e.mul = BMAP::COLS_PER_TILE_DIV;
+	if (s.bn == 256)
+		return launch_g8p<pf::E16Part<BF>, BMAP, 2, 2>(f, A, lda, M, K, kb, bm, N + Nd, e, st, 0, Nd ? N : -1, Kd, s.nkc);
+	if constexpr (BMAP::COLS_PER_TILE_DIV == 1) {
+		if (s.bn == 192)
+			return launch_g8p<pf::E16Part<BF>, BMAP, 2, 1>(f, A, lda, M, K, kb, bm, N + Nd, e, st, 0, Nd ? N : -1, Kd, s.nkc);
+		return launch_g8p<pf::E16Part<BF>, BMAP, 1, 1>(f, A, lda, M, K, kb, bm, N + Nd, e, st, 0, Nd ? N : -1, Kd, s.nkc);
+	}
+	set_err("prefill GEMM: a gated pair's K slices have width 256");
+	return YALM_ERR_UNSUPPORTED;
+}
+
 // c_split / K2: columns [c_split, N) run K2 (gemm8p_kernel); c_split = N: one depth
 template <class EPI, class BMAP, int FJ0, int FJ1>
 int launch_g8p(const PfForms &f, const uint16_t *A, int lda, int M, int K, int kb, const BMAP &bm, int N,
-               const EPI &epi, hipStream_t st, int c0, int c_split = -1, int K2 = 0) {
+               const EPI &epi, hipStream_t st, int c0, int c_split, int K2, int nkc) {
 	auto kern = pf::gemm8p_kernel<EPI, BMAP, FJ0, FJ1>;
 	constexpr size_t lds = pf::gemm8p_lds<FJ0, FJ1>();
 	constexpr int BN = 64 * (FJ0 + FJ1);
@@ -154,14 +234,16 @@ int launch_g8p(const PfForms &f, const uint16_t *A, int lda, int M, int K, int k
 		HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
 		attr = true;
 	}
-	const int nwg = ((M + pf::G_BM - 1) / pf::G_BM) * (N / BN);
-	// more tiles than CUs: one persistent workgroup per CU walks them
-	const int ncu = (int)device_cu_count();
+	const int tiles_m = (M + pf::G_BM - 1) / pf::G_BM;
 	// (two depths: one workgroup per tile, so the hardware balances them longest first)
 	const bool two = c_split >= 0 && c_split < N;
-	const int grid = f.persist && nwg > ncu && !two ? ncu : nwg;
+	const int ks1 = pf::epi_partial<EPI>::value ? slices(K, nkc) : 1, ks2 = pf::epi_partial<EPI>::value && two ? slices(K2, nkc) : 1;
+	const int nwg = tiles_m * ((two ? c_split : N) / BN * ks1 + (two ? N - c_split : 0) / BN * ks2);
+	// more tiles than CUs: one persistent workgroup per CU walks them
+	const int ncu = (int)device_cu_count();
+	const int grid = f.persist && nwg > ncu && !two && !pf::epi_partial<EPI>::value ? ncu : nwg;
 	hipLaunchKernelGGL(kern, dim3(grid), dim3(pf::G_THREADS), lds, st, A, lda, M, K, kb, bm, N, epi, c0,
-	                   two ? c_split : N, two ? K2 : K);
+	                   two ? c_split : N, two ? K2 : K, nkc);
 	HIPCHK(hipGetLastError());
 	return YALM_OK;
 }
@@ -354,6 +436,28 @@ int launch_rmsnorm(bool split, const PfForms &f, const float *X, const float *w,
 	             : launch_rmsnorm_t<false>(f, X, w, dim, T, eps, Xn, range, st);
 }
 
+// X += scale * (sum of the partials), Xn = the next norm's operand (prefill_skinny.h); w null: no norm
+template <bool SPLIT>
+int launch_reduce_norm_t(const float *part, int KS, int T, float *X, int dim, float scale, const float *w, float eps,
+                         uint16_t *Xn, unsigned *range, hipStream_t st) {
+	const size_t kstride = (size_t)((T + 15) / 16 * 16) * dim;
+	const int nt = std::min(1024, (dim / 4 + 63) / 64 * 64), nv = (dim / 4 + nt - 1) / nt;
+	if (nv == 1)
+		pf::reduce_norm_rows_kernel<SPLIT, 1><<<T, nt, 0, st>>>(part, KS, kstride, X, dim, scale, w, eps, Xn, range);
+	else if (nv == 2)
+		pf::reduce_norm_rows_kernel<SPLIT, 2><<<T, nt, 0, st>>>(part, KS, kstride, X, dim, scale, w, eps, Xn, range);
+	else
+		pf::reduce_norm_rows_kernel<SPLIT, 4><<<T, nt, 0, st>>>(part, KS, kstride, X, dim, scale, w, eps, Xn, range);
+	HIPCHK(hipGetLastError());
+	return YALM_OK;
+}
+int launch_reduce_norm(bool split, const float *part, int KS, int T, float *X, int dim, float scale, const float *w,
+                       float eps, uint16_t *Xn, unsigned *range, hipStream_t st) {
+	return split ? launch_reduce_norm_t<true>(part, KS, T, X, dim, scale, w, eps, Xn, range, st)
+	             : launch_reduce_norm_t<false>(part, KS, T, X, dim, scale, w, eps, Xn, range, st);
+}
+constexpr int REDUCE_NORM_MAX_DIM = 4 * 1024 * 4; // the row in registers: 4 float4 of 1024 threads
+
 template <int D, bool SPLIT>
 int launch_attn_prefill_t(const uint16_t *Q, const uint16_t *kc, const uint16_t *vc, int T, int pos0, int n_heads,
 						  int n_kv, uint16_t *O, hipStream_t st) {
@@ -424,7 +528,7 @@ int ensure_bufs(yalm_decoder_s *d) {
 							 3 * (size_t)c.dim * c.hidden_dim;
 		TRY(pf_alloc(d, (void **)&b.wdq, 2 * std::max(layer, (size_t)c.vocab_size * c.dim)));
 	}
-	{ // short-prompt split-K partials: the largest [KS][64][Np] of the layer's GEMMs
+	{ // split-K partials; short prompts: the largest [KS][64][Np] of the layer's GEMMs
 		const int kv_dim = c.n_kv_heads * c.head_dim, TP = SK_MAX_T;
 		const int np_qkv = (int)q_dim + 2 * kv_dim;
 		// (QKV: 2 KS partial slots, the k | v GEMM's)
@@ -434,6 +538,9 @@ int ensure_bufs(yalm_decoder_s *d) {
 		    (size_t)std::max(1, sk_pick_ks({{2 * c.hidden_dim, c.dim, 1}}, TP)) * 2 * c.hidden_dim,
 		    (size_t)std::max(1, sk_pick_ks({{c.dim, c.hidden_dim, 1}}, TP)) * c.dim};
 		b.skp_floats = (size_t)TP * *std::max_element(sz, sz + 4);
+		// K slices of the large tiles: at most 128 MB, which plan_split keeps to
+		const size_t widest = std::max({(size_t)np_qkv, (size_t)c.dim, (size_t)2 * c.hidden_dim});
+		b.skp_floats = std::max(b.skp_floats, std::min((size_t)32 << 20, 16 * (cap + 15) / 16 * 16 * widest));
 		TRY(pf_alloc(d, (void **)&b.skp, b.skp_floats * 4));
 	}
 	b.cap = (int)cap;
@@ -454,6 +561,11 @@ int enqueue_glu_t(yalm_decoder_s *d, const yalm_block_weights &w, int T, float h
 	e.range = range;
 	e.lo_off = SPLIT ? c.hidden_dim : 0;
 	pf::BRowsGlu<64> bm{(const uint16_t *)w.w1, (const uint16_t *)w.w3};
+	const SplitPlan s = plan_split(f, PG_GLU, T, 2 * c.hidden_dim, sp * c.dim, 0, 0, true, d->pf.skp_floats);
+	if (s.ks > 1) {
+		TRY(launch_split(f, s, d->pf.Xn, sp * c.dim, T, sp * c.dim, c.dim, bm, 2 * c.hidden_dim, 0, 0, d->pf.skp, d->stream));
+		return launch_skinny_reduce<true>(d->pf.skp, s.ks, s.ks, 2 * c.hidden_dim, T, 2 * c.hidden_dim, e, d->stream);
+	}
 	if (bn == 256)
 		return launch_g16_t<pf::E16Glu<ACT, SPLIT>, pf::BRowsGlu<64>, 256, 2>(f, d->pf.Xn, sp * c.dim, T, sp * c.dim, c.dim,
                                                                      bm, 2 * c.hidden_dim, e, d->stream);
@@ -511,6 +623,24 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 	const bool split = f.split;
 	const int sp = split ? 2 : 1;
 	const int bn_qkv_all = pick_bn(f, PG_QKV, T, q_dim + 2 * kv_dim, false);
+	// too few tiles for the chip: K slices. Wo's and W2's partials, and a short prompt's, are
+	// summed by the launch that also adds the residual and makes the next product's operand
+	const size_t pcap = b.skp_floats;
+	const SplitPlan s_qkv = split ? plan_split(f, PG_QKV, T, q_dim + 2 * kv_dim, 2 * c.dim, 0, 0, false, pcap)
+	                              : plan_split(f, PG_QKV, T, q_dim, c.dim, 2 * kv_dim, 2 * c.dim, false, pcap);
+	const SplitPlan s_wo = plan_split(f, PG_WO, T, c.dim, sp * q_dim, 0, 0, false, pcap);
+	const SplitPlan s_w2 = plan_split(f, PG_W2, T, c.dim, sp * c.hidden_dim, 0, 0, false, pcap);
+	const bool fused_norm = f.wnorm && c.dim <= REDUCE_NORM_MAX_DIM;
+	auto reduce_norm = [&](int KS, float scale, const float *w, bool xsplit, unsigned *range) -> int {
+		if (!fused_norm) { // (rows too wide for the fused kernel's registers)
+			pf::E16Residual e;
+			e.x = b.X, e.ldx = c.dim, e.M = T, e.scale = scale;
+			TRY(launch_skinny_reduce<false>(b.skp, KS, KS, c.dim, T, c.dim, e, st));
+			return w ? launch_rmsnorm(xsplit, f, b.X, w, c.dim, T, c.norm_eps, b.Xn, range, st) : YALM_OK;
+		}
+		return launch_reduce_norm(xsplit, b.skp, KS, T, b.X, c.dim, scale, w, c.norm_eps, b.Xn, range, st);
+	};
+	bool normed = false; // Xn holds this layer's attention input already
 	for (int l = 0; l < c.n_layers; ++l) {
 		yalm_block_weights w = d->b[l];
 		if (fp8) { // this layer's weights as f16 (exact), in the scratch the previous layer's GEMMs are done with
@@ -523,7 +653,8 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 		// the k | v columns' (their cache rows then carry one f16 rounding, infer.cpp:299)
 		unsigned *rg = b.range + (size_t)l * RG_N;
 		const int he = hexp ? hexp[l] : 0;
-		TRY(launch_rmsnorm(true, f, b.X, w.rms_att, c.dim, T, c.norm_eps, b.Xn, rg + RG_XATT, st));
+		if (!normed)
+			TRY(launch_rmsnorm(true, f, b.X, w.rms_att, c.dim, T, c.norm_eps, b.Xn, rg + RG_XATT, st));
 		{
 			pf::BSrc qkv{};
 			qkv.p[0] = (const uint16_t *)w.wq;
@@ -554,12 +685,22 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 				                  st));
 				TRY(launch_skinny_reduce<false>(b.skp, ks_qkv, 2 * ks_qkv, q_dim, T, np, e, st));
 			} else {
+				const int np = q_dim + 2 * kv_dim;
 				if (split) { // q | k | v all over [hi | lo], Q stored [hi | lo]
 					pf::E16QKVt<true> es;
 					es.q = e.q, es.kc = e.kc, es.vc = e.vc, es.rope = e.rope, es.M = e.M, es.q_dim = e.q_dim;
 					es.kv_dim = e.kv_dim, es.head_dim = e.head_dim, es.pos0 = e.pos0, es.clip = e.clip;
 					es.range = e.range, es.q_lo = q_dim;
-					TRY(launch_plain(f, bn_qkv_all, b.Xn, 2 * c.dim, T, 2 * c.dim, c.dim, qkv, q_dim + 2 * kv_dim, es, st));
+					if (s_qkv.ks > 1) {
+						TRY(launch_split(f, s_qkv, b.Xn, 2 * c.dim, T, 2 * c.dim, c.dim, pf::BRowsPlain{qkv}, np, 0, 0, b.skp, st));
+						TRY(launch_skinny_reduce<false>(b.skp, s_qkv.ks, s_qkv.ks, np, T, np, es, st));
+					} else {
+						TRY(launch_plain(f, bn_qkv_all, b.Xn, 2 * c.dim, T, 2 * c.dim, c.dim, qkv, np, es, st));
+					}
+				} else if (s_qkv.ks > 1) {
+					TRY(launch_split(f, s_qkv, b.Xn, 2 * c.dim, T, c.dim, c.dim, pf::BRowsPlain{qkv}, q_dim, 2 * kv_dim,
+					                 2 * c.dim, b.skp, st));
+					TRY(launch_skinny_reduce<false>(b.skp, s_qkv.ks, s_qkv.ks2, q_dim, T, np, e, st));
 				} else if (qkv1) { // one launch: the k | v tiles (K = 2 dim) first, then the q tiles (K = dim)
 					TRY((launch_g8p<pf::E16QKV, pf::BRowsPlain, 2, 2>(f, b.Xn, 2 * c.dim, T, c.dim, c.dim,
 					                                                   pf::BRowsPlain{qkv}, q_dim + 2 * kv_dim, e, st,
@@ -572,20 +713,22 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 		}
 		TRY(launch_attn_prefill(b.Q, w.key_cache, w.value_cache, T, pos0, c.n_heads, c.n_kv_heads, c.head_dim, b.O,
 								st, split));
-		{
+		if (small || s_wo.ks > 1) {
+			if (small)
+				TRY(launch_skinny(f, b.O, q_dim, T, q_dim, q_dim, pf::BRowsPlain{one(w.wo, c.dim)}, c.dim, ks_wo, 0, c.dim,
+				                  b.skp, st));
+			else
+				TRY(launch_split(f, s_wo, b.O, sp * q_dim, T, sp * q_dim, q_dim, pf::BRowsPlain{one(w.wo, c.dim)}, c.dim, 0, 0,
+				                 b.skp, st));
+			TRY(reduce_norm(small ? ks_wo : s_wo.ks, 1.0f, w.rms_ffn, split, rg + RG_XFFN));
+		} else {
 			pf::E16Residual e;
 			e.x = b.X;
 			e.ldx = c.dim;
 			e.M = T;
-			if (small) {
-				TRY(launch_skinny(f, b.O, q_dim, T, q_dim, q_dim, pf::BRowsPlain{one(w.wo, c.dim)}, c.dim, ks_wo, 0, c.dim,
-				                  b.skp, st));
-				TRY(launch_skinny_reduce<false>(b.skp, ks_wo, ks_wo, c.dim, T, c.dim, e, st));
-			} else {
-				TRY(launch_plain(f, bn_wo, b.O, sp * q_dim, T, sp * q_dim, q_dim, one(w.wo, c.dim), c.dim, e, st));
-			}
+			TRY(launch_plain(f, bn_wo, b.O, sp * q_dim, T, sp * q_dim, q_dim, one(w.wo, c.dim), c.dim, e, st));
+			TRY(launch_rmsnorm(split, f, b.X, w.rms_ffn, c.dim, T, c.norm_eps, b.Xn, rg + RG_XFFN, st));
 		}
-		TRY(launch_rmsnorm(split, f, b.X, w.rms_ffn, c.dim, T, c.norm_eps, b.Xn, rg + RG_XFFN, st));
 		const float hscale = ldexpf(1.0f, -he);
 		if (small) {
 			const pf::BRowsGlu<64> bm{(const uint16_t *)w.w1, (const uint16_t *)w.w3};
@@ -604,26 +747,33 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 			TRY(c.act == YALM_SILU ? enqueue_glu<1>(d, w, T, hscale, rg + RG_H)
 								   : enqueue_glu<0>(d, w, T, hscale, rg + RG_H));
 		}
-		{
+		// the next norm: the next layer's (its operand [hi | lo] in either form), or the final one
+		const bool last = l + 1 == c.n_layers;
+		const float *w_next = last ? (want_lp ? d->rms_final : nullptr) : d->b[l + 1].rms_att;
+		normed = small || s_w2.ks > 1;
+		if (normed) {
+			if (small)
+				TRY(launch_skinny(f, b.H, c.hidden_dim, T, c.hidden_dim, c.hidden_dim, pf::BRowsPlain{one(w.w2, c.dim)},
+				                  c.dim, ks_w2, 0, c.dim, b.skp, st));
+			else
+				TRY(launch_split(f, s_w2, b.H, sp * c.hidden_dim, T, sp * c.hidden_dim, c.hidden_dim,
+				                 pf::BRowsPlain{one(w.w2, c.dim)}, c.dim, 0, 0, b.skp, st));
+			TRY(reduce_norm(small ? ks_w2 : s_w2.ks, ldexpf(1.0f, he), w_next, last ? split : true, rg + RG_N + RG_XATT));
+		} else {
 			pf::E16Residual e;
 			e.x = b.X;
 			e.ldx = c.dim;
 			e.M = T;
 			e.scale = ldexpf(1.0f, he);
-			if (small) {
-				TRY(launch_skinny(f, b.H, c.hidden_dim, T, c.hidden_dim, c.hidden_dim, pf::BRowsPlain{one(w.w2, c.dim)},
-				                  c.dim, ks_w2, 0, c.dim, b.skp, st));
-				TRY(launch_skinny_reduce<false>(b.skp, ks_w2, ks_w2, c.dim, T, c.dim, e, st));
-			} else {
-				TRY(launch_plain(f, bn_w2, b.H, sp * c.hidden_dim, T, sp * c.hidden_dim, c.hidden_dim, one(w.w2, c.dim),
-								 c.dim, e, st));
-			}
+			TRY(launch_plain(f, bn_w2, b.H, sp * c.hidden_dim, T, sp * c.hidden_dim, c.hidden_dim, one(w.w2, c.dim),
+			                 c.dim, e, st));
 		}
 	}
 	if (!want_lp)
 		return YALM_OK;
-	TRY(launch_rmsnorm(split, f, b.X, d->rms_final, c.dim, T, c.norm_eps, b.Xn,
-	                   b.range + (size_t)c.n_layers * RG_N + RG_XATT, st));
+	if (!normed)
+		TRY(launch_rmsnorm(split, f, b.X, d->rms_final, c.dim, T, c.norm_eps, b.Xn,
+		                   b.range + (size_t)c.n_layers * RG_N + RG_XATT, st));
 	const int cls_bn = pick_bn(f, PG_CLS, T, c.vocab_size, false);
 	const int ntiles = cls_bn ? c.vocab_size / cls_bn : 1;
 	pf::E16Logits e;
@@ -821,8 +971,18 @@ extern "C" int yalm_gemm_f16(float *c, const uint16_t *a, const uint16_t *w, int
 	e16.ldc = N;
 	e16.M = M;
 	const PfForms f = g_test_forms; // a test hook: the forms set by yalm_set_prefill_forms(NULL, ...)
-	TRY(launch_plain(f, pick_bn(f, PG_TEST, M, N, false), (const uint16_t *)da.p, K, M, K, K, one(dw.p, N), N, e16,
-	                 nullptr));
+	const size_t cap = (size_t)32 << 20; // as a decoder's (ensure_bufs)
+	const SplitPlan s = plan_split(f, PG_TEST, M, N, K, 0, 0, false, cap);
+	HostDev dp;
+	if (s.ks > 1) { // K slices, summed by the reduce kernel the prefill uses
+		TRY(hd(dp, nullptr, (size_t)s.ks * ((M + 15) / 16 * 16) * N * 4));
+		TRY(launch_split(f, s, (const uint16_t *)da.p, K, M, K, K, pf::BRowsPlain{one(dw.p, N)}, N, 0, 0, (float *)dp.p,
+		                 nullptr));
+		TRY(launch_skinny_reduce<false>((const float *)dp.p, s.ks, s.ks, N, M, N, e16, nullptr));
+	} else {
+		TRY(launch_plain(f, pick_bn(f, PG_TEST, M, N, false), (const uint16_t *)da.p, K, M, K, K, one(dw.p, N), N, e16,
+		                 nullptr));
+	}
 	HIPCHK(hipDeviceSynchronize());
 	HIPCHK(hipMemcpy(c, dc.p, (size_t)M * N * 4, hipMemcpyDeviceToHost));
 	return YALM_OK;

@@ -198,6 +198,34 @@ struct E16GluB {
 	}
 };
 
+// Split K: the slice's f32 partial tile, part[m][B row index] of its slot (gemm8p_kernel adds slot
+// x kstride). B row index = output column, or, over BRowsGlu<64> rows, twice the hidden column
+// (mul 2): 32 W1 rows, then the same 32 W3 rows, as skinny_reduce_kernel<.., GLU> reads them.
+template <bool BFOP = false>
+struct E16Part {
+	static constexpr bool NEEDS_LDS = false;
+	static constexpr bool PARTIAL = true;
+	static constexpr bool BF16 = BFOP;
+	float *red = nullptr;
+	float *part;
+	size_t kstride;
+	int ld, M, mul = 1;
+	template <int FI, int FJ>
+	__device__ __forceinline__ void apply(f32x4_t (&acc)[FI][FJ], int m0, int n0, int lane, int, int) const {
+#pragma unroll
+		for (int i = 0; i < FI; ++i)
+#pragma unroll
+			for (int r = 0; r < 4; ++r) {
+				const int m = m0 + 16 * i + crow16(r, lane);
+				if (m >= M)
+					continue;
+#pragma unroll
+				for (int j = 0; j < FJ; ++j)
+					part[(size_t)m * ld + n0 * mul + 16 * j + (lane & 15)] = acc[i][j][r];
+			}
+	}
+};
+
 struct E16Residual { // X[m][n] += scale C  (fused_matmul_add_residuals, per row)
 	static constexpr bool NEEDS_LDS = false;
 	float *red = nullptr;
@@ -594,10 +622,23 @@ constexpr int P8_HT = 128 * G_BK; // f16 per A half-tile (128 rows)
 // (twice the work) come first in dispatch order, each class keeping its own XCD-aware
 // order: with one workgroup per tile the hardware then hands the K tiles to the CUs the
 // K2 tiles leave free (longest first).
+//
+// Split K (nkc < the depth in K tiles; an EPI with PARTIAL, E16Part): a tile's K range is cut into
+// slices of nkc K tiles (the last one shorter), one item per (slice, tile), each leaving its f32
+// partial tile in its own slot; skinny_reduce_kernel / reduce_norm_rows_kernel sum the slots in
+// slice order. What it is for: a prompt of a few hundred rows has 2-4 row tiles, so Wo and W2 (N =
+// dim) are 32-64 tiles of 256 x 256 on 256 CUs whatever their depth (Mistral-7B, 391 rows: Wo + W2
+// 261 us a layer, 1/8 of the chip). A deep tile (K2) has as many more slices as it is deeper, all
+// of the same length. Order: slice slowest, so the tiles of one XCD share the same K columns of A.
+template <class EPI, class = void>
+struct epi_partial : std::false_type {};
+template <class EPI>
+struct epi_partial<EPI, std::void_t<decltype(EPI::PARTIAL)>> : std::bool_constant<EPI::PARTIAL> {};
+
 template <class EPI, class BMAP, int FJ0 = 2, int FJ1 = 2>
 __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__restrict__ A, int lda, int M, int K,
                                                              int kb, BMAP bm, int N, EPI epi, int c0, int c_split,
-                                                             int K2) {
+                                                             int K2, int nkc) {
 	constexpr int FI = 8, FJ = FJ0 + FJ1, TM = 128, TN = 16 * FJ, BN = 4 * TN;
 	constexpr int HB0 = 64 * FJ0 * G_BK, HB1 = 64 * FJ1 * G_BK; // f16 per B half-tile
 	constexpr int OFF[4] = {0, P8_HT, 2 * P8_HT, 2 * P8_HT + HB0}; // Am0, Am1, Bn0, Bn1 in a buffer
@@ -610,9 +651,11 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
 	const int wr = wave >> 2, wc = wave & 3;
 
 	const int tiles_m = (M + G_BM - 1) / G_BM, tiles_n = N / BN;
-	const int nwg = tiles_m * tiles_n;
-	const int tn_split = c_split / BN;             // column tiles with depth K
-	const int nwg2 = tiles_m * (tiles_n - tn_split); // tiles with depth K2, dispatched first
+	const int tn_split = c_split / BN; // column tiles with depth K
+	const int ks1 = epi_partial<EPI>::value ? (K / G_BK + nkc - 1) / nkc : 1;
+	const int ks2 = epi_partial<EPI>::value ? (K2 / G_BK + nkc - 1) / nkc : 1;
+	const int nwg2 = tiles_m * (tiles_n - tn_split) * ks2; // items with depth K2, dispatched first
+	const int nwg = tiles_m * tn_split * ks1 + nwg2;
 	// one tile per workgroup, or (grid smaller than the tile count) a persistent loop over
 	// tiles b, b + grid, ...: the next tile's LDS-DMA prologue follows this tile's epilogue
 	// stores without a workgroup exit and dispatch in between
@@ -626,8 +669,15 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
 			const int q = n / 8, rr = n % 8, xcd = wg % 8, idx = wg / 8;
 			wg = (xcd < rr ? xcd * (q + 1) : rr * (q + 1) + (xcd - rr) * q) + idx;
 		}
+		int ks = 0; // the K slice
+		if constexpr (epi_partial<EPI>::value) {
+			const int per = tiles_m * (deep ? tiles_n - tn_split : tn_split);
+			ks = wg / per;
+			wg -= ks * per;
+		}
 		const int tm = wg % tiles_m, tn = wg / tiles_m + (deep ? tn_split : 0);
 		const int Kt = deep ? K2 : K;
+		const int kt0 = ks * nkc; // first K tile of the slice
 		const int row0 = tm * G_BM;
 		const int colB = c0 + tn * (BN / BMAP::COLS_PER_TILE_DIV); // c0: first column of this launch
 
@@ -658,7 +708,7 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
 		}
 		// half-tile h (0 Am0, 1 Am1, 2 Bn0, 3 Bn1) of K tile kt into buffer buf
 		auto stage = [&](int buf, int h, int kt) {
-			const int k0 = kt * G_BK;
+			const int k0 = (epi_partial<EPI>::value ? kt0 + kt : kt) * G_BK;
 			const int kw = k0 < kb ? k0 : k0 - kb; // B wrap
 			uint16_t *base = smem + buf * BUFE + OFF[h];
 			if (h < 2) {
@@ -687,7 +737,7 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
 				acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 		half8_t a[4][2], b0[FJ0][2], b1[FJ1][2];
 
-		const int nk = Kt / G_BK;
+		const int nk = epi_partial<EPI>::value ? min(Kt / G_BK - kt0, nkc) : Kt / G_BK;
 		// prologue = the previous iteration's stages p3 .. p8 for K tiles 0 (E) and 1 (O)
 		const int k1 = nk > 1 ? 1 : 0;
 		stage(0, 0, 0);
@@ -810,6 +860,8 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
 		EPI e = epi;
 		if constexpr (EPI::NEEDS_LDS)
 			e.red = (float *)smem;
+		if constexpr (epi_partial<EPI>::value)
+			e.part += (size_t)ks * e.kstride;
 		const int n0 = BMAP::COLS_PER_TILE_DIV == 1 ? colB + wc * TN : colB + wc * (TN / 2);
 		e.template apply<FI, FJ>(acc, row0 + wr * TM, n0, lane, wc, 4);
 	}
