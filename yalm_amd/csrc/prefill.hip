@@ -147,7 +147,7 @@ int pick_bn(const PfForms &f, int kind, int M, int n_eff, bool glu, bool ragged 
 // A GEMM of few rows on the large tiles: tile width bn, K in slices of nkc K tiles (ks of them; ks2 of
 // the deeper columns). ks = 1: not split.
 struct SplitPlan {
-	int bn = 0, nkc = 1 << 24, ks = 1, ks2 = 1;
+	int bn = 0, nkc = 1 << 24, ks = 1, ks2 = 1, n = 0;
 };
 int slices(int K, int nkc) { return (K / pf::BK + nkc - 1) / nkc; }
 
@@ -159,7 +159,9 @@ int slices(int K, int nkc) { return (K / pf::BK + nkc - 1) / nkc; }
 // (Nd of depth Kd) count by their own slices. Split only where that model gains a tenth: the partials are
 // extra bytes. Mistral-7B, 391 rows, QKV + Wo + W2 of a layer: 425 us whole, 129 us + 28 us of sums in slices.
 constexpr float T8P_KT[3] = {1.05f, 1.3f, 1.55f}, T8P_TILE = 5.0f; // widths 128, 192, 256
-SplitPlan plan_split(const PfForms &f, int kind, int M, int N, int K, int Nd, int Kd, bool glu, size_t cap) {
+// ragged: the last tile may reach past N (n: the columns as whole tiles).
+SplitPlan plan_split(const PfForms &f, int kind, int M, int Nt, int K, int Nd, int Kd, bool glu, size_t cap,
+                     bool ragged = false) {
 	SplitPlan best;
 	if (!f.ksplit || !f.p8 || f.g16[kind] > 0)
 		return best;
@@ -167,7 +169,7 @@ SplitPlan plan_split(const PfForms &f, int kind, int M, int N, int K, int Nd, in
 	const int nk = K / pf::BK, nkd = Nd ? Kd / pf::BK : 0;
 	float whole = 0.0f, least = 0.0f;
 	for (int w = 0; w < 3; ++w) {
-		const int bn = 128 + 64 * w;
+		const int bn = 128 + 64 * w, N = ragged ? (Nt + bn - 1) / bn * bn : Nt;
 		if (N % bn || Nd % bn || (glu && bn != 256))
 			continue;
 		for (int ks = 1; ks <= 16; ++ks) {
@@ -189,7 +191,7 @@ SplitPlan plan_split(const PfForms &f, int kind, int M, int N, int K, int Nd, in
 			t += 3.0f + (float)((long)k1 * N + (long)k2 * Nd) * M * 8.0f / 5e6f;
 			if (least == 0.0f || t < least) {
 				least = t;
-				best = {bn, nkc, k1, k2};
+				best = {bn, nkc, k1, k2, N};
 			}
 		}
 	}
@@ -913,13 +915,34 @@ extern "C" int yalm_prefill_time(yalm_decoder d, int n, int iters, float *avg_ms
 	return YALM_OK;
 }
 
-// The layer-list engine's door to the large-tile GEMM (seq.hip; device pointers, asynchronous
-// on st): C [M][ldc] f32 = act(A [M][lda] bf16 . W [N][K]^T bf16 (+ bias[n])), act: E16StoreF32B. Same tiles, phases
-// and tile-width choice as the f16 prefill GEMMs (an N that is no multiple of 128 takes a last tile that
-// reaches past it); YALM_ERR_UNSUPPORTED (nothing launched) when the shape does not fit them: K % 64,
-// N below one tile, rows not 16-byte aligned.
+// bf16 partials of a few rows (T <= SK_MAX_T): the weight rows streamed once (skinny_gemm_lds_kernel)
+template <class BMAP>
+static int launch_skinny_bf16(const uint16_t *A, int lda, int T, int K, const BMAP &bm, int N, int KS, float *part,
+                              hipStream_t st) {
+	const int mt = (T + 15) / 16, KC = K / KS;
+	auto kern = mt == 1 ? pf::skinny_gemm_lds_kernel<1, BMAP, true> : mt == 2 ? pf::skinny_gemm_lds_kernel<2, BMAP, true>
+	            : mt == 3 ? pf::skinny_gemm_lds_kernel<3, BMAP, true> : pf::skinny_gemm_lds_kernel<4, BMAP, true>;
+	static bool attr[4] = {};
+	if (!attr[mt - 1]) {
+		HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+		                           32768 + (int)pf::SKL_RING_BYTES));
+		attr[mt - 1] = true;
+	}
+	hipLaunchKernelGGL(kern, dim3((N / pf::SK_ROWS) * KS), dim3(256), (size_t)16 * mt * KC * 2 + pf::SKL_RING_BYTES, st, A,
+	                   lda, T, K, K, bm, N, KC, 0, N, part);
+	HIPCHK(hipGetLastError());
+	return YALM_OK;
+}
+
+// The layer-list engine's door to the prefill GEMMs (seq.hip; device pointers, asynchronous
+// on st): C [M][ldc] f32 = act(A [M][lda] bf16 . W [N][K]^T bf16 (+ bias[n])), act: E16StoreF32B. The same
+// forms as the f16 prefill's: up to 64 rows the streamed split-K kernel (a 16-row product of [2048][2048] on the
+// general kernel's 64 x 64 tiles is 32 workgroups, 60-100 us; so 8 + 4 us), else the large tiles, in K slices
+// where plan_split says so (part: part_floats of scratch for the partials), else whole (an N that is no multiple
+// of the tile takes a last tile that reaches past it). YALM_ERR_UNSUPPORTED (nothing launched) when the shape
+// does not fit them: K % 64, N below one tile, rows not 16-byte aligned.
 int pf_gemm_bf16(const uint16_t *A, int lda, int M, int K, const uint16_t *W, int N, float *C, int ldc,
-                 const float *bias, int act, hipStream_t st) {
+                 const float *bias, int act, float *part, size_t part_floats, hipStream_t st) {
 	static const PfForms f = pf_forms_default();
 	if (M <= 0 || K % pf::BK != 0 || lda % 8 != 0 || ((size_t)A | (size_t)W) % 16 != 0)
 		return YALM_ERR_UNSUPPORTED;
@@ -934,13 +957,26 @@ int pf_gemm_bf16(const uint16_t *A, int lda, int M, int K, const uint16_t *W, in
 	e.M = M;
 	e.N = N;
 	e.act = act;
+	if (M <= SK_MAX_T) {
+		const int TP = 16 * ((M + 15) / 16), np = (N + pf::SK_ROWS - 1) / pf::SK_ROWS * pf::SK_ROWS;
+		const int ks = sk_pick_ks({{np, K, 1}}, TP);
+		if (ks > 0 && (size_t)ks * TP * np <= part_floats) {
+			TRY(launch_skinny_bf16(A, lda, M, K, pf::BRowsRagged{W, N}, np, ks, part, st));
+			return launch_skinny_reduce<false>(part, ks, ks, np, M, np, e, st);
+		}
+	}
+	const SplitPlan s = plan_split(f, PG_TEST, M, N, K, 0, 0, false, part_floats, ragged);
+	if (s.ks > 1) {
+		TRY((launch_split<pf::BRowsRagged, true>(f, s, A, lda, M, K, K, pf::BRowsRagged{W, N}, s.n, 0, 0, part, st)));
+		return launch_skinny_reduce<false>(part, s.ks, s.ks, s.n, M, s.n, e, st);
+	}
 	return launch_rows(f, bn, A, lda, M, K, K, pf::BRowsRagged{W, N}, (N + bn - 1) / bn * bn, e, st);
 }
 
 // The same door for a gated pair: C [M][ldc] f32 = act(A Wg^T) (.) (A Wu^T) over `hidden` units
 // (mode / limit: E16GluB), the two matrices' rows interleaved per wave as in the f16 prefill.
 int pf_gemm_glu_bf16(const uint16_t *A, int lda, int M, int K, const uint16_t *Wg, const uint16_t *Wu, int hidden,
-                     float *C, int ldc, int mode, float limit, hipStream_t st) {
+                     float *C, int ldc, int mode, float limit, float *part, size_t part_floats, hipStream_t st) {
 	static const PfForms f = pf_forms_default();
 	if (M <= 0 || K % pf::BK != 0 || lda % 8 != 0 || ((size_t)A | (size_t)Wg | (size_t)Wu) % 16 != 0)
 		return YALM_ERR_UNSUPPORTED;
@@ -952,6 +988,21 @@ int pf_gemm_glu_bf16(const uint16_t *A, int lda, int M, int K, const uint16_t *W
 	e.mode = mode;
 	e.limit = limit;
 	pf::BRowsGlu<64> bm{Wg, Wu};
+	const int N = 2 * hidden;
+	if (!bn)
+		return YALM_ERR_UNSUPPORTED;
+	if (M <= SK_MAX_T) {
+		const int TP = 16 * ((M + 15) / 16), ks = sk_pick_ks({{N, K, 1}}, TP);
+		if (ks > 0 && (size_t)ks * TP * N <= part_floats) {
+			TRY(launch_skinny_bf16(A, lda, M, K, bm, N, ks, part, st));
+			return launch_skinny_reduce<true>(part, ks, ks, N, M, N, e, st);
+		}
+	}
+	const SplitPlan s = plan_split(f, PG_GLU, M, N, K, 0, 0, true, part_floats);
+	if (s.ks > 1) {
+		TRY((launch_split<pf::BRowsGlu<64>, true>(f, s, A, lda, M, K, K, bm, N, 0, 0, part, st)));
+		return launch_skinny_reduce<true>(part, s.ks, s.ks, N, M, N, e, st);
+	}
 	if (bn == 256)
 		return launch_g16_t<pf::E16GluB, pf::BRowsGlu<64>, 256, 2>(f, A, lda, M, K, K, bm, 2 * hidden, e, st);
 	if (bn == 128)

@@ -135,7 +135,7 @@ constexpr int SKL_NS = 3;                      // ring stages
 constexpr int SKL_STAGE = SK_ROWS * SKL_KS;    // f16 per stage (16 KB)
 constexpr size_t SKL_RING_BYTES = (size_t)SKL_NS * SKL_STAGE * 2;
 
-template <int MT, class BMAP>
+template <int MT, class BMAP, bool BF = false> // BF: bf16 operands (the layer-list engine's products)
 __global__ __launch_bounds__(256) void skinny_gemm_lds_kernel(const uint16_t *__restrict__ A, int lda, int T, int K,
                                                               int kb, BMAP bm, int N, int KC, int c0, int Np,
                                                               float *__restrict__ part) {
@@ -189,7 +189,7 @@ __global__ __launch_bounds__(256) void skinny_gemm_lds_kernel(const uint16_t *__
 #pragma unroll
 			for (int m = 0; m < MT; ++m) {
 				const half8_t a = sk_afrag<MT>(as, KC, 16 * m + n, st * SKL_KS + 32 * j + 8 * q);
-				acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, acc[m], 0, 0, 0);
+				acc[m] = mfma16<BF>(a, b, acc[m]);
 			}
 		}
 	}

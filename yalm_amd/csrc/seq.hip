@@ -26,10 +26,11 @@
 // library built from the shim and this unit alone has no prefill unit, and every product then
 // runs on this unit's general-shape kernels.
 int pf_gemm_bf16(const uint16_t *A, int lda, int M, int K, const uint16_t *W, int N, float *C, int ldc,
-                 const float *bias, int act, hipStream_t st) __attribute__((weak));
+                 const float *bias, int act, float *part, size_t part_floats, hipStream_t st) __attribute__((weak));
 
 int pf_gemm_glu_bf16(const uint16_t *A, int lda, int M, int K, const uint16_t *Wg, const uint16_t *Wu, int hidden,
-                     float *C, int ldc, int mode, float limit, hipStream_t st) __attribute__((weak));
+                     float *C, int ldc, int mode, float limit, float *part, size_t part_floats, hipStream_t st)
+    __attribute__((weak));
 
 struct yalm_seq_s {
 	yalm_seq_config c{};
@@ -66,6 +67,8 @@ struct yalm_seq_s {
 	int ldz = 0;
 	float *inv_freq = nullptr;
 	uint16_t *a16 = nullptr;     // [cap][bw] bf16 copy of a product's activations (large-tile GEMM operand)
+	float *gpart = nullptr;      // f32 partials of those products' K slices (at most 128 MB)
+	size_t gpart_floats = 0;
 	int *tok = nullptr, *want = nullptr;
 	float *logits = nullptr;     // [LOGIT_ROWS][vocab]
 	int *idx = nullptr, *counts = nullptr, *lists = nullptr;
@@ -533,8 +536,14 @@ static int create_seq(const yalm_seq_config *config, const yalm_seq_weights *w, 
 	STRY(sallocT(q, &q->Z, cap * zw));
 	for (int i = 0; i < 4; ++i)
 		STRY(sallocT(q, &q->B[i], cap * bw));
-	if (bf && pf_gemm_bf16)
+	if (bf && pf_gemm_bf16) {
 		STRY(sallocT(q, &q->a16, cap * bw));
+		size_t widest = std::max({bw, (size_t)zw, (size_t)c.width});
+		for (const yalm_seq_layer &l : q->L)
+			widest = std::max({widest, (size_t)2 * l.ff, (size_t)2 * l.shared_ff});
+		q->gpart_floats = std::min((size_t)32 << 20, 16 * (cap + 15) / 16 * 16 * (widest + 256));
+		STRY(sallocT(q, &q->gpart, q->gpart_floats));
+	}
 	STRY(sallocT(q, &q->tok, cap + 1));
 	q->tok += 1; // [-1]: the token before the portion's first
 	STRY(sallocT(q, &q->prev, 1));
@@ -733,11 +742,12 @@ static int gemm(Seq *q, const GemmArgs &a, int batches = 1, int max_m = -1, bool
 		max_m = a.M;
 	if (f32w || q->c.weight_dtype == YALM_F32)
 		return gemm_t<WF32>(q, a, batches, max_m);
-	// plain products of long portions whose shape fits the large-tile GEMM of the prefill unit
+	// plain products of portions whose shape fits the GEMMs of the prefill unit (max_m <= GEMV_MAX_M: the
+	// activations stay f32)
 	const bool pair = a.W2 != nullptr && (a.epi == EPI_GLU_GELU || a.epi == EPI_GLU_CLAMP || a.epi == EPI_GLU_SILU) && !a.bias;
 	const bool single = !a.W2 && (a.epi == EPI_NONE || a.epi == EPI_GELU || a.epi == EPI_RELU2 || a.epi == EPI_GELU_ERF);
 	const int act1 = a.epi == EPI_GELU ? 1 : (a.epi == EPI_RELU2 ? 2 : (a.epi == EPI_GELU_ERF ? 3 : 0)); // the large-tile door's activation
-	if (q->a16 && batches == 1 && max_m >= 2 * GB_BM && !a.rows && !a.row_scale && !a.gate && !a.w_sel && a.z_split == 0 && a.ldw == a.K &&
+	if (q->a16 && batches == 1 && max_m > GEMV_MAX_M && !a.rows && !a.row_scale && !a.gate && !a.w_sel && a.z_split == 0 && a.ldw == a.K &&
 	    a.K % 64 == 0 && (pair ? a.N % 64 == 0 : (single && a.N >= 128))) {
 		const size_t n8 = (size_t)a.M * (a.K / 8);
 		seq_to_bf16_kernel<<<(unsigned)std::min<size_t>((n8 + SEQ_THREADS - 1) / SEQ_THREADS, 4096), SEQ_THREADS, 0,
@@ -745,8 +755,10 @@ static int gemm(Seq *q, const GemmArgs &a, int batches = 1, int max_m = -1, bool
 		HIPCHK(hipGetLastError());
 		const int rc =
 		    pair ? pf_gemm_glu_bf16(q->a16, a.K, a.M, a.K, (const uint16_t *)a.W, (const uint16_t *)a.W2, a.N, a.C, a.ldc,
-		                            a.epi == EPI_GLU_GELU ? 1 : (a.epi == EPI_GLU_CLAMP ? 2 : 3), a.limit, q->stream)
-		         : pf_gemm_bf16(q->a16, a.K, a.M, a.K, (const uint16_t *)a.W, a.N, a.C, a.ldc, a.bias, act1, q->stream);
+		                            a.epi == EPI_GLU_GELU ? 1 : (a.epi == EPI_GLU_CLAMP ? 2 : 3), a.limit, q->gpart,
+		                            q->gpart_floats, q->stream)
+		         : pf_gemm_bf16(q->a16, a.K, a.M, a.K, (const uint16_t *)a.W, a.N, a.C, a.ldc, a.bias, act1, q->gpart,
+		                        q->gpart_floats, q->stream);
 		if (rc != YALM_ERR_UNSUPPORTED)
 			return rc;
 	}
