@@ -158,7 +158,8 @@ int slices(int K, int nkc) { return (K / pf::BK + nkc - 1) / nkc; }
 // 10 us of a 391-row reduce + norm). The whole is the rounds that the busiest CU walks; the deeper columns
 // (Nd of depth Kd) count by their own slices. Split only where that model gains a tenth: the partials are
 // extra bytes. Mistral-7B, 391 rows, QKV + Wo + W2 of a layer: 425 us whole, 129 us + 28 us of sums in slices.
-constexpr float T8P_KT[3] = {1.05f, 1.3f, 1.55f}, T8P_TILE = 5.0f; // widths 128, 192, 256
+// (a whole tile's epilogue, with its bias, activation or rotation, costs more than a slice's plain stores)
+constexpr float T8P_KT[3] = {1.05f, 1.3f, 1.55f}, T8P_TILE = 5.0f, T8P_EPI = 4.0f; // widths 128, 192, 256
 // ragged: the last tile may reach past N (n: the columns as whole tiles).
 SplitPlan plan_split(const PfForms &f, int kind, int M, int Nt, int K, int Nd, int Kd, bool glu, size_t cap,
                      bool ragged = false) {
@@ -174,16 +175,16 @@ SplitPlan plan_split(const PfForms &f, int kind, int M, int Nt, int K, int Nd, i
 			continue;
 		for (int ks = 1; ks <= 16; ++ks) {
 			const int nkc = (nk + ks - 1) / ks;
-			if (ks > 1 && (nkc < 8 || nkc == (nk + ks - 2) / (ks - 1)))
+			if (ks > 1 && (nkc < 4 || nkc == (nk + ks - 2) / (ks - 1)))
 				continue;
 			const int k1 = (nk + nkc - 1) / nkc, k2 = Nd ? (nkd + nkc - 1) / nkc : 1;
 			if (ks > 1 && (size_t)std::max(k1, k2) * TP * (N + Nd) > cap)
 				break;
 			// (not split, two depths: the deep tiles alone, or the mean over the CUs)
 			const long items = tm * (N / bn * k1 + Nd / bn * k2);
-			float t = (float)((items + ncu - 1) / ncu) * (nkc * T8P_KT[w] + T8P_TILE);
+			float t = (float)((items + ncu - 1) / ncu) * (nkc * T8P_KT[w] + T8P_TILE + (ks == 1 ? T8P_EPI : 0.0f));
 			if (ks == 1 && Nd)
-				t = std::max((float)nkd, (float)(tm * (N / bn * nk + Nd / bn * nkd)) / ncu) * T8P_KT[w] + T8P_TILE;
+				t = std::max((float)nkd, (float)(tm * (N / bn * nk + Nd / bn * nkd)) / ncu) * T8P_KT[w] + T8P_TILE + T8P_EPI;
 			if (ks == 1) {
 				whole = whole == 0.0f ? t : std::min(whole, t);
 				continue;
