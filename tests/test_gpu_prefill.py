@@ -325,6 +325,36 @@ def test_fp8_prefill_equals_f16_twin(cfg_name, n):
             R.lib.yalm_free(p)
 
 
+@pytest.mark.parametrize("dims", [(1536, 4096, 12, 4), (768, 1536, 6, 2), (640, 1152, 5, 5)])
+@pytest.mark.parametrize("n,split", [(4, False), (33, False), (64, True), (65, False), (300, True), (300, False), (700, False)])
+def test_fp8_prefill_reads_bytes_as_f16_twin(dims, n, split):
+    """The E5M2 bytes read as they are by each GEMM (streamed short prompts; tiles of 128, 192 and 256 columns, whole
+    and in K slices; the gated pair; the two-depth QKV; the classifier) against the f16 twin's kernels: bit for bit,
+    log p and the next step's logits (which read the caches), in both precision forms."""
+    dim, hidden, nh, nkv = dims
+    cfg8 = M.ModelConfig(dim=dim, hidden_dim=hidden, head_dim=128, n_layers=2, n_heads=nh, n_kv_heads=nkv,
+                         vocab_size=1920, max_seq_len=704, rope_theta=1e6, act=M.SILU, weight_dtype=M.F8E5M2)
+    t8 = M.synth_host_tensors(cfg8, seed=5)
+    cfg16, t16 = _f16_twin(cfg8, t8)
+    R = rt()
+    dm8, dm16 = R.DeviceModel.from_arrays(cfg8, t8), R.DeviceModel.from_arrays(cfg16, t16)
+    d8, d16, base = R.Decoder(dm8), R.Decoder(dm16), R.Decoder(dm8)
+    try:
+        tok = np.random.default_rng(n).integers(0, cfg8.vocab_size, size=n).astype(np.int32)
+        for d in (d8, d16, base):
+            d.set_prefill_forms("ksplit:0,8p:0" if d is base else "")  # base: the f16 copies, whole 2-phase tiles
+            d.set_prefill_precision(R.PREFILL_SPLIT if split else R.PREFILL_FAST)
+        lp8, lp16, lpb = d8.prefill(tok), d16.prefill(tok), base.prefill(tok)
+        np.testing.assert_array_equal(lp8, lp16)
+        assert np.max(np.abs(lp8 - lpb)) < (2e-4 if split else LP_ATOL / 2)  # another order of the same sums
+        # the next step in the f16 engine over either cache (the two engines' own steps differ in their order of sums)
+        nxt = [d.forward(7, n) for d in (d8, d16)]
+        np.testing.assert_allclose(nxt[0], nxt[1], rtol=0, atol=1e-4 * np.max(np.abs(nxt[1])))
+    finally:
+        for h in (d8, d16, base, dm8, dm16):
+            h.close()
+
+
 def test_prefill_range_guard_scales_glu_output():
     """a GLU product above 65504 (the f16 range; the reference keeps it in
     f32, infer.cpp:360-375) must not become inf. models.REALISTIC's spike layer gives one at

@@ -118,9 +118,10 @@ int pf_alloc(yalm_decoder_s *d, void **p, size_t bytes) {
 // BN for a GEMM of M x N (n_eff = B rows: 2 x hidden for the GLU); 0 = none fits. A
 // forced width that does not divide N falls back to the automatic choice. ragged: no width needs to
 // divide N (BRowsRagged), the last tile counts whole.
-int pick_bn(const PfForms &f, int kind, int M, int n_eff, bool glu, bool ragged = false) {
+// e5m2: the widths of the 8-phase kernel alone (it reads the bytes as they are).
+int pick_bn(const PfForms &f, int kind, int M, int n_eff, bool glu, bool ragged = false, bool e5m2 = false) {
 	static const int cands[4] = {128, 192, 256, 320};
-	auto fits = [&](int bn) { return (n_eff % bn == 0 || (ragged && bn <= 256)) && (!glu || bn == 128 || bn == 256); };
+	auto fits = [&](int bn) { return (!e5m2 || (bn <= 256 && (!glu || bn == 256))) && (n_eff % bn == 0 || (ragged && bn <= 256)) && (!glu || bn == 128 || bn == 256); };
 	const int form = f.g16[kind];
 	if (form > 0 && fits(form) && (form == 128 || form == 192 || form == 256 || form == 320))
 		return form;
@@ -230,7 +231,7 @@ template <class EPI, class BMAP, int FJ0, int FJ1>
 int launch_g8p(const PfForms &f, const uint16_t *A, int lda, int M, int K, int kb, const BMAP &bm, int N,
                const EPI &epi, hipStream_t st, int c0, int c_split, int K2, int nkc) {
 	auto kern = pf::gemm8p_kernel<EPI, BMAP, FJ0, FJ1>;
-	constexpr size_t lds = pf::gemm8p_lds<FJ0, FJ1>();
+	constexpr size_t lds = pf::gemm8p_lds<FJ0, FJ1, sizeof(pf::bmap_elt<BMAP>)>();
 	constexpr int BN = 64 * (FJ0 + FJ1);
 	static bool attr = false;
 	if (!attr) {
@@ -264,17 +265,22 @@ int launch_g16_t(const PfForms &f, const uint16_t *A, int lda, int M, int K, int
 		if constexpr (BN == 128 && BMAP::COLS_PER_TILE_DIV == 1) // GLU rows pair per 64-col wave
 			return launch_g8p<EPI, BMAP, 1, 1>(f, A, lda, M, K, kb, bm, N, epi, st, c0);
 	}
-	auto kern = pf::gemm16_kernel<EPI, BMAP, BN, WM>;
-	constexpr size_t lds = pf::gemm16_lds<BN>();
-	static bool attr = false;
-	if (!attr) {
-		HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-		attr = true;
+	if constexpr (sizeof(pf::bmap_elt<BMAP>) == 1) {
+		set_err("prefill GEMM: E5M2 weights run on the 8-phase kernel (widths 128, 192, 256)");
+		return YALM_ERR_UNSUPPORTED;
+	} else {
+		auto kern = pf::gemm16_kernel<EPI, BMAP, BN, WM>;
+		constexpr size_t lds = pf::gemm16_lds<BN>();
+		static bool attr = false;
+		if (!attr) {
+			HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+			attr = true;
+		}
+		const int nwg = ((M + pf::G_BM - 1) / pf::G_BM) * (N / BN);
+		hipLaunchKernelGGL(kern, dim3(nwg), dim3(pf::G_THREADS), lds, st, A, lda, M, K, kb, bm, N, epi, c0);
+		HIPCHK(hipGetLastError());
+		return YALM_OK;
 	}
-	const int nwg = ((M + pf::G_BM - 1) / pf::G_BM) * (N / BN);
-	hipLaunchKernelGGL(kern, dim3(nwg), dim3(pf::G_THREADS), lds, st, A, lda, M, K, kb, bm, N, epi, c0);
-	HIPCHK(hipGetLastError());
-	return YALM_OK;
 }
 
 // C = A · W^T through the large-tile kernel at width bn (pick_bn; 0: no width fits)
@@ -295,10 +301,36 @@ int launch_rows(const PfForms &f, int bn, const uint16_t *A, int lda, int M, int
 	return YALM_ERR_UNSUPPORTED;
 }
 
+// Weight rows from up to 3 matrices laid end to end: f16, or E5M2 bytes read as they are (e5m2)
+struct WSrc {
+	const void *p[3];
+	int end[3];
+	bool e5m2;
+};
+template <class F>
+int with_rows(const WSrc &b, F launch) {
+	if (b.e5m2) {
+		pf::BRowsPlain8 r;
+		for (int i = 0; i < 3; ++i)
+			r.p[i] = (const uint8_t *)b.p[i], r.end[i] = b.end[i];
+		return launch(r);
+	}
+	pf::BRowsPlain r;
+	for (int i = 0; i < 3; ++i)
+		r.src.p[i] = (const uint16_t *)b.p[i], r.src.end[i] = b.end[i];
+	return launch(r);
+}
+// ... and a gated pair's two matrices
+template <class F>
+int with_glu(const void *w1, const void *w3, bool e5m2, F launch) {
+	if (e5m2)
+		return launch(pf::BRowsGlu<64, uint8_t>{(const uint8_t *)w1, (const uint8_t *)w3});
+	return launch(pf::BRowsGlu<64>{(const uint16_t *)w1, (const uint16_t *)w3});
+}
 template <class EPI>
-int launch_plain(const PfForms &f, int bn, const uint16_t *A, int lda, int M, int K, int kb, const pf::BSrc &b,
+int launch_plain(const PfForms &f, int bn, const uint16_t *A, int lda, int M, int K, int kb, const WSrc &b,
                  int N, const EPI &epi, hipStream_t st, int c0 = 0) {
-	return launch_rows(f, bn, A, lda, M, K, kb, pf::BRowsPlain{b}, N, epi, st, c0);
+	return with_rows(b, [&](const auto &bm) { return launch_rows(f, bn, A, lda, M, K, kb, bm, N, epi, st, c0); });
 }
 
 // ---- short prompts (T <= SK_MAX_T): split-K skinny GEMMs (prefill_skinny.h)
@@ -337,7 +369,10 @@ int sk_pick_ks(std::initializer_list<SkGemm> kn, int TP) {
 template <int MT, class BMAP>
 int launch_skinny_mt(const PfForms &f, const uint16_t *A, int lda, int T, int K, int kb, const BMAP &bm, int N,
                      int KS, int c0, int Np, float *part, hipStream_t st) {
-	auto kern = f.skl ? pf::skinny_gemm_lds_kernel<MT, BMAP> : pf::skinny_gemm_kernel<MT, BMAP>;
+	auto kern = pf::skinny_gemm_lds_kernel<MT, BMAP>;
+	if constexpr (sizeof(pf::bmap_elt<BMAP>) == 2)
+		if (!f.skl)
+			kern = pf::skinny_gemm_kernel<MT, BMAP>;
 	static bool attr[2] = {false, false};
 	if (!attr[f.skl]) {
 		HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -378,17 +413,20 @@ int launch_skinny_reduce(const float *part, int KS, int KS2, int c_split, int T,
 	return YALM_OK;
 }
 
-pf::BSrc one(const void *w, int rows) {
-	pf::BSrc b{};
-	b.p[0] = b.p[1] = b.p[2] = (const uint16_t *)w;
-	b.end[0] = b.end[1] = b.end[2] = rows;
-	return b;
-}
+WSrc one(const void *w, int rows, bool e5m2 = false) { return WSrc{{w, w, w}, {rows, rows, rows}, e5m2}; }
 
-// fp8 models: the tensors (E5M2 bytes, n elements each) dequantised to f16 into b.wdq, end
+// fp8 models in the forms that cannot read the bytes (yalm_set_prefill_forms' other tilings, a classifier of
+// width-320 tiles): the tensors (E5M2 bytes, n elements each) dequantised to f16 into b.wdq, end
 // to end; returns their f16 copies in `out` (prefill.h e5m2_to_f16_kernel)
 int dequant(yalm_decoder_s *d, std::initializer_list<std::pair<const void *, size_t>> t, const uint16_t **out,
 			hipStream_t st) {
+	if (!d->pf.wdq) { // one layer's weights, or the classifier's
+		const yalm_config &c = d->c;
+		const size_t q_dim = (size_t)c.n_heads * c.head_dim;
+		const size_t layer = (q_dim + 2 * (size_t)c.n_kv_heads * c.head_dim) * c.dim + (size_t)c.dim * q_dim +
+							 3 * (size_t)c.dim * c.hidden_dim;
+		TRY(pf_alloc(d, (void **)&d->pf.wdq, 2 * std::max(layer, (size_t)c.vocab_size * c.dim)));
+	}
 	pf::DqSegs s{};
 	size_t off = 0, pieces = 0;
 	for (auto &p : t) {
@@ -526,11 +564,6 @@ int ensure_bufs(yalm_decoder_s *d) {
 	TRY(pf_alloc(d, (void **)&b.lp, cap * 4));
 	TRY(pf_alloc(d, (void **)&b.rope, cap * c.head_dim * 4));
 	TRY(pf_alloc(d, (void **)&b.range, (size_t)(c.n_layers + 1) * RG_N * 4));
-	if (c.weight_dtype == YALM_F8E5M2) { // the f16 copy of one layer's weights, or of the classifier
-		const size_t layer = ((size_t)q_dim + 2 * (size_t)c.n_kv_heads * c.head_dim) * c.dim + (size_t)c.dim * q_dim +
-							 3 * (size_t)c.dim * c.hidden_dim;
-		TRY(pf_alloc(d, (void **)&b.wdq, 2 * std::max(layer, (size_t)c.vocab_size * c.dim)));
-	}
 	{ // split-K partials; short prompts: the largest [KS][64][Np] of the layer's GEMMs
 		const int kv_dim = c.n_kv_heads * c.head_dim, TP = SK_MAX_T;
 		const int np_qkv = (int)q_dim + 2 * kv_dim;
@@ -551,10 +584,10 @@ int ensure_bufs(yalm_decoder_s *d) {
 }
 
 template <int ACT, bool SPLIT>
-int enqueue_glu_t(yalm_decoder_s *d, const yalm_block_weights &w, int T, float hscale, unsigned *range) {
+int enqueue_glu_t(yalm_decoder_s *d, const yalm_block_weights &w, int T, float hscale, unsigned *range, bool e5m2) {
 	const yalm_config &c = d->c;
 	const PfForms &f = d->pf_forms;
-	const int bn = pick_bn(f, PG_GLU, T, 2 * c.hidden_dim, true);
+	const int bn = pick_bn(f, PG_GLU, T, 2 * c.hidden_dim, true, false, e5m2);
 	const int sp = SPLIT ? 2 : 1; // split-operand form: A = [hi | lo] (K = 2 dim), H rows [hi | lo]
 	pf::E16Glu<ACT, SPLIT> e;
 	e.h = d->pf.H;
@@ -563,26 +596,28 @@ int enqueue_glu_t(yalm_decoder_s *d, const yalm_block_weights &w, int T, float h
 	e.hscale = hscale;
 	e.range = range;
 	e.lo_off = SPLIT ? c.hidden_dim : 0;
-	pf::BRowsGlu<64> bm{(const uint16_t *)w.w1, (const uint16_t *)w.w3};
 	const SplitPlan s = plan_split(f, PG_GLU, T, 2 * c.hidden_dim, sp * c.dim, 0, 0, true, d->pf.skp_floats);
-	if (s.ks > 1) {
-		TRY(launch_split(f, s, d->pf.Xn, sp * c.dim, T, sp * c.dim, c.dim, bm, 2 * c.hidden_dim, 0, 0, d->pf.skp, d->stream));
-		return launch_skinny_reduce<true>(d->pf.skp, s.ks, s.ks, 2 * c.hidden_dim, T, 2 * c.hidden_dim, e, d->stream);
-	}
-	if (bn == 256)
-		return launch_g16_t<pf::E16Glu<ACT, SPLIT>, pf::BRowsGlu<64>, 256, 2>(f, d->pf.Xn, sp * c.dim, T, sp * c.dim, c.dim,
-                                                                     bm, 2 * c.hidden_dim, e, d->stream);
-	if (bn == 128)
-		return launch_g16_t<pf::E16Glu<ACT, SPLIT>, pf::BRowsGlu<64>, 128, 4>(f, d->pf.Xn, sp * c.dim, T, sp * c.dim, c.dim,
-                                                                     bm, 2 * c.hidden_dim, e, d->stream);
-	set_err("prefill GLU GEMM: 2 x hidden_dim must divide by 128 (or by a forced width of 128 / 256)");
-	return YALM_ERR_UNSUPPORTED;
+	return with_glu(w.w1, w.w3, e5m2, [&](const auto &bm) -> int {
+		using BM = std::decay_t<decltype(bm)>;
+		if (s.ks > 1) {
+			TRY(launch_split(f, s, d->pf.Xn, sp * c.dim, T, sp * c.dim, c.dim, bm, 2 * c.hidden_dim, 0, 0, d->pf.skp, d->stream));
+			return launch_skinny_reduce<true>(d->pf.skp, s.ks, s.ks, 2 * c.hidden_dim, T, 2 * c.hidden_dim, e, d->stream);
+		}
+		if (bn == 256)
+			return launch_g16_t<pf::E16Glu<ACT, SPLIT>, BM, 256, 2>(f, d->pf.Xn, sp * c.dim, T, sp * c.dim, c.dim, bm,
+			                                                        2 * c.hidden_dim, e, d->stream);
+		if (bn == 128)
+			return launch_g16_t<pf::E16Glu<ACT, SPLIT>, BM, 128, 4>(f, d->pf.Xn, sp * c.dim, T, sp * c.dim, c.dim, bm,
+			                                                        2 * c.hidden_dim, e, d->stream);
+		set_err("prefill GLU GEMM: 2 x hidden_dim must divide by 128 (or by a forced width of 128 / 256)");
+		return YALM_ERR_UNSUPPORTED;
+	});
 }
 
 template <int ACT>
-int enqueue_glu(yalm_decoder_s *d, const yalm_block_weights &w, int T, float hscale, unsigned *range) {
-	return d->pf_forms.split ? enqueue_glu_t<ACT, true>(d, w, T, hscale, range)
-	                         : enqueue_glu_t<ACT, false>(d, w, T, hscale, range);
+int enqueue_glu(yalm_decoder_s *d, const yalm_block_weights &w, int T, float hscale, unsigned *range, bool e5m2) {
+	return d->pf_forms.split ? enqueue_glu_t<ACT, true>(d, w, T, hscale, range, e5m2)
+	                         : enqueue_glu_t<ACT, false>(d, w, T, hscale, range, e5m2);
 }
 
 // The whole prefill on d->stream: T rows at positions pos0 .. pos0 + T - 1. hexp[l] (null:
@@ -603,15 +638,18 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 	const int half = c.head_dim / 2;
 	pf::rope_table_kernel<<<(T * half + 255) / 256, 256, 0, st>>>(d->inv_freq, half, T, pos0, b.rope);
 	HIPCHK(hipGetLastError());
+	// fp8: every GEMM reads the E5M2 bytes (gemm8p_kernel, skinny_gemm_lds_kernel) with the slices and K order of
+	// the f16 twin, so the results are its bit for bit; forms that name other kernels run on f16 copies
+	const bool raw8 = fp8 && f.p8 && f.skl && f.g16[PG_QKV] < 0 && f.g16[PG_WO] < 0 && f.g16[PG_GLU] < 0 && f.g16[PG_W2] < 0;
 	// GEMM widths are the same for every layer
-	const int bn_q = pick_bn(f, PG_QKV, T, q_dim, false);
-	const int bn_kv = pick_bn(f, PG_QKV, T, 2 * kv_dim, false);
+	const int bn_q = pick_bn(f, PG_QKV, T, q_dim, false, false, raw8);
+	const int bn_kv = pick_bn(f, PG_QKV, T, 2 * kv_dim, false, false, raw8);
 	// q and k | v in one two-depth launch at width 256 (gemm8p_kernel): the two launches'
 	// tiles balanced over the chip instead of one round each (Llama-3B at T 4096: q 82 us
 	// at width 192 + k | v 115 us at 128)
 	const bool qkv1 = f.qkv1 && f.p8 && f.g16[PG_QKV] < 0 && q_dim % 256 == 0 && (2 * kv_dim) % 256 == 0;
-	const int bn_wo = pick_bn(f, PG_WO, T, c.dim, false);
-	const int bn_w2 = pick_bn(f, PG_W2, T, c.dim, false);
+	const int bn_wo = pick_bn(f, PG_WO, T, c.dim, false, false, raw8);
+	const int bn_w2 = pick_bn(f, PG_W2, T, c.dim, false, false, raw8);
 	// short prompts: split-K skinny GEMMs (the 256-row tiles would leave most CUs idle)
 	const int TP = 16 * ((T + 15) / 16);
 	const int ks_qkv = sk_pick_ks({{q_dim, c.dim, 1}, {2 * kv_dim, 2 * c.dim, 2}}, TP);
@@ -625,7 +663,7 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 	// carries an f16 rounding the reference's f32 lacks; sp = operand width factor
 	const bool split = f.split;
 	const int sp = split ? 2 : 1;
-	const int bn_qkv_all = pick_bn(f, PG_QKV, T, q_dim + 2 * kv_dim, false);
+	const int bn_qkv_all = pick_bn(f, PG_QKV, T, q_dim + 2 * kv_dim, false, false, raw8);
 	// too few tiles for the chip: K slices. Wo's and W2's partials, and a short prompt's, are
 	// summed by the launch that also adds the residual and makes the next product's operand
 	const size_t pcap = b.skp_floats;
@@ -646,7 +684,7 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 	bool normed = false; // Xn holds this layer's attention input already
 	for (int l = 0; l < c.n_layers; ++l) {
 		yalm_block_weights w = d->b[l];
-		if (fp8) { // this layer's weights as f16 (exact), in the scratch the previous layer's GEMMs are done with
+		if (fp8 && !raw8) { // this layer's weights as f16 (exact), in the scratch the previous layer's GEMMs are done with
 			const uint16_t *p[7];
 			const size_t qd = (size_t)q_dim * c.dim, kd = (size_t)kv_dim * c.dim, hd = (size_t)c.hidden_dim * c.dim;
 			TRY(dequant(d, {{w.wq, qd}, {w.wk, kd}, {w.wv, kd}, {w.wo, qd}, {w.w1, hd}, {w.w2, hd}, {w.w3, hd}}, p, st));
@@ -659,13 +697,7 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 		if (!normed)
 			TRY(launch_rmsnorm(true, f, b.X, w.rms_att, c.dim, T, c.norm_eps, b.Xn, rg + RG_XATT, st));
 		{
-			pf::BSrc qkv{};
-			qkv.p[0] = (const uint16_t *)w.wq;
-			qkv.p[1] = (const uint16_t *)w.wk;
-			qkv.p[2] = (const uint16_t *)w.wv;
-			qkv.end[0] = q_dim;
-			qkv.end[1] = q_dim + kv_dim;
-			qkv.end[2] = q_dim + 2 * kv_dim;
+			const WSrc qkv{{w.wq, w.wk, w.wv}, {q_dim, q_dim + kv_dim, q_dim + 2 * kv_dim}, raw8};
 			pf::E16QKV e;
 			e.q = b.Q;
 			e.kc = w.key_cache;
@@ -681,11 +713,12 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 			// QKV + clip + RoPE as two GEMMs: q (K = dim over hi) and k | v from column
 			// q_dim (K = 2 dim over hi | lo, the B rows wrapping at dim)
 			if (small) {
-				const pf::BRowsPlain bm{qkv};
 				const int np = q_dim + 2 * kv_dim;
-				TRY(launch_skinny(f, b.Xn, 2 * c.dim, T, c.dim, c.dim, bm, q_dim, ks_qkv, 0, np, b.skp, st));
-				TRY(launch_skinny(f, b.Xn, 2 * c.dim, T, 2 * c.dim, c.dim, bm, 2 * kv_dim, 2 * ks_qkv, q_dim, np, b.skp,
-				                  st));
+				TRY(with_rows(qkv, [&](const auto &bm) -> int {
+					TRY(launch_skinny(f, b.Xn, 2 * c.dim, T, c.dim, c.dim, bm, q_dim, ks_qkv, 0, np, b.skp, st));
+					return launch_skinny(f, b.Xn, 2 * c.dim, T, 2 * c.dim, c.dim, bm, 2 * kv_dim, 2 * ks_qkv, q_dim, np, b.skp,
+					                     st);
+				}));
 				TRY(launch_skinny_reduce<false>(b.skp, ks_qkv, 2 * ks_qkv, q_dim, T, np, e, st));
 			} else {
 				const int np = q_dim + 2 * kv_dim;
@@ -695,19 +728,23 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 					es.kv_dim = e.kv_dim, es.head_dim = e.head_dim, es.pos0 = e.pos0, es.clip = e.clip;
 					es.range = e.range, es.q_lo = q_dim;
 					if (s_qkv.ks > 1) {
-						TRY(launch_split(f, s_qkv, b.Xn, 2 * c.dim, T, 2 * c.dim, c.dim, pf::BRowsPlain{qkv}, np, 0, 0, b.skp, st));
+						TRY(with_rows(qkv, [&](const auto &bm) {
+							return launch_split(f, s_qkv, b.Xn, 2 * c.dim, T, 2 * c.dim, c.dim, bm, np, 0, 0, b.skp, st);
+						}));
 						TRY(launch_skinny_reduce<false>(b.skp, s_qkv.ks, s_qkv.ks, np, T, np, es, st));
 					} else {
 						TRY(launch_plain(f, bn_qkv_all, b.Xn, 2 * c.dim, T, 2 * c.dim, c.dim, qkv, np, es, st));
 					}
 				} else if (s_qkv.ks > 1) {
-					TRY(launch_split(f, s_qkv, b.Xn, 2 * c.dim, T, c.dim, c.dim, pf::BRowsPlain{qkv}, q_dim, 2 * kv_dim,
-					                 2 * c.dim, b.skp, st));
+					TRY(with_rows(qkv, [&](const auto &bm) {
+						return launch_split(f, s_qkv, b.Xn, 2 * c.dim, T, c.dim, c.dim, bm, q_dim, 2 * kv_dim, 2 * c.dim, b.skp, st);
+					}));
 					TRY(launch_skinny_reduce<false>(b.skp, s_qkv.ks, s_qkv.ks2, q_dim, T, np, e, st));
 				} else if (qkv1) { // one launch: the k | v tiles (K = 2 dim) first, then the q tiles (K = dim)
-					TRY((launch_g8p<pf::E16QKV, pf::BRowsPlain, 2, 2>(f, b.Xn, 2 * c.dim, T, c.dim, c.dim,
-					                                                   pf::BRowsPlain{qkv}, q_dim + 2 * kv_dim, e, st,
-					                                                   0, q_dim, 2 * c.dim)));
+					TRY(with_rows(qkv, [&](const auto &bm) {
+						return launch_g8p<pf::E16QKV, std::decay_t<decltype(bm)>, 2, 2>(
+						    f, b.Xn, 2 * c.dim, T, c.dim, c.dim, bm, q_dim + 2 * kv_dim, e, st, 0, q_dim, 2 * c.dim);
+					}));
 				} else {
 					TRY(launch_plain(f, bn_q, b.Xn, 2 * c.dim, T, c.dim, c.dim, qkv, q_dim, e, st));
 					TRY(launch_plain(f, bn_kv, b.Xn, 2 * c.dim, T, 2 * c.dim, c.dim, qkv, 2 * kv_dim, e, st, q_dim));
@@ -717,26 +754,24 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 		TRY(launch_attn_prefill(b.Q, w.key_cache, w.value_cache, T, pos0, c.n_heads, c.n_kv_heads, c.head_dim, b.O,
 								st, split));
 		if (small || s_wo.ks > 1) {
-			if (small)
-				TRY(launch_skinny(f, b.O, q_dim, T, q_dim, q_dim, pf::BRowsPlain{one(w.wo, c.dim)}, c.dim, ks_wo, 0, c.dim,
-				                  b.skp, st));
-			else
-				TRY(launch_split(f, s_wo, b.O, sp * q_dim, T, sp * q_dim, q_dim, pf::BRowsPlain{one(w.wo, c.dim)}, c.dim, 0, 0,
-				                 b.skp, st));
+			TRY(with_rows(one(w.wo, c.dim, raw8), [&](const auto &bm) {
+				return small ? launch_skinny(f, b.O, q_dim, T, q_dim, q_dim, bm, c.dim, ks_wo, 0, c.dim, b.skp, st)
+				             : launch_split(f, s_wo, b.O, sp * q_dim, T, sp * q_dim, q_dim, bm, c.dim, 0, 0, b.skp, st);
+			}));
 			TRY(reduce_norm(small ? ks_wo : s_wo.ks, 1.0f, w.rms_ffn, split, rg + RG_XFFN));
 		} else {
 			pf::E16Residual e;
 			e.x = b.X;
 			e.ldx = c.dim;
 			e.M = T;
-			TRY(launch_plain(f, bn_wo, b.O, sp * q_dim, T, sp * q_dim, q_dim, one(w.wo, c.dim), c.dim, e, st));
+			TRY(launch_plain(f, bn_wo, b.O, sp * q_dim, T, sp * q_dim, q_dim, one(w.wo, c.dim, raw8), c.dim, e, st));
 			TRY(launch_rmsnorm(split, f, b.X, w.rms_ffn, c.dim, T, c.norm_eps, b.Xn, rg + RG_XFFN, st));
 		}
 		const float hscale = ldexpf(1.0f, -he);
 		if (small) {
-			const pf::BRowsGlu<64> bm{(const uint16_t *)w.w1, (const uint16_t *)w.w3};
-			TRY(launch_skinny(f, b.Xn, c.dim, T, c.dim, c.dim, bm, 2 * c.hidden_dim, ks_glu, 0, 2 * c.hidden_dim, b.skp,
-			                  st));
+			TRY(with_glu(w.w1, w.w3, raw8, [&](const auto &bm) {
+				return launch_skinny(f, b.Xn, c.dim, T, c.dim, c.dim, bm, 2 * c.hidden_dim, ks_glu, 0, 2 * c.hidden_dim, b.skp, st);
+			}));
 			if (c.act == YALM_SILU) {
 				pf::E16Glu<1> e;
 				e.h = b.H, e.ldh = c.hidden_dim, e.M = T, e.hscale = hscale, e.range = rg + RG_H;
@@ -747,20 +782,19 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 				TRY(launch_skinny_reduce<true>(b.skp, ks_glu, ks_glu, 2 * c.hidden_dim, T, 2 * c.hidden_dim, e, st));
 			}
 		} else {
-			TRY(c.act == YALM_SILU ? enqueue_glu<1>(d, w, T, hscale, rg + RG_H)
-								   : enqueue_glu<0>(d, w, T, hscale, rg + RG_H));
+			TRY(c.act == YALM_SILU ? enqueue_glu<1>(d, w, T, hscale, rg + RG_H, raw8)
+								   : enqueue_glu<0>(d, w, T, hscale, rg + RG_H, raw8));
 		}
 		// the next norm: the next layer's (its operand [hi | lo] in either form), or the final one
 		const bool last = l + 1 == c.n_layers;
 		const float *w_next = last ? (want_lp ? d->rms_final : nullptr) : d->b[l + 1].rms_att;
 		normed = small || s_w2.ks > 1;
 		if (normed) {
-			if (small)
-				TRY(launch_skinny(f, b.H, c.hidden_dim, T, c.hidden_dim, c.hidden_dim, pf::BRowsPlain{one(w.w2, c.dim)},
-				                  c.dim, ks_w2, 0, c.dim, b.skp, st));
-			else
-				TRY(launch_split(f, s_w2, b.H, sp * c.hidden_dim, T, sp * c.hidden_dim, c.hidden_dim,
-				                 pf::BRowsPlain{one(w.w2, c.dim)}, c.dim, 0, 0, b.skp, st));
+			TRY(with_rows(one(w.w2, c.dim, raw8), [&](const auto &bm) {
+				const int h = c.hidden_dim;
+				return small ? launch_skinny(f, b.H, h, T, h, h, bm, c.dim, ks_w2, 0, c.dim, b.skp, st)
+				             : launch_split(f, s_w2, b.H, sp * h, T, sp * h, h, bm, c.dim, 0, 0, b.skp, st);
+			}));
 			TRY(reduce_norm(small ? ks_w2 : s_w2.ks, ldexpf(1.0f, he), w_next, last ? split : true, rg + RG_N + RG_XATT));
 		} else {
 			pf::E16Residual e;
@@ -768,8 +802,8 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 			e.ldx = c.dim;
 			e.M = T;
 			e.scale = ldexpf(1.0f, he);
-			TRY(launch_plain(f, bn_w2, b.H, sp * c.hidden_dim, T, sp * c.hidden_dim, c.hidden_dim, one(w.w2, c.dim),
-			                 c.dim, e, st));
+			TRY(launch_plain(f, bn_w2, b.H, sp * c.hidden_dim, T, sp * c.hidden_dim, c.hidden_dim,
+			                 one(w.w2, c.dim, raw8), c.dim, e, st));
 		}
 	}
 	if (!want_lp)
@@ -788,12 +822,14 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 	e.ntiles = ntiles;
 	e.red = nullptr;
 	const void *wcls = d->wcls;
-	if (fp8) {
+	const bool cls8 = raw8 && f.g16[PG_CLS] < 0 && cls_bn <= 256; // (the f16 twin's tile width decides the sums' order)
+	if (fp8 && !cls8) {
 		const uint16_t *p[1];
 		TRY(dequant(d, {{d->wcls, (size_t)c.vocab_size * c.dim}}, p, st));
 		wcls = p[0];
 	}
-	TRY(launch_plain(f, cls_bn, b.Xn, sp * c.dim, T, sp * c.dim, c.dim, one(wcls, c.vocab_size), c.vocab_size, e, st));
+	TRY(launch_plain(f, cls_bn, b.Xn, sp * c.dim, T, sp * c.dim, c.dim, one(wcls, c.vocab_size, cls8), c.vocab_size,
+	                 e, st));
 	pf::logprob_kernel<<<T, 256, 0, st>>>(b.pmax, b.psum, b.tgt_logit, b.tgt, T, ntiles, b.lp);
 	HIPCHK(hipGetLastError());
 	return YALM_OK;
@@ -1027,9 +1063,10 @@ extern "C" int yalm_gemm_f16(float *c, const uint16_t *a, const uint16_t *w, int
 	const SplitPlan s = plan_split(f, PG_TEST, M, N, K, 0, 0, false, cap);
 	HostDev dp;
 	if (s.ks > 1) { // K slices, summed by the reduce kernel the prefill uses
+		const uint16_t *wp = (const uint16_t *)dw.p;
 		TRY(hd(dp, nullptr, (size_t)s.ks * ((M + 15) / 16 * 16) * N * 4));
-		TRY(launch_split(f, s, (const uint16_t *)da.p, K, M, K, K, pf::BRowsPlain{one(dw.p, N)}, N, 0, 0, (float *)dp.p,
-		                 nullptr));
+		TRY(launch_split(f, s, (const uint16_t *)da.p, K, M, K, K, pf::BRowsPlain{{{wp, wp, wp}, {N, N, N}}}, N, 0, 0,
+		                 (float *)dp.p, nullptr));
 		TRY(launch_skinny_reduce<false>((const float *)dp.p, s.ks, s.ks, N, M, N, e16, nullptr));
 	} else {
 		TRY(launch_plain(f, pick_bn(f, PG_TEST, M, N, false), (const uint16_t *)da.p, K, M, K, K, one(dw.p, N), N, e16,

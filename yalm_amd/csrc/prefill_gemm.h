@@ -65,6 +65,7 @@ __device__ __forceinline__ f32x4_t mfma16(const half8_t &a, const half8_t &b, co
 // ---------------------------------------------------------------- B row policies
 struct BRowsPlain { // W rows n0 + r from up to 3 row-major [rows][K] matrices laid end to end
 	BSrc src;
+	using elt = uint16_t;
 	static constexpr int COLS_PER_TILE_DIV = 1; // output columns per tile = BN
 	__device__ __forceinline__ const uint16_t *row(int n0, int r, int K) const {
 		const int n = n0 + r;
@@ -74,11 +75,27 @@ struct BRowsPlain { // W rows n0 + r from up to 3 row-major [rows][K] matrices l
 	}
 };
 
+// The same over E5M2 bytes: 16 K columns per 16-byte piece; the GEMM expands a byte to the f16 with bits
+// b << 8 as it reads a fragment (gemm8p_kernel).
+struct BRowsPlain8 {
+	const uint8_t *p[3];
+	int end[3];
+	using elt = uint8_t;
+	static constexpr int COLS_PER_TILE_DIV = 1;
+	__device__ __forceinline__ const uint8_t *row(int n0, int r, int K) const {
+		const int n = n0 + r;
+		const int s = n < end[0] ? 0 : (n < end[1] ? 1 : 2);
+		const int start = s == 0 ? 0 : end[s - 1];
+		return p[s] + (size_t)(n - start) * K;
+	}
+};
+
 // One matrix of `rows` rows that need not be a multiple of the tile's width: the last tile's rows past
 // the end repeat the last row, and the epilogue leaves their columns out.
 struct BRowsRagged {
 	const uint16_t *w;
 	int rows;
+	using elt = uint16_t;
 	static constexpr int COLS_PER_TILE_DIV = 1;
 	__device__ __forceinline__ const uint16_t *row(int n0, int r, int K) const {
 		return w + (size_t)min(n0 + r, rows - 1) * K;
@@ -87,11 +104,12 @@ struct BRowsRagged {
 
 // GLU: a tile covers BN / 2 hidden columns h0 .. ; wave column wc's TN B rows are
 // TN / 2 W1 rows then the same TN / 2 W3 rows (h0 + wc * TN / 2 + ..).
-template <int TN>
+template <int TN, class ELT = uint16_t>
 struct BRowsGlu {
-	const uint16_t *w1, *w3;
+	const ELT *w1, *w3;
+	using elt = ELT;
 	static constexpr int COLS_PER_TILE_DIV = 2;
-	__device__ __forceinline__ const uint16_t *row(int h0, int r, int K) const {
+	__device__ __forceinline__ const ELT *row(int h0, int r, int K) const {
 		const int wc = r / TN, within = r % TN;
 		const int mat = within / (TN / 2);
 		const int hc = h0 + wc * (TN / 2) + within % (TN / 2);
@@ -519,6 +537,21 @@ __device__ __forceinline__ half8_t g16frag(const uint16_t *lds, int r, int s, in
 	return *(const half8_t *)(lds + r * G_BK + 8 * (kc ^ (r & 7)));
 }
 
+// The same fragment of an E5M2 image: rows of 64 bytes, 16-byte chunk c of row r at c ^ ((r >> 2) & 3) (four rows
+// span the 64 banks, so 16 rows' reads of one chunk column spread over all of them), read as 8 bytes ...
+__device__ __forceinline__ uint2 g8frag(const uint16_t *lds, int r, int s, int lane) {
+	const int q = lane >> 4, c = (2 * s + (q >> 1)) ^ ((r >> 2) & 3);
+	return *(const uint2 *)((const char *)lds + r * G_BK + 16 * c + 8 * (q & 1));
+}
+// ... and expanded: byte b is the f16 with bits b << 8 (exact).
+__device__ __forceinline__ half8_t e5m2x8(const uint2 &v) {
+	const u32x4_t o = {__builtin_amdgcn_perm(v.x, v.x, 0x010c000cu), __builtin_amdgcn_perm(v.x, v.x, 0x030c020cu),
+	                   __builtin_amdgcn_perm(v.y, v.y, 0x010c000cu), __builtin_amdgcn_perm(v.y, v.y, 0x030c020cu)};
+	return __builtin_bit_cast(half8_t, o);
+}
+template <class BMAP>
+using bmap_elt = typename BMAP::elt;
+
 // C tile [256][BN] of C = A · B^T, B rows through BMAP. 8 waves as WM x (8 / WM).
 template <class EPI, class BMAP, int BN, int WM>
 __global__ __launch_bounds__(G_THREADS, 1) void gemm16_kernel(const uint16_t *__restrict__ A, int lda, int M, int K,
@@ -656,6 +689,10 @@ constexpr int P8_HT = 128 * G_BK; // f16 per A half-tile (128 rows)
 // order: with one workgroup per tile the hardware then hands the K tiles to the CUs the
 // K2 tiles leave free (longest first).
 //
+// E5M2 weights (a BMAP of bytes): the B half-tiles hold bytes (half the LDS-DMAs), a fragment is expanded to f16
+// after the phase's barrier, 4 v_perm per 16-deep-by-16 fragment beside 8 MFMAs. Before, a pass wrote and read
+// an f16 copy of every layer (Mistral-7B: 131 us a layer, 4.2 of the 20.9 ms of a 1001-row prompt).
+//
 // Split K (nkc < the depth in K tiles; an EPI with PARTIAL, E16Part): a tile's K range is cut into
 // slices of nkc K tiles (the last one shorter), one item per (slice, tile), each leaving its f32
 // partial tile in its own slot; skinny_reduce_kernel / reduce_norm_rows_kernel sum the slots in
@@ -673,11 +710,21 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
                                                              int kb, BMAP bm, int N, EPI epi, int c0, int c_split,
                                                              int K2, int nkc) {
 	constexpr int FI = 8, FJ = FJ0 + FJ1, TM = 128, TN = 16 * FJ, BN = 4 * TN;
-	constexpr int HB0 = 64 * FJ0 * G_BK, HB1 = 64 * FJ1 * G_BK; // f16 per B half-tile
+	using elt = bmap_elt<BMAP>;
+	constexpr int EB = sizeof(elt); // bytes per weight
+	static_assert(EB == 1 || EB == 2, "f16 / bf16 or E5M2 weights");
+	constexpr int HB0 = 32 * FJ0 * G_BK * EB, HB1 = 32 * FJ1 * G_BK * EB; // 16-bit words per B half-tile
 	constexpr int OFF[4] = {0, P8_HT, 2 * P8_HT, 2 * P8_HT + HB0}; // Am0, Am1, Bn0, Bn1 in a buffer
 	constexpr int BUFE = 2 * P8_HT + HB0 + HB1;
-	constexpr int INFLIGHT = FJ0 + FJ1 + 4;
-	static_assert(FJ0 >= 1 && FJ1 >= 1 && FJ0 <= 3 && FJ1 <= 3, "quadrant widths");
+	// LDS-DMAs of a wave per B half-tile (1 KB each: 8 rows of f16, 16 of E5M2). A half-tile of 64 E5M2 rows is 4
+	// of them: waves 0-3 stage Bn0's, waves 4-7 Bn1's
+	constexpr int NB0 = EB == 2 ? FJ0 : (FJ0 + 1) / 2, NB1 = EB == 2 ? FJ1 : (FJ1 + 1) / 2;
+	constexpr bool HALF0 = EB == 1 && FJ0 == 1, HALF1 = EB == 1 && FJ1 == 1;
+	static_assert(FJ0 >= 1 && FJ1 >= 1 && FJ0 <= 3 && FJ1 <= 3 && (EB == 2 || (FJ0 <= 2 && FJ1 <= 2)), "quadrant widths");
+	// in flight after a phase's wait: the last 4 phases' stages, one of each half-tile (a wave without a share of
+	// Bn1 has one fewer)
+	constexpr int INFLIGHT = 4 + NB0 + NB1 - (HALF0 && HALF1 ? 1 : 0);
+	constexpr bool UNEVEN = HALF0 != HALF1;
 	extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
 	const int lane = threadIdx.x & 63;
 	const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -718,7 +765,7 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
 		// + (lane >> 3), 16-byte chunk lane & 7 read from source chunk (lane & 7) ^ (lr & 7)
 		// (the swizzle g16frag undoes)
 		uint32_t aoff[2][2]; // [m half][i]: element offset into A
-		const uint16_t *bp[2][3];
+		const elt *bp[2][3];
 	#pragma unroll
 		for (int i = 0; i < 2; ++i) {
 			const int lr = (2 * wave + i) * 8 + (lane >> 3);
@@ -727,17 +774,19 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
 			aoff[0][i] = (uint32_t)min(row0 + ra, M - 1) * lda + sw;
 			aoff[1][i] = (uint32_t)min(row0 + ra + 64, M - 1) * lda + sw;
 		}
+		// (E5M2: 16 rows of 64 bytes per instruction, source chunk (lane & 3) ^ ((lr >> 2) & 3), g8frag)
+		const int w0 = HALF0 ? wave & 3 : wave, w1 = HALF1 ? wave & 3 : wave;
+		auto brow = [&](int inst) { return EB == 2 ? inst * 8 + (lane >> 3) : inst * 16 + (lane >> 2); };
+		auto bsw = [&](int lr) { return EB == 2 ? 8 * ((lane & 7) ^ (lr & 7)) : 16 * ((lane & 3) ^ ((lr >> 2) & 3)); };
 	#pragma unroll
-		for (int i = 0; i < FJ0; ++i) {
-			const int lr = (FJ0 * wave + i) * 8 + (lane >> 3);
-			const int sw = 8 * ((lane & 7) ^ (lr & 7));
-			bp[0][i] = bm.row(colB, (lr / (16 * FJ0)) * TN + lr % (16 * FJ0), kb) + sw;
+		for (int i = 0; i < NB0; ++i) {
+			const int lr = brow(NB0 * w0 + i);
+			bp[0][i] = bm.row(colB, (lr / (16 * FJ0)) * TN + lr % (16 * FJ0), kb) + bsw(lr);
 		}
 	#pragma unroll
-		for (int i = 0; i < FJ1; ++i) {
-			const int lr = (FJ1 * wave + i) * 8 + (lane >> 3);
-			const int sw = 8 * ((lane & 7) ^ (lr & 7));
-			bp[1][i] = bm.row(colB, (lr / (16 * FJ1)) * TN + 16 * FJ0 + lr % (16 * FJ1), kb) + sw;
+		for (int i = 0; i < NB1; ++i) {
+			const int lr = brow(NB1 * w1 + i);
+			bp[1][i] = bm.row(colB, (lr / (16 * FJ1)) * TN + 16 * FJ0 + lr % (16 * FJ1), kb) + bsw(lr);
 		}
 		// half-tile h (0 Am0, 1 Am1, 2 Bn0, 3 Bn1) of K tile kt into buffer buf
 		auto stage = [&](int buf, int h, int kt) {
@@ -750,16 +799,24 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
 					__builtin_amdgcn_global_load_lds((const void *)(A + aoff[h][i] + k0),
 					                                 (YALM_LDS void *)(base + (2 * wave + i) * 8 * G_BK), 16, 0, 0);
 			} else if (h == 2) {
+				if (!HALF0 || wave < 4)
 	#pragma unroll
-				for (int i = 0; i < FJ0; ++i)
-					__builtin_amdgcn_global_load_lds((const void *)(bp[0][i] + kw),
-					                                 (YALM_LDS void *)(base + (FJ0 * wave + i) * 8 * G_BK), 16, 0, 0);
+					for (int i = 0; i < NB0; ++i)
+						__builtin_amdgcn_global_load_lds((const void *)(bp[0][i] + kw),
+						                                 (YALM_LDS void *)(base + (NB0 * w0 + i) * 512), 16, 0, 0);
 			} else {
+				if (!HALF1 || (wave >= 4) == HALF0) // (2, 1): waves 0-3; (1, 1): waves 4-7
 	#pragma unroll
-				for (int i = 0; i < FJ1; ++i)
-					__builtin_amdgcn_global_load_lds((const void *)(bp[1][i] + kw),
-					                                 (YALM_LDS void *)(base + (FJ1 * wave + i) * 8 * G_BK), 16, 0, 0);
+					for (int i = 0; i < NB1; ++i)
+						__builtin_amdgcn_global_load_lds((const void *)(bp[1][i] + kw),
+						                                 (YALM_LDS void *)(base + (NB1 * w1 + i) * 512), 16, 0, 0);
 			}
+		};
+		auto wait_older = [&]() { // all but the last 4 phases' stages have landed
+			if (UNEVEN && wave >= 4)
+				asm volatile("s_waitcnt vmcnt(%0)" ::"n"(INFLIGHT - 1) : "memory");
+			else
+				asm volatile("s_waitcnt vmcnt(%0)" ::"n"(INFLIGHT) : "memory");
 		};
 
 		f32x4_t acc[FI][FJ];
@@ -769,6 +826,7 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
 			for (int j = 0; j < FJ; ++j)
 				acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 		half8_t a[4][2], b0[FJ0][2], b1[FJ1][2];
+		uint2 r0[FJ0][2], r1[FJ1][2]; // E5M2: the fragments as read
 
 		const int nk = epi_partial<EPI>::value ? min(Kt / G_BK - kt0, nkc) : Kt / G_BK;
 		// prologue = the previous iteration's stages p3 .. p8 for K tiles 0 (E) and 1 (O)
@@ -779,7 +837,7 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
 		stage(0, 1, 0);
 		stage(1, 0, k1);
 		stage(1, 2, k1);
-		asm volatile("s_waitcnt vmcnt(%0)" ::"n"(INFLIGHT) : "memory"); // Am0, Bn0 of K tile 0
+		wait_older(); // Am0, Bn0 of K tile 0
 		asm volatile("s_barrier" ::: "memory");
 		if (wr == 1)
 			asm volatile("s_barrier" ::: "memory"); // wave row 1 runs one barrier behind
@@ -798,7 +856,26 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
 			for (int j = 0; j < FJ0; ++j)
 	#pragma unroll
 				for (int ks = 0; ks < 2; ++ks)
-					b0[j][ks] = g16frag(s, wc * 16 * FJ0 + 16 * j + (lane & 15), ks, lane);
+					if constexpr (EB == 2)
+						b0[j][ks] = g16frag(s, wc * 16 * FJ0 + 16 * j + (lane & 15), ks, lane);
+					else
+						r0[j][ks] = g8frag(s, wc * 16 * FJ0 + 16 * j + (lane & 15), ks, lane);
+		};
+		auto cv_b0 = [&]() {
+			if constexpr (EB == 1)
+	#pragma unroll
+				for (int j = 0; j < FJ0; ++j)
+	#pragma unroll
+					for (int ks = 0; ks < 2; ++ks)
+						b0[j][ks] = e5m2x8(r0[j][ks]);
+		};
+		auto cv_b1 = [&]() {
+			if constexpr (EB == 1)
+	#pragma unroll
+				for (int j = 0; j < FJ1; ++j)
+	#pragma unroll
+					for (int ks = 0; ks < 2; ++ks)
+						b1[j][ks] = e5m2x8(r1[j][ks]);
 		};
 		auto rd_b1 = [&](int buf) {
 			const uint16_t *s = smem + buf * BUFE + OFF[3];
@@ -806,13 +883,16 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
 			for (int j = 0; j < FJ1; ++j)
 	#pragma unroll
 				for (int ks = 0; ks < 2; ++ks)
-					b1[j][ks] = g16frag(s, wc * 16 * FJ1 + 16 * j + (lane & 15), ks, lane);
+					if constexpr (EB == 2)
+						b1[j][ks] = g16frag(s, wc * 16 * FJ1 + 16 * j + (lane & 15), ks, lane);
+					else
+						r1[j][ks] = g8frag(s, wc * 16 * FJ1 + 16 * j + (lane & 15), ks, lane);
 		};
 		// {stage (or drain), barrier, MFMAs on quadrant (mh, nh), barrier}
 		auto sync_stage = [&](int sbuf, int sh, int skt) {
 			if (skt < nk) {
 				stage(sbuf, sh, skt);
-				asm volatile("s_waitcnt vmcnt(%0)" ::"n"(INFLIGHT) : "memory");
+				wait_older();
 			} else {
 				asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 			}
@@ -852,10 +932,12 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
 			rd_a(0, 0);
 			rd_b0(0);
 			sync_stage(1, 3, ko); // p1: Bn1 O(2i+1)
+			cv_b0();
 			mfma_n0(0);
 			sync_end();
 			rd_b1(0);
 			sync_stage(1, 1, ko); // p2: Am1 O(2i+1)
+			cv_b1();
 			mfma_n1(0);
 			sync_end();
 			rd_a(0, 1);
@@ -871,10 +953,12 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
 			rd_a(1, 0);
 			rd_b0(1);
 			sync_stage(0, 3, ke + 2); // p5: Bn1 E(2i+2)
+			cv_b0();
 			mfma_n0(0);
 			sync_end();
 			rd_b1(1);
 			sync_stage(0, 1, ke + 2); // p6: Am1 E(2i+2)
+			cv_b1();
 			mfma_n1(0);
 			sync_end();
 			rd_a(1, 1);
@@ -900,9 +984,9 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
 	}
 }
 
-template <int FJ0 = 2, int FJ1 = 2>
+template <int FJ0 = 2, int FJ1 = 2, int EB = 2>
 constexpr size_t gemm8p_lds() {
-	return (size_t)2 * (2 * P8_HT + 64 * (FJ0 + FJ1) * G_BK) * sizeof(uint16_t);
+	return (size_t)2 * (2 * P8_HT * sizeof(uint16_t) + 64 * (FJ0 + FJ1) * G_BK * EB);
 }
 
 } // namespace pf

@@ -125,15 +125,15 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(const uint16_t *__rest
 // The same partials with the weight rows staged through LDS by LDS-DMA, so every
 // wave-instruction reads 4 rows x 256 contiguous bytes (skinny_gemm_kernel's register
 // loads read 16 rows x 64 B per instruction: half cache lines, 16 DRAM rows at once).
-// Each wave owns its 16 weight rows in a 3-stage ring of 128-column stages (4 KB per
+// Each wave owns its 16 weight rows in a 3-stage ring of 256-byte-wide stages (4 KB per
 // wave per stage): no workgroup barrier in the loop, one counted vmcnt per stage. The
 // 16-byte chunks of a row are XOR-swizzled by the row (source side of the DMA) so the
 // MFMA B-fragment reads (16 rows x one chunk) spread over the banks. LDS: the A chunk
 // (<= 32 KB) + 48 KB of ring: two workgroups per CU.
-constexpr int SKL_KS = 128;                    // K columns per stage
+constexpr int SKL_ROWB = 256;                  // bytes per weight row and stage: 128 f16 / bf16 columns, 256 E5M2
 constexpr int SKL_NS = 3;                      // ring stages
-constexpr int SKL_STAGE = SK_ROWS * SKL_KS;    // f16 per stage (16 KB)
-constexpr size_t SKL_RING_BYTES = (size_t)SKL_NS * SKL_STAGE * 2;
+constexpr int SKL_STAGE = SK_ROWS * SKL_ROWB;  // bytes per stage (16 KB)
+constexpr size_t SKL_RING_BYTES = (size_t)SKL_NS * SKL_STAGE;
 
 template <int MT, class BMAP, bool BF = false> // BF: bf16 operands (the layer-list engine's products)
 __global__ __launch_bounds__(256) void skinny_gemm_lds_kernel(const uint16_t *__restrict__ A, int lda, int T, int K,
@@ -141,8 +141,10 @@ __global__ __launch_bounds__(256) void skinny_gemm_lds_kernel(const uint16_t *__
                                                               float *__restrict__ part) {
 	extern __shared__ __attribute__((aligned(16))) uint16_t sm[];
 	constexpr int TP = 16 * MT;
-	uint16_t *const as = sm;                                      // [TP][KC], swizzled as skinny_gemm_kernel
-	uint16_t *const ring = sm + (size_t)TP * KC;                  // [SKL_NS][64 rows][SKL_KS]
+	using elt = bmap_elt<BMAP>;
+	constexpr int EB = sizeof(elt), KSTG = SKL_ROWB / EB; // columns per stage
+	uint16_t *const as = sm;                              // [TP][KC], swizzled as skinny_gemm_kernel
+	char *const ring = (char *)(sm + (size_t)TP * KC);    // [SKL_NS][64 rows][SKL_ROWB]
 	const int nblk = N / SK_ROWS;
 	const int nb = blockIdx.x % nblk, ks = blockIdx.x / nblk;
 	const int k0 = ks * KC;
@@ -151,23 +153,23 @@ __global__ __launch_bounds__(256) void skinny_gemm_lds_kernel(const uint16_t *__
 	const int cb = c0 + nb * SK_ROWS;      // the workgroup's first B row (output column)
 	const int col = cb + 16 * wave;        // the wave's
 	const int kw0 = k0 < kb ? k0 : k0 - kb; // B wrap (a K chunk never straddles kb)
-	const int nst = KC / SKL_KS;
+	const int nst = KC / KSTG;
 	// DMA geometry: instruction i of a stage covers the wave's rows 4 i .. 4 i + 3, lane
 	// l row 4 i + (l >> 4), LDS slot l & 15 <- source chunk (l & 15) ^ row
-	const uint16_t *src[4];
+	const elt *src[4];
 #pragma unroll
 	for (int i = 0; i < 4; ++i) {
 		const int rr = 4 * i + (lane >> 4);
-		src[i] = bm.row(cb / BMAP::COLS_PER_TILE_DIV, 16 * wave + rr, kb) + kw0 + 8 * ((lane & 15) ^ rr);
+		src[i] = bm.row(cb / BMAP::COLS_PER_TILE_DIV, 16 * wave + rr, kb) + kw0 + 16 / EB * ((lane & 15) ^ rr);
 	}
-	uint16_t *const wring = ring + wave * 16 * SKL_KS; // this wave's rows in every stage
+	char *const wring = ring + wave * 16 * SKL_ROWB; // this wave's rows in every stage
 	auto issue = [&](int st) { // stage st (clamped: past the chunk it re-reads the last stage, an L2 hit)
 		const int sc = st < nst ? st : nst - 1;
-		uint16_t *dst = wring + (st % SKL_NS) * SKL_STAGE;
+		char *dst = wring + (st % SKL_NS) * SKL_STAGE;
 #pragma unroll
 		for (int i = 0; i < 4; ++i)
-			__builtin_amdgcn_global_load_lds((const void *)(src[i] + sc * SKL_KS),
-			                                 (YALM_LDS void *)(dst + 4 * i * SKL_KS), 16, 0, 0);
+			__builtin_amdgcn_global_load_lds((const void *)(src[i] + sc * KSTG),
+			                                 (YALM_LDS void *)(dst + 4 * i * SKL_ROWB), 16, 0, 0);
 	};
 	issue(0);
 	issue(1);
@@ -182,13 +184,17 @@ __global__ __launch_bounds__(256) void skinny_gemm_lds_kernel(const uint16_t *__
 		asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // stage st - 1's B reads are done...
 		issue(st + 2); // ...before its slot is re-staged
 		asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); // stage st landed (2 stages x 4 behind it)
-		const uint16_t *bst = wring + (st % SKL_NS) * SKL_STAGE + n * SKL_KS;
+		const char *bst = wring + (st % SKL_NS) * SKL_STAGE + n * SKL_ROWB;
 #pragma unroll
-		for (int j = 0; j < SKL_KS / 32; ++j) {
-			const half8_t b = *(const half8_t *)(bst + 8 * ((4 * j + q) ^ n));
+		for (int j = 0; j < KSTG / 32; ++j) {
+			half8_t b;
+			if constexpr (EB == 2)
+				b = *(const half8_t *)(bst + 16 * ((4 * j + q) ^ n));
+			else // E5M2: 8 of a chunk's 16 columns
+				b = e5m2x8(*(const uint2 *)(bst + 16 * ((2 * j + (q >> 1)) ^ n) + 8 * (q & 1)));
 #pragma unroll
 			for (int m = 0; m < MT; ++m) {
-				const half8_t a = sk_afrag<MT>(as, KC, 16 * m + n, st * SKL_KS + 32 * j + 8 * q);
+				const half8_t a = sk_afrag<MT>(as, KC, 16 * m + n, st * KSTG + 32 * j + 8 * q);
 				acc[m] = mfma16<BF>(a, b, acc[m]);
 			}
 		}
