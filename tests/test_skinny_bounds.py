@@ -1,114 +1,125 @@
-"""CPU: the address range of the short-prompt (T <= 64) skinny GEMMs, bounded on the host
-(the r4y illegal-address question of the LDS-DMA skinny form).
+"""CPU: the address range of the short-prompt (T <= 64) streamed GEMMs, bounded on the host.
 
-The index arithmetic of yalm_amd/csrc/prefill_skinny.h is restated here for every GEMM
-the prefill launches at T = 1..64 (prefill.hip enqueue_prefill, the `small` path) at the
-production shapes: sk_stage_a's A-row reads (rows clamped to T - 1, columns inside the
-K chunk) and skinny_gemm_lds_kernel's weight-row DMA sources (rows of the workgroup's
-64-row block, columns inside the chunk, the clamped tail stages), against the sizes of
-the buffers they read (PrefillBufs, the weight tensors). The K split sk_pick_ks is
-restated too, with its invariants (KC a multiple of the 128-column DMA stage, the A chunk
-within 32 KB of LDS, no chunk straddling the B wrap of the k | v GEMM).
+The index arithmetic of yalm_amd/csrc/prefill_skinny.h (stream_gemm_kernel) and prefill.hip
+(plan_stream) is restated here for every GEMM the prefill launches at T = 1..64 (enqueue_prefill,
+the `small` path) at the production shapes: the A-row and weight-row DMA sources (rows clamped to
+T - 1, the workgroup's rows inside the matrix, columns inside the slice), the LDS destinations of
+every stage inside the ring, the partial slots inside their buffer, and the K slices, which cover K
+once each.
 """
+import math
+
 import pytest
 
 from yalm_amd import models as M
 
-SK_ROWS, SK_U = 64, 8
-SK_KSTEP = 32 * SK_U
-SKL_KS = 128
-SK_AMAX = 8
-SK_MAX_T = 64
+SK_MAX_T, KSTG, CUS = 64, 128, 256
 
 
-def sk_pick_ks(kn, TP):
-    """prefill.hip sk_pick_ks: kn = [(N, K, mult)]."""
-    best, kmin, wg1 = -1, 1 << 30, 0
-    for N, K, mult in kn:
-        kmin = min(kmin, K // mult)
-        wg1 += N // SK_ROWS * mult
-    for ks in range(1, kmin // SK_KSTEP + 1):
-        ok = True
-        for N, K, mult in kn:
-            s = ks * mult
-            ok = ok and K % s == 0 and (K // s) % SK_KSTEP == 0 and TP * (K // s) * 2 <= 32768
-        if not ok:
+def sk_rows(T):
+    return 16 if T <= 16 else 32 if T <= 32 else 64
+
+
+def sk_cols(T):
+    return 64 if T <= 32 else 128
+
+
+def plan_stream(T, N, nst, cap):
+    """prefill.hip plan_stream."""
+    blocks, rows = -(-N // sk_cols(T)), sk_rows(T)
+    slots = CUS * (2 if T <= 32 else 1)
+    best, least = None, 0.0
+    for ks in range(1, min(16, nst) + 1):
+        nsc = -(-nst // ks)
+        k = -(-nst // nsc)
+        floats = k * rows * blocks * sk_cols(T)
+        if k != ks or (ks > 1 and (nsc < 2 or floats > cap)):
             continue
-        best = ks
-        if wg1 * ks >= 512:
-            break
+        items = blocks * ks
+        t = math.ceil(items / slots) * (nsc * max(0.7, 1.27 * min(1.0, items / slots)) + 2.0)
+        if ks > 1:
+            t += 4.0 + floats * 8.0 / 5e6
+        if best is None or t < least:
+            best, least = (ks, nsc), t
     return best
 
 
-def a_max_elem(T, lda, K, KS):
-    """Largest f16 element index (exclusive end of a 16-byte read) sk_stage_a touches in A."""
-    MT = (T + 15) // 16
-    TP = 16 * MT
-    KC = K // KS
-    cpr, nch = KC // 8, TP * KC // 8
-    assert nch <= 256 * SK_AMAX, "the A chunk must fit one round of loads"
-    hi = 0
-    for ks in range(KS):
-        k0 = ks * KC
-        i = nch - 1  # the largest chunk index (later u clamp to it)
-        for i in range(max(0, nch - 2 * cpr), nch):  # the last rows' chunks: the largest addresses
-            r, c = divmod(i, cpr)
-            hi = max(hi, min(r, T - 1) * lda + k0 + 8 * c + 8)
-    return hi
-
-
-def b_max(N_rows_block_end, kb, K, KS):
-    """(largest B row + 1, largest B column + 1) the DMA sources reach: rows of the last
-    64-row block, columns of the clamped last 128-column stage of the last chunk."""
-    KC = K // KS
-    assert KC % SKL_KS == 0
-    nst = KC // SKL_KS
-    col_hi = 0
-    for ks in range(KS):
-        k0 = ks * KC
-        assert not (k0 < kb < k0 + KC), "a K chunk straddles the B wrap"
-        kw0 = k0 if k0 < kb else k0 - kb
-        col_hi = max(col_hi, kw0 + (nst - 1) * SKL_KS + 8 * 15 + 8)
-    return N_rows_block_end, col_hi
+def stream_cfg(T, eb, dual):
+    """StreamCfg: (waves, MT, stage bytes, ring depth, weight / A DMAs per wave)."""
+    mt, nw = {16: (1, 4), 32: (2, 4), 64: (4, 8)}[sk_rows(T)]
+    wb, ab = nw * 16 * KSTG * eb, 16 * mt * KSTG * 2
+    sb = wb + ab * (2 if dual else 1)
+    fit2, fit1 = 81920 // sb, 163840 // sb
+    ns = min(fit2, 6) if fit2 >= 3 else min(fit1, 4)
+    assert ns >= 2 and ns * sb <= 163840 and 4 * mt % nw == 0
+    return nw, mt, wb, ab, sb, ns, KSTG * eb // 64, 4 * mt // nw
 
 
 CFGS = {"mistral-7b": M.MISTRAL_7B, "llama-3.2-3b": M.LLAMA_32_3B,
         "gqa-d128": M.ModelConfig(dim=512, hidden_dim=1024, head_dim=128, n_layers=3, n_heads=4, n_kv_heads=2,
                                   vocab_size=1024, max_seq_len=320, rope_theta=1e6),
         "d768": M.ModelConfig(dim=768, hidden_dim=1536, head_dim=128, n_layers=2, n_heads=6, n_kv_heads=2,
-                              vocab_size=1920, max_seq_len=320, rope_theta=1e6)}
+                              vocab_size=1920, max_seq_len=40, rope_theta=1e6)}
 
 
+@pytest.mark.parametrize("eb", [1, 2])
 @pytest.mark.parametrize("name", list(CFGS))
-def test_skinny_gemm_reads_stay_inside_their_buffers(name):
+def test_stream_gemm_stays_inside_its_buffers(name, eb):
     c = CFGS[name]
-    cap = c.max_seq_len
-    q_dim, kv_dim = c.q_dim, c.kv_dim
-    # PrefillBufs allocations in f16 elements (prefill.hip ensure_bufs)
-    xn_elems = cap * c.dim * 2
-    o_elems = cap * q_dim * 2
-    h_elems = cap * c.hidden_dim * 2
-    for T in range(1, SK_MAX_T + 1):
-        TP = 16 * ((T + 15) // 16)
-        ks_qkv = sk_pick_ks([(q_dim, c.dim, 1), (2 * kv_dim, 2 * c.dim, 2)], TP)
-        ks_wo = sk_pick_ks([(c.dim, q_dim, 1)], TP)
-        ks_glu = sk_pick_ks([(2 * c.hidden_dim, c.dim, 1)], TP)
-        ks_w2 = sk_pick_ks([(c.dim, c.hidden_dim, 1)], TP)
-        assert min(ks_qkv, ks_wo, ks_glu, ks_w2) > 0, (T, ks_qkv, ks_wo, ks_glu, ks_w2)
-        # (A buffer, lda, K, kb, KS, B rows, B row width = kb)
-        gemms = [
-            ("q", xn_elems, 2 * c.dim, c.dim, c.dim, ks_qkv, q_dim),
-            ("k|v", xn_elems, 2 * c.dim, 2 * c.dim, c.dim, 2 * ks_qkv, 2 * kv_dim),
-            ("wo", o_elems, q_dim, q_dim, q_dim, ks_wo, c.dim),
-            ("glu", xn_elems, c.dim, c.dim, c.dim, ks_glu, 2 * c.hidden_dim),
-            ("w2", h_elems, c.hidden_dim, c.hidden_dim, c.hidden_dim, ks_w2, c.dim),
-        ]
-        for g, a_elems, lda, K, kb, KS, nrows in gemms:
-            hi = a_max_elem(T, lda, K, KS)
-            assert hi <= a_elems, (name, T, g, hi, a_elems)
-            assert hi <= T * lda, (name, T, g, "A read past row T - 1")
-            assert (T * lda if T > 0 else 0) <= a_elems
-            assert nrows % SK_ROWS == 0, (name, g, nrows)
-            rows_end, col_hi = b_max(nrows, kb, K, KS)
-            assert col_hi <= kb, (name, T, g, col_hi, kb)
-            assert (K // KS) * TP * 2 <= 32768, (name, T, g)
+    cap16 = -(-c.max_seq_len // 16) * 16
+    np_qkv = c.q_dim + 2 * c.kv_dim
+    skp = min(32 << 20, 16 * max(cap16, SK_MAX_T) * (max(np_qkv, c.dim, 2 * c.hidden_dim) + 64))
+    for T in range(1, min(SK_MAX_T, c.max_seq_len) + 1):
+        # (lda, K, B row width, columns, halves of A, GLU)
+        gemms = [("qkv", 2 * c.dim, c.dim, np_qkv, True, False), ("wo", c.q_dim, c.q_dim, c.dim, False, False),
+                 ("glu", c.dim, c.dim, 2 * c.hidden_dim, False, True), ("w2", c.hidden_dim, c.hidden_dim, c.dim, False, False)]
+        for g, lda, K, N, dual, glu in gemms:
+            nw, mt, wb, ab, sb, ns, nwi, na = stream_cfg(T, eb, dual)
+            assert K % KSTG == 0 and N % (16 * nw) == 0, (name, g)
+            ks, nsc = plan_stream(T, N, K // KSTG, skp)
+            slices = [(i * nsc, min(nsc, K // KSTG - i * nsc)) for i in range(ks)]
+            assert all(n > 0 for _, n in slices) and sum(n for _, n in slices) == K // KSTG
+            assert ks == 1 or ks * 16 * mt * N <= skp
+            for lane in range(64):
+                for wave in range(nw):
+                    for i in range(na):  # A: 4 rows of 256 bytes per DMA
+                        r = 4 * (wave * na + i) + (lane >> 4)
+                        assert r < 16 * mt and 8 * ((lane & 15) ^ (r & 15)) + 8 <= KSTG
+                        assert (wave * na + i + 1) * 1024 <= ab
+                    for i in range(nwi):
+                        rr = 4 * i + (lane >> 4) if eb == 2 else 8 * i + (lane >> 3)
+                        ch = (lane & 15) ^ rr if eb == 2 else (lane & 7) ^ ((rr >> 1) & 7)
+                        assert rr < 16 and (16 // eb) * ch + 16 // eb <= KSTG
+                        assert (wave * nwi + i + 1) * 1024 <= wb
+            st0, n = slices[-1]
+            k_end = (st0 + n) * KSTG
+            assert k_end <= K and (min(16 * mt - 1, T - 1) * lda + k_end + (K if dual else 0)) <= T * lda
+
+
+@pytest.mark.parametrize("eb", [1, 2])
+def test_stream_gemm_fragments_read_what_the_dma_wrote(eb):
+    """The swizzle of the DMA's source and of the fragment reads: lane (n, q) of k-step j gets the 8 columns
+    32 j + 8 q .. of row n, for A and weights, and no bank is read twice by 32 lanes of one weight read."""
+    a_lds, w_lds = {}, {}
+    for lane in range(64):
+        for i in range(4):
+            r = 4 * i + (lane >> 4)
+            a_lds[i * 1024 + lane * 16] = (r, 8 * ((lane & 15) ^ (r & 15)))
+        for i in range(KSTG * eb // 64):
+            rr = 4 * i + (lane >> 4) if eb == 2 else 8 * i + (lane >> 3)
+            ch = (lane & 15) ^ rr if eb == 2 else (lane & 7) ^ ((rr >> 1) & 7)
+            w_lds[i * 1024 + lane * 16] = (rr, 16 // eb * ch)
+    for j in range(4):
+        banks = [set(), set()]
+        for lane in range(64):
+            n, q = lane & 15, lane >> 4
+            assert a_lds[n * 256 + 16 * ((4 * j + q) ^ n)] == (n, 32 * j + 8 * q)
+            if eb == 2:
+                at, off = n * 256 + 16 * ((4 * j + q) ^ n), 0
+            else:
+                at, off = n * 128 + 16 * ((2 * j + (q >> 1)) ^ ((n >> 1) & 7)), 8 * (q & 1)
+            row, col = w_lds[at]
+            assert (row, col + off) == (n, 32 * j + 8 * q)
+            if eb == 1:
+                banks[lane >> 5].add((at + off) % 256)
+        assert eb == 2 or all(len(b) == 32 for b in banks)

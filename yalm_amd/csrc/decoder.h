@@ -90,9 +90,9 @@ struct PrefillBufs {
 struct PfForms {
 	int g16[6] = {-1, -1, -1, -1, -1, -1}; // qkv, wo, glu, w2, cls, test
 	bool p8 = true, persist = true;
-	bool no_skinny = false; // T <= 64: split-K skinny GEMMs (prefill_skinny.h) unless set
+	bool no_skinny = false; // T <= 64: streamed GEMMs (prefill_skinny.h) unless set
 	bool qkv1 = true;       // the q and k | v GEMMs as ONE two-depth launch when BN 256 fits both
-	bool skl = true;        // skinny GEMMs: weight rows staged by LDS-DMA (prefill_skinny.h)
+	bool skl = true;        // streamed GEMMs: LDS-DMA stages stay in flight (false: every stage drained)
 	bool split = false;     // split-operand precision form (yalm_set_prefill_precision): every f16
 							// activation operand as [hi | lo], the large-tile GEMMs at every T
 	bool ksplit = true;     // large tiles: K split over workgroups where the tiles leave CUs idle (gemm8p_kernel)

@@ -25,7 +25,7 @@
 // explicitly through yalm_set_prefill_forms: "qkv:256,wo:128,..." forces widths, 8p:0
 // the 2-phase kernel, persist:0 one workgroup per tile, skinny:0 the large tiles at
 // T <= 64 too (prefill_skinny.h otherwise), qkv1:0 the q and k | v GEMMs as two
-// launches, skl:0 the skinny GEMMs' weights as register loads instead of LDS-DMA stages,
+// launches, skl:0 the streamed short-prompt GEMMs with every stage drained,
 // ksplit:0 no K slices (plan_split), wnorm:0 the workgroup-per-row norm kernel instead of one wave per row.
 // The production library reads no environment for them; the A/B build (-DYALM_AB)
 // takes a decoder's initial forms from YALM_PF_FORMS (same syntax).
@@ -333,81 +333,77 @@ int launch_plain(const PfForms &f, int bn, const uint16_t *A, int lda, int M, in
 	return with_rows(b, [&](const auto &bm) { return launch_rows(f, bn, A, lda, M, K, kb, bm, N, epi, st, c0); });
 }
 
-// ---- short prompts (T <= SK_MAX_T): split-K skinny GEMMs (prefill_skinny.h)
+// ---- short prompts (T <= SK_MAX_T): streamed GEMMs (prefill_skinny.h)
 constexpr int SK_MAX_T = 64;
+// rows of a streamed GEMM: 16, 32 (4 waves of 16 weight rows, two workgroups per CU) or 64 (8 waves, one)
+int sk_rows(int T) { return T <= 16 ? 16 : T <= 32 ? 32 : 64; }
+int sk_cols(int T) { return T <= 32 ? 64 : 128; }
 
-// K splits of a skinny GEMM: every K chunk a multiple of the kernel's 256-column step
-// and <= 64 KB of A rows in LDS; the fewest splits that give >= 512 workgroups (the
-// weight stream needs the whole chip), else the most. kn: (N, K, mult) of each GEMM
-// sharing one partial buffer, split mult x KS ways (the k | v GEMM over [hi | lo], K =
-// 2 dim, takes 2 KS splits of the q GEMM's chunk size, so no chunk straddles the B
-// wrap at dim).
-struct SkGemm {
-	int N, K, mult;
+// K slices of a streamed GEMM of N columns over nst stages of 128: ks slices of nsc stages. Rounds of the
+// workgroups that fit the chip at once, a stage costing its share of HBM (2 x 16 KB or 32 KB of a CU's 26
+// GB/ms, 1.27 us with every CU busy) or, with few workgroups, the latency behind its ring (0.7 us), 2 us to
+// fill the ring, and for several slices a second launch that reads the partials (cap floats). The same for
+// f16 and E5M2 weights, so an fp8 model sums in its f16 twin's order.
+struct StreamPlan {
+	int ks = 0, nsc = 0;
 };
-int sk_pick_ks(std::initializer_list<SkGemm> kn, int TP) {
-	int best = -1, kmin = 1 << 30, wg1 = 0;
-	for (auto &p : kn) {
-		kmin = std::min(kmin, p.K / p.mult);
-		wg1 += p.N / pf::SK_ROWS * p.mult;
-	}
-	for (int ks = 1; ks <= kmin / pf::SK_KSTEP; ++ks) {
-		bool ok = true;
-		for (auto &p : kn) {
-			const int s = ks * p.mult;
-			ok = ok && p.K % s == 0 && (p.K / s) % pf::SK_KSTEP == 0 && (size_t)TP * (p.K / s) * 2 <= 32768;
-		}
-		if (!ok)
+StreamPlan plan_stream(int T, int N, int nst, size_t cap) {
+	const int blocks = (N + sk_cols(T) - 1) / sk_cols(T), rows = sk_rows(T);
+	const float slots = (float)device_cu_count() * (T <= 32 ? 2 : 1);
+	StreamPlan best;
+	float least = 0.0f;
+	for (int ks = 1; ks <= 16 && ks <= nst; ++ks) {
+		const int nsc = (nst + ks - 1) / ks, k = (nst + nsc - 1) / nsc;
+		const size_t floats = (size_t)k * rows * blocks * sk_cols(T);
+		if (k != ks || (ks > 1 && (nsc < 2 || floats > cap)))
 			continue;
-		best = ks;
-		if (wg1 * ks >= 512)
-			break;
+		const float items = (float)blocks * ks;
+		float t = std::ceil(items / slots) * (nsc * std::max(0.7f, 1.27f * std::min(1.0f, items / slots)) + 2.0f);
+		if (ks > 1)
+			t += 4.0f + (float)floats * 8.0f / 5e6f;
+		if (!best.ks || t < least) {
+			least = t;
+			best = {ks, nsc};
+		}
 	}
 	return best;
 }
 
-template <int MT, class BMAP>
-int launch_skinny_mt(const PfForms &f, const uint16_t *A, int lda, int T, int K, int kb, const BMAP &bm, int N,
-                     int KS, int c0, int Np, float *part, hipStream_t st) {
-	auto kern = pf::skinny_gemm_lds_kernel<MT, BMAP>;
-	if constexpr (sizeof(pf::bmap_elt<BMAP>) == 2)
-		if (!f.skl)
-			kern = pf::skinny_gemm_kernel<MT, BMAP>;
-	static bool attr[2] = {false, false};
-	if (!attr[f.skl]) {
-		HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-		                           32768 + (int)pf::SKL_RING_BYTES));
-		attr[f.skl] = true;
+// GLU: over BRowsGlu rows (N = 2 x hidden, the epilogue's columns are hidden units). plan.ks == 1: the epilogue
+// runs in the launch, else partials for launch_skinny_reduce / launch_reduce_norm. DUAL: columns >= c_split
+// over [hi | lo].
+template <int MT, int NW, class BMAP, bool DUAL, bool GLU, class EPI, bool BF>
+int launch_stream_t(const PfForms &f, const StreamPlan &p, const uint16_t *A, int lda, int T, int K, int kb, const BMAP &bm,
+                    int N, int c_split, float *part, const EPI &epi, hipStream_t st) {
+	using C = pf::StreamCfg<MT, NW, BMAP, DUAL>;
+	auto kern = pf::stream_gemm_kernel<MT, NW, BMAP, DUAL, GLU, EPI, BF>;
+	static bool attr = false;
+	if (!attr) {
+		HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::LDS));
+		attr = true;
 	}
-	const int KC = K / KS;
-	const size_t lds = (size_t)16 * MT * KC * sizeof(uint16_t) + (f.skl ? pf::SKL_RING_BYTES : 0);
-	hipLaunchKernelGGL(kern, dim3((N / pf::SK_ROWS) * KS), dim3(256), lds, st, A, lda, T, K, kb, bm, N, KC, c0, Np,
-	                   part);
+	const int nblk = (N + 16 * NW - 1) / (16 * NW);
+	hipLaunchKernelGGL(kern, dim3(nblk * p.ks), dim3(64 * NW), C::LDS, st, A, lda, T, K / C::KSTG, kb, bm, nblk, p.nsc,
+	                   c_split, nblk * 16 * NW, part, epi, (int)!f.skl);
 	HIPCHK(hipGetLastError());
 	return YALM_OK;
 }
-
-template <class BMAP>
-int launch_skinny(const PfForms &f, const uint16_t *A, int lda, int T, int K, int kb, const BMAP &bm, int N, int KS,
-                  int c0, int Np, float *part, hipStream_t st) {
-	switch ((T + 15) / 16) {
-	case 1:
-		return launch_skinny_mt<1>(f, A, lda, T, K, kb, bm, N, KS, c0, Np, part, st);
-	case 2:
-		return launch_skinny_mt<2>(f, A, lda, T, K, kb, bm, N, KS, c0, Np, part, st);
-	case 3:
-		return launch_skinny_mt<3>(f, A, lda, T, K, kb, bm, N, KS, c0, Np, part, st);
-	default:
-		return launch_skinny_mt<4>(f, A, lda, T, K, kb, bm, N, KS, c0, Np, part, st);
-	}
+template <bool DUAL, bool GLU, bool BF, class BMAP, class EPI>
+int launch_stream(const PfForms &f, const StreamPlan &p, const uint16_t *A, int lda, int T, int K, int kb, const BMAP &bm,
+                  int N, int c_split, float *part, const EPI &epi, hipStream_t st) {
+	if (T <= 16)
+		return launch_stream_t<1, 4, BMAP, DUAL, GLU, EPI, BF>(f, p, A, lda, T, K, kb, bm, N, c_split, part, epi, st);
+	if (T <= 32)
+		return launch_stream_t<2, 4, BMAP, DUAL, GLU, EPI, BF>(f, p, A, lda, T, K, kb, bm, N, c_split, part, epi, st);
+	return launch_stream_t<4, 8, BMAP, DUAL, GLU, EPI, BF>(f, p, A, lda, T, K, kb, bm, N, c_split, part, epi, st);
 }
 
 // columns < c_split sum KS partials, the others KS2
 template <bool GLU, class EPI>
 int launch_skinny_reduce(const float *part, int KS, int KS2, int c_split, int T, int Np, const EPI &epi,
-                         hipStream_t st) {
-	const int TP = 16 * ((T + 15) / 16);
-	const int waves = (TP / 16) * (Np / 64);
+                         hipStream_t st, int TP = 0) { // TP: rows of a slot (default: T in whole 16s)
+	TP = TP ? TP : 16 * ((T + 15) / 16);
+	const int waves = ((T + 15) / 16) * (Np / 64);
 	pf::skinny_reduce_kernel<4, GLU, EPI><<<(waves + 3) / 4, 256, 0, st>>>(part, KS, KS2, c_split, TP, T, Np, epi);
 	HIPCHK(hipGetLastError());
 	return YALM_OK;
@@ -480,8 +476,8 @@ int launch_rmsnorm(bool split, const PfForms &f, const float *X, const float *w,
 // X += scale * (sum of the partials), Xn = the next norm's operand (prefill_skinny.h); w null: no norm
 template <bool SPLIT>
 int launch_reduce_norm_t(const float *part, int KS, int T, float *X, int dim, float scale, const float *w, float eps,
-                         uint16_t *Xn, unsigned *range, hipStream_t st) {
-	const size_t kstride = (size_t)((T + 15) / 16 * 16) * dim;
+                         uint16_t *Xn, unsigned *range, hipStream_t st, int TP) {
+	const size_t kstride = (size_t)TP * dim;
 	const int nt = std::min(1024, (dim / 4 + 63) / 64 * 64), nv = (dim / 4 + nt - 1) / nt;
 	if (nv == 1)
 		pf::reduce_norm_rows_kernel<SPLIT, 1><<<T, nt, 0, st>>>(part, KS, kstride, X, dim, scale, w, eps, Xn, range);
@@ -493,9 +489,9 @@ int launch_reduce_norm_t(const float *part, int KS, int T, float *X, int dim, fl
 	return YALM_OK;
 }
 int launch_reduce_norm(bool split, const float *part, int KS, int T, float *X, int dim, float scale, const float *w,
-                       float eps, uint16_t *Xn, unsigned *range, hipStream_t st) {
-	return split ? launch_reduce_norm_t<true>(part, KS, T, X, dim, scale, w, eps, Xn, range, st)
-	             : launch_reduce_norm_t<false>(part, KS, T, X, dim, scale, w, eps, Xn, range, st);
+                       float eps, uint16_t *Xn, unsigned *range, hipStream_t st, int TP) {
+	return split ? launch_reduce_norm_t<true>(part, KS, T, X, dim, scale, w, eps, Xn, range, st, TP)
+	             : launch_reduce_norm_t<false>(part, KS, T, X, dim, scale, w, eps, Xn, range, st, TP);
 }
 constexpr int REDUCE_NORM_MAX_DIM = 4 * 1024 * 4; // the row in registers: 4 float4 of 1024 threads
 
@@ -564,19 +560,9 @@ int ensure_bufs(yalm_decoder_s *d) {
 	TRY(pf_alloc(d, (void **)&b.lp, cap * 4));
 	TRY(pf_alloc(d, (void **)&b.rope, cap * c.head_dim * 4));
 	TRY(pf_alloc(d, (void **)&b.range, (size_t)(c.n_layers + 1) * RG_N * 4));
-	{ // split-K partials; short prompts: the largest [KS][64][Np] of the layer's GEMMs
-		const int kv_dim = c.n_kv_heads * c.head_dim, TP = SK_MAX_T;
-		const int np_qkv = (int)q_dim + 2 * kv_dim;
-		// (QKV: 2 KS partial slots, the k | v GEMM's)
-		const size_t sz[4] = {
-		    (size_t)2 * std::max(1, sk_pick_ks({{(int)q_dim, c.dim, 1}, {2 * kv_dim, 2 * c.dim, 2}}, TP)) * np_qkv,
-		    (size_t)std::max(1, sk_pick_ks({{c.dim, (int)q_dim, 1}}, TP)) * c.dim,
-		    (size_t)std::max(1, sk_pick_ks({{2 * c.hidden_dim, c.dim, 1}}, TP)) * 2 * c.hidden_dim,
-		    (size_t)std::max(1, sk_pick_ks({{c.dim, c.hidden_dim, 1}}, TP)) * c.dim};
-		b.skp_floats = (size_t)TP * *std::max_element(sz, sz + 4);
-		// K slices of the large tiles: at most 128 MB, which plan_split keeps to
-		const size_t widest = std::max({(size_t)np_qkv, (size_t)c.dim, (size_t)2 * c.hidden_dim});
-		b.skp_floats = std::max(b.skp_floats, std::min((size_t)32 << 20, 16 * (cap + 15) / 16 * 16 * widest));
+	{ // f32 partials of K slices, at most 128 MB: plan_split and plan_stream keep to it
+		const size_t widest = std::max({q_dim + 2 * (size_t)c.n_kv_heads * c.head_dim, (size_t)c.dim, (size_t)2 * c.hidden_dim});
+		b.skp_floats = std::min((size_t)32 << 20, 16 * std::max((cap + 15) / 16 * 16, (size_t)SK_MAX_T) * (widest + 64));
 		TRY(pf_alloc(d, (void **)&b.skp, b.skp_floats * 4));
 	}
 	b.cap = (int)cap;
@@ -650,13 +636,14 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 	const bool qkv1 = f.qkv1 && f.p8 && f.g16[PG_QKV] < 0 && q_dim % 256 == 0 && (2 * kv_dim) % 256 == 0;
 	const int bn_wo = pick_bn(f, PG_WO, T, c.dim, false, false, raw8);
 	const int bn_w2 = pick_bn(f, PG_W2, T, c.dim, false, false, raw8);
-	// short prompts: split-K skinny GEMMs (the 256-row tiles would leave most CUs idle)
-	const int TP = 16 * ((T + 15) / 16);
-	const int ks_qkv = sk_pick_ks({{q_dim, c.dim, 1}, {2 * kv_dim, 2 * c.dim, 2}}, TP);
-	const int ks_wo = sk_pick_ks({{c.dim, q_dim, 1}}, TP);
-	const int ks_glu = sk_pick_ks({{2 * c.hidden_dim, c.dim, 1}}, TP);
-	const int ks_w2 = sk_pick_ks({{c.dim, c.hidden_dim, 1}}, TP);
-	const bool small = T <= SK_MAX_T && !f.no_skinny && !f.split && ks_qkv > 0 && ks_wo > 0 && ks_glu > 0 && ks_w2 > 0;
+	// short prompts: streamed GEMMs (the 256-row tiles would leave most CUs idle)
+	const bool small = T <= SK_MAX_T && !f.no_skinny && !f.split;
+	const int TP = small ? sk_rows(T) : (T + 15) / 16 * 16; // rows of a partial slot
+	const int nstg = pf::StreamCfg<1, 4, pf::BRowsPlain, false>::KSTG;
+	const StreamPlan p_qkv = plan_stream(T, q_dim + 2 * kv_dim, c.dim / nstg, b.skp_floats);
+	const StreamPlan p_wo = plan_stream(T, c.dim, q_dim / nstg, b.skp_floats);
+	const StreamPlan p_glu = plan_stream(T, 2 * c.hidden_dim, c.dim / nstg, b.skp_floats);
+	const StreamPlan p_w2 = plan_stream(T, c.dim, c.hidden_dim / nstg, b.skp_floats);
 	// the split-operand precision form (yalm_set_prefill_precision): every activation operand
 	// [hi | lo] -- the normalised x of all three norms, Q, P (attention.h SPLIT), O and H --
 	// each GEMM over K = 2 x its depth with the B rows wrapping (prefill_gemm.h), so no operand
@@ -676,10 +663,19 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 		if (!fused_norm) { // (rows too wide for the fused kernel's registers)
 			pf::E16Residual e;
 			e.x = b.X, e.ldx = c.dim, e.M = T, e.scale = scale;
-			TRY(launch_skinny_reduce<false>(b.skp, KS, KS, c.dim, T, c.dim, e, st));
+			TRY(launch_skinny_reduce<false>(b.skp, KS, KS, c.dim, T, c.dim, e, st, TP));
 			return w ? launch_rmsnorm(xsplit, f, b.X, w, c.dim, T, c.norm_eps, b.Xn, range, st) : YALM_OK;
 		}
-		return launch_reduce_norm(xsplit, b.skp, KS, T, b.X, c.dim, scale, w, c.norm_eps, b.Xn, range, st);
+		return launch_reduce_norm(xsplit, b.skp, KS, T, b.X, c.dim, scale, w, c.norm_eps, b.Xn, range, st, TP);
+	};
+	// a streamed product: one slice runs the epilogue itself, several leave partials to be reduced
+	auto stream = [&](auto DUALc, auto GLUc, const StreamPlan &p, const uint16_t *A, int lda, int K, const auto &bm, int N,
+	                  int c_split, const auto &e) -> int {
+		constexpr bool DUAL = decltype(DUALc)::value, GLU = decltype(GLUc)::value;
+		if (p.ks == 1)
+			return launch_stream<DUAL, GLU, false>(f, p, A, lda, T, K, K, bm, N, c_split, nullptr, e, st);
+		TRY((launch_stream<DUAL, GLU, false>(f, p, A, lda, T, K, K, bm, N, c_split, b.skp, pf::NoEpi{}, st)));
+		return launch_skinny_reduce<GLU>(b.skp, p.ks, p.ks, N, T, N, e, st, TP);
 	};
 	bool normed = false; // Xn holds this layer's attention input already
 	for (int l = 0; l < c.n_layers; ++l) {
@@ -713,13 +709,10 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 			// QKV + clip + RoPE as two GEMMs: q (K = dim over hi) and k | v from column
 			// q_dim (K = 2 dim over hi | lo, the B rows wrapping at dim)
 			if (small) {
-				const int np = q_dim + 2 * kv_dim;
-				TRY(with_rows(qkv, [&](const auto &bm) -> int {
-					TRY(launch_skinny(f, b.Xn, 2 * c.dim, T, c.dim, c.dim, bm, q_dim, ks_qkv, 0, np, b.skp, st));
-					return launch_skinny(f, b.Xn, 2 * c.dim, T, 2 * c.dim, c.dim, bm, 2 * kv_dim, 2 * ks_qkv, q_dim, np, b.skp,
-					                     st);
+				// one launch: q over hi, k | v over [hi | lo]
+				TRY(with_rows(qkv, [&](const auto &bm) {
+					return stream(std::true_type{}, std::false_type{}, p_qkv, b.Xn, 2 * c.dim, c.dim, bm, q_dim + 2 * kv_dim, q_dim, e);
 				}));
-				TRY(launch_skinny_reduce<false>(b.skp, ks_qkv, 2 * ks_qkv, q_dim, T, np, e, st));
 			} else {
 				const int np = q_dim + 2 * kv_dim;
 				if (split) { // q | k | v all over [hi | lo], Q stored [hi | lo]
@@ -755,10 +748,11 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 								st, split));
 		if (small || s_wo.ks > 1) {
 			TRY(with_rows(one(w.wo, c.dim, raw8), [&](const auto &bm) {
-				return small ? launch_skinny(f, b.O, q_dim, T, q_dim, q_dim, bm, c.dim, ks_wo, 0, c.dim, b.skp, st)
+				return small ? launch_stream<false, false, false>(f, p_wo, b.O, q_dim, T, q_dim, q_dim, bm, c.dim, c.dim, b.skp,
+				                                                  pf::NoEpi{}, st)
 				             : launch_split(f, s_wo, b.O, sp * q_dim, T, sp * q_dim, q_dim, bm, c.dim, 0, 0, b.skp, st);
 			}));
-			TRY(reduce_norm(small ? ks_wo : s_wo.ks, 1.0f, w.rms_ffn, split, rg + RG_XFFN));
+			TRY(reduce_norm(small ? p_wo.ks : s_wo.ks, 1.0f, w.rms_ffn, split, rg + RG_XFFN));
 		} else {
 			pf::E16Residual e;
 			e.x = b.X;
@@ -769,18 +763,13 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 		}
 		const float hscale = ldexpf(1.0f, -he);
 		if (small) {
-			TRY(with_glu(w.w1, w.w3, raw8, [&](const auto &bm) {
-				return launch_skinny(f, b.Xn, c.dim, T, c.dim, c.dim, bm, 2 * c.hidden_dim, ks_glu, 0, 2 * c.hidden_dim, b.skp, st);
-			}));
-			if (c.act == YALM_SILU) {
-				pf::E16Glu<1> e;
+			auto glu = [&](auto e) -> int {
 				e.h = b.H, e.ldh = c.hidden_dim, e.M = T, e.hscale = hscale, e.range = rg + RG_H;
-				TRY(launch_skinny_reduce<true>(b.skp, ks_glu, ks_glu, 2 * c.hidden_dim, T, 2 * c.hidden_dim, e, st));
-			} else {
-				pf::E16Glu<0> e;
-				e.h = b.H, e.ldh = c.hidden_dim, e.M = T, e.hscale = hscale, e.range = rg + RG_H;
-				TRY(launch_skinny_reduce<true>(b.skp, ks_glu, ks_glu, 2 * c.hidden_dim, T, 2 * c.hidden_dim, e, st));
-			}
+				return with_glu(w.w1, w.w3, raw8, [&](const auto &bm) {
+					return stream(std::false_type{}, std::true_type{}, p_glu, b.Xn, c.dim, c.dim, bm, 2 * c.hidden_dim, 2 * c.hidden_dim, e);
+				});
+			};
+			TRY(c.act == YALM_SILU ? glu(pf::E16Glu<1>{}) : glu(pf::E16Glu<0>{}));
 		} else {
 			TRY(c.act == YALM_SILU ? enqueue_glu<1>(d, w, T, hscale, rg + RG_H, raw8)
 								   : enqueue_glu<0>(d, w, T, hscale, rg + RG_H, raw8));
@@ -792,10 +781,10 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 		if (normed) {
 			TRY(with_rows(one(w.w2, c.dim, raw8), [&](const auto &bm) {
 				const int h = c.hidden_dim;
-				return small ? launch_skinny(f, b.H, h, T, h, h, bm, c.dim, ks_w2, 0, c.dim, b.skp, st)
+				return small ? launch_stream<false, false, false>(f, p_w2, b.H, h, T, h, h, bm, c.dim, c.dim, b.skp, pf::NoEpi{}, st)
 				             : launch_split(f, s_w2, b.H, sp * h, T, sp * h, h, bm, c.dim, 0, 0, b.skp, st);
 			}));
-			TRY(reduce_norm(small ? ks_w2 : s_w2.ks, ldexpf(1.0f, he), w_next, last ? split : true, rg + RG_N + RG_XATT));
+			TRY(reduce_norm(small ? p_w2.ks : s_w2.ks, ldexpf(1.0f, he), w_next, last ? split : true, rg + RG_N + RG_XATT));
 		} else {
 			pf::E16Residual e;
 			e.x = b.X;
@@ -952,23 +941,16 @@ extern "C" int yalm_prefill_time(yalm_decoder d, int n, int iters, float *avg_ms
 	return YALM_OK;
 }
 
-// bf16 partials of a few rows (T <= SK_MAX_T): the weight rows streamed once (skinny_gemm_lds_kernel)
-template <class BMAP>
-static int launch_skinny_bf16(const uint16_t *A, int lda, int T, int K, const BMAP &bm, int N, int KS, float *part,
-                              hipStream_t st) {
-	const int mt = (T + 15) / 16, KC = K / KS;
-	auto kern = mt == 1 ? pf::skinny_gemm_lds_kernel<1, BMAP, true> : mt == 2 ? pf::skinny_gemm_lds_kernel<2, BMAP, true>
-	            : mt == 3 ? pf::skinny_gemm_lds_kernel<3, BMAP, true> : pf::skinny_gemm_lds_kernel<4, BMAP, true>;
-	static bool attr[4] = {};
-	if (!attr[mt - 1]) {
-		HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
-		                           32768 + (int)pf::SKL_RING_BYTES));
-		attr[mt - 1] = true;
-	}
-	hipLaunchKernelGGL(kern, dim3((N / pf::SK_ROWS) * KS), dim3(256), (size_t)16 * mt * KC * 2 + pf::SKL_RING_BYTES, st, A,
-	                   lda, T, K, K, bm, N, KC, 0, N, part);
-	HIPCHK(hipGetLastError());
-	return YALM_OK;
+// bf16 products of a few rows (M <= SK_MAX_T): the weight rows streamed once, in one or several K slices
+template <bool GLU, class BMAP, class EPI>
+static int stream_bf16(const PfForms &f, const uint16_t *A, int lda, int M, int K, const BMAP &bm, int N, const EPI &e,
+                       float *part, size_t part_floats, hipStream_t st) {
+	const StreamPlan p = plan_stream(M, N, K / 128, part_floats);
+	const int np = (N + sk_cols(M) - 1) / sk_cols(M) * sk_cols(M);
+	if (p.ks == 1)
+		return launch_stream<false, GLU, true>(f, p, A, lda, M, K, K, bm, N, np, nullptr, e, st);
+	TRY((launch_stream<false, GLU, true>(f, p, A, lda, M, K, K, bm, N, np, part, pf::NoEpi{}, st)));
+	return launch_skinny_reduce<GLU>(part, p.ks, p.ks, np, M, np, e, st, sk_rows(M));
 }
 
 // The layer-list engine's door to the prefill GEMMs (seq.hip; device pointers, asynchronous
@@ -994,14 +976,8 @@ int pf_gemm_bf16(const uint16_t *A, int lda, int M, int K, const uint16_t *W, in
 	e.M = M;
 	e.N = N;
 	e.act = act;
-	if (M <= SK_MAX_T) {
-		const int TP = 16 * ((M + 15) / 16), np = (N + pf::SK_ROWS - 1) / pf::SK_ROWS * pf::SK_ROWS;
-		const int ks = sk_pick_ks({{np, K, 1}}, TP);
-		if (ks > 0 && (size_t)ks * TP * np <= part_floats) {
-			TRY(launch_skinny_bf16(A, lda, M, K, pf::BRowsRagged{W, N}, np, ks, part, st));
-			return launch_skinny_reduce<false>(part, ks, ks, np, M, np, e, st);
-		}
-	}
+	if (M <= SK_MAX_T && K % 128 == 0)
+		return stream_bf16<false>(f, A, lda, M, K, pf::BRowsRagged{W, N}, N, e, part, part_floats, st);
 	const SplitPlan s = plan_split(f, PG_TEST, M, N, K, 0, 0, false, part_floats, ragged);
 	if (s.ks > 1) {
 		TRY((launch_split<pf::BRowsRagged, true>(f, s, A, lda, M, K, K, pf::BRowsRagged{W, N}, s.n, 0, 0, part, st)));
@@ -1028,13 +1004,8 @@ int pf_gemm_glu_bf16(const uint16_t *A, int lda, int M, int K, const uint16_t *W
 	const int N = 2 * hidden;
 	if (!bn)
 		return YALM_ERR_UNSUPPORTED;
-	if (M <= SK_MAX_T) {
-		const int TP = 16 * ((M + 15) / 16), ks = sk_pick_ks({{N, K, 1}}, TP);
-		if (ks > 0 && (size_t)ks * TP * N <= part_floats) {
-			TRY(launch_skinny_bf16(A, lda, M, K, bm, N, ks, part, st));
-			return launch_skinny_reduce<true>(part, ks, ks, N, M, N, e, st);
-		}
-	}
+	if (M <= SK_MAX_T && K % 128 == 0 && N % sk_cols(M) == 0)
+		return stream_bf16<true>(f, A, lda, M, K, bm, N, e, part, part_floats, st);
 	const SplitPlan s = plan_split(f, PG_GLU, M, N, K, 0, 0, true, part_floats);
 	if (s.ks > 1) {
 		TRY((launch_split<pf::BRowsGlu<64>, true>(f, s, A, lda, M, K, K, bm, N, 0, 0, part, st)));

@@ -1,211 +1,172 @@
 // prefill_skinny.h — the prefill's GEMMs for a SHORT prompt (T <= 64 rows: the
 // CLI's prompt hydration, main.cpp:91-97 in the reference, runs T one-token
-// forwards there). At small T the 256-row tiles of prefill_gemm.h leave most CUs
-// idle (Llama-3B Wo / W2, N 3072: 12-16 tiles) and the GEMM is a weight stream, not
-// MFMA work: every weight byte is read once, for T <= 64 rows.
+// forwards there), and the sums of K slices. At small T the 256-row tiles of
+// prefill_gemm.h leave most CUs idle (Llama-3B Wo / W2, N 3072: 12-16 tiles) and the
+// GEMM is a weight stream, not MFMA work: every weight byte is read once, for T <= 64 rows.
 //
-//   skinny_gemm_kernel: split-K. Workgroup = 4 waves x 16 weight rows (64 rows of
-//     B) x KC columns of K; the A rows of its K chunk (T padded to 16 MT) are staged
-//     once in LDS (XOR-swizzled 16-byte chunks), the weight rows stream straight
-//     into registers (lane (row r, group q) reads 16 B at k + 8 q: 16 rows x 64 B per
-//     wave-instruction, U of them in flight) and feed v_mfma_f32_16x16x32_f16 with the
-//     TOKENS as the A operand and the weight rows as B. Each wave leaves its f32
-//     [16 MT][16] partial in part[ks][row][col].
+//   stream_gemm_kernel: a workgroup owns 16 weight rows per wave and a slice of K; weight
+//     rows and A rows (tokens) come through one ring of LDS-DMA stages; the TOKENS are the
+//     MFMA's A operand, the weight rows B. One slice: the epilogue runs in the launch;
+//     several: each leaves f32 partials part[ks][row][col].
 //   skinny_reduce_kernel: per (16 rows x 16 FJ columns) wave block, the KS partials
 //     summed in ks order (deterministic) into the 16x16 MFMA C layout, then the same
 //     epilogue object as the large-tile GEMM (prefill_gemm.h E16*: RoPE + cache
 //     write, residual add, GLU).
-// Columns k >= kb of A wrap to B column k - kb (the split-f16 K / V operand); a K chunk
-// never straddles kb (the host splits the k | v GEMM in 2 KS chunks of the q GEMM's size).
+//   reduce_norm_rows_kernel: the same for a residual product, with the next row norm.
 #pragma once
 
 #include "prefill_gemm.h"
 
 namespace pf {
 
-constexpr int SK_ROWS = 64;    // B rows per workgroup (16 per wave)
-constexpr int SK_U = 8;        // weight loads in flight per lane (8 x 32 k)
-constexpr int SK_KSTEP = 32 * SK_U;
+// C = A · W^T for T <= 16 MT rows. Workgroup = NW waves x 16 weight rows, stages of 128 K columns
+// (ROWB bytes per weight row) in a ring of NS: per stage a wave DMAs its own 16 weight rows and its
+// share of the A rows, all waves read A. One barrier per stage publishes the stage that landed and
+// frees the slot of the one before it, which the next DMA refills.
+//
+// What bounds it is the weight stream: 16 NW ROWB bytes a stage with NS - 1 stages in flight, two
+// workgroups per CU where the ring fits 80 KB (64-96 KB in flight per CU: HBM latency x bandwidth is about
+// 55 KB per CU), else one. A slice may be the whole of K: a gated pair of 448 row blocks is one round of
+// workgroups that never refill their pipeline, and its epilogue needs no partials. (The form before it
+// staged a whole A chunk per workgroup and so cut K into chunks of at most 32 KB of A: at 13 rows, W1 | W3 of
+// Mistral-7B was 1792 workgroups, 52.4 + 4.7 us for 235 MB.)
+//
+// DUAL: columns >= c_split take A = [hi | lo], kb columns apart, against the same weights (the split-f16
+// K / V operand): the weight fragment is read once for both halves.
+//
+// 16-byte chunks are XOR-swizzled on the source side of the DMA so that 16 rows' fragment reads of one
+// chunk column spread over the banks: A (256-byte rows) by row & 15, f16 weights the same, E5M2 (128-byte
+// rows, two per 256 bytes) by (row >> 1) & 7.
+template <int MT, int NW, class BMAP, bool DUAL>
+struct StreamCfg {
+	static constexpr int EB = sizeof(bmap_elt<BMAP>);
+	static constexpr int KSTG = 128, ROWB = KSTG * EB;
+	static constexpr int WB = NW * 16 * ROWB, AB = 16 * MT * KSTG * 2; // stage bytes: weights, one half of A
+	static constexpr int SB = WB + AB * (DUAL ? 2 : 1);
+	static constexpr int FIT2 = 81920 / SB, FIT1 = 163840 / SB;
+	static constexpr int NS = FIT2 >= 3 ? (FIT2 < 6 ? FIT2 : 6) : (FIT1 < 4 ? FIT1 : 4);
+	static constexpr int NWI = ROWB / 64;          // weight DMAs per wave and stage: 16 ROWB bytes, 1 KB each
+	static constexpr int NA = 4 * MT / NW;         // A DMAs per wave, stage and half
+	static constexpr size_t RED = (size_t)NW * MT * 16 * 17 * 4; // the epilogue's sums
+	static constexpr size_t LDS = (size_t)NS * SB > RED ? (size_t)NS * SB : RED;
+	static_assert(NA * NW == 4 * MT && NS >= 2, "shape");
+};
+struct NoEpi {}; // partials
 
-// lds: [16 MT][KC] f16, 16-byte chunk c of row r stored at chunk c ^ (r & 15)
-template <int MT>
-__device__ __forceinline__ half8_t sk_afrag(const uint16_t *lds, int KC, int row, int k) {
-	const int c = (k >> 3) ^ (row & 15);
-	return *(const half8_t *)(lds + (size_t)row * KC + 8 * c);
-}
-
-// A rows [0, TP) x columns [k0, k0 + KC) into LDS, 16-byte chunk c of row r at c ^ (r & 15)
-// (rows past T are zeros). TP * KC <= 16384 f16 (32 KB: the host's K split) = at most
-// SK_AMAX chunks per thread, all loaded before any is stored: one memory round trip.
-// (A loop of load -> LDS store per chunk waited vmcnt(0) per chunk -- and for the weight
-// loads issued before it: 8 serial round trips per workgroup.)
-constexpr int SK_AMAX = 8;
-template <int MT>
-__device__ __forceinline__ void sk_stage_a(uint16_t *as, const uint16_t *__restrict__ A, int lda, int T, int k0,
-                                           int KC) {
-	constexpr int TP = 16 * MT;
-	const int cpr = KC / 8, nch = TP * cpr, tid = threadIdx.x;
-	u32x4_t v[SK_AMAX];
-#pragma unroll
-	for (int u = 0; u < SK_AMAX; ++u) {
-		const int i = min(tid + 256 * u, nch - 1);
-		const int r = i / cpr, c = i % cpr;
-		v[u] = *(const u32x4_t *)(A + (size_t)min(r, T - 1) * lda + k0 + 8 * c);
-	}
-#pragma unroll
-	for (int u = 0; u < SK_AMAX; ++u) {
-		const int i = tid + 256 * u;
-		if (i < nch) {
-			const int r = i / cpr, c = i % cpr;
-			*(u32x4_t *)(as + (size_t)r * KC + 8 * (c ^ (r & 15))) = r < T ? v[u] : u32x4_t{0u, 0u, 0u, 0u};
-		}
-	}
-}
-
-// C[:, c0 .. c0 + N) partials over K columns of A (row stride lda; B rows kb wide,
-// wrapping), K chunks of KC: part[ks][row][c] with row stride Np (c absolute).
-template <int MT, class BMAP>
-__global__ __launch_bounds__(256) void skinny_gemm_kernel(const uint16_t *__restrict__ A, int lda, int T, int K,
-                                                          int kb, BMAP bm, int N, int KC, int c0, int Np,
-                                                          float *__restrict__ part) {
-	extern __shared__ __attribute__((aligned(16))) uint16_t as[];
-	const int nblk = N / SK_ROWS;
-	const int nb = blockIdx.x % nblk, ks = blockIdx.x / nblk;
-	const int k0 = ks * KC;
-	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-	constexpr int TP = 16 * MT;
-	// ---- this wave's 16 weight rows (through the row policy: plain / QKV segments / GLU)
-	const int cb = c0 + nb * SK_ROWS;           // the workgroup's first B row index (output column)
-	const int col = cb + 16 * wave;              // the wave's
-	const int kw0 = k0 < kb ? k0 : k0 - kb;      // B wrap (a K chunk never straddles kb)
-	// row policy: tile base = first output column (plain) or first hidden column (GLU:
-	// 64 B rows = 32 W1 rows then the same 32 W3 rows, BRowsGlu<64>)
-	const uint16_t *wrow =
-	    bm.row(cb / BMAP::COLS_PER_TILE_DIV, 16 * wave + (lane & 15), kb) + kw0 + 8 * (lane >> 4);
-	// ---- the weight stream: a ring of SK_U 16-byte loads per lane (32 K columns each),
-	// the first SK_U issued before the A chunk is staged; every consumed slot is refilled
-	// SK_U steps ahead, unconditionally (past the chunk it re-reads step 0, an L2 hit:
-	// a conditional refill makes hipcc drain vmcnt to 0 before every load). Round 4's
-	// first cut loaded SK_U steps, waited, computed, loaded the next SK_U: one full
-	// memory latency per 256 K columns (Mistral T = 1 prefill: 3.8 TB/s).
-	const int nst = KC / 32;
-	half8_t b[SK_U];
-#pragma unroll
-	for (int u = 0; u < SK_U; ++u)
-		b[u] = __builtin_bit_cast(half8_t, load_nt16(wrow + 32 * (u < nst ? u : 0)));
-	sk_stage_a<MT>(as, A, lda, T, k0, KC);
-	__syncthreads();
-	f32x4_t acc[MT];
-#pragma unroll
-	for (int m = 0; m < MT; ++m)
-		acc[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-	for (int j0 = 0; j0 < nst; j0 += SK_U) {
-#pragma unroll
-		for (int u = 0; u < SK_U; ++u) {
-			const int j = j0 + u;
-			if (j < nst) {
-#pragma unroll
-				for (int m = 0; m < MT; ++m) {
-					const half8_t a = sk_afrag<MT>(as, KC, 16 * m + (lane & 15), 32 * j + 8 * (lane >> 4));
-					acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[u], acc[m], 0, 0, 0);
-				}
-			}
-			b[u] = __builtin_bit_cast(half8_t, load_nt16(wrow + 32 * (j + SK_U < nst ? j + SK_U : 0)));
-		}
-	}
-	// ---- partial: element r of acc[m] is row 16 m + 4 (lane >> 4) + r, column col + (lane & 15)
-	float *pp = part + (size_t)ks * TP * Np;
-#pragma unroll
-	for (int m = 0; m < MT; ++m)
-#pragma unroll
-		for (int r = 0; r < 4; ++r)
-			pp[(size_t)(16 * m + crow16(r, lane)) * Np + col + (lane & 15)] = acc[m][r];
-}
-
-// The same partials with the weight rows staged through LDS by LDS-DMA, so every
-// wave-instruction reads 4 rows x 256 contiguous bytes (skinny_gemm_kernel's register
-// loads read 16 rows x 64 B per instruction: half cache lines, 16 DRAM rows at once).
-// Each wave owns its 16 weight rows in a 3-stage ring of 256-byte-wide stages (4 KB per
-// wave per stage): no workgroup barrier in the loop, one counted vmcnt per stage. The
-// 16-byte chunks of a row are XOR-swizzled by the row (source side of the DMA) so the
-// MFMA B-fragment reads (16 rows x one chunk) spread over the banks. LDS: the A chunk
-// (<= 32 KB) + 48 KB of ring: two workgroups per CU.
-constexpr int SKL_ROWB = 256;                  // bytes per weight row and stage: 128 f16 / bf16 columns, 256 E5M2
-constexpr int SKL_NS = 3;                      // ring stages
-constexpr int SKL_STAGE = SK_ROWS * SKL_ROWB;  // bytes per stage (16 KB)
-constexpr size_t SKL_RING_BYTES = (size_t)SKL_NS * SKL_STAGE;
-
-template <int MT, class BMAP, bool BF = false> // BF: bf16 operands (the layer-list engine's products)
-__global__ __launch_bounds__(256) void skinny_gemm_lds_kernel(const uint16_t *__restrict__ A, int lda, int T, int K,
-                                                              int kb, BMAP bm, int N, int KC, int c0, int Np,
-                                                              float *__restrict__ part) {
-	extern __shared__ __attribute__((aligned(16))) uint16_t sm[];
-	constexpr int TP = 16 * MT;
+template <int MT, int NW, class BMAP, bool DUAL, bool GLU, class EPI, bool BF>
+__global__ __launch_bounds__(64 * NW) void stream_gemm_kernel(const uint16_t *__restrict__ A, int lda, int T, int nst_all,
+                                                              int kb, BMAP bm, int nblk, int nsc, int c_split, int Np,
+                                                              float *__restrict__ part, EPI epi, int drain) {
+	using C = StreamCfg<MT, NW, BMAP, DUAL>;
 	using elt = bmap_elt<BMAP>;
-	constexpr int EB = sizeof(elt), KSTG = SKL_ROWB / EB; // columns per stage
-	uint16_t *const as = sm;                              // [TP][KC], swizzled as skinny_gemm_kernel
-	char *const ring = (char *)(sm + (size_t)TP * KC);    // [SKL_NS][64 rows][SKL_ROWB]
-	const int nblk = N / SK_ROWS;
+	constexpr int EB = C::EB, NS = C::NS, CW = C::NWI + C::NA;
+	extern __shared__ __attribute__((aligned(16))) char smem_c[];
 	const int nb = blockIdx.x % nblk, ks = blockIdx.x / nblk;
-	const int k0 = ks * KC;
-	const int tid = threadIdx.x, lane = tid & 63;
-	const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-	const int cb = c0 + nb * SK_ROWS;      // the workgroup's first B row (output column)
-	const int col = cb + 16 * wave;        // the wave's
-	const int kw0 = k0 < kb ? k0 : k0 - kb; // B wrap (a K chunk never straddles kb)
-	const int nst = KC / KSTG;
-	// DMA geometry: instruction i of a stage covers the wave's rows 4 i .. 4 i + 3, lane
-	// l row 4 i + (l >> 4), LDS slot l & 15 <- source chunk (l & 15) ^ row
-	const elt *src[4];
+	const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const int n = lane & 15, q = lane >> 4;
+	const int cb = nb * 16 * NW;        // the workgroup's first B row (output column)
+	const bool dual = DUAL && cb >= c_split;
+	const int st0 = ks * nsc, nst = min(nsc, nst_all - st0);
+	const int k0 = st0 * C::KSTG;
+	const elt *wsrc[C::NWI];
 #pragma unroll
-	for (int i = 0; i < 4; ++i) {
-		const int rr = 4 * i + (lane >> 4);
-		src[i] = bm.row(cb / BMAP::COLS_PER_TILE_DIV, 16 * wave + rr, kb) + kw0 + 16 / EB * ((lane & 15) ^ rr);
+	for (int i = 0; i < C::NWI; ++i) {
+		const int rr = EB == 2 ? 4 * i + (lane >> 4) : 8 * i + (lane >> 3);
+		const int ch = EB == 2 ? (lane & 15) ^ rr : (lane & 7) ^ ((rr >> 1) & 7);
+		wsrc[i] = bm.row(cb / BMAP::COLS_PER_TILE_DIV, 16 * wave + rr, kb) + k0 + 16 / EB * ch;
 	}
-	char *const wring = ring + wave * 16 * SKL_ROWB; // this wave's rows in every stage
-	auto issue = [&](int st) { // stage st (clamped: past the chunk it re-reads the last stage, an L2 hit)
-		const int sc = st < nst ? st : nst - 1;
-		char *dst = wring + (st % SKL_NS) * SKL_STAGE;
+	const uint16_t *asrc[C::NA];
 #pragma unroll
-		for (int i = 0; i < 4; ++i)
-			__builtin_amdgcn_global_load_lds((const void *)(src[i] + sc * KSTG),
-			                                 (YALM_LDS void *)(dst + 4 * i * SKL_ROWB), 16, 0, 0);
+	for (int i = 0; i < C::NA; ++i) { // rows past T repeat the last one (their results are dropped)
+		const int r = 4 * (wave * C::NA + i) + (lane >> 4);
+		asrc[i] = A + (size_t)min(r, T - 1) * lda + k0 + 8 * ((lane & 15) ^ (r & 15));
+	}
+	// the workgroups walk the slice's columns from different stages on: rows are a power of two apart, so
+	// workgroups in step would all read the same HBM channels
+	const int rot = nb % nst;
+	auto issue = [&](int st) {
+		char *const base = smem_c + (st % NS) * C::SB;
+		st = st + rot < nst ? st + rot : st + rot - nst;
+#pragma unroll
+		for (int i = 0; i < C::NWI; ++i)
+			__builtin_amdgcn_global_load_lds((const void *)(wsrc[i] + st * C::KSTG),
+			                                 (YALM_LDS void *)(base + (wave * C::NWI + i) * 1024), 16, 0, 0);
+#pragma unroll
+		for (int i = 0; i < C::NA; ++i)
+			__builtin_amdgcn_global_load_lds((const void *)(asrc[i] + st * C::KSTG),
+			                                 (YALM_LDS void *)(base + C::WB + (wave * C::NA + i) * 1024), 16, 0, 0);
+		if (DUAL && dual)
+#pragma unroll
+			for (int i = 0; i < C::NA; ++i)
+				__builtin_amdgcn_global_load_lds((const void *)(asrc[i] + kb + st * C::KSTG),
+				                                 (YALM_LDS void *)(base + C::WB + C::AB + (wave * C::NA + i) * 1024), 16, 0, 0);
 	};
-	issue(0);
-	issue(1);
-	sk_stage_a<MT>(as, A, lda, T, k0, KC);
-	__syncthreads();
+	for (int st = 0; st < min(NS - 1, nst); ++st)
+		issue(st);
 	f32x4_t acc[MT];
 #pragma unroll
 	for (int m = 0; m < MT; ++m)
 		acc[m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-	const int n = lane & 15, q = lane >> 4;
 	for (int st = 0; st < nst; ++st) {
-		asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // stage st - 1's B reads are done...
-		issue(st + 2); // ...before its slot is re-staged
-		asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); // stage st landed (2 stages x 4 behind it)
-		const char *bst = wring + (st % SKL_NS) * SKL_STAGE + n * SKL_ROWB;
+		// stage st has landed: the NS - 2 stages after it stay in flight (near the slice's end: drain)
+		if (st + NS - 2 >= nst || drain)
+			asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+		else if (DUAL && dual)
+			asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * (CW + C::NA)) : "memory");
+		else
+			asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * CW) : "memory");
+		raw_barrier(); // ... every wave's share of it, and everyone is done reading stage st - 1
+		if (st + NS - 1 < nst)
+			issue(st + NS - 1);
+		const char *const base = smem_c + (st % NS) * C::SB;
+		const char *const bst = base + wave * 16 * C::ROWB + n * C::ROWB;
+		const uint16_t *const as = (const uint16_t *)(base + C::WB);
 #pragma unroll
-		for (int j = 0; j < KSTG / 32; ++j) {
+		for (int j = 0; j < 4; ++j) {
 			half8_t b;
 			if constexpr (EB == 2)
 				b = *(const half8_t *)(bst + 16 * ((4 * j + q) ^ n));
 			else // E5M2: 8 of a chunk's 16 columns
-				b = e5m2x8(*(const uint2 *)(bst + 16 * ((2 * j + (q >> 1)) ^ n) + 8 * (q & 1)));
+				b = e5m2x8(*(const uint2 *)(bst + 16 * ((2 * j + (q >> 1)) ^ ((n >> 1) & 7)) + 8 * (q & 1)));
 #pragma unroll
 			for (int m = 0; m < MT; ++m) {
-				const half8_t a = sk_afrag<MT>(as, KC, 16 * m + n, st * KSTG + 32 * j + 8 * q);
-				acc[m] = mfma16<BF>(a, b, acc[m]);
+				const uint16_t *const ap = as + (16 * m + n) * C::KSTG + 8 * ((4 * j + q) ^ n);
+				acc[m] = mfma16<BF>(*(const half8_t *)ap, b, acc[m]);
+				if (DUAL && dual)
+					acc[m] = mfma16<BF>(*(const half8_t *)(ap + C::AB / 2), b, acc[m]);
 			}
 		}
 	}
-	asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the clamped tail stages, before the wave exits
-	float *pp = part + (size_t)ks * TP * Np;
+	if constexpr (std::is_same<EPI, NoEpi>::value) {
+		float *pp = part + (size_t)ks * 16 * MT * Np + cb + 16 * wave + n;
 #pragma unroll
-	for (int m = 0; m < MT; ++m)
+		for (int m = 0; m < MT; ++m)
 #pragma unroll
-		for (int r = 0; r < 4; ++r)
-			pp[(size_t)(16 * m + crow16(r, lane)) * Np + col + n] = acc[m][r];
+			for (int r = 0; r < 4; ++r)
+				pp[(size_t)(16 * m + crow16(r, lane)) * Np] = acc[m][r];
+	} else {
+		// the waves' columns meet in LDS: a wave then runs the epilogue of one 16-row tile x 64 columns
+		raw_barrier();
+		float *const red = (float *)smem_c;
+#pragma unroll
+		for (int m = 0; m < MT; ++m)
+#pragma unroll
+			for (int r = 0; r < 4; ++r)
+				red[((wave * MT + m) * 16 + crow16(r, lane)) * 17 + n] = acc[m][r];
+		raw_barrier();
+		for (int task = wave; task < MT * (NW / 4); task += NW) {
+			const int m = task % MT, g = task / MT;
+			if (16 * m >= T)
+				continue;
+			f32x4_t a2[1][4];
+#pragma unroll
+			for (int j = 0; j < 4; ++j)
+#pragma unroll
+				for (int r = 0; r < 4; ++r)
+					a2[0][j][r] = red[(((4 * g + j) * MT + m) * 16 + crow16(r, lane)) * 17 + n];
+			epi.template apply<1, 4>(a2, 16 * m, GLU ? cb / 2 + 32 * g : cb + 64 * g, lane, 0, 1);
+		}
+	}
 }
 
 // One wave per (16 rows, 16 FJ columns) block of C: the KS partials summed

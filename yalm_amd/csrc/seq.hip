@@ -67,7 +67,7 @@ struct yalm_seq_s {
 	int ldz = 0;
 	float *inv_freq = nullptr;
 	uint16_t *a16 = nullptr;     // [cap][bw] bf16 copy of a product's activations (large-tile GEMM operand)
-	float *gpart = nullptr;      // f32 partials of those products' K slices (at most 128 MB)
+	float *gpart = nullptr;      // f32 partials of those products' K slices (at most 32 MB)
 	size_t gpart_floats = 0;
 	int *tok = nullptr, *want = nullptr;
 	float *logits = nullptr;     // [LOGIT_ROWS][vocab]
@@ -541,7 +541,7 @@ static int create_seq(const yalm_seq_config *config, const yalm_seq_weights *w, 
 		size_t widest = std::max({bw, (size_t)zw, (size_t)c.width});
 		for (const yalm_seq_layer &l : q->L)
 			widest = std::max({widest, (size_t)2 * l.ff, (size_t)2 * l.shared_ff});
-		q->gpart_floats = std::min((size_t)32 << 20, 16 * (cap + 15) / 16 * 16 * (widest + 256));
+		q->gpart_floats = std::min((size_t)8 << 20, 16 * std::max((cap + 15) / 16 * 16, (size_t)64) * (widest + 256));
 		STRY(sallocT(q, &q->gpart, q->gpart_floats));
 	}
 	STRY(sallocT(q, &q->tok, cap + 1));
