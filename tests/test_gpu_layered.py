@@ -137,6 +137,51 @@ PORTIONS = [
 ]
 
 
+# block, head and rank sizes at the limits of the few-token kernels (128-channel recurrence blocks and the smallest,
+# 16; a latent rank of 256 and one that is no multiple of 8; value heads wider than key heads; 4 of 16 experts)
+FEW = C.config([
+    ("rglru", C.rglru(width=256, blocks=2, conv=4), C.moe(ff=32, experts=16, top=4, groups=4, keep=2)),
+    ("latent_attention", C.latent(heads=5, dim=32, vdim=32, kv_rank=256, q_rank=64, scale=0.18), C.dense(ff=96)),
+    ("delta", C.delta(heads=4, kv_heads=2, dim=16, vdim=160, conv=1), C.moe(ff=16, experts=5, top=5, groups=1, keep=1)),
+    ("rglru", C.rglru(width=48, blocks=3, conv=2), None),
+    ("latent_attention", C.latent(heads=3, dim=24, vdim=16, kv_rank=52, q_rank=32, scale=0.2), C.dense(ff=40)),
+    ("delta", C.delta(heads=2, kv_heads=2, dim=256, vdim=8, conv=16), None),
+], width=128, vocab=211)
+
+
+@pytest.mark.parametrize("portions", [[1] * 40, [8, 1, 7, 2, 6, 3, 5, 4, 8, 8], [15, 1, 1, 15, 8, 40, 1, 8]],
+                         ids=["ones", "few", "across"])
+def test_few_token_kernels(rt, portions):
+    """Steps of 1 to 8 tokens, across the 16-key tiles of the split attention and between long portions."""
+    from yalm_amd import models as M
+
+    model, dec, w = build(rt, FEW, M.F32, seed=12, max_tokens=100)
+    try:
+        tok = C.tokens(FEW, sum(portions), 4)
+        got = run_portions(dec, tok, portions)
+        assert close_enough(got, R.forward(FEW, w, tok), "f32")
+    finally:
+        dec.close()
+        model.close()
+
+
+@pytest.mark.parametrize("n", [9, 16, 17, 32, 33, 64, 65, 130, 255])
+def test_few_row_products_bf16(rt, n):
+    """Products of 9 to 255 rows on the prefill unit: streamed in one or several K slices, large tiles in slices."""
+    from yalm_amd import models as M
+
+    cfg = C.config([("rglru", C.rglru(width=256, blocks=4, conv=4), C.dense(ff=1024)),
+                    ("delta", C.delta(heads=2, kv_heads=1, dim=64, vdim=64, conv=3), C.dense(ff=512))], width=512, vocab=391)
+    model, dec, w = build(rt, cfg, M.BF16, seed=3)
+    try:
+        tok = C.tokens(cfg, n, 5)
+        got = dec.step(tok, list(range(n)))
+        assert close_enough(got, R.forward(cfg, w, tok), "bf16")
+    finally:
+        dec.close()
+        model.close()
+
+
 @pytest.mark.parametrize("cfg", [C.MIXED, C.ODD], ids=["mixed", "odd"])
 @pytest.mark.parametrize("sizes", PORTIONS, ids=[str(i) for i in range(len(PORTIONS))])
 def test_portions_of_any_size(rt, cfg, sizes):

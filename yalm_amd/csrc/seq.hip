@@ -561,7 +561,7 @@ static int create_seq(const yalm_seq_config *config, const yalm_seq_weights *w, 
 				max_h = std::max(max_h, l.heads);
 				max_rank = std::max(max_rank, l.kv_rank);
 			}
-		q->att_splits = std::max(1, std::min(32, cdiv(c.max_tokens, 2 * ATT_KT)));
+		q->att_splits = std::max(1, std::min(64, cdiv(c.max_tokens, ATS_KT)));
 		size_t part = (size_t)(4 * ATT_BR + GEMV_MAX_M * max_h) * q->att_splits * (att_rank4(max_rank) + 4);
 		// attn: the keys a single token can see, split so that a workgroup walks one tile (up to 64 splits)
 		q->attn_splits.assign(q->L.size(), 1);
@@ -781,7 +781,8 @@ static GemmArgs plain(const float *A, int lda, const void *W, int ldw, float *C,
 template <class CT>
 static int attn_t(Seq *q, const float *Qa, const void *cache, int rank, int H, int n, float scale, float *ctx) {
 	const int NR = n * H;
-	if (sizeof(CT) == 2 && NR > 4 * ATT_BR) { // portions over a bf16 cache: the MFMA form
+	const bool few = NR <= 4 * ATT_BR || n <= GEMV_MAX_M;
+	if (sizeof(CT) == 2 && !few) { // portions over a bf16 cache: the MFMA form
 		const dim3 gm(cdiv(NR, ATM_BR));
 		const int ks = cdiv(rank, 32);
 #define ATM_LAUNCH(KS)                                                                                                 \
@@ -795,20 +796,29 @@ static int attn_t(Seq *q, const float *Qa, const void *cache, int rank, int H, i
 		HIPCHK(hipGetLastError());
 		return YALM_OK;
 	}
-	// few rows (single tokens, short portions): the visible keys are split over workgroups
-	const int S = NR <= 4 * ATT_BR ? q->att_splits : 1;
-	const dim3 g(cdiv(NR, ATT_BR), S);
-	const size_t lds = att_lds_bytes(rank);
 	const int na = cdiv(att_rank4(rank), 64);
+	// few rows (single tokens, short portions): the visible keys are split over workgroups
+	if (few) {
+		const dim3 gs(cdiv(NR, ATT_BR), q->att_splits);
+#define ATS_LAUNCH(NA)                                                                                                 \
+	seq_latent_split_kernel<CT, NA><<<gs, SEQ_THREADS, ats_lds_bytes(rank), q->stream>>>(Qa, (const CT *)cache, rank, H, NR, \
+	                                                                                    scale, q->st, q->att_part)
+		if (na <= 1) ATS_LAUNCH(1);
+		else if (na <= 2) ATS_LAUNCH(2);
+		else ATS_LAUNCH(4);
+#undef ATS_LAUNCH
+		seq_latent_merge_kernel<<<NR, SEQ_THREADS, 0, q->stream>>>(q->att_part, q->att_splits, rank, ctx);
+		HIPCHK(hipGetLastError());
+		return YALM_OK;
+	}
+	const dim3 g(cdiv(NR, ATT_BR));
+	const size_t lds = att_lds_bytes(rank);
 #define ATT_LAUNCH(NA)                                                                                                 \
-	seq_latent_attn_kernel<CT, NA><<<g, SEQ_THREADS, lds, q->stream>>>(Qa, (const CT *)cache, rank, H, NR, scale, q->st, ctx, \
-	                                                                  q->att_part)
+	seq_latent_attn_kernel<CT, NA><<<g, SEQ_THREADS, lds, q->stream>>>(Qa, (const CT *)cache, rank, H, NR, scale, q->st, ctx)
 	if (na <= 1) ATT_LAUNCH(1);
 	else if (na <= 2) ATT_LAUNCH(2);
 	else ATT_LAUNCH(4);
 #undef ATT_LAUNCH
-	if (S > 1)
-		seq_latent_merge_kernel<<<NR, SEQ_THREADS, 0, q->stream>>>(q->att_part, S, rank, ctx);
 	HIPCHK(hipGetLastError());
 	return YALM_OK;
 }
@@ -874,6 +884,12 @@ static int mixer_rglru(Seq *q, int li, int n) {
 		GemmArgs a = plain(q->In, c.width, l.w_in, c.width, q->Z, 2 * W, n, 2 * W, c.width);
 		a.bias = l.in_bias;
 		TRY(gemm(q, a));
+	}
+	if (n <= SEQ_CONV_STEP_T && bs <= 128 && bs % 16 == 0 && ((size_t)l.gate_a | (size_t)l.gate_i) % 16 == 0) { // all of it in one launch
+		seq_rglru_step_kernel<<<l.blocks, 1024, 0, q->stream>>>(q->Z, 2 * W, W, bs, l.conv, l.conv_w, l.conv_b, q->conv[li], l.gate_a,
+		                                                        l.gate_a_b, l.gate_i, l.gate_i_b, l.lam, q->S[li], so, n);
+		HIPCHK(hipGetLastError());
+		return gemm(q, plain(so, W, l.w_o, W, q->Yout, c.width, n, c.width, W));
 	}
 	TRY(conv_launch(q, q->Z, 2 * W, W, W, l.conv, l.conv_w, l.conv_b, 0, q->conv[li], u, n));
 	{ // both block-diagonal gates in f32, one launch: batches [0, blocks) recurrence gate, the rest input gate
@@ -945,6 +961,9 @@ static int delta_launch(Seq *q, const float *qkv, int ldq, int qo, int ko, int v
 	return YALM_OK;
 }
 
+// seq_delta_out_kernel: few tokens share their heads over workgroups (one of 16 heads: 6.2 us for one token)
+static dim3 out_grid(int n, int H) { return dim3(n, n <= 64 ? cdiv(H, SEQ_THREADS / 64) : 1); }
+
 static int mixer_delta(Seq *q, int li, int n) {
 	const yalm_seq_layer &l = q->L[li];
 	const yalm_seq_config &c = q->c;
@@ -955,11 +974,17 @@ static int mixer_delta(Seq *q, int li, int n) {
 	// one decay per head and key channel: its inputs, then the decays, follow the [n][2 H] factors
 	float *gv = l.decay_rank > 0 ? bg + (size_t)n * 2 * H : nullptr;
 	TRY(gemm(q, plain(q->In, c.width, l.w_in, c.width, q->Z, zin, n, zin, c.width)));
-	TRY(conv_launch(q, q->Z, zin, 0, cc, l.conv, l.conv_w, nullptr, 1, q->conv[li], qkv, n));
-	if (gv) // the low-rank decay's second factor
-		TRY(gemm(q, plain(q->Z + acol, zin, l.w_a2, l.decay_rank, gv, H * D, n, H * D, l.decay_rank)));
-	seq_delta_prep_kernel<<<n, SEQ_THREADS, 0, q->stream>>>(qkv, cc, KH, D, q->Z, zin, bcol, acol, H, l.a_log, l.dt_bias,
-	                                                        bg, gv);
+	if (!gv && n <= SEQ_CONV_STEP_T && D <= SEQ_THREADS && V <= SEQ_THREADS) { // convolution and preparation in one launch
+		seq_delta_front_kernel<<<2 * KH + H, SEQ_THREADS, 0, q->stream>>>(q->Z, zin, KH, D, H, V, l.conv, l.conv_w, q->conv[li],
+		                                                                  bcol, acol, l.a_log, l.dt_bias, qkv, cc, bg, n);
+	} else {
+		TRY(conv_launch(q, q->Z, zin, 0, cc, l.conv, l.conv_w, nullptr, 1, q->conv[li], qkv, n));
+		if (gv) // the low-rank decay's second factor
+			TRY(gemm(q, plain(q->Z + acol, zin, l.w_a2, l.decay_rank, gv, H * D, n, H * D, l.decay_rank)));
+		const dim3 pg(n, n <= 64 ? cdiv(2 * KH, SEQ_THREADS / 64) : 1); // few tokens: their heads over workgroups
+		seq_delta_prep_kernel<<<pg, SEQ_THREADS, 0, q->stream>>>(qkv, cc, KH, D, q->Z, zin, bcol, acol, H, l.a_log, l.dt_bias, bg,
+		                                                         gv);
+	}
 	HIPCHK(hipGetLastError());
 	const float *gl = q->Z;
 	int ldg = zin, gc = gcol;
@@ -970,7 +995,7 @@ static int mixer_delta(Seq *q, int li, int n) {
 		gc = 0;
 	}
 	TRY(delta_launch(q, qkv, cc, 0, CQ, 2 * CQ, KH, D, H, V, bg, gv, nullptr, q->S[li], o, n, WALK_DELTA));
-	seq_delta_out_kernel<<<n, SEQ_THREADS, 0, q->stream>>>(o, H, V, l.out_norm, c.norm_eps, gl, ldg, gc, on,
+	seq_delta_out_kernel<<<out_grid(n, H), SEQ_THREADS, 0, q->stream>>>(o, H, V, l.out_norm, c.norm_eps, gl, ldg, gc, on,
 	                                                       l.gate_act == YALM_GATE_SIGMOID);
 	HIPCHK(hipGetLastError());
 	return gemm(q, plain(on, CV, l.w_o, CV, q->Yout, c.width, n, c.width, CV));
@@ -1020,7 +1045,7 @@ static int mixer_memory(Seq *q, int li, int n) {
 		mg.cap = 0.0f;
 	}
 	TRY(delta_launch(q, Z, ldz, 0, H * D, 2 * H * D, H, D, H, V, nullptr, nullptr, nullptr, q->S[li], o, n, WALK_MEMORY, mg));
-	seq_delta_out_kernel<<<n, SEQ_THREADS, 0, q->stream>>>(o, H, V, l.out_norm, c.norm_eps, Z, ldz, gcol, on, 1, V, 1);
+	seq_delta_out_kernel<<<out_grid(n, H), SEQ_THREADS, 0, q->stream>>>(o, H, V, l.out_norm, c.norm_eps, Z, ldz, gcol, on, 1, V, 1);
 	HIPCHK(hipGetLastError());
 	return gemm(q, plain(on, HV, l.w_o, HV, q->Yout, c.width, n, c.width, HV));
 }
@@ -1043,7 +1068,7 @@ static int mixer_gla(Seq *q, int li, int n) {
 	MemGates mg{};
 	mg.scale = 1.0f / std::sqrt((float)D);
 	TRY(delta_launch(q, q->Z, zin, 0, HD, 2 * HD, H, D, H, V, nullptr, gv, nullptr, q->S[li], o, n, WALK_GLA, mg));
-	seq_delta_out_kernel<<<n, SEQ_THREADS, 0, q->stream>>>(o, H, V, l.out_norm, c.norm_eps, q->Z, zin, gcol, on,
+	seq_delta_out_kernel<<<out_grid(n, H), SEQ_THREADS, 0, q->stream>>>(o, H, V, l.out_norm, c.norm_eps, q->Z, zin, gcol, on,
 	                                                       l.gate_act == YALM_GATE_SIGMOID);
 	HIPCHK(hipGetLastError());
 	return gemm(q, plain(on, HV, l.w_o, HV, q->Yout, c.width, n, c.width, HV));
@@ -1464,7 +1489,8 @@ static int ff_moe(Seq *q, int li, int n, const PostNorm *pn = nullptr) {
 	const int E = l.experts, ER = E + l.identity, top = l.top, ff = l.ff, slots = n * top;
 	float *hx = q->B[0], *yx = q->B[1], *hs = q->B[2], *ys = q->B[3];
 	// a choice that is one wave's work: more waves for the logits
-	const bool one_wave = l.router_kind == YALM_ROUTER_SOFTMAX_NORMED || l.router_kind == YALM_ROUTER_SIGMOID_TOP;
+	const bool one_wave = l.router_kind == YALM_ROUTER_SOFTMAX_TOP || l.router_kind == YALM_ROUTER_SOFTMAX_NORMED ||
+	                      l.router_kind == YALM_ROUTER_SIGMOID_TOP;
 	auto router = one_wave ? seq_router_kernel<1024> : seq_router_kernel<SEQ_THREADS>;
 	const int rth = one_wave ? 1024 : SEQ_THREADS;
 	size_t lds = (2 * ER + l.groups) * sizeof(float);
@@ -1616,12 +1642,24 @@ static int post_close(Seq *q, const float *wb, int n, const yalm_seq_layer *moe)
 // moe: the layer's routed experts feed the norm (their combine happens inside it) instead of Y
 static int add_norm(Seq *q, const float *wb, const float *w_next, int n, const yalm_seq_layer *moe) {
 	const int w = q->c.width;
-	if (!moe && w <= 16 * SEQ_THREADS) { // the row in registers
-#define AN_LAUNCH(E)                                                                                                   \
-	seq_add_norm_reg_kernel<E><<<n, SEQ_THREADS, 0, q->stream>>>(q->X, q->Y, wb, q->c.norm_eps, w, w_next, q->Hn, q->nk, q->c.residual_scale)
-		if (w <= 4 * SEQ_THREADS) AN_LAUNCH(4);
-		else if (w <= 8 * SEQ_THREADS) AN_LAUNCH(8);
-		else AN_LAUNCH(16);
+	if (w <= 16 * SEQ_THREADS) { // the row in registers
+		Combine cb;
+		if (moe)
+			cb = {q->B[1], combine_wt(q, *moe), moe->top, moe->shared_ff > 0 ? q->B[3] : nullptr,
+			      moe->shared_ff > 0 && moe->shared_sg ? q->sgate : nullptr, q->idx, moe->experts, moe->identity > 0 ? q->In : nullptr};
+#define AN_LAUNCH(E, C)                                                                                                \
+	seq_add_norm_reg_kernel<E, C><<<n, SEQ_THREADS, 0, q->stream>>>(q->X, q->Y, wb, q->c.norm_eps, w, w_next, q->Hn, q->nk, \
+	                                                                q->c.residual_scale, cb)
+		if (w <= 4 * SEQ_THREADS) {
+			if (moe) AN_LAUNCH(4, true);
+			else AN_LAUNCH(4, false);
+		} else if (w <= 8 * SEQ_THREADS) {
+			if (moe) AN_LAUNCH(8, true);
+			else AN_LAUNCH(8, false);
+		} else {
+			if (moe) AN_LAUNCH(16, true);
+			else AN_LAUNCH(16, false);
+		}
 #undef AN_LAUNCH
 	} else {
 		seq_add_norm_kernel<<<n, SEQ_THREADS, w * sizeof(float), q->stream>>>(
@@ -1665,7 +1703,23 @@ static int enqueue_portion(Seq *q, const int *tokens_dev, int n) {
 		bg = Bigram{q->bigram, c.bigram_buckets, c.bigram_mul_prev, c.bigram_mul_cur, q->prev};
 	// no row statistics: elementwise (in the greedy loop the one workgroup that also passes the previous token on)
 	const int eb = q->nk == NK_TANH && !q->embed_norm && (tokens_dev || !bg.table) ? cdiv(c.width, SEQ_THREADS) : 1;
-	if (c.weight_dtype == YALM_F32)
+	if (q->nk != NK_TANH && !q->embed_norm && !bg.table && c.width <= 16 * SEQ_THREADS && c.width % 2 == 0) { // the row in registers
+#define EM_ARGS                                                                                                        \
+	q->st, tokens_dev, q->embed, q->inv_freq, c.width, c.vocab, c.embed_scale, q->X, first_norm, c.norm_eps, q->Hn, q->nk,  \
+	    q->L[0].pre_add, first_norm2, q->Hn2
+#define EM_LAUNCH(P)                                                                                                   \
+	do {                                                                                                               \
+		if (c.weight_dtype == YALM_F32)                                                                                \
+			seq_embed_reg_kernel<WF32, P><<<n, SEQ_THREADS, 0, q->stream>>>(EM_ARGS);                                  \
+		else                                                                                                           \
+			seq_embed_reg_kernel<WBF16, P><<<n, SEQ_THREADS, 0, q->stream>>>(EM_ARGS);                                 \
+	} while (0)
+		if (c.width <= 4 * SEQ_THREADS) EM_LAUNCH(2);
+		else if (c.width <= 8 * SEQ_THREADS) EM_LAUNCH(4);
+		else EM_LAUNCH(8);
+#undef EM_LAUNCH
+#undef EM_ARGS
+	} else if (c.weight_dtype == YALM_F32)
 		seq_embed_kernel<WF32><<<dim3(n, eb), SEQ_THREADS, 0, q->stream>>>(q->st, tokens_dev, q->embed, q->inv_freq, c.width,
 		                                                         c.vocab, c.embed_scale, q->X, first_norm, c.norm_eps,
 		                                                         q->Hn, q->nk, q->L[0].pre_add, q->embed_norm, first_norm2,

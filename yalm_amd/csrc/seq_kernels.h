@@ -197,6 +197,80 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_embed_kernel(const StepState 
 	}
 }
 
+// The same for rows of up to 2 P SEQ_THREADS entries, without an embedding norm, token pairs or tanh norms: a thread owns P pairs
+// of entries (one angle each) in registers, all loads in flight together. (The general kernel's three passes over
+// the row, with a sine and a cosine branch per entry, took 13.5 us for one token of width 2048.)
+template <class WT, int P>
+__global__ __launch_bounds__(SEQ_THREADS) void seq_embed_reg_kernel(const StepState *__restrict__ st,
+                                                                    const int *__restrict__ tokens,
+                                                                    const void *__restrict__ emb,
+                                                                    const float *__restrict__ inv_freq, int width,
+                                                                    int vocab, float scale, float *__restrict__ X,
+                                                                    const float *__restrict__ w_next, float eps,
+                                                                    float *__restrict__ Hn, int nk,
+                                                                    const float *__restrict__ pre_add,
+                                                                    const float *__restrict__ w_next2,
+                                                                    float *__restrict__ Hn2) {
+	__shared__ float red[SEQ_THREADS / 64];
+	const int t = blockIdx.x;
+	const int tok = min(max(tokens ? tokens[t] : st->token, 0), vocab - 1);
+	const float p = (float)(st->pos + t);
+	float v[P][2], w[P][2];
+#pragma unroll
+	for (int e = 0; e < P; ++e) {
+		const int i = 2 * (threadIdx.x + e * SEQ_THREADS), ic = min(i, width - 2);
+		float s = 0.0f, c = 0.0f;
+		if (inv_freq)
+			sincosf(p * inv_freq[ic >> 1], &s, &c);
+#pragma unroll
+		for (int k = 0; k < 2; ++k) {
+			v[e][k] = wload<WT>(emb, (size_t)tok * width + ic + k) * scale + (k ? c : s);
+			if (pre_add)
+				v[e][k] += pre_add[ic + k];
+			w[e][k] = w_next ? w_next[ic + k] : 0.0f;
+		}
+	}
+	float ss = 0.0f, sm = 0.0f;
+#pragma unroll
+	for (int e = 0; e < P; ++e) {
+		const int i = 2 * (threadIdx.x + e * SEQ_THREADS);
+		if (i < width)
+#pragma unroll
+			for (int k = 0; k < 2; ++k) {
+				X[(size_t)t * width + i + k] = v[e][k];
+				ss = fmaf(v[e][k], v[e][k], ss);
+				sm += v[e][k];
+			}
+	}
+	if (!w_next)
+		return;
+	float mu = 0.0f;
+	if (nk_centred(nk)) {
+		mu = block_sum(sm, red) / (float)width;
+		ss = 0.0f;
+#pragma unroll
+		for (int e = 0; e < P; ++e)
+			if (2 * (int)(threadIdx.x + e * SEQ_THREADS) < width)
+#pragma unroll
+				for (int k = 0; k < 2; ++k)
+					ss = fmaf(v[e][k] - mu, v[e][k] - mu, ss);
+	}
+	const float r = 1.0f / sqrtf(block_sum(ss, red) / (float)width + eps);
+#pragma unroll
+	for (int e = 0; e < P; ++e) {
+		const int i = 2 * (threadIdx.x + e * SEQ_THREADS);
+		if (i >= width)
+			continue;
+#pragma unroll
+		for (int k = 0; k < 2; ++k) {
+			const float u = (v[e][k] - mu) * r;
+			Hn[(size_t)t * width + i + k] = u * w[e][k] + norm_bias(nk, w_next, width, i + k);
+			if (w_next2)
+				Hn2[(size_t)t * width + i + k] = u * w_next2[i + k] + norm_bias(nk, w_next2, width, i + k);
+		}
+	}
+}
+
 // ------------------------------------------------------------------ norms
 // out[row(t)] = norm(in[t]) * w * post, one workgroup per row. rows != null: the input row
 // is rows[t] (gather). pos_rows: the output row is st->pos + t (a cache write).
@@ -282,20 +356,74 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_norm2_kernel(const float *__r
 // Rows of up to E * SEQ_THREADS entries without a combine: the row of Y, the row of X and both
 // weight vectors are loaded at once (one memory round trip instead of one per pass) and the
 // row lives in registers.
-template <int E>
+// COMB: the routed experts' combine in place of Y (Combine), its rows loaded with the others: the
+// passes over LDS of the general kernel below took 17 us for one row of 2048, 40 us for 2048 rows.
+struct Combine {
+	const float *Yx = nullptr, *wt = nullptr;
+	int top = 0;
+	const float *Ys = nullptr, *sgate = nullptr;
+	const int *idx = nullptr;
+	int n_exp = 0;
+	const float *hid = nullptr;
+};
+// Slot k of token t in the routed experts' combine: the row its expert computed (Yx [slot][n]), or,
+// for a choice past the `n_exp` experts (an identity output), the feed-forward's own input row.
+__device__ __forceinline__ const float *combine_row(const float *Yx, const int *idx, int n_exp, const float *hid, int t,
+                                                    int top, int k, int n) {
+	const size_t slot = (size_t)t * top + k;
+	return (hid && idx[slot] >= n_exp) ? hid + (size_t)t * n : Yx + slot * n;
+}
+
+// The weight of a choice in the combine; wt == nullptr: 1 (the weight has been applied to the expert's input).
+__device__ __forceinline__ float combine_weight(const float *wt, size_t slot) {
+	return wt ? wt[slot] : 1.0f;
+}
+template <int E, bool COMB = false>
 __global__ __launch_bounds__(SEQ_THREADS) void seq_add_norm_reg_kernel(float *__restrict__ X,
                                                                        const float *__restrict__ Y,
                                                                        const float *__restrict__ wb, float eps, int n,
                                                                        const float *__restrict__ w_next,
-                                                                       float *__restrict__ Hn, int nk, float rs) {
+                                                                       float *Hn, int nk, float rs, Combine cb = Combine{}) {
 	__shared__ float red[SEQ_THREADS / 64];
 	const int t = blockIdx.x;
 	float y[E], x[E], b[E], wn[E], bb[E], nb[E]; // bb, nb: the biases of layer norms that have one
+	if constexpr (COMB) { // four choices' rows in flight at a time, summed in slot order, the shared expert's last
+#pragma unroll
+		for (int e = 0; e < E; ++e)
+			y[e] = 0.0f;
+		for (int k0 = 0; k0 < cb.top; k0 += 4) {
+			float v[4][E], w[4];
+#pragma unroll
+			for (int u = 0; u < 4; ++u) {
+				const int k = min(k0 + u, cb.top - 1);
+				const float *row = combine_row(cb.Yx, cb.idx, cb.n_exp, cb.hid, t, cb.top, k, n);
+				w[u] = combine_weight(cb.wt, (size_t)t * cb.top + k);
+#pragma unroll
+				for (int e = 0; e < E; ++e)
+					v[u][e] = row[min((int)threadIdx.x + e * SEQ_THREADS, n - 1)];
+			}
+#pragma unroll
+			for (int u = 0; u < 4; ++u)
+				if (k0 + u < cb.top)
+#pragma unroll
+					for (int e = 0; e < E; ++e)
+						y[e] = fmaf(w[u], v[u][e], y[e]);
+		}
+		if (cb.Ys) {
+			const float sg = cb.sgate ? cb.sgate[t] : 1.0f;
+#pragma unroll
+			for (int e = 0; e < E; ++e)
+				y[e] = fmaf(sg, cb.Ys[(size_t)t * n + min((int)threadIdx.x + e * SEQ_THREADS, n - 1)], y[e]);
+		}
+	}
 #pragma unroll
 	for (int e = 0; e < E; ++e) {
 		const int i = threadIdx.x + e * SEQ_THREADS;
 		const bool in = i < n;
-		y[e] = in ? Y[(size_t)t * n + i] : 0.0f;
+		if constexpr (COMB)
+			y[e] = in ? y[e] : 0.0f;
+		else
+			y[e] = in ? Y[(size_t)t * n + i] : 0.0f;
 		x[e] = in ? X[(size_t)t * n + i] : 0.0f;
 		b[e] = in ? wb[i] : 0.0f;
 		wn[e] = (in && w_next) ? w_next[i] : 0.0f;
@@ -369,19 +497,6 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_add_norm_reg_kernel(float *__
 		if (i < n)
 			Hn[(size_t)t * n + i] = x[e] * r2 * wn[e] + nb[e];
 	}
-}
-
-// Slot k of token t in the routed experts' combine: the row its expert computed (Yx [slot][n]), or,
-// for a choice past the `n_exp` experts (an identity output), the feed-forward's own input row.
-__device__ __forceinline__ const float *combine_row(const float *Yx, const int *idx, int n_exp, const float *hid, int t,
-                                                    int top, int k, int n) {
-	const size_t slot = (size_t)t * top + k;
-	return (hid && idx[slot] >= n_exp) ? hid + (size_t)t * n : Yx + slot * n;
-}
-
-// The weight of a choice in the combine; wt == nullptr: 1 (the weight has been applied to the expert's input).
-__device__ __forceinline__ float combine_weight(const float *wt, size_t slot) {
-	return wt ? wt[slot] : 1.0f;
 }
 
 // Yx != null: Y is not read; its row is the routed experts' combine sum_k wt[t][k] Yx[t top + k]
@@ -1738,6 +1853,92 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_rglru_scan_kernel(const float
 	state[c] = S;
 }
 
+// A few tokens (T <= SEQ_CONV_STEP_T) of the recurrent block between its two projections, one launch: a workgroup per
+// diagonal block of bs channels (bs <= 128, a multiple of 16). 1024 threads: four threads per gate row keep a quarter
+// of its weights in registers (2 bs rows: recurrence gates, then input gates), the convolved inputs, gates and the
+// block's channels meet in LDS. What bounds it is one CU's read of the block's 2 bs^2 f32 weights (128 KB at bs 128)
+// behind one memory round trip. (Convolution, gates and recurrence were three launches of 4.4-4.7 us.)
+__global__ __launch_bounds__(1024) void seq_rglru_step_kernel(const float *__restrict__ Z, int ldz, int W, int bs, int taps,
+                                                              const float *__restrict__ cw, const float *__restrict__ cb,
+                                                              float *__restrict__ cstate, const float *__restrict__ ga,
+                                                              const float *__restrict__ gab, const float *__restrict__ gi,
+                                                              const float *__restrict__ gib, const float *__restrict__ lam,
+                                                              float *__restrict__ state, float *__restrict__ out, int T) {
+	__shared__ __attribute__((aligned(16))) float us[128];
+	__shared__ float gs[256];
+	const int tid = threadIdx.x, b0 = blockIdx.x * bs;
+	const int row = tid >> 2, qt = tid & 3, per = bs >> 2; // per: this thread's weights of its row (<= 32)
+	const bool gate = row < 2 * bs;
+	const bool second = row >= bs;
+	float4_t wr[8];
+	{
+		const float *wp = (second ? gi : ga) + (size_t)blockIdx.x * bs * bs + (size_t)(gate ? (second ? row - bs : row) : 0) * bs + qt * per;
+#pragma unroll
+		for (int k = 0; k < 8; ++k)
+			wr[k] = *(const float4_t *)(wp + min(4 * k, per - 4));
+	}
+	const float gb = gate && qt == 0 ? (second ? gib[b0 + row - bs] : gab[b0 + row]) : 0.0f;
+	const int c = b0 + min(tid, bs - 1);
+	const bool ch = tid < bs; // these threads also own a channel
+	float win[SEQ_MAX_TAPS], wv[SEQ_MAX_TAPS], S = 0.0f, sp = 0.0f, bias = 0.0f;
+	if (ch) {
+#pragma unroll
+		for (int j = 0; j < SEQ_MAX_TAPS; ++j) {
+			win[j] = (j < taps - 1) ? cstate[(size_t)j * W + c] : 0.0f;
+			wv[j] = j < taps ? cw[(size_t)c * taps + j] : 0.0f;
+		}
+		S = state[c];
+		sp = sq_softplus(lam[c]);
+		bias = cb[c];
+	}
+	for (int t = 0; t < T; ++t) {
+		float u = 0.0f, y = 0.0f;
+		if (ch) {
+			const float cur = Z[(size_t)t * ldz + W + c];
+			y = Z[(size_t)t * ldz + c];
+			u = bias;
+#pragma unroll
+			for (int j = 0; j < SEQ_MAX_TAPS; ++j)
+				if (j < taps)
+					u = fmaf(wv[j], (j == taps - 1) ? cur : win[j], u);
+#pragma unroll
+			for (int j = 0; j < SEQ_MAX_TAPS - 1; ++j)
+				if (j < taps - 1)
+					win[j] = (j + 1 < taps - 1) ? win[j + 1] : cur;
+			us[tid] = u;
+		}
+		__syncthreads();
+		float a = 0.0f, a2 = 0.0f;
+#pragma unroll
+		for (int k = 0; k < 8; ++k)
+			if (4 * k < per) {
+				const float4_t x = *(const float4_t *)(us + qt * per + 4 * k);
+				a = fmaf(wr[k][0], x[0], a);
+				a2 = fmaf(wr[k][1], x[1], a2);
+				a = fmaf(wr[k][2], x[2], a);
+				a2 = fmaf(wr[k][3], x[3], a2);
+			}
+		a += a2;
+		a += dpp<0xB1>(a); // the row's four threads are neighbours
+		a += dpp<0x4E>(a);
+		if (gate && qt == 0)
+			gs[row] = sq_sigmoid(a + gb);
+		__syncthreads();
+		if (ch) {
+			const float la = -8.0f * gs[tid] * sp;
+			S = fmaf(expf(la), S, sqrtf(-expm1f(2.0f * la)) * (gs[bs + tid] * u));
+			out[(size_t)t * W + c] = S * sq_gelu_tanh(y);
+		}
+	}
+	if (ch) {
+		state[c] = S;
+#pragma unroll
+		for (int j = 0; j < SEQ_MAX_TAPS; ++j)
+			if (j < taps - 1)
+				cstate[(size_t)j * W + c] = win[j];
+	}
+}
+
 // Long portions: everything that does not depend on the carried state is evaluated for all
 // tokens at once (R <- a, I <- sqrt(1 - a^2) i u, U <- gelu_tanh(gate branch)), so that the
 // sequential walk below is one fused multiply-add per token and channel.
@@ -1779,7 +1980,7 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_rglru_walk_kernel(const float
 // (convolved, silu); Z columns bcol.. = beta logits, acol.. = decay inputs. BG [T][2 H]: beta,
 // per-head decay. GV != nullptr: one decay per head and key channel instead, GV [T][H D] holds
 // the decay inputs on entry (no bias yet; dt_bias is [H D]) and the decays on return, and the
-// per-head decay of BG is 1. One workgroup per token.
+// per-head decay of BG is 1. The workgroups of a token (gridDim.y) share its heads.
 __global__ __launch_bounds__(SEQ_THREADS) void seq_delta_prep_kernel(float *__restrict__ QKV, int ldq, int KH, int D,
                                                                      const float *__restrict__ Z, int ldz, int bcol,
                                                                      int acol, int H, const float *__restrict__ a_log,
@@ -1790,7 +1991,7 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_delta_prep_kernel(float *__re
 	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
 	float *row = QKV + (size_t)t * ldq;
 	const float qs = 1.0f / sqrtf((float)D);
-	for (int seg = wave; seg < 2 * KH; seg += SEQ_THREADS / 64) {
+	for (int seg = blockIdx.y * (SEQ_THREADS / 64) + wave; seg < 2 * KH; seg += gridDim.y * (SEQ_THREADS / 64)) {
 		float *x = row + (size_t)seg * D;
 		float ss = 0.0f;
 		for (int i = lane; i < D; i += 64)
@@ -1800,16 +2001,69 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_delta_prep_kernel(float *__re
 		for (int i = lane; i < D; i += 64)
 			x[i] *= r;
 	}
-	for (int h = threadIdx.x; h < H; h += SEQ_THREADS) {
+	for (int h = threadIdx.x; h < H && blockIdx.y == 0; h += SEQ_THREADS) {
 		BG[(size_t)t * 2 * H + h] = sq_sigmoid(Z[(size_t)t * ldz + bcol + h]);
 		BG[(size_t)t * 2 * H + H + h] =
 		    GV ? 1.0f : expf(-expf(a_log[h]) * sq_softplus(Z[(size_t)t * ldz + acol + h] + dt_bias[h]));
 	}
 	if (GV)
-		for (int i = threadIdx.x; i < H * D; i += SEQ_THREADS) {
+		for (int i = blockIdx.y * SEQ_THREADS + threadIdx.x; i < H * D; i += gridDim.y * SEQ_THREADS) {
 			float *g = GV + (size_t)t * H * D + i;
 			*g = expf(-expf(a_log[i / D]) * sq_softplus(*g + dt_bias[i]));
 		}
+}
+
+// A few tokens (T <= SEQ_CONV_STEP_T) of the delta rule's convolution, silu and preparation in one launch: a workgroup
+// per head segment of q | k | v (a thread per channel, D, V <= SEQ_THREADS), which walks the tokens with the channel's window
+// in registers, stores the new state and scales q and k segments to unit length; a value head's
+// workgroup also works out its beta and decay. (Two launches before: 4.8 + 5.4 us for one token, both latency.)
+__global__ __launch_bounds__(SEQ_THREADS) void seq_delta_front_kernel(const float *__restrict__ Z, int ldz, int KH, int D,
+                                                                      int H, int V, int taps, const float *__restrict__ w,
+                                                                      float *__restrict__ state, int bcol, int acol,
+                                                                      const float *__restrict__ a_log,
+                                                                      const float *__restrict__ dt_bias,
+                                                                      float *__restrict__ QKV, int C,
+                                                                      float *__restrict__ BG, int T) {
+	__shared__ float red[SEQ_THREADS / 64];
+	const int seg = blockIdx.x, tid = threadIdx.x;
+	const bool value = seg >= 2 * KH;
+	const int h = seg - 2 * KH, n = value ? V : D;
+	const int c = min((value ? 2 * KH * D + h * V : seg * D) + min(tid, n - 1), C - 1);
+	const bool in = tid < n;
+	float win[SEQ_MAX_TAPS], wv[SEQ_MAX_TAPS];
+#pragma unroll
+	for (int j = 0; j < SEQ_MAX_TAPS; ++j) {
+		win[j] = (j < taps - 1) ? state[(size_t)j * C + c] : 0.0f;
+		wv[j] = j < taps ? w[(size_t)c * taps + j] : 0.0f;
+	}
+	const float qs = seg < KH ? 1.0f / sqrtf((float)D) : 1.0f;
+	for (int t = 0; t < T; ++t) {
+		const float cur = Z[(size_t)t * ldz + c];
+		float acc = 0.0f;
+#pragma unroll
+		for (int j = 0; j < SEQ_MAX_TAPS; ++j)
+			if (j < taps)
+				acc = fmaf(wv[j], (j == taps - 1) ? cur : win[j], acc);
+		float v = sq_silu(acc);
+		if (!value) {
+			const float ss = block_sum(in ? v * v : 0.0f, red);
+			v *= (1.0f / sqrtf(ss + 1e-6f)) * qs;
+		} else if (tid == 0) {
+			BG[(size_t)t * 2 * H + h] = sq_sigmoid(Z[(size_t)t * ldz + bcol + h]);
+			BG[(size_t)t * 2 * H + H + h] = expf(-expf(a_log[h]) * sq_softplus(Z[(size_t)t * ldz + acol + h] + dt_bias[h]));
+		}
+		if (in)
+			QKV[(size_t)t * C + c] = v;
+#pragma unroll
+		for (int j = 0; j < SEQ_MAX_TAPS - 1; ++j) // shift the window by one token
+			if (j < taps - 1)
+				win[j] = (j + 1 < taps - 1) ? win[j + 1] : cur;
+	}
+	if (in)
+#pragma unroll
+		for (int j = 0; j < SEQ_MAX_TAPS; ++j)
+			if (j < taps - 1)
+				state[(size_t)j * C + c] = win[j];
 }
 
 // Selective state-space layer: per token and head dt = softplus(step + dt_bias[h]) and the
@@ -2141,7 +2395,7 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_delta_kernel(const float *__r
 // heads, or wstride = vdim: one per head), times the output gate: silu (sig == 0) or sigmoid (sig != 0) of the gate logits Gl [t][ldg],
 // head h's at column gcol + h V (out may alias Gl when both rows have the same layout: every
 // entry is read before the same entry is written). divided: O rows hold vdim + 1 entries per head, the
-// last one a divisor of the others. One workgroup per token, a wave per head.
+// last one a divisor of the others. A wave per head, the heads of a token shared by gridDim.y workgroups.
 __global__ __launch_bounds__(SEQ_THREADS) void seq_delta_out_kernel(const float *__restrict__ O, int H, int V,
                                                                     const float *__restrict__ w, float eps,
                                                                     const float *Gl, int ldg, int gcol,
@@ -2149,7 +2403,7 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_delta_out_kernel(const float 
                                                                     int divided = 0) {
 	const int t = blockIdx.x;
 	const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-	for (int h = wave; h < H; h += SEQ_THREADS / 64) {
+	for (int h = blockIdx.y * (SEQ_THREADS / 64) + wave; h < H; h += gridDim.y * (SEQ_THREADS / 64)) {
 		const int VS = V + (divided ? 1 : 0);
 		const float *o = O + ((size_t)t * H + h) * VS;
 		const float dv = divided ? 1.0f / o[V] : 1.0f;
@@ -2197,9 +2451,7 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_gated_part_norm_kernel(const 
 #define ATT_BR 16
 #define ATT_KT 64
 // LDS rows are padded to a multiple of 4 floats (zeros) so that both phases read 16 bytes
-// at a time. Key splits (gridDim.y = S > 1, single tokens and short portions): split s walks
-// its share of the visible keys and leaves (sums, running maximum, running sum) per row in
-// `part` for seq_latent_merge_kernel; S == 1 writes the normalised sums to Ctx.
+// at a time. Single tokens and short portions: seq_latent_split_kernel.
 __host__ __device__ inline int att_rank4(int rank) {
 	return (rank + 3) & ~3;
 }
@@ -2208,8 +2460,7 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_latent_attn_kernel(const floa
                                                                       const CT *__restrict__ cache, int rank, int H,
                                                                       int NR, float scale,
                                                                       const StepState *__restrict__ st,
-                                                                      float *__restrict__ Ctx,
-                                                                      float *__restrict__ part) {
+                                                                      float *__restrict__ Ctx) {
 	extern __shared__ __attribute__((aligned(16))) float lds[];
 	const int rank4 = att_rank4(rank), ldc = rank4 + 4, q4n = rank4 >> 2;
 	float *qs = lds;                      // [ATT_BR][rank4]
@@ -2217,19 +2468,11 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_latent_attn_kernel(const floa
 	float *ps = cs + ATT_KT * ldc;        // [ATT_BR][ATT_KT]
 	float *alpha = ps + ATT_BR * ATT_KT;  // [ATT_BR]
 	float *lsum = alpha + ATT_BR;         // [ATT_BR]
-	float *mfin = lsum + ATT_BR;          // [ATT_BR]
 	const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
 	const int r0 = blockIdx.x * ATT_BR;
-	const int S = gridDim.y, split = blockIdx.y;
 	const int pos0 = st->pos;
 	const int rlast = min(r0 + ATT_BR, NR) - 1;
-	const int nkeys = pos0 + rlast / H + 1; // keys visible to the workgroup's last row
-	int k_begin = 0, k_end = nkeys;
-	if (S > 1) {
-		const int chunk = (((nkeys + S - 1) / S) + ATT_KT - 1) & ~(ATT_KT - 1);
-		k_begin = split * chunk;
-		k_end = min(nkeys, k_begin + chunk);
-	}
+	const int k_end = pos0 + rlast / H + 1; // keys visible to the workgroup's last row
 	for (int i = tid; i < ATT_BR * rank4; i += SEQ_THREADS) {
 		const int r = r0 + i / rank4, d = i % rank4;
 		qs[i] = (r < NR && d < rank) ? Qa[(size_t)r * rank + d] * scale : 0.0f;
@@ -2247,7 +2490,7 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_latent_attn_kernel(const floa
 		lrun[i] = 0.0f;
 		lim[i] = r < NR ? min(pos0 + r / H, k_end - 1) : -1;
 	}
-	for (int kt = k_begin; kt < k_end; kt += ATT_KT) {
+	for (int kt = 0; kt < k_end; kt += ATT_KT) {
 		__syncthreads(); // the previous tile's sums have read cs / ps
 		if (rank % 8 == 0 && (size_t)cache % 16 == 0) { // 8 latent entries per load
 			const int v8n = rank >> 3;
@@ -2343,10 +2586,8 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_latent_attn_kernel(const floa
 	}
 	if (lane == 0) {
 #pragma unroll
-		for (int i = 0; i < 4; ++i) {
+		for (int i = 0; i < 4; ++i)
 			lsum[wave * 4 + i] = lrun[i];
-			mfin[wave * 4 + i] = mrun[i];
-		}
 	}
 	__syncthreads();
 #pragma unroll
@@ -2356,26 +2597,144 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_latent_attn_kernel(const floa
 			const int r = u / q4n, d4 = u % q4n;
 			if (r0 + r >= NR)
 				continue;
-			if (S == 1) {
-				const float inv = 1.0f / lsum[r];
+			const float inv = 1.0f / lsum[r];
 #pragma unroll
-				for (int e = 0; e < 4; ++e)
-					if (4 * d4 + e < rank)
-						Ctx[(size_t)(r0 + r) * rank + 4 * d4 + e] = acc[a][e] * inv;
-			} else {
-				float *pp = part + ((size_t)(r0 + r) * S + split) * (rank4 + 4);
-				*(float4_t *)(pp + 4 * d4) = acc[a];
-				if (d4 == 0) {
-					pp[rank4] = mfin[r];
-					pp[rank4 + 1] = lsum[r];
-				}
-			}
+			for (int e = 0; e < 4; ++e)
+				if (4 * d4 + e < rank)
+					Ctx[(size_t)(r0 + r) * rank + 4 * d4 + e] = acc[a][e] * inv;
 		}
 	}
 }
 static inline size_t att_lds_bytes(int rank) {
 	const int r4 = att_rank4(rank);
-	return sizeof(float) * ((size_t)ATT_BR * r4 + (size_t)ATT_KT * (r4 + 4) + ATT_BR * ATT_KT + 3 * ATT_BR);
+	return sizeof(float) * ((size_t)ATT_BR * r4 + (size_t)ATT_KT * (r4 + 4) + ATT_BR * ATT_KT + 2 * ATT_BR);
+}
+// Single tokens and short portions: the same, the visible keys split over gridDim.y workgroups per ATT_BR rows, in tiles
+// of ATS_KT keys: 16 rows x 16 keys, a score per thread, so a token at a short context is a handful of workgroups of one tile
+// each (64-key tiles, a workgroup of 16 rows walking them alone: 34 us at 86 keys, LDS reads of one CU). A split leaves
+// (sums, running maximum, running sum) per row in `part` for seq_latent_merge_kernel; one without keys leaves (0, -max, 0).
+#define ATS_KT 16
+template <class CT, int NA4>
+__global__ __launch_bounds__(SEQ_THREADS) void seq_latent_split_kernel(const float *__restrict__ Qa,
+                                                                       const CT *__restrict__ cache, int rank, int H, int NR,
+                                                                       float scale, const StepState *__restrict__ st,
+                                                                       float *__restrict__ part) {
+	extern __shared__ __attribute__((aligned(16))) float lds[];
+	const int rank4 = att_rank4(rank), ldc = rank4 + 4, q4n = rank4 >> 2;
+	float *qs = lds;                     // [ATT_BR][rank4 + 4]
+	float *cs = qs + ATT_BR * ldc;       // [ATS_KT][rank4 + 4]
+	float *ps = cs + ATS_KT * ldc;       // [ATT_BR][ATS_KT]
+	float *alpha = ps + ATT_BR * ATS_KT; // [ATT_BR]
+	const int tid = threadIdx.x, row = tid >> 4, key = tid & 15;
+	const int r0 = blockIdx.x * ATT_BR, S = gridDim.y, split = blockIdx.y;
+	const int pos0 = st->pos;
+	const int nkeys = pos0 + (min(r0 + ATT_BR, NR) - 1) / H + 1; // keys visible to the workgroup's last row
+	const int chunk = (((nkeys + S - 1) / S) + ATS_KT - 1) & ~(ATS_KT - 1);
+	const int k_begin = split * chunk, k_end = min(nkeys, k_begin + chunk);
+	const int lim = r0 + row < NR ? min(pos0 + (r0 + row) / H, k_end - 1) : -1;
+	float4_t acc[NA4];
+#pragma unroll
+	for (int a = 0; a < NA4; ++a)
+		acc[a] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+	float mrun = -FLT_MAX, lrun = 0.0f;
+	if (k_begin < k_end)
+		for (int i = tid; i < ATT_BR * rank4; i += SEQ_THREADS) {
+			const int r = i / rank4, d = i % rank4;
+			qs[r * ldc + d] = (r0 + r < NR && d < rank) ? Qa[(size_t)(r0 + r) * rank + d] * scale : 0.0f;
+		}
+	const bool vec = rank % 8 == 0 && (size_t)cache % 16 == 0; // 8 latent entries per load
+	for (int kt = k_begin; kt < k_end; kt += ATS_KT) {
+		__syncthreads(); // the previous tile's sums have read cs / ps
+		if (vec) {
+			const int v8n = rank >> 3;
+			for (int i = tid; i < ATS_KT * v8n; i += SEQ_THREADS) {
+				const int jj = i / v8n, d = (i % v8n) * 8, j = min(kt + jj, k_end - 1); // (keys past the end are masked)
+				float4_t lo, hi;
+				if constexpr (sizeof(CT) == 2) {
+					float f[8];
+					WBF16::unpack(load16(cache + (size_t)j * rank + d), f);
+					lo = float4_t{f[0], f[1], f[2], f[3]};
+					hi = float4_t{f[4], f[5], f[6], f[7]};
+				} else {
+					lo = *(const float4_t *)(cache + (size_t)j * rank + d);
+					hi = *(const float4_t *)(cache + (size_t)j * rank + d + 4);
+				}
+				*(float4_t *)(cs + jj * ldc + d) = lo;
+				*(float4_t *)(cs + jj * ldc + d + 4) = hi;
+			}
+		} else {
+			for (int i = tid; i < ATS_KT * rank4; i += SEQ_THREADS) {
+				const int jj = i / rank4, d = i % rank4, j = min(kt + jj, k_end - 1);
+				float v = 0.0f;
+				if (d < rank) {
+					if constexpr (sizeof(CT) == 2)
+						v = bf2f(cache[(size_t)j * rank + d]);
+					else
+						v = cache[(size_t)j * rank + d];
+				}
+				cs[jj * ldc + d] = v;
+			}
+		}
+		__syncthreads();
+		{
+			float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+			const float4_t *cj = (const float4_t *)(cs + key * ldc), *qj = (const float4_t *)(qs + row * ldc);
+#pragma unroll 8
+			for (int d = 0; d < q4n; ++d) {
+				const float4_t c = cj[d], qv = qj[d];
+#pragma unroll
+				for (int e = 0; e < 4; ++e)
+					s[e] = fmaf(qv[e], c[e], s[e]);
+			}
+			const bool vis = kt + key <= lim;
+			const float sv = vis ? (s[0] + s[1]) + (s[2] + s[3]) : -FLT_MAX;
+			const float mnew = fmaxf(mrun, row16_max(sv));
+			const float p = vis ? expf(sv - mnew) : 0.0f;
+			const float al = expf(mrun - mnew); // 1 while nothing is visible yet, 0 at the first key
+			lrun = lrun * al + row16_sum(p);
+			mrun = mnew;
+			ps[row * ATS_KT + key] = p;
+			if (key == 0)
+				alpha[row] = al;
+		}
+		__syncthreads();
+#pragma unroll
+		for (int a = 0; a < NA4; ++a) {
+			const int u = tid + a * SEQ_THREADS;
+			if (u < ATT_BR * q4n) {
+				const int r = u / q4n, d4 = u % q4n;
+				float4_t v = acc[a] * alpha[r];
+				const float4_t *pr = (const float4_t *)(ps + r * ATS_KT);
+#pragma unroll
+				for (int j4 = 0; j4 < ATS_KT / 4; ++j4) {
+					const float4_t p = pr[j4];
+#pragma unroll
+					for (int e = 0; e < 4; ++e) {
+						const float4_t c = *(const float4_t *)(cs + (4 * j4 + e) * ldc + 4 * d4);
+#pragma unroll
+						for (int x = 0; x < 4; ++x)
+							v[x] = fmaf(p[e], c[x], v[x]);
+					}
+				}
+				acc[a] = v;
+			}
+		}
+	}
+	const int stride = rank4 + 4;
+	if (key == 0 && r0 + row < NR) {
+		float *pp = part + ((size_t)(r0 + row) * S + split) * stride;
+		pp[rank4] = mrun;
+		pp[rank4 + 1] = lrun;
+	}
+#pragma unroll
+	for (int a = 0; a < NA4; ++a) {
+		const int u = tid + a * SEQ_THREADS;
+		if (u < ATT_BR * q4n && r0 + u / q4n < NR)
+			*(float4_t *)(part + ((size_t)(r0 + u / q4n) * S + split) * stride + 4 * (u % q4n)) = acc[a];
+	}
+}
+static inline size_t ats_lds_bytes(int rank) {
+	return sizeof(float) * ((size_t)(ATT_BR + ATS_KT) * (att_rank4(rank) + 4) + ATT_BR * ATS_KT + ATT_BR);
 }
 // Ctx[r] = sum_s e^(m_s - M) acc_s / sum_s e^(m_s - M) l_s over the key splits of row r
 // (times gate[r] if given; gate_e: times sigmoid of the row's own gate logits, row r = token
@@ -2683,7 +3042,6 @@ __global__ __launch_bounds__(NT) void seq_router_kernel(const float *__restrict_
 		return;
 	}
 	float *gsc = sc + E; // [G]
-	__shared__ float red[SEQ_THREADS / 64];
 	if (kind >= 3) { // one wave: a lane owns experts lane, lane + 64, ... and only touches their entries
 		if (wave != 0)
 			return;
@@ -2789,55 +3147,58 @@ __global__ __launch_bounds__(NT) void seq_router_kernel(const float *__restrict_
 		}
 		return;
 	}
-	if constexpr (NT == SEQ_THREADS) { // kind 0
-		float mx = -FLT_MAX;
-		for (int e = threadIdx.x; e < E; e += SEQ_THREADS)
+	if (kind == 0) { // one wave: softmax, the best groups, the best experts among them (ties: the lower index)
+		if (wave != 0)
+			return;
+		float mx = -FLT_MAX, sum = 0.0f;
+		for (int e = lane; e < E; e += 64)
 			mx = fmaxf(mx, sc[e]);
 		mx = wave_max(mx);
-		if (lane == 0)
-			red[wave] = mx;
-		__syncthreads();
-		mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-		float sum = 0.0f;
-		for (int e = threadIdx.x; e < E; e += SEQ_THREADS) {
+		for (int e = lane; e < E; e += 64) {
 			const float v = expf(sc[e] - mx);
 			sc[e] = v;
 			sum += v;
 		}
-		sum = block_sum(sum, red);
-		const float inv = 1.0f / sum;
+		const float inv = 1.0f / wave_sum(sum);
+		__threadfence_block(); // the scores written by other lanes of this wave
 		const int gs = E / G;
-		for (int g = threadIdx.x; g < G; g += SEQ_THREADS) {
-			float m = -1.0f;
-			for (int e = g * gs; e < (g + 1) * gs; ++e)
-				m = fmaxf(m, sc[e]);
-			gsc[g] = m;
-		}
-		__syncthreads();
-		if (threadIdx.x != 0)
-			return;
-		unsigned long long allowed = 0ull; // groups that may be chosen from (G <= 64)
-		for (int k = 0; k < keep; ++k) {
-			int best = -1;
-			float bv = -2.0f;
-			for (int g = 0; g < G; ++g)
-				if (!((allowed >> g) & 1ull) && gsc[g] > bv) {
-					bv = gsc[g];
-					best = g;
+		float gm = -1.0f; // lane g: the best score of group g (G <= 64)
+		if (lane < G)
+			for (int e = lane * gs; e < (lane + 1) * gs; ++e)
+				gm = fmaxf(gm, sc[e]);
+		auto take = [&](float v, int i, int none) { // the largest v over the wave, its lowest index
+#pragma unroll
+			for (int d = 32; d > 0; d >>= 1) {
+				const float ov = __shfl_xor(v, d);
+				const int oi = __shfl_xor(i, d);
+				if (ov > v || (ov == v && oi < i)) {
+					v = ov;
+					i = oi;
 				}
-			allowed |= 1ull << best;
+			}
+			return v > -1.0f ? i : none;
+		};
+		unsigned long long allowed = 0ull; // groups that may be chosen from
+		for (int k = 0; k < keep; ++k) {
+			const bool open = lane < G && !((allowed >> lane) & 1ull);
+			const int g = take(open ? gm : -2.0f, open ? lane : 64, 64);
+			if (g < 64)
+				allowed |= 1ull << g;
 		}
 		for (int k = 0; k < top; ++k) {
-			int best = 0;
 			float bv = -1.0f;
-			for (int e = 0; e < E; ++e)
+			int best = E;
+			for (int e = lane; e < E; e += 64)
 				if (((allowed >> (e / gs)) & 1ull) && sc[e] > bv) {
 					bv = sc[e];
 					best = e;
 				}
-			idx[(size_t)t * top + k] = best;
-			wt[(size_t)t * top + k] = bv * inv * rscale;
-			sc[best] = -1.0f; // taken
+			best = take(bv, best, 0);
+			if ((best & 63) == lane) {
+				idx[(size_t)t * top + k] = best;
+				wt[(size_t)t * top + k] = sc[best] * inv * rscale;
+				sc[best] = -1.0f; // taken
+			}
 		}
 	}
 }
