@@ -71,6 +71,7 @@ struct yalm_seq_s {
 	size_t gpart_floats = 0;
 	int *tok = nullptr, *want = nullptr;
 	float *logits = nullptr;     // [LOGIT_ROWS][vocab]
+	float *logits_pinned = nullptr; // [PINNED_ROWS][vocab] on the host, made by the first step that returns a few rows
 	int *idx = nullptr, *counts = nullptr, *lists = nullptr;
 	float *wt = nullptr, *sgate = nullptr;
 	int cur_pos = 0;             // the position the portion being enqueued starts at (host copy of st->pos)
@@ -104,7 +105,26 @@ struct yalm_seq_s {
 };
 typedef yalm_seq_s Seq;
 
-enum { LOGIT_ROWS = 64, SEQ_PORTION_CAP = 4096 };
+enum { LOGIT_ROWS = 64, SEQ_PORTION_CAP = 4096, STEP_ARGS = 64, PINNED_ROWS = 4 };
+static_assert(STEP_ARGS <= LOGIT_ROWS, "a step whose rows travel as arguments asks for one batch of logits");
+// A short step's tokens and asked rows, as kernel arguments.
+struct StepArgs {
+	int tok[STEP_ARGS], want[STEP_ARGS];
+};
+static __global__ void seq_begin_kernel(StepState *st, int pos, int *tok, int n, int *want, int n_want, bool pair, int prev,
+                                        StepArgs a) {
+	const int i = threadIdx.x;
+	if (i < n)
+		tok[i] = a.tok[i];
+	if (i < n_want)
+		want[i] = a.want[i];
+	if (i == 0) {
+		st->token = 0;
+		st->pos = pos;
+		if (pair)
+			tok[-1] = prev;
+	}
+}
 
 static int salloc(Seq *q, void **p, size_t bytes) {
 	*p = nullptr;
@@ -341,6 +361,8 @@ static void destroy_seq(Seq *q) {
 		(void)hipGraphDestroy(q->greedy_graph);
 	for (void *p : q->allocs)
 		(void)hipFree(p);
+	if (q->logits_pinned)
+		(void)hipHostFree(q->logits_pinned);
 	if (q->own_stream && q->stream)
 		(void)hipStreamDestroy(q->stream);
 	delete q;
@@ -1841,12 +1863,25 @@ extern "C" int yalm_seq_step(yalm_seq q, const int *tokens, int n, const int *wa
 	const yalm_seq_config &c = q->c;
 	int wi = 0;
 	q->dump_n = 0;
+	// up to STEP_ARGS tokens and asked rows travel as kernel arguments (a copy from the caller's memory and the wait
+	// for it cost more than a small launch); a few rows of logits come back through pinned memory
+	const bool args = n <= STEP_ARGS && n_want <= STEP_ARGS && n <= q->cap;
+	const bool pinned = n_want > 0 && n_want <= PINNED_ROWS;
+	if (pinned && !q->logits_pinned)
+		HIPCHK(hipHostMalloc((void **)&q->logits_pinned, (size_t)PINNED_ROWS * c.vocab * sizeof(float), hipHostMallocDefault));
 	for (int t0 = 0; t0 < n; t0 += q->cap) {
 		const int m = std::min(q->cap, n - t0);
-		HIPCHK(hipMemcpyAsync(q->tok, tokens + t0, (size_t)m * sizeof(int), hipMemcpyHostToDevice, q->stream));
-		set_step_kernel<<<1, 1, 0, q->stream>>>(q->st, 0, q->host_pos, 0);
-		if (q->bigram)
-			seq_fill_int_kernel<<<1, 1, 0, q->stream>>>(q->tok - 1, 1, q->host_prev);
+		if (args) {
+			StepArgs sa;
+			std::copy(tokens, tokens + n, sa.tok);
+			std::copy(want, want + n_want, sa.want);
+			seq_begin_kernel<<<1, 64, 0, q->stream>>>(q->st, q->host_pos, q->tok, n, q->want, n_want, q->bigram != nullptr, q->host_prev, sa);
+		} else {
+			HIPCHK(hipMemcpyAsync(q->tok, tokens + t0, (size_t)m * sizeof(int), hipMemcpyHostToDevice, q->stream));
+			set_step_kernel<<<1, 1, 0, q->stream>>>(q->st, 0, q->host_pos, 0);
+			if (q->bigram)
+				seq_fill_int_kernel<<<1, 1, 0, q->stream>>>(q->tok - 1, 1, q->host_prev);
+		}
 		HIPCHK(hipGetLastError());
 		q->cur_pos = q->host_pos;
 		if (q->dump_on) {
@@ -1865,17 +1900,20 @@ extern "C" int yalm_seq_step(yalm_seq q, const int *tokens, int n, const int *wa
 			std::vector<int> rel(k);
 			for (int i = 0; i < k; ++i)
 				rel[i] = want[wi + i] - t0;
-			HIPCHK(hipMemcpyAsync(q->want, rel.data(), (size_t)k * sizeof(int), hipMemcpyHostToDevice, q->stream));
-			HIPCHK(hipStreamSynchronize(q->stream)); // rel leaves scope
+			if (!args) {
+				HIPCHK(hipMemcpyAsync(q->want, rel.data(), (size_t)k * sizeof(int), hipMemcpyHostToDevice, q->stream));
+				HIPCHK(hipStreamSynchronize(q->stream)); // rel leaves scope
+			}
 			TRY(enqueue_logits(q, q->want, k));
-			HIPCHK(hipMemcpyAsync(logits_host + (size_t)wi * c.vocab, q->logits, (size_t)k * c.vocab * sizeof(float),
-			                      hipMemcpyDeviceToHost, q->stream));
+			const size_t bytes = (size_t)k * c.vocab * sizeof(float);
+			float *const out = logits_host + (size_t)wi * c.vocab;
+			HIPCHK(hipMemcpyAsync(pinned ? q->logits_pinned : out, q->logits, bytes, hipMemcpyDeviceToHost, q->stream));
 			HIPCHK(hipStreamSynchronize(q->stream));
+			if (pinned)
+				memcpy(out, q->logits_pinned, bytes);
 			wi += k;
 		}
 	}
-	if (n_want)
-		HIPCHK(hipStreamSynchronize(q->stream));
 	return YALM_OK;
 }
 

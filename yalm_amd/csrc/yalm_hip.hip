@@ -366,6 +366,10 @@ static int attn_wo_init(yalm_decoder_s *d) {
 	return YALM_OK;
 }
 
+// The logits buffer: vocab_full words rounded up to a 128-byte line, then the error word's line.
+static size_t logits_words(int vocab_full) { return ((size_t)vocab_full + 31) / 32 * 32; }
+static size_t logits_bytes(const yalm_decoder_s *d) { return sizeof(float) * (logits_words(d->vocab_full) + 1); }
+
 // After a sync: report (once) a bounded spin that gave up -- the fused attention + Wo
 // launch waiting for its heads, or an IPC exchange waiting for a peer.
 int awo_check(yalm_decoder_s *d) {
@@ -690,7 +694,7 @@ static int enqueue_forward(yalm_decoder_s *d, int which) {
 		if (which == GRAPH_LOGITS) { // every rank's vocabulary slice, side by side
 			tpx_collect_kernel<<<TPX_COLLECT_WG, 256, 0, d->stream>>>(tpx_ex(d, 2 * L), d->c.vocab_size, 1, d->logits);
 			HIPCHK(hipGetLastError());
-			HIPCHK(hipMemcpyAsync(d->logits_pinned, d->logits, sizeof(float) * d->vocab_full, hipMemcpyDeviceToHost,
+			HIPCHK(hipMemcpyAsync(d->logits_pinned, d->logits, logits_bytes(d), hipMemcpyDeviceToHost,
 			                      d->stream));
 		} else { // local first max, pushed; every rank's pair gathered and picked in the same launch
 			argmax_tp_kernel<<<1, 1024, 0, d->stream>>>(d->logits_local, d->c.vocab_size, d->step, d->tokens,
@@ -705,7 +709,7 @@ static int enqueue_forward(yalm_decoder_s *d, int which) {
 			set_err("ncclAllGather (logits) failed");
 			return YALM_ERR_HIP;
 		}
-		HIPCHK(hipMemcpyAsync(d->logits_pinned, d->logits, sizeof(float) * d->vocab_full, hipMemcpyDeviceToHost,
+		HIPCHK(hipMemcpyAsync(d->logits_pinned, d->logits, logits_bytes(d), hipMemcpyDeviceToHost,
 		                      d->stream));
 	} else if (!d->comm) {
 		argmax_kernel<<<1, 1024, 0, d->stream>>>(d->logits, d->c.vocab_size, d->step, d->tokens, d->tokens_cap);
@@ -858,8 +862,7 @@ static int create_decoder(const yalm_config *config, const yalm_model_weights *w
 	    (r = dalloc(d, (void **)&d->xb2, sizeof(float) * q_dim)) ||
 	    (r = dalloc(d, (void **)&d->hb, sizeof(float) * c.hidden_dim)) ||
 	    (r = dalloc(d, (void **)&d->part, sizeof(unsigned long long) * (size_t)c.n_heads * nsplit * (c.head_dim + 2))) ||
-	    (r = dalloc(d, (void **)&d->awo_err, sizeof(unsigned) * AWO_REPL_STRIDE)) ||
-	    (r = dalloc(d, (void **)&d->logits, sizeof(float) * vocab_full)) ||
+	    (r = dalloc(d, (void **)&d->logits, sizeof(float) * (logits_words(vocab_full) + AWO_REPL_STRIDE))) ||
 	    (r = dalloc(d, (void **)&d->xs, sizeof(float) * c.dim)) ||
 	    (r = dalloc(d, (void **)&d->amax, sizeof(float) * 2)) ||
 	    (r = dalloc(d, (void **)&d->amax_all, sizeof(float) * 2 * tp_size)) ||
@@ -887,10 +890,12 @@ static int create_decoder(const yalm_config *config, const yalm_model_weights *w
 		if (!bw.value_cache && (r = dalloc(d, (void **)&bw.value_cache, kvb)))
 			return fail(r);
 	}
+	// the in-launch waits' error word follows the logits, so a forward's one copy to the host brings both
+	d->awo_err = (unsigned *)d->logits + logits_words(vocab_full);
 	d->logits_local = d->logits;
 	if (tp_size > 1 && (r = dalloc(d, (void **)&d->logits_local, sizeof(float) * c.vocab_size)))
 		return fail(r);
-	if (hipHostMalloc((void **)&d->logits_pinned, sizeof(float) * vocab_full, hipHostMallocDefault) != hipSuccess) {
+	if (hipHostMalloc((void **)&d->logits_pinned, logits_bytes(d), hipHostMallocDefault) != hipSuccess) {
 		set_err("hipHostMalloc failed");
 		return fail(YALM_ERR_HIP);
 	}
@@ -1115,7 +1120,9 @@ extern "C" int yalm_forward(yalm_decoder d, int token, int pos, int mode, float 
 	d->host_pos = pos; // OUTPUT / HYDRATE forwards do not advance the device position
 	if (which == GRAPH_LOGITS) {
 		HIPCHK(hipStreamSynchronize(d->stream));
-		TRY(awo_check(d));
+		// (the error word came with the logits: a second copy and wait cost 20 us a forward)
+		if (d->ipc || ((const unsigned *)d->logits_pinned)[logits_words(d->vocab_full)])
+			TRY(awo_check(d));
 		if (logits_host)
 			memcpy(logits_host, d->logits_pinned, sizeof(float) * d->vocab_full);
 	}
