@@ -54,6 +54,8 @@ struct yalm_seq_s {
 	const void *bigram = nullptr;
 	int host_prev = -1;
 	int *prev = nullptr;
+	char *slab = nullptr;        // salloc
+	size_t slab_left = 0;
 	std::vector<int> side_of;    // per layer: index in L of its second mixer, or -1 (sides follow the n_layers entries)
 	std::vector<float *> rel_dist; // attn with a distance bias: [rel_far + 1][heads], the bucketed table per distance
 	std::vector<int> rel_far;
@@ -105,6 +107,7 @@ struct yalm_seq_s {
 };
 typedef yalm_seq_s Seq;
 
+enum { ROWS_MAX_M = 256 }; // bf16 batches of at most this many rows: seq_rows_kernel
 enum { LOGIT_ROWS = 64, SEQ_PORTION_CAP = 4096, STEP_ARGS = 64, PINNED_ROWS = 4 };
 static_assert(STEP_ARGS <= LOGIT_ROWS, "a step whose rows travel as arguments asks for one batch of logits");
 // A short step's tokens and asked rows, as kernel arguments.
@@ -126,11 +129,27 @@ static __global__ void seq_begin_kernel(StepState *st, int pos, int *tok, int n,
 	}
 }
 
+// Zeroed device memory of the decoder's lifetime; small buffers are cut from slabs (an allocation and its fill cost
+// 20 us and more each, and a decoder has some thirty).
 static int salloc(Seq *q, void **p, size_t bytes) {
+	constexpr size_t SLAB = (size_t)1 << 20;
 	*p = nullptr;
-	HIPCHK(hipMalloc(p, bytes ? bytes : 1));
+	const size_t need = (std::max<size_t>(bytes, 1) + 255) / 256 * 256;
+	if (need <= SLAB / 8 && need <= q->slab_left) {
+		*p = q->slab;
+		q->slab += need;
+		q->slab_left -= need;
+		return YALM_OK;
+	}
+	const bool slab = need <= SLAB / 8;
+	const size_t size = slab ? SLAB : need;
+	HIPCHK(hipMalloc(p, size));
 	q->allocs.push_back(*p);
-	HIPCHK(hipMemset(*p, 0, bytes ? bytes : 1));
+	HIPCHK(hipMemset(*p, 0, size));
+	if (slab) {
+		q->slab = (char *)*p + need;
+		q->slab_left = SLAB - need;
+	}
 	return YALM_OK;
 }
 template <class T>
@@ -564,7 +583,11 @@ static int create_seq(const yalm_seq_config *config, const yalm_seq_weights *w, 
 		for (const yalm_seq_layer &l : q->L)
 			widest = std::max({widest, (size_t)2 * l.ff, (size_t)2 * l.shared_ff});
 		q->gpart_floats = std::min((size_t)8 << 20, 16 * std::max((cap + 15) / 16 * 16, (size_t)64) * (widest + 256));
-		STRY(sallocT(q, &q->gpart, q->gpart_floats));
+		if (hipMalloc((void **)&q->gpart, q->gpart_floats * sizeof(float)) != hipSuccess) { // (written before it is read)
+			set_err("hipMalloc failed");
+			return fail(YALM_ERR_HIP);
+		}
+		q->allocs.push_back(q->gpart);
 	}
 	STRY(sallocT(q, &q->tok, cap + 1));
 	q->tok += 1; // [-1]: the token before the portion's first
@@ -733,9 +756,41 @@ extern "C" int yalm_seq_pos(yalm_seq q, int *pos) {
 }
 
 // ------------------------------------------------------------------ launches
+// seq_rows_kernel's loads: 16-byte pieces of whole steps, in every batch
+template <class WT>
+static bool rows_ok(const GemmArgs &a) {
+	constexpr int E = WT::BYTES == 2 ? 8 : 4;
+	const size_t wp = (size_t)a.W | (size_t)a.W2 | (size_t)(a.z_split ? a.W_b : nullptr) | ((size_t)a.w_bs * WT::BYTES);
+	const size_t ap = (size_t)a.A | (size_t)a.a_bs * 4;
+	return !a.own_b && a.K % (4 * E) == 0 && a.ldw % E == 0 && a.lda % 4 == 0 && (wp | ap) % 16 == 0;
+}
+template <class WT, bool F32OP>
+static int rows_launch(Seq *q, const GemmArgs &a, int batches, int max_m) {
+	const int mt = max_m <= 16 ? 1 : max_m <= 32 ? 2 : 4;
+	const dim3 g(cdiv(a.N, 16), cdiv(max_m, 16 * mt), batches);
+#define ROWS_LAUNCH(GLU, MT) seq_rows_kernel<WT, F32OP, GLU, MT><<<g, SEQ_THREADS, 0, q->stream>>>(a)
+	if (a.W2) {
+		if (mt == 1) ROWS_LAUNCH(true, 1);
+		else if (mt == 2) ROWS_LAUNCH(true, 2);
+		else ROWS_LAUNCH(true, 4);
+	} else {
+		if (mt == 1) ROWS_LAUNCH(false, 1);
+		else if (mt == 2) ROWS_LAUNCH(false, 2);
+		else ROWS_LAUNCH(false, 4);
+	}
+#undef ROWS_LAUNCH
+	HIPCHK(hipGetLastError());
+	return YALM_OK;
+}
 template <class WT>
 static int gemm_t(Seq *q, const GemmArgs &a, int batches, int max_m) {
 	const bool glu = a.W2 != nullptr;
+	// 2 to 8 tokens in either type, and f32 portions: f32 products on the matrix cores
+	if (max_m > 1 && (WT::BYTES == 4 || max_m <= GEMV_MAX_M) && rows_ok<WT>(a))
+		return rows_launch<WT, true>(q, a, batches, max_m);
+	// bf16 batches (heads, experts' row lists) of few rows: the general tiles are mostly empty
+	if (WT::BYTES == 2 && max_m > GEMV_MAX_M && batches > 1 && max_m <= ROWS_MAX_M && rows_ok<WT>(a))
+		return rows_launch<WT, WT::BYTES == 4>(q, a, batches, max_m);
 	if (max_m <= GEMV_MAX_M) {
 		const dim3 g(cdiv(a.own_b ? std::max(a.N, a.N_b) : a.N, SEQ_THREADS / 64), 1, batches);
 		if (glu)

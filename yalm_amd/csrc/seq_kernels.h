@@ -1282,6 +1282,124 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_gemv_kernel(GemmArgs a) {
 	}
 }
 
+// ---- a few rows on the matrix cores, any batches and row lists: a workgroup owns 16 weight rows and up to 16 MT
+// result rows, its four waves a quarter of K each; weights and activations go from memory to registers
+// (lane (n, q): row n, E consecutive columns), U steps in flight, the quarters meet in LDS. F32OP: f32 products
+// (v_mfma_f32_16x16x4_f32: every operand and sum f32, bf16 weights widened exactly) for f32 models and for 2 to
+// 8 tokens of bf16 ones; else activations rounded to bf16 as in every longer portion. What bounds it is the weight
+// stream up to 16-32 rows (f32 MFMA: 512 weight bytes per 128 cycles of a SIMD), beyond that the f32 products.
+// Against it: 8 tokens as GEMVs read the activations once per weight row (1.17 ms a portion for 0.50 of
+// one token, width 2048), and f32 portions ran as FMA tiles of 64 x 64 on few workgroups (14-22 ms for 12 to 250
+// tokens, width 1536-2048). The workgroups start at different columns (in step they read the same HBM channels).
+typedef float f32x4r_t __attribute__((ext_vector_type(4)));
+template <class WT, bool F32OP, bool GLU, int MT>
+__global__ __launch_bounds__(SEQ_THREADS) void seq_rows_kernel(GemmArgs a) {
+	const GemmBatch b = gemm_batch<WT>(a, blockIdx.z);
+	const int m0 = blockIdx.y * 16 * MT, n0 = blockIdx.x * 16;
+	if (m0 >= b.M || n0 >= b.N)
+		return;
+	constexpr int E = WT::BYTES == 2 ? 8 : 4, STEP = 4 * E; // columns per lane and step, per wave and step
+	constexpr int U = MT == 4 ? 2 : 4;
+	__shared__ float red[(GLU ? 2 : 1) * 4 * MT * 16 * 17];
+	const int lane = threadIdx.x & 63, n = lane & 15, q = lane >> 4;
+	const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const char *w = b.W + (size_t)min(n0 + n, b.N - 1) * b.ldw * WT::BYTES + (size_t)q * 16;
+	const char *w2 = GLU ? b.W2 + (size_t)min(n0 + n, b.N - 1) * b.ldw * WT::BYTES + (size_t)q * 16 : nullptr;
+	const float *ar[MT];
+#pragma unroll
+	for (int m = 0; m < MT; ++m) {
+		const int mm = min(m0 + 16 * m + n, b.M - 1), s = b.rows ? b.rows[mm] : mm;
+		ar[m] = b.A + (size_t)(b.rows ? s / a.a_div : s) * b.lda + q * E;
+	}
+	const int mt = __builtin_amdgcn_readfirstlane(min(MT, (b.M - m0 + 15) / 16));
+	const int steps = b.K / STEP, per = (steps + 3) / 4;
+	const int s0 = min(wave * per, steps), cnt = min(steps - s0, per);
+	const int rot = cnt > 0 ? (int)(blockIdx.x % cnt) : 0;
+	f32x4r_t acc[MT], acc2[GLU ? MT : 1];
+#pragma unroll
+	for (int m = 0; m < MT; ++m) {
+		acc[m] = f32x4r_t{0.f, 0.f, 0.f, 0.f};
+		if constexpr (GLU)
+			acc2[m] = f32x4r_t{0.f, 0.f, 0.f, 0.f};
+	}
+	for (int i0 = 0; i0 < cnt; i0 += U) {
+		u32x4_t wv[U], wv2[GLU ? U : 1];
+		float4_t xv[U][MT][E / 4];
+#pragma unroll
+		for (int u = 0; u < U; ++u) {
+			const int i = min(i0 + u, cnt - 1);
+			const int k = (s0 + (i + rot < cnt ? i + rot : i + rot - cnt)) * STEP;
+			wv[u] = load_nt16(w + (size_t)k * WT::BYTES);
+			if constexpr (GLU)
+				wv2[u] = load_nt16(w2 + (size_t)k * WT::BYTES);
+#pragma unroll
+			for (int m = 0; m < MT; ++m)
+				if (m < mt)
+#pragma unroll
+					for (int e = 0; e < E / 4; ++e)
+						xv[u][m][e] = *(const float4_t *)(ar[m] + k + 4 * e);
+		}
+#pragma unroll
+		for (int u = 0; u < U; ++u) {
+			if (i0 + u >= cnt)
+				break;
+			if constexpr (F32OP) {
+				float wf[E], wf2[E];
+				WT::unpack(wv[u], wf);
+				if constexpr (GLU)
+					WT::unpack(wv2[u], wf2);
+#pragma unroll
+				for (int e = 0; e < E; ++e)
+#pragma unroll
+					for (int m = 0; m < MT; ++m)
+						if (m < mt) {
+							acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[u][m][e >> 2][e & 3], wf[e], acc[m], 0, 0, 0);
+							if constexpr (GLU)
+								acc2[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[u][m][e >> 2][e & 3], wf2[e], acc2[m], 0, 0, 0);
+						}
+			} else {
+				typedef __bf16 rows_bf16x8 __attribute__((ext_vector_type(8)));
+#pragma unroll
+				for (int m = 0; m < MT; ++m)
+					if (m < mt) {
+						uint16_t h[8];
+#pragma unroll
+						for (int e = 0; e < 8; ++e)
+							h[e] = f2bf(xv[u][m][(e >> 2) % (E / 4)][e & 3]);
+						u32x4_t p;
+#pragma unroll
+						for (int e = 0; e < 4; ++e)
+							p[e] = h[2 * e] | ((uint32_t)h[2 * e + 1] << 16);
+						const rows_bf16x8 av = __builtin_bit_cast(rows_bf16x8, p);
+						acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, __builtin_bit_cast(rows_bf16x8, wv[u]), acc[m], 0, 0, 0);
+						if constexpr (GLU)
+							acc2[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, __builtin_bit_cast(rows_bf16x8, wv2[u]), acc2[m], 0, 0, 0);
+					}
+			}
+		}
+	}
+	constexpr int QS = MT * 16 * 17; // one wave's sums
+#pragma unroll
+	for (int m = 0; m < MT; ++m)
+#pragma unroll
+		for (int r = 0; r < 4; ++r) { // C/D: column = lane & 15, row = 4 (lane >> 4) + r
+			red[wave * QS + (16 * m + 4 * q + r) * 17 + n] = acc[m][r];
+			if constexpr (GLU)
+				red[(4 + wave) * QS + (16 * m + 4 * q + r) * 17 + n] = acc2[m][r];
+		}
+	__syncthreads();
+	for (int i = threadIdx.x; i < 16 * mt * 16; i += SEQ_THREADS) {
+		const int r = i >> 4, c = i & 15, m = m0 + r;
+		if (m >= b.M || n0 + c >= b.N)
+			continue;
+		const float *rp = red + r * 17 + c;
+		const float v = (rp[0] + rp[QS]) + (rp[2 * QS] + rp[3 * QS]);
+		const float v2 = GLU ? (rp[4 * QS] + rp[5 * QS]) + (rp[6 * QS] + rp[7 * QS]) : 0.0f;
+		const int rc = (b.rows && !a.c_dense) ? b.rows[m] : m;
+		b.C[(size_t)rc * b.ldc + n0 + c] = epi_out(a, b, rc, n0 + c, v, v2);
+	}
+}
+
 // ---- one token, the previous sublayer's closing norm (rms or layer) folded in: x' = x + rs norm(y) wb is what
 // the product reads when sublayers read the stream itself. Every workgroup rebuilds x' once
 // (a thread KI groups of 4 entries, the row's statistics over the workgroup) into LDS, while
