@@ -764,23 +764,40 @@ static bool rows_ok(const GemmArgs &a) {
 	const size_t ap = (size_t)a.A | (size_t)a.a_bs * 4;
 	return !a.own_b && a.K % (4 * E) == 0 && a.ldw % E == 0 && a.lda % 4 == 0 && (wp | ap) % 16 == 0;
 }
-template <class WT, bool F32OP>
-static int rows_launch(Seq *q, const GemmArgs &a, int batches, int max_m) {
-	const int mt = max_m <= 16 ? 1 : max_m <= 32 ? 2 : 4;
-	const dim3 g(cdiv(a.N, 16), cdiv(max_m, 16 * mt), batches);
-#define ROWS_LAUNCH(GLU, MT) seq_rows_kernel<WT, F32OP, GLU, MT><<<g, SEQ_THREADS, 0, q->stream>>>(a)
-	if (a.W2) {
-		if (mt == 1) ROWS_LAUNCH(true, 1);
-		else if (mt == 2) ROWS_LAUNCH(true, 2);
-		else ROWS_LAUNCH(true, 4);
-	} else {
-		if (mt == 1) ROWS_LAUNCH(false, 1);
-		else if (mt == 2) ROWS_LAUNCH(false, 2);
-		else ROWS_LAUNCH(false, 4);
+template <class WT, bool F32OP, bool GLU, int MT, int NW>
+static int rows_launch_t(Seq *q, const GemmArgs &a, const dim3 &g) {
+	auto kern = seq_rows_kernel<WT, F32OP, GLU, MT, NW>;
+	constexpr size_t lds = (size_t)(GLU ? 2 : 1) * NW * MT * 16 * 17 * sizeof(float);
+	if constexpr (lds > 65536) {
+		static bool attr = false;
+		if (!attr) {
+			HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+			attr = true;
+		}
 	}
-#undef ROWS_LAUNCH
+	hipLaunchKernelGGL(kern, g, dim3(64 * NW), lds, q->stream, a);
 	HIPCHK(hipGetLastError());
 	return YALM_OK;
+}
+template <class WT, bool F32OP, bool GLU, int MT>
+static int rows_launch_nw(Seq *q, const GemmArgs &a, int batches, int max_m) {
+	const dim3 g(cdiv(a.N, 16), cdiv(max_m, 16 * MT), batches);
+	// about 16 waves a CU, each with at least two rounds of loads
+	const long wgs = (long)g.x * g.y * g.z, steps = a.K / (WT::BYTES == 2 ? 32 : 16);
+	const int u = MT == 4 ? 2 : 4;
+	if (wgs * 8 <= 256 * 16 && steps >= 8 * 2 * u) {
+		if constexpr (!(GLU && MT == 4)) // (16 waves leave a wave 128 registers)
+			if (wgs * 16 <= 256 * 16 && steps >= 16 * 2 * u)
+				return rows_launch_t<WT, F32OP, GLU, MT, 16>(q, a, g);
+		return rows_launch_t<WT, F32OP, GLU, MT, 8>(q, a, g);
+	}
+	return rows_launch_t<WT, F32OP, GLU, MT, 4>(q, a, g);
+}
+template <class WT, bool F32OP>
+static int rows_launch(Seq *q, const GemmArgs &a, int batches, int max_m) {
+#define ROWS_LAUNCH(MT) (a.W2 ? rows_launch_nw<WT, F32OP, true, MT>(q, a, batches, max_m) : rows_launch_nw<WT, F32OP, false, MT>(q, a, batches, max_m))
+	return max_m <= 16 ? ROWS_LAUNCH(1) : max_m <= 32 ? ROWS_LAUNCH(2) : ROWS_LAUNCH(4);
+#undef ROWS_LAUNCH
 }
 template <class WT>
 static int gemm_t(Seq *q, const GemmArgs &a, int batches, int max_m) {
@@ -1584,7 +1601,8 @@ static int ff_moe(Seq *q, int li, int n, const PostNorm *pn = nullptr) {
 	const int epi = glu ? glu_epi(l, EPI_GLU_CLAMP) : plain_epi(l);
 	// a few tokens: one batch per (token, choice), its expert's matrices picked on the device; the shared
 	// expert is the last batch
-	if (n <= GEMV_MAX_M) {
+	// (several tokens that choose more often than there are experts share an expert's weights as longer portions do)
+	if (n <= GEMV_MAX_M && slots <= E) {
 		const bool shared = l.shared_ff > 0;
 		GemmArgs a = plain(q->In, c.width, glu ? l.w_gate : l.w_up, c.width, hx, ff, 1, ff, c.width);
 		a.W2 = glu ? l.w_up : nullptr;

@@ -1283,8 +1283,9 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_gemv_kernel(GemmArgs a) {
 }
 
 // ---- a few rows on the matrix cores, any batches and row lists: a workgroup owns 16 weight rows and up to 16 MT
-// result rows, its four waves a quarter of K each; weights and activations go from memory to registers
-// (lane (n, q): row n, E consecutive columns), U steps in flight, the quarters meet in LDS. F32OP: f32 products
+// result rows, its NW waves a share of K each (as many as fill the chip: the chain of loads of one wave is what a
+// product of few workgroups waits for: 60 rows of [1536][5376] f32, 96 workgroups, 78 us with 4 waves); weights and activations go from memory to registers
+// (lane (n, q): row n, E consecutive columns), U steps in flight, the shares meet in LDS. F32OP: f32 products
 // (v_mfma_f32_16x16x4_f32: every operand and sum f32, bf16 weights widened exactly) for f32 models and for 2 to
 // 8 tokens of bf16 ones; else activations rounded to bf16 as in every longer portion. What bounds it is the weight
 // stream up to 16-32 rows (f32 MFMA: 512 weight bytes per 128 cycles of a SIMD), beyond that the f32 products.
@@ -1292,15 +1293,15 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_gemv_kernel(GemmArgs a) {
 // one token, width 2048), and f32 portions ran as FMA tiles of 64 x 64 on few workgroups (14-22 ms for 12 to 250
 // tokens, width 1536-2048). The workgroups start at different columns (in step they read the same HBM channels).
 typedef float f32x4r_t __attribute__((ext_vector_type(4)));
-template <class WT, bool F32OP, bool GLU, int MT>
-__global__ __launch_bounds__(SEQ_THREADS) void seq_rows_kernel(GemmArgs a) {
+template <class WT, bool F32OP, bool GLU, int MT, int NW>
+__global__ __launch_bounds__(64 * NW) void seq_rows_kernel(GemmArgs a) {
 	const GemmBatch b = gemm_batch<WT>(a, blockIdx.z);
 	const int m0 = blockIdx.y * 16 * MT, n0 = blockIdx.x * 16;
 	if (m0 >= b.M || n0 >= b.N)
 		return;
 	constexpr int E = WT::BYTES == 2 ? 8 : 4, STEP = 4 * E; // columns per lane and step, per wave and step
 	constexpr int U = MT == 4 ? 2 : 4;
-	__shared__ float red[(GLU ? 2 : 1) * 4 * MT * 16 * 17];
+	extern __shared__ float red[]; // [GLU ? 2 : 1][NW][16 MT][17]
 	const int lane = threadIdx.x & 63, n = lane & 15, q = lane >> 4;
 	const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const char *w = b.W + (size_t)min(n0 + n, b.N - 1) * b.ldw * WT::BYTES + (size_t)q * 16;
@@ -1312,7 +1313,7 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_rows_kernel(GemmArgs a) {
 		ar[m] = b.A + (size_t)(b.rows ? s / a.a_div : s) * b.lda + q * E;
 	}
 	const int mt = __builtin_amdgcn_readfirstlane(min(MT, (b.M - m0 + 15) / 16));
-	const int steps = b.K / STEP, per = (steps + 3) / 4;
+	const int steps = b.K / STEP, per = (steps + NW - 1) / NW;
 	const int s0 = min(wave * per, steps), cnt = min(steps - s0, per);
 	const int rot = cnt > 0 ? (int)(blockIdx.x % cnt) : 0;
 	f32x4r_t acc[MT], acc2[GLU ? MT : 1];
@@ -1385,16 +1386,21 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_rows_kernel(GemmArgs a) {
 		for (int r = 0; r < 4; ++r) { // C/D: column = lane & 15, row = 4 (lane >> 4) + r
 			red[wave * QS + (16 * m + 4 * q + r) * 17 + n] = acc[m][r];
 			if constexpr (GLU)
-				red[(4 + wave) * QS + (16 * m + 4 * q + r) * 17 + n] = acc2[m][r];
+				red[(NW + wave) * QS + (16 * m + 4 * q + r) * 17 + n] = acc2[m][r];
 		}
 	__syncthreads();
-	for (int i = threadIdx.x; i < 16 * mt * 16; i += SEQ_THREADS) {
+	for (int i = threadIdx.x; i < 16 * mt * 16; i += 64 * NW) {
 		const int r = i >> 4, c = i & 15, m = m0 + r;
 		if (m >= b.M || n0 + c >= b.N)
 			continue;
 		const float *rp = red + r * 17 + c;
-		const float v = (rp[0] + rp[QS]) + (rp[2 * QS] + rp[3 * QS]);
-		const float v2 = GLU ? (rp[4 * QS] + rp[5 * QS]) + (rp[6 * QS] + rp[7 * QS]) : 0.0f;
+		float v = 0.0f, v2 = 0.0f;
+#pragma unroll
+		for (int k = 0; k < NW; ++k) {
+			v += rp[k * QS];
+			if constexpr (GLU)
+				v2 += rp[(NW + k) * QS];
+		}
 		const int rc = (b.rows && !a.c_dense) ? b.rows[m] : m;
 		b.C[(size_t)rc * b.ldc + n0 + c] = epi_out(a, b, rc, n0 + c, v, v2);
 	}
