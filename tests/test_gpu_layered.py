@@ -165,6 +165,31 @@ def test_few_token_kernels(rt, portions):
         model.close()
 
 
+@pytest.mark.parametrize("width", [8, 136, 1024, 1032, 2056, 4096, 4104])
+def test_token_seams_inside_products(rt, width):
+    """Single tokens: the norms between sublayers inside the next product's or the router's launch (rows of at most 4096
+    entries), against the same steps with their own launches (as when every layer's stream is kept)."""
+    from yalm_amd import models as M
+
+    cfg = C.config([("rglru", C.rglru(width=32, blocks=2, conv=2), C.moe(ff=24, experts=6, top=5, groups=2, keep=2)),
+                    ("delta", C.delta(heads=2, kv_heads=1, dim=16, vdim=16, conv=3), C.dense(ff=24)),
+                    ("latent_attention", C.latent(heads=2, dim=16, vdim=16, kv_rank=24, q_rank=16, scale=0.25), None),
+                    ("rglru", C.rglru(width=32, blocks=2, conv=2), C.moe(ff=16, experts=4, top=1, groups=1, keep=1))],
+                   width=width, vocab=97)
+    model, dec, w = build(rt, cfg, M.F32, seed=8)
+    try:
+        tok = C.tokens(cfg, 12, 3)
+        got = run_portions(dec, tok, [1] * 12)
+        dec.reset()
+        dec.layer_dump(True)
+        apart = run_portions(dec, tok, [1] * 12)
+        assert rel_err(got, apart).max() < 5e-5  # the same sums in another order
+        assert close_enough(got, R.forward(cfg, w, tok), "f32")
+    finally:
+        dec.close()
+        model.close()
+
+
 @pytest.mark.parametrize("n", [9, 16, 17, 32, 33, 64, 65, 130, 255])
 def test_few_row_products_bf16(rt, n):
     """Products of 9 to 255 rows on the prefill unit: streamed in one or several K slices, large tiles in slices."""

@@ -60,8 +60,12 @@ struct yalm_seq_s {
 	std::vector<float *> rel_dist; // attn with a distance bias: [rel_far + 1][heads], the bucketed table per distance
 	std::vector<int> rel_far;
 	const float *In = nullptr;   // what a sublayer reads: Hn (pre_norm) or X itself
-	float *Xalt = nullptr, *Xbase = nullptr; // single tokens without opening norms: the stream alternates between two rows
-	const float *pend_wb = nullptr; // a closing norm not yet applied: X += norm(Y) pend_wb, owed to the next product
+	float *Xalt = nullptr, *Xbase = nullptr; // single tokens: the stream alternates between two rows
+	// a seam not yet applied, owed to the next product: X += norm(Y) pend_wb, Hn = norm(X) pend_next where sublayers open
+	// with a norm; Y the combine of pend_moe's experts if given
+	const float *pend_wb = nullptr, *pend_next = nullptr;
+	const yalm_seq_layer *pend_moe = nullptr;
+	bool hn_final = false; // the portion (one token) has left its final norm in Hn
 	int nk = NK_RMS;             // the kind of the model's norms
 	// a pair whose two mixers share one input projection: where the mixer being enqueued finds its
 	// columns of the result, and that result's row length (nullptr: the mixer projects for itself)
@@ -626,8 +630,7 @@ static int create_seq(const yalm_seq_config *config, const yalm_seq_weights *w, 
 	q->nk = c.norm_kind;
 	q->In = c.pre_norm ? q->Hn : q->X;
 	q->Xbase = q->X;
-	if (!c.pre_norm)
-		STRY(sallocT(q, &q->Xalt, (size_t)c.width));
+	STRY(sallocT(q, &q->Xalt, (size_t)c.width));
 	// position frequencies 10000^(-2 i / width), evaluated in double
 	if (c.pos_embed) {
 		std::vector<float> f((c.width + 1) / 2);
@@ -917,13 +920,15 @@ static int attn_t(Seq *q, const float *Qa, const void *cache, int rank, int H, i
 	return YALM_OK;
 }
 
+static int gemm_in(Seq *q, GemmArgs a);
+
 static int mixer_latent(Seq *q, int li, int n) {
 	const yalm_seq_layer &l = q->L[li];
 	const yalm_seq_config &c = q->c;
 	const bool bf = c.weight_dtype == YALM_BF16;
 	const int zin = in_rows(l), H = l.heads, D = l.dim, V = l.vdim, rk = l.kv_rank;
 	float *cq = q->B[0], *qh = q->B[1], *qa = q->B[2], *ctx = q->B[3];
-	TRY(gemm(q, plain(q->In, c.width, l.w_in, c.width, q->Z, zin, n, zin, c.width)));
+	TRY(gemm_in(q, plain(q->In, c.width, l.w_in, c.width, q->Z, zin, n, zin, c.width)));
 	if (l.kv_from >= 0)
 		seq_norm_kernel<float><<<n, SEQ_THREADS, 0, q->stream>>>(q->Z, zin, l.q_norm, c.norm_eps, l.q_rank, cq, l.q_rank,
 		                                                         nullptr, q->st, 0);
@@ -977,7 +982,7 @@ static int mixer_rglru(Seq *q, int li, int n) {
 	{
 		GemmArgs a = plain(q->In, c.width, l.w_in, c.width, q->Z, 2 * W, n, 2 * W, c.width);
 		a.bias = l.in_bias;
-		TRY(gemm(q, a));
+		TRY(gemm_in(q, a));
 	}
 	if (n <= SEQ_CONV_STEP_T && bs <= 128 && bs % 16 == 0 && ((size_t)l.gate_a | (size_t)l.gate_i) % 16 == 0) { // all of it in one launch
 		seq_rglru_step_kernel<<<l.blocks, 1024, 0, q->stream>>>(q->Z, 2 * W, W, bs, l.conv, l.conv_w, l.conv_b, q->conv[li], l.gate_a,
@@ -1067,7 +1072,7 @@ static int mixer_delta(Seq *q, int li, int n) {
 	float *qkv = q->B[0], *bg = q->B[1], *o = q->B[2], *on = q->B[3];
 	// one decay per head and key channel: its inputs, then the decays, follow the [n][2 H] factors
 	float *gv = l.decay_rank > 0 ? bg + (size_t)n * 2 * H : nullptr;
-	TRY(gemm(q, plain(q->In, c.width, l.w_in, c.width, q->Z, zin, n, zin, c.width)));
+	TRY(gemm_in(q, plain(q->In, c.width, l.w_in, c.width, q->Z, zin, n, zin, c.width)));
 	if (!gv && n <= SEQ_CONV_STEP_T && D <= SEQ_THREADS && V <= SEQ_THREADS) { // convolution and preparation in one launch
 		seq_delta_front_kernel<<<2 * KH + H, SEQ_THREADS, 0, q->stream>>>(q->Z, zin, KH, D, H, V, l.conv, l.conv_w, q->conv[li],
 		                                                                  bcol, acol, l.a_log, l.dt_bias, qkv, cc, bg, n);
@@ -1105,7 +1110,7 @@ static int mixer_ssm(Seq *q, int li, int n) {
 	const int H = l.heads, P = l.vdim, N = l.ssm_state, G = l.ssm_groups;
 	const int inner = H * P, GN = G * N, cc = inner + 2 * GN, zin = in_rows(l);
 	float *xbc = q->B[0], *bg = q->B[1], *y = q->B[2], *yn = q->B[3];
-	TRY(gemm(q, plain(q->In, c.width, l.w_in, c.width, q->Z, zin, n, zin, c.width)));
+	TRY(gemm_in(q, plain(q->In, c.width, l.w_in, c.width, q->Z, zin, n, zin, c.width)));
 	TRY(conv_launch(q, q->Z, zin, inner, cc, l.conv, l.conv_w, l.conv_b, 1, q->conv[li], xbc, n));
 	seq_ssm_prep_kernel<<<cdiv(n * H, SEQ_THREADS), SEQ_THREADS, 0, q->stream>>>(q->Z, zin, inner + cc, H, l.a_log,
 	                                                                            l.dt_bias, bg, n);
@@ -1153,7 +1158,7 @@ static int mixer_gla(Seq *q, int li, int n) {
 	const int H = l.heads, D = l.dim, V = l.vdim, zin = in_rows(l), HD = H * D, HV = H * V;
 	const int gcol = 2 * HD + HV, acol = gcol + HV;
 	float *gv = q->B[0], *o = q->B[1], *on = q->B[2];
-	TRY(gemm(q, plain(q->In, c.width, l.w_in, c.width, q->Z, zin, n, zin, c.width)));
+	TRY(gemm_in(q, plain(q->In, c.width, l.w_in, c.width, q->Z, zin, n, zin, c.width)));
 	GemmArgs a = plain(q->Z + acol, zin, l.w_a2, l.decay_rank, gv, HD, n, HD, l.decay_rank);
 	a.bias = l.dt_bias;
 	a.epi = EPI_SIG_ROOT;
@@ -1168,45 +1173,71 @@ static int mixer_gla(Seq *q, int li, int n) {
 	return gemm(q, plain(on, HV, l.w_o, HV, q->Yout, c.width, n, c.width, HV));
 }
 
-// ---- the closing norm of a single token, owed to the product that reads the stream next
+// ---- the seam after a single token's sublayer, owed to the product that reads the stream next
 static int add_norm(Seq *q, const float *wb, const float *w_next, int n, const yalm_seq_layer *moe);
+static Combine combine_of(const Seq *q, const yalm_seq_layer *moe);
 
 static bool an_foldable(const Seq *q, int n) {
-	return n == 1 && !q->c.pre_norm && q->c.block_kind == YALM_BLOCK_SERIAL && q->nk != NK_TANH && !q->dump_on && q->Xalt && q->c.width % 8 == 0 && q->c.width <= 8 * 1024;
+	return n == 1 && q->c.block_kind == YALM_BLOCK_SERIAL && q->nk != NK_TANH && !q->dump_on && q->c.width % 8 == 0 &&
+	       q->c.width <= 8 * 1024;
+}
+static void settled(Seq *q) {
+	q->pend_wb = q->pend_next = nullptr;
+	q->pend_moe = nullptr;
 }
 static int flush_norm(Seq *q, int n) {
 	if (!q->pend_wb)
 		return YALM_OK;
-	const float *wb = q->pend_wb;
-	q->pend_wb = nullptr;
-	return add_norm(q, wb, nullptr, n, nullptr);
+	const float *wb = q->pend_wb, *next = q->pend_next;
+	const yalm_seq_layer *moe = q->pend_moe;
+	settled(q);
+	return add_norm(q, wb, next, n, moe);
 }
-template <class WT>
+// Every workgroup of seq_gemv_an_kernel reads the seam's operands while others write results: no overlap.
+static bool an_apart(const Seq *q, const GemmArgs &a) {
+	const Combine cb = combine_of(q, q->pend_moe);
+	auto apart = [&](const float *p, size_t n) { return !p || a.C + a.N <= p || p + n <= a.C; };
+	const size_t w = q->c.width;
+	return apart(q->Y, w) && apart(cb.Yx, w * cb.top) && apart(cb.Ys, w) && apart(q->Xbase, w) && apart(q->Xalt, w) && apart(q->Hn, w);
+}
+template <class WT, bool GLU, bool COMB>
 static int gemv_an_t(Seq *q, const GemmArgs &a) {
 	const int K = a.K, ki = cdiv(K, 1024);
-	const dim3 g(cdiv(a.N, (SEQ_THREADS / 64) * GAN_RPW));
+	// two rows a wave, the second's loads under the first's sums, once one row a wave is two workgroups on every CU
+	const int rpw = a.N > 2048 ? 2 : 1;
+	const dim3 g(cdiv(a.N, (SEQ_THREADS / 64) * rpw));
+	float *const to = q->X == q->Xbase ? q->Xalt : q->Xbase;
 #define GA_LAUNCH(KI)                                                                                                  \
-	seq_gemv_an_kernel<WT, KI><<<g, SEQ_THREADS, (size_t)K * sizeof(float), q->stream>>>(                              \
-	    q->X, q->Y, q->pend_wb, q->c.norm_eps, q->nk, q->c.residual_scale, K, q->X == q->Xbase ? q->Xalt : q->Xbase, a.W, a.N, a.C,    \
-	    a.bias, a.epi)
+	seq_gemv_an_kernel<WT, KI, GLU, COMB><<<g, SEQ_THREADS, (size_t)K * sizeof(float), q->stream>>>(                   \
+	    q->X, q->Y, q->pend_wb, q->c.norm_eps, q->nk, q->c.residual_scale, K, to, q->pend_next, q->Hn,                 \
+	    (const char *)a.W, (const char *)a.W2, a.N, a.C, a.bias, a.epi, a.limit, rpw, combine_of(q, q->pend_moe))
 	if (ki <= 1) GA_LAUNCH(1);
 	else if (ki <= 2) GA_LAUNCH(2);
-	else if (ki <= 4) GA_LAUNCH(4);
-	else GA_LAUNCH(8);
+	else if (GLU || COMB || ki <= 4) GA_LAUNCH(4);
+	else if constexpr (!GLU && !COMB) GA_LAUNCH(8);
 #undef GA_LAUNCH
 	HIPCHK(hipGetLastError());
-	q->X = q->X == q->Xbase ? q->Xalt : q->Xbase; // the stream now lives in the other row
-	q->In = q->X;
-	q->pend_wb = nullptr;
+	q->X = to; // the stream now lives in the other row
+	if (!q->c.pre_norm)
+		q->In = q->X;
+	settled(q);
 	return YALM_OK;
 }
-// A product whose A operand is the sublayer input q->In. With a closing norm owed and a single
-// token, the norm + residual sum run inside the product's kernel; else the norm first.
+template <class WT>
+static int gemv_an(Seq *q, const GemmArgs &a) {
+	if (q->pend_moe)
+		return a.W2 ? gemv_an_t<WT, true, true>(q, a) : gemv_an_t<WT, false, true>(q, a);
+	return a.W2 ? gemv_an_t<WT, true, false>(q, a) : gemv_an_t<WT, false, false>(q, a);
+}
+// A product whose A operand is the sublayer input q->In. With a seam owed and a single token, it runs inside the
+// product's kernel; else before it.
 static int gemm_in(Seq *q, GemmArgs a) {
 	if (q->pend_wb) {
-		if (a.M == 1 && !a.W2 && (a.epi == EPI_NONE || a.epi == EPI_GELU) && a.ldw == a.K && a.K == q->c.width &&
-		    (size_t)a.W % 16 == 0 && !a.rows && !a.w_sel && a.z_split == 0 && a.A == q->In)
-			return q->c.weight_dtype == YALM_F32 ? gemv_an_t<WF32>(q, a) : gemv_an_t<WBF16>(q, a);
+		// (rows past 4096 entries: only the plain form has the registers for them)
+		const bool wide = a.K > 4096 && (a.W2 || q->pend_moe || q->pend_next);
+		if (a.M == 1 && !wide && (q->pend_next || !q->c.pre_norm) && a.ldw == a.K && a.K == q->c.width && ((size_t)a.W | (size_t)a.W2 | (size_t)q->pend_wb | (size_t)q->pend_next) % 16 == 0 &&
+		    !a.rows && !a.w_sel && !a.gate && !a.row_scale && a.z_split == 0 && a.A == q->In && an_apart(q, a))
+			return q->c.weight_dtype == YALM_F32 ? gemv_an<WF32>(q, a) : gemv_an<WBF16>(q, a);
 		TRY(flush_norm(q, a.M));
 		a.A = q->In;
 	}
@@ -1440,7 +1471,7 @@ static int mixer_latent_direct(Seq *q, int li, int n) {
 	const int klo = attn_first_key(l.mask_kind, l.mask_size, q->cur_pos), rows = q->cur_pos + n - klo;
 	const bool absorbed_ok = n == 1 || (bf && n > GEMV_MAX_M && KR <= 512 && rk <= 128) || attn_fma_fits(H, 1, KR, rk, n);
 	const bool expand = l.w_ukv && n > 1 && rows <= q->ex_rows && (n >= 32 || !absorbed_ok);
-	TRY(gemm(q, plain(q->In, c.width, l.w_in, c.width, q->Z, zin, n, zin, c.width)));
+	TRY(gemm_in(q, plain(q->In, c.width, l.w_in, c.width, q->Z, zin, n, zin, c.width)));
 	const size_t rot_lds = (size_t)std::max(l.rot_dims, 2) * sizeof(float);
 	const float *kv_w = l.kv_from < 0 ? l.kv_norm : nullptr; // another layer's cache rows: queries (and gate) only
 	const float *ge = l.out_gate == 2 ? q->Z + (zin - H * V) : nullptr; // elementwise gate logits close the projection
@@ -1568,14 +1599,17 @@ static int ff_dense(Seq *q, int li, int n, float *out) {
 	a.W2 = l.w_up;
 	a.epi = glu_epi(l, EPI_GLU_GELU);
 	a.limit = l.limit;
-	TRY(gemm(q, a));
+	TRY(gemm_in(q, a));
 	return gemm(q, plain(q->B[0], l.ff, l.w_down, l.ff, out, c.width, n, c.width, l.ff));
 }
 
 // pn: the seam that makes this feed-forward's input, not yet applied (post_routes)
+static bool route_lds(const Seq *q, const yalm_seq_layer &l) { // the row and the scores within the router's LDS
+	return (size_t)q->c.width + 2 * (l.experts + l.identity) <= 12 * 1024;
+}
 static bool post_routes(const Seq *q, const yalm_seq_layer &l) {
 	return q->c.block_kind == YALM_BLOCK_POST && l.ff_kind == YALM_FF_MOE && l.router_kind >= YALM_ROUTER_SOFTMAX_NORMED &&
-	       (size_t)q->c.width + 2 * (l.experts + l.identity) <= 12 * 1024;
+	       route_lds(q, l);
 }
 static int ff_moe(Seq *q, int li, int n, const PostNorm *pn = nullptr) {
 	const yalm_seq_layer &l = q->L[li];
@@ -1586,9 +1620,9 @@ static int ff_moe(Seq *q, int li, int n, const PostNorm *pn = nullptr) {
 	const bool one_wave = l.router_kind == YALM_ROUTER_SOFTMAX_TOP || l.router_kind == YALM_ROUTER_SOFTMAX_NORMED ||
 	                      l.router_kind == YALM_ROUTER_SIGMOID_TOP;
 	auto router = one_wave ? seq_router_kernel<1024> : seq_router_kernel<SEQ_THREADS>;
-	const int rth = one_wave ? 1024 : SEQ_THREADS;
+	const int rth = one_wave || pn ? 1024 : SEQ_THREADS;
 	size_t lds = (2 * ER + l.groups) * sizeof(float);
-	if (pn) { // the post-norm seam before this feed-forward, in the router's launch
+	if (pn) { // the seam before this feed-forward, in the router's launch
 		router = seq_router_kernel<1024, true>;
 		lds += ((c.width + 3) & ~3) * sizeof(float);
 	}
@@ -1679,6 +1713,12 @@ static int ff_moe(Seq *q, int li, int n, const PostNorm *pn = nullptr) {
 static const float *combine_wt(const Seq *q, const yalm_seq_layer &l) {
 	return l.expert_in_weighted ? nullptr : q->wt;
 }
+static Combine combine_of(const Seq *q, const yalm_seq_layer *moe) {
+	if (!moe)
+		return Combine{};
+	return Combine{q->B[1], combine_wt(q, *moe), moe->top, moe->shared_ff > 0 ? q->B[3] : nullptr,
+	               moe->shared_ff > 0 && moe->shared_sg ? q->sgate : nullptr, q->idx, moe->experts, moe->identity > 0 ? q->In : nullptr};
+}
 
 // The seam after a parallel block: both sublayers' results join the stream (the experts' combine
 // happens here), the next entry's pre_add and opening norm follow in the same launch.
@@ -1738,10 +1778,7 @@ static int post_close(Seq *q, const float *wb, int n, const yalm_seq_layer *moe)
 static int add_norm(Seq *q, const float *wb, const float *w_next, int n, const yalm_seq_layer *moe) {
 	const int w = q->c.width;
 	if (w <= 16 * SEQ_THREADS) { // the row in registers
-		Combine cb;
-		if (moe)
-			cb = {q->B[1], combine_wt(q, *moe), moe->top, moe->shared_ff > 0 ? q->B[3] : nullptr,
-			      moe->shared_ff > 0 && moe->shared_sg ? q->sgate : nullptr, q->idx, moe->experts, moe->identity > 0 ? q->In : nullptr};
+		const Combine cb = combine_of(q, moe);
 #define AN_LAUNCH(E, C)                                                                                                \
 	seq_add_norm_reg_kernel<E, C><<<n, SEQ_THREADS, 0, q->stream>>>(q->X, q->Y, wb, q->c.norm_eps, w, w_next, q->Hn, q->nk, \
 	                                                                q->c.residual_scale, cb)
@@ -1777,18 +1814,21 @@ static int enqueue_portion(Seq *q, const int *tokens_dev, int n) {
 	const bool par = c.block_kind == YALM_BLOCK_PARALLEL;
 	// a parallel block whose feed-forward has a norm of its own reads Hn2 = norm2(x)
 	const float *first_norm2 = (par && q->L[0].ff_kind != YALM_FF_NONE) ? q->L[0].norm2 : nullptr;
-	if (!pre) { // every portion starts in the same row of the stream (the greedy graph's pointers are static)
-		q->X = q->Xbase;
+	q->X = q->Xbase; // every portion starts in the same row of the stream (the greedy graph's pointers are static)
+	if (!pre)
 		q->In = q->X;
-	}
-	q->pend_wb = nullptr;
+	settled(q);
+	q->hn_final = false;
 	const bool fold = an_foldable(q, n);
-	// the closing norm of a sublayer: applied now, or owed to the product that reads the stream next
+	// the seam after a sublayer: applied now, or owed to the product that reads the stream next (identity outputs read the
+	// row that the seam rewrites: now)
 	auto close = [&](const float *wb, const float *w_next, const yalm_seq_layer *moe) {
 		if (c.block_kind == YALM_BLOCK_POST)
 			return post_close(q, wb, n, moe);
-		if (fold && !moe && !w_next) {
+		if (fold && !(moe && moe->identity > 0)) {
 			q->pend_wb = wb;
+			q->pend_next = w_next;
+			q->pend_moe = moe;
 			return (int)YALM_OK;
 		}
 		return add_norm(q, wb, w_next, n, moe);
@@ -1847,8 +1887,8 @@ static int enqueue_portion(Seq *q, const int *tokens_dev, int n) {
 		const yalm_seq_layer &l = q->L[li];
 		const float *next = pre && li + 1 < c.n_layers ? q->L[li + 1].norm1 : nullptr;
 		const int side = q->side_of[li];
-		if (l.mixer != YALM_MIX_ATTN || side >= 0)
-			TRY(flush_norm(q, n)); // only a lone attention mixer's input projection takes an owed norm
+		if (l.mixer == YALM_MIX_MEMORY || side >= 0)
+			TRY(flush_norm(q, n)); // the other mixers' input projections take an owed seam
 		q->Yout = q->Y;
 		const int own = in_rows(l), joint = side >= 0 && !q->L[side].w_in ? own + in_rows(q->L[side]) : 0;
 		if (joint) { // both mixers' input projections as one product
@@ -1893,12 +1933,19 @@ static int enqueue_portion(Seq *q, const int *tokens_dev, int n) {
 		if (l.ff_kind == YALM_FF_NONE) {
 			TRY(close(l.norm1b, next, nullptr));
 		} else {
-			const bool routed = post_routes(q, l); // the seam runs in the router's launch
-			const PostNorm pn{q->X, q->Y, l.norm1b, c.norm_eps, c.stream_scale, c.residual_scale, q->nk};
+			bool routed = post_routes(q, l); // the seam runs in the router's launch
+			PostNorm pn{q->X, q->Y, l.norm1b, c.norm_eps, c.stream_scale, c.residual_scale, q->nk};
 			if (!routed)
 				TRY(close(l.norm1b, pre ? l.norm2 : nullptr, nullptr));
-			if (l.ff_kind != YALM_FF_PLAIN)
-				TRY(flush_norm(q, n));
+			if (l.ff_kind == YALM_FF_MOE && q->pend_wb) {
+				if (q->pend_next && route_lds(q, l)) { // an owed seam with an opening norm, too
+					routed = true;
+					pn.w_next = q->pend_next;
+					pn.Hn = q->Hn;
+					settled(q);
+				} else
+					TRY(flush_norm(q, n));
+			}
 			TRY(l.ff_kind == YALM_FF_DENSE ? ff_dense(q, li, n, q->Y)
 			                               : (l.ff_kind == YALM_FF_PLAIN ? ff_plain(q, li, n, q->Y)
 			                                                             : ff_moe(q, li, n, routed ? &pn : nullptr)));
@@ -1908,6 +1955,10 @@ static int enqueue_portion(Seq *q, const int *tokens_dev, int n) {
 			HIPCHK(hipMemcpyAsync(q->dump + (size_t)li * n * c.width, q->X, (size_t)n * c.width * sizeof(float),
 			                      hipMemcpyDeviceToDevice, q->stream));
 	}
+	if (q->pend_wb && c.logit_scale == 1.0f) { // a single token's last seam: the final norm is its opening norm
+		q->pend_next = q->final_norm;
+		q->hn_final = true;
+	}
 	return flush_norm(q, n); // the last sublayer's norm, if still owed
 }
 
@@ -1915,9 +1966,9 @@ static int enqueue_portion(Seq *q, const int *tokens_dev, int n) {
 static int enqueue_logits(Seq *q, const int *rows_dev, int n_rows) {
 	const yalm_seq_config &c = q->c;
 	const dim3 ng(n_rows, q->nk == NK_TANH ? cdiv(c.width, SEQ_THREADS) : 1);
-	seq_norm_kernel<float><<<ng, SEQ_THREADS, 0, q->stream>>>(q->X, c.width, q->final_norm, c.norm_eps, c.width,
-	                                                              q->Hn, c.width, rows_dev, q->st, 0, q->nk,
-	                                                              c.logit_scale);
+	if (!q->hn_final)
+		seq_norm_kernel<float><<<ng, SEQ_THREADS, 0, q->stream>>>(q->X, c.width, q->final_norm, c.norm_eps, c.width,
+		                                                          q->Hn, c.width, rows_dev, q->st, 0, q->nk, c.logit_scale);
 	HIPCHK(hipGetLastError());
 	GemmArgs a = plain(q->Hn, c.width, q->head, c.width, q->logits, c.vocab, n_rows, c.vocab, c.width);
 	if (c.logit_softcap > 0.0f) {

@@ -1406,110 +1406,189 @@ __global__ __launch_bounds__(64 * NW) void seq_rows_kernel(GemmArgs a) {
 	}
 }
 
-// ---- one token, the previous sublayer's closing norm (rms or layer) folded in: x' = x + rs norm(y) wb is what
-// the product reads when sublayers read the stream itself. Every workgroup rebuilds x' once
-// (a thread KI groups of 4 entries, the row's statistics over the workgroup) into LDS, while
-// its waves' first weight rows are already in flight; then each wave multiplies RPW weight
-// rows: C[n] = epi(W[n] . x' + bias[n]). Workgroup 0 also writes x' to Xout, a second buffer
-// (the other workgroups still read X). K % 8 == 0, K <= 1024 KI, rows of W contiguous and
-// 16-byte aligned. Dynamic LDS: K floats.
-#define GAN_RPW 2
-template <class WT, int KI>
+// ---- one token, the seam before the product folded in: x' = x + rs norm(y) wb (norms with row statistics), y the
+// previous sublayer's result or (COMB) the routed experts' combine, and, where sublayers open with a norm,
+// h = norm(x') w_next; the product reads h (x' without w_next). Every workgroup rebuilds the row once (a thread KI groups
+// of 4 entries, statistics over the workgroup) into LDS, while its waves' first weight rows are already in flight; then
+// each wave multiplies rpw weight rows (GLU: pairs of rows). Workgroup 0 also writes x' to Xout, a second buffer (the other
+// workgroups still read X), and h to Hn. K % 8 == 0, K <= 1024 KI, rows of W contiguous and 16-byte aligned; nothing read
+// here is among the results. Dynamic LDS: K floats. A launch between two small products costs its 5 us: of a token of width
+// 2048 in 9 layers the 11 seams took 61 us and the products and routers that now hold them 111 us; these take 118 us.
+template <class WT, int KI, bool GLU, bool COMB>
 __global__ __launch_bounds__(SEQ_THREADS) void seq_gemv_an_kernel(const float *__restrict__ X, const float *__restrict__ Y,
                                                                   const float *__restrict__ wb, float eps, int nk, float rs,
-                                                                  int K,
-                                                                  float *__restrict__ Xout, const void *__restrict__ W,
-                                                                  int N, float *__restrict__ C,
-                                                                  const float *__restrict__ bias, int epi) {
+                                                                  int K, float *__restrict__ Xout,
+                                                                  const float *__restrict__ w_next, float *__restrict__ Hn,
+                                                                  const char *__restrict__ W, const char *__restrict__ W2, int N,
+                                                                  float *__restrict__ C, const float *__restrict__ bias, int epi,
+                                                                  float limit, int rpw, Combine cb) {
 	extern __shared__ __attribute__((aligned(16))) float xs[];
 	__shared__ float red[SEQ_THREADS / 64];
 	constexpr int KE = 2 * KI;                 // steps of 512 entries over a weight row
 	constexpr int NL = WT::BYTES == 2 ? 1 : 2; // 16-byte loads per 8 weights
 	const int tid = threadIdx.x, lane = tid & 63;
-	const int n0 = (blockIdx.x * (SEQ_THREADS / 64) + (tid >> 6)) * GAN_RPW;
-	u32x4_t wv[KE][NL];
+	const int n0 = (blockIdx.x * (SEQ_THREADS / 64) + (tid >> 6)) * rpw;
+	u32x4_t wv[KE][NL], wv2[GLU ? KE : 1][NL];
 	auto fetch = [&](int n) {
-		const char *w = (const char *)W + (size_t)n * K * WT::BYTES;
+		const size_t row = (size_t)n * K * WT::BYTES;
 #pragma unroll
 		for (int u = 0; u < KE; ++u) {
 			const int k = u * 512 + lane * 8;
 #pragma unroll
-			for (int i = 0; i < NL; ++i)
-				wv[u][i] = (n < N && k < K) ? load_nt16(w + (size_t)k * WT::BYTES + 16 * i) : u32x4_t{0, 0, 0, 0};
+			for (int i = 0; i < NL; ++i) {
+				const size_t off = row + (size_t)k * WT::BYTES + 16 * i;
+				wv[u][i] = (n < N && k < K) ? load_nt16(W + off) : u32x4_t{0, 0, 0, 0};
+				if constexpr (GLU)
+					wv2[u][i] = (n < N && k < K) ? load_nt16(W2 + off) : u32x4_t{0, 0, 0, 0};
+			}
 		}
 	};
 	fetch(n0);
-	float4_t x[KI], y[KI], b[KI], bb[KI]; // bb: the bias of a layer norm that has one
-	float sm = 0.0f;
+	float4_t x[KI], y[KI], b[KI], wn[KI];
 #pragma unroll
 	for (int i = 0; i < KI; ++i) {
 		const int k = 4 * (tid + SEQ_THREADS * i);
 		const bool in = k < K;
-		y[i] = in ? *(const float4_t *)(Y + k) : float4_t{0, 0, 0, 0};
 		x[i] = in ? *(const float4_t *)(X + k) : float4_t{0, 0, 0, 0};
 		b[i] = in ? *(const float4_t *)(wb + k) : float4_t{0, 0, 0, 0};
-		bb[i] = (in && nk == NK_LAYER_B) ? *(const float4_t *)(wb + K + k) * rs : float4_t{0, 0, 0, 0};
-		sm += (y[i][0] + y[i][1]) + (y[i][2] + y[i][3]);
+		wn[i] = (in && w_next) ? *(const float4_t *)(w_next + k) : float4_t{0, 0, 0, 0};
+		if constexpr (!COMB)
+			y[i] = in ? *(const float4_t *)(Y + k) : float4_t{0, 0, 0, 0};
 	}
-	if (nk_centred(nk)) { // entries past the row's end stay 0
-		const float mu = block_sum(sm, red) / (float)K;
+	if constexpr (COMB) { // four choices' rows in flight at a time, summed in slot order, the shared expert's last
+#pragma unroll
+		for (int i = 0; i < KI; ++i)
+			y[i] = float4_t{0, 0, 0, 0};
+		for (int k0 = 0; k0 < cb.top; k0 += 4) {
+			float4_t v[4][KI];
+			float w[4];
+#pragma unroll
+			for (int u = 0; u < 4; ++u) {
+				const int c = min(k0 + u, cb.top - 1);
+				w[u] = combine_weight(cb.wt, c);
+#pragma unroll
+				for (int i = 0; i < KI; ++i)
+					v[u][i] = *(const float4_t *)(cb.Yx + (size_t)c * K + min(4 * (tid + SEQ_THREADS * i), K - 4));
+			}
+#pragma unroll
+			for (int u = 0; u < 4; ++u)
+				if (k0 + u < cb.top)
+#pragma unroll
+					for (int i = 0; i < KI; ++i)
+#pragma unroll
+						for (int e = 0; e < 4; ++e)
+							y[i][e] = fmaf(w[u], v[u][i][e], y[i][e]);
+		}
+		if (cb.Ys) {
+			const float sg = cb.sgate ? cb.sgate[0] : 1.0f;
+#pragma unroll
+			for (int i = 0; i < KI; ++i) {
+				const float4_t v = *(const float4_t *)(cb.Ys + min(4 * (tid + SEQ_THREADS * i), K - 4));
+#pragma unroll
+				for (int e = 0; e < 4; ++e)
+					y[i][e] = fmaf(sg, v[e], y[i][e]);
+			}
+		}
+#pragma unroll
+		for (int i = 0; i < KI; ++i)
+			if (4 * (tid + SEQ_THREADS * i) >= K)
+				y[i] = float4_t{0, 0, 0, 0};
+	}
+	auto sum4 = [&](const float4_t *v) {
+		float s = 0.0f;
+#pragma unroll
+		for (int i = 0; i < KI; ++i)
+			s += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
+		return s;
+	};
+	auto squares = [&](const float4_t *v) {
+		float s = 0.0f;
+#pragma unroll
+		for (int i = 0; i < KI; ++i)
+#pragma unroll
+			for (int e = 0; e < 4; ++e)
+				s = fmaf(v[i][e], v[i][e], s);
+		return s;
+	};
+	auto centre = [&](float4_t *v, float mu) { // entries past the row's end stay 0
 #pragma unroll
 		for (int i = 0; i < KI; ++i)
 			if (4 * (tid + SEQ_THREADS * i) < K)
 #pragma unroll
 				for (int e = 0; e < 4; ++e)
-					y[i][e] -= mu;
-	}
-	float ss = 0.0f;
-#pragma unroll
-	for (int i = 0; i < KI; ++i)
-#pragma unroll
-		for (int e = 0; e < 4; ++e)
-			ss = fmaf(y[i][e], y[i][e], ss);
-	const float r = rs / sqrtf(block_sum(ss, red) / (float)K + eps);
+					v[i][e] -= mu;
+	};
+	if (nk_centred(nk))
+		centre(y, block_sum(sum4(y), red) / (float)K);
+	const float r = rs / sqrtf(block_sum(squares(y), red) / (float)K + eps);
 #pragma unroll
 	for (int i = 0; i < KI; ++i) {
 		const int k = 4 * (tid + SEQ_THREADS * i);
 		if (k >= K)
-			continue;
+			continue; // x is 0 there
 #pragma unroll
 		for (int e = 0; e < 4; ++e)
-			x[i][e] = fmaf(y[i][e] * r, b[i][e], x[i][e] + bb[i][e]);
-		*(float4_t *)(xs + k) = x[i];
+			x[i][e] = fmaf(y[i][e] * r, b[i][e], x[i][e] + rs * norm_bias(nk, wb, K, k + e));
 		if (blockIdx.x == 0)
 			*(float4_t *)(Xout + k) = x[i];
 	}
-	__syncthreads();
+	if (w_next) {
+		if (nk_centred(nk))
+			centre(x, block_sum(sum4(x), red) / (float)K);
+		const float r2 = 1.0f / sqrtf(block_sum(squares(x), red) / (float)K + eps);
 #pragma unroll
-	for (int j = 0; j < GAN_RPW; ++j) {
+		for (int i = 0; i < KI; ++i) {
+			const int k = 4 * (tid + SEQ_THREADS * i);
+			if (k >= K)
+				continue;
+#pragma unroll
+			for (int e = 0; e < 4; ++e)
+				x[i][e] = x[i][e] * r2 * wn[i][e] + norm_bias(nk, w_next, K, k + e);
+			if (blockIdx.x == 0)
+				*(float4_t *)(Hn + k) = x[i];
+		}
+	}
+#pragma unroll
+	for (int i = 0; i < KI; ++i) {
+		const int k = 4 * (tid + SEQ_THREADS * i);
+		if (k < K)
+			*(float4_t *)(xs + k) = x[i];
+	}
+	__syncthreads();
+	GemmArgs a;
+	a.epi = epi;
+	for (int j = 0; j < rpw; ++j) {
 		const int n = n0 + j;
-		float acc = 0.0f;
+		float acc = 0.0f, acc2 = 0.0f;
 #pragma unroll
 		for (int u = 0; u < KE; ++u) {
 			const int k = u * 512 + lane * 8;
 			if (k >= K)
 				continue;
-			float wf[8];
-			if constexpr (WT::BYTES == 2) {
-				WT::unpack(wv[u][0], wf);
-			} else {
-				WT::unpack(wv[u][0], wf);
-				WT::unpack(wv[u][NL - 1], wf + 4);
-			}
 			const float4_t x0 = *(const float4_t *)(xs + k), x1 = *(const float4_t *)(xs + k + 4);
+			auto dot = [&](const u32x4_t *w, float s) {
+				float wf[8];
+				WT::unpack(w[0], wf);
+				if constexpr (WT::BYTES != 2)
+					WT::unpack(w[NL - 1], wf + 4);
 #pragma unroll
-			for (int e = 0; e < 4; ++e) {
-				acc = fmaf(wf[e], x0[e], acc);
-				acc = fmaf(wf[4 + e], x1[e], acc);
-			}
+				for (int e = 0; e < 4; ++e) {
+					s = fmaf(wf[e], x0[e], s);
+					s = fmaf(wf[4 + e], x1[e], s);
+				}
+				return s;
+			};
+			acc = dot(wv[u], acc);
+			if constexpr (GLU)
+				acc2 = dot(wv2[u], acc2);
 		}
-		if (j + 1 < GAN_RPW)
+		if (j + 1 < rpw)
 			fetch(n + 1); // the next row's loads run under this row's reduction
 		acc = wave_sum(acc);
-		if (lane == 0 && n < N) {
-			const float v = acc + (bias ? bias[n] : 0.0f);
-			C[n] = epi == EPI_GELU ? sq_gelu_tanh(v) : v;
-		}
+		if constexpr (GLU)
+			acc2 = wave_sum(acc2);
+		if (lane == 0 && n < N)
+			C[n] = epi_apply(a, acc, acc2, bias ? bias[n] : 0.0f, limit);
 	}
 }
 
@@ -3055,6 +3134,9 @@ struct PostNorm {
 	const float *Y = nullptr, *wb = nullptr;
 	float eps = 0.0f, alpha = 1.0f, rs = 1.0f;
 	int nk = NK_RMS;
+	// the seam of a serial block instead: x <- x + rs norm(y) wb, and the row is norm(x) w_next, written to Hn
+	const float *w_next = nullptr;
+	float *Hn = nullptr;
 };
 template <int NT>
 __device__ __forceinline__ float block_sum_of(float v, float *red) { // block_sum over NT threads
@@ -3088,7 +3170,33 @@ __global__ __launch_bounds__(NT) void seq_router_kernel(const float *__restrict_
 		const float *y = pn.Y + (size_t)t * width;
 		const int n = width;
 		float sm = 0.0f, ss = 0.0f;
-		for (int i = threadIdx.x; i < n; i += NT) { // each thread re-reads the entries it wrote
+		const bool serial = pn.w_next != nullptr; // the row so far: y, normed and added to x first
+		if (serial) {
+			for (int i = threadIdx.x; i < n; i += NT) {
+				const float v = y[i];
+				sm += v;
+				ss = fmaf(v, v, ss);
+			}
+			float mu = 0.0f;
+			if (nk_centred(pn.nk)) {
+				mu = block_sum_of<NT>(sm, pred) / (float)n;
+				ss = 0.0f;
+				for (int i = threadIdx.x; i < n; i += NT) {
+					const float d = y[i] - mu;
+					ss = fmaf(d, d, ss);
+				}
+			}
+			const float r = pn.rs / sqrtf(block_sum_of<NT>(ss, pred) / (float)n + pn.eps);
+			sm = ss = 0.0f;
+			for (int i = threadIdx.x; i < n; i += NT) {
+				const float v = x[i] + ((y[i] - mu) * r * pn.wb[i] + pn.rs * norm_bias(pn.nk, pn.wb, n, i));
+				row[i] = v;
+				x[i] = v;
+				sm += v;
+				ss = fmaf(v, v, ss);
+			}
+		}
+		for (int i = threadIdx.x; i < n && !serial; i += NT) { // each thread re-reads the entries it wrote
 			const float v = fmaf(pn.alpha, x[i], pn.rs * y[i]);
 			row[i] = v;
 			sm += v;
@@ -3105,11 +3213,13 @@ __global__ __launch_bounds__(NT) void seq_router_kernel(const float *__restrict_
 		}
 		if (pn.nk != NK_TANH)
 			r = 1.0f / sqrtf(block_sum_of<NT>(ss, pred) / (float)n + pn.eps);
+		const float *wo = serial ? pn.w_next : pn.wb;
+		float *out = serial ? pn.Hn + (size_t)t * width : x;
 		for (int i = threadIdx.x; i < n; i += NT) {
-			const float v = pn.nk == NK_TANH ? tanh_norm(pn.wb, n, i, row[i])
-			                                 : fmaf((row[i] - mu) * r, pn.wb[i], norm_bias(pn.nk, pn.wb, n, i));
+			const float v = pn.nk == NK_TANH ? tanh_norm(wo, n, i, row[i])
+			                                 : fmaf((row[i] - mu) * r, wo[i], norm_bias(pn.nk, wo, n, i));
 			row[i] = v;
-			x[i] = v;
+			out[i] = v;
 		}
 		__syncthreads();
 		h = row;
