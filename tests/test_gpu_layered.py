@@ -190,6 +190,25 @@ def test_token_seams_inside_products(rt, width):
         model.close()
 
 
+@pytest.mark.parametrize("rank", [8, 36, 64, 100, 132, 256])
+def test_latent_portions_bf16(rt, rank):
+    """Latent attention of portions on the matrix cores: ranks within and past a 32-deep step, row blocks and key tiles
+    with remainders, portions that start at keys of earlier ones."""
+    from yalm_amd import models as M
+
+    cfg = C.config([("latent_attention", C.latent(heads=5, dim=16, vdim=16, kv_rank=rank, q_rank=32, scale=0.3), None),
+                    ("latent_attention", C.latent(heads=5, dim=16, vdim=16, kv_rank=rank, q_rank=32, scale=0.3), None)],
+                   width=64, vocab=101)
+    model, dec, w = build(rt, cfg, M.BF16, seed=9)
+    try:
+        tok = C.tokens(cfg, 145, 6)
+        got = run_portions(dec, tok, [70, 1, 13, 33, 28])
+        assert close_enough(got, R.forward(cfg, w, tok), "bf16")
+    finally:
+        dec.close()
+        model.close()
+
+
 @pytest.mark.parametrize("n", [9, 16, 17, 32, 33, 64, 65, 130, 255])
 def test_few_row_products_bf16(rt, n):
     """Products of 9 to 255 rows on the prefill unit: streamed in one or several K slices, large tiles in slices."""

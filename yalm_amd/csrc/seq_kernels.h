@@ -2976,8 +2976,15 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_latent_merge_kernel(const flo
 // v_mfma_f32_16x16x32_bf16 products with f32 accumulation whose f32 operands (q~ * scale, the
 // softmax weights) enter as hi + lo bf16 pairs (hi = bf16(x), lo = bf16(x - hi): 16 significant
 // bits), the cached latent being bf16 already. Maximum, exponentials, running sums and the
-// rescaling of the sums stay f32, in the MFMA's C layout (row = 4 (lane >> 4) + reg, column =
-// lane & 15), where a row's 16 columns are the 16 lanes of a DPP row. KS = ceil(rank / 32).
+// rescaling of the sums stay f32. KS = ceil(rank / 32). Both products are computed transposed,
+// S^T = C Q^T and O^T = C^T P^T (C/D layout: row = 4 (lane >> 4) + reg, column = lane & 15): a lane's scores all belong to
+// one query row, column lane & 15, so the maximum takes two exchanges between lanes, the sums none until the end, and the
+// weights a lane holds, keys 4 q + e and 16 + 4 q + e (q = lane >> 4), are its own B fragment of the second product; the
+// transposed tile keeps its keys in that order. A tile comes through registers, loaded while the tile before is worked on:
+// a thread holds 4 keys x 8 entries and writes them by rows (16 bytes) and, turned round in registers, by columns (8 bytes).
+// Workgroups take the row blocks with the most keys first, so a CU's two workgroups see equally many keys together.
+// The LDS reads (32 KB a wave and tile) and the matrix cores are about even. 2048 rows of 16 heads, rank 256: 513 us with
+// the weights through LDS and the transposed tile written 2 bytes at a time (16 lanes on a bank), 167 us so.
 typedef float f32x4a_t __attribute__((ext_vector_type(4)));
 #define ATM_BR 64
 #define ATM_KT 32
@@ -2988,125 +2995,144 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_latent_attn_mfma_kernel(const
                                                                            const StepState *__restrict__ st,
                                                                            float *__restrict__ Ctx) {
 	constexpr int R32 = 32 * KS, NT = 2 * KS; // padded rank, 16-wide output tiles
-	constexpr int LDC = R32 + 8, LDT = ATM_KT + 8, LDP = ATM_KT + 8;
+	constexpr int LDC = R32 + 8, LDT = ATM_KT + 8;
+	constexpr int ND8 = R32 / 8; // 8-entry pieces of a latent; ATM_KT / 4 * ND8 <= SEQ_THREADS
 	__shared__ __attribute__((aligned(16))) uint16_t Cs[ATM_KT * LDC]; // [key][latent entry]
-	__shared__ __attribute__((aligned(16))) uint16_t CsT[R32 * LDT];   // [latent entry][key]
-	__shared__ __attribute__((aligned(16))) uint16_t Ps[4][2][16 * LDP]; // per wave: weights hi / lo [row][key]
+	__shared__ __attribute__((aligned(16))) uint16_t CsT[R32 * LDT];   // [latent entry][8 q + 4 h + e: key 16 h + 4 q + e]
 	const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
 	const int lr = lane & 15, lq = lane >> 4;
-	const int r0 = blockIdx.x * ATM_BR;
+	const int nb = gridDim.x, hb = (nb + 1) / 2, bx = blockIdx.x;
+	const int r0 = (bx < hb ? nb - 1 - bx : bx - hb) * ATM_BR;
 	const int pos0 = st->pos;
 	const int rlast = min(r0 + ATM_BR, NR) - 1;
 	const int nkeys = pos0 + rlast / H + 1;
-	// this lane's A-operand row of q~ (row lr of the wave), as hi / lo fragments per 32-deep step
+	const int row = r0 + wave * 16 + lr; // this lane's query row
+	// its B-operand entries of q~, as hi / lo fragments per 32-deep step
 	bf16x8_t qh[KS], ql[KS];
-	{
-		const int r = r0 + wave * 16 + lr;
 #pragma unroll
-		for (int sst = 0; sst < KS; ++sst) {
-			u32x4_t hi = {0, 0, 0, 0}, lo = {0, 0, 0, 0};
+	for (int sst = 0; sst < KS; ++sst) {
+		u32x4_t hi = {0, 0, 0, 0}, lo = {0, 0, 0, 0};
 #pragma unroll
-			for (int e = 0; e < 8; ++e) {
-				const int d = 32 * sst + 8 * lq + e;
-				const float x = (r < NR && d < rank) ? Qa[(size_t)r * rank + d] * scale : 0.0f;
-				const uint16_t hb = f2bf(x);
-				const uint16_t lb = f2bf(x - bf2f(hb));
-				hi[e >> 1] |= (uint32_t)hb << (16 * (e & 1));
-				lo[e >> 1] |= (uint32_t)lb << (16 * (e & 1));
-			}
-			qh[sst] = __builtin_bit_cast(bf16x8_t, hi);
-			ql[sst] = __builtin_bit_cast(bf16x8_t, lo);
+		for (int e = 0; e < 8; ++e) {
+			const int d = 32 * sst + 8 * lq + e;
+			const float x = (row < NR && d < rank) ? Qa[(size_t)row * rank + d] * scale : 0.0f;
+			const uint16_t hb16 = f2bf(x);
+			const uint16_t lb16 = f2bf(x - bf2f(hb16));
+			hi[e >> 1] |= (uint32_t)hb16 << (16 * (e & 1));
+			lo[e >> 1] |= (uint32_t)lb16 << (16 * (e & 1));
 		}
+		qh[sst] = __builtin_bit_cast(bf16x8_t, hi);
+		ql[sst] = __builtin_bit_cast(bf16x8_t, lo);
 	}
-	int lim[4];
-	float mrun[4], lrun[4];
-#pragma unroll
-	for (int g = 0; g < 4; ++g) {
-		const int r = r0 + wave * 16 + 4 * lq + g;
-		lim[g] = r < NR ? pos0 + r / H : -1;
-		mrun[g] = -FLT_MAX;
-		lrun[g] = 0.0f;
-	}
+	const int lim = row < NR ? pos0 + row / H : -1;
+	float mrun = -FLT_MAX, lrun = 0.0f; // lrun: of this lane's keys only
 	f32x4a_t oacc[NT];
 #pragma unroll
 	for (int n = 0; n < NT; ++n)
 		oacc[n] = f32x4a_t{0.0f, 0.0f, 0.0f, 0.0f};
 	const bool cvec = rank % 8 == 0 && (size_t)cache % 16 == 0;
-	for (int kt = 0; kt < nkeys; kt += ATM_KT) {
-		__syncthreads(); // the previous tile's products have read Cs / CsT / Ps
-		for (int v = tid; v < ATM_KT * (R32 / 8); v += SEQ_THREADS) {
-			const int jj = v / (R32 / 8), d8 = (v % (R32 / 8)) * 8, j = kt + jj;
-			u32x4_t w = {0, 0, 0, 0};
-			if (j < nkeys) {
-				const uint16_t *src = cache + (size_t)j * rank + d8;
-				if (cvec && d8 + 8 <= rank) {
-					w = load16(src);
-				} else {
+	const int kg = tid & 7, d8 = (tid >> 3) * 8; // the thread's 4 keys and 8 entries of a tile
+	const bool stages = tid < ATM_KT / 4 * ND8;
+	u32x4_t w[4];
+	auto load_tile = [&](int kt) {
 #pragma unroll
-					for (int e = 0; e < 8; ++e)
-						if (d8 + e < rank)
-							w[e >> 1] |= (uint32_t)src[e] << (16 * (e & 1));
-				}
+		for (int k = 0; k < 4; ++k) {
+			const int j = kt + 4 * kg + k;
+			w[k] = u32x4_t{0, 0, 0, 0};
+			if (!stages || j >= nkeys)
+				continue;
+			const uint16_t *src = cache + (size_t)j * rank + d8;
+			if (cvec && d8 + 8 <= rank) {
+				w[k] = load16(src);
+			} else {
+#pragma unroll
+				for (int e = 0; e < 8; ++e)
+					if (d8 + e < rank)
+						w[k][e >> 1] |= (uint32_t)src[e] << (16 * (e & 1));
 			}
-			*(u32x4_t *)(Cs + jj * LDC + d8) = w;
+		}
+	};
+	load_tile(0);
+	for (int kt = 0; kt < nkeys; kt += ATM_KT) {
+		__syncthreads(); // the previous tile's products have read Cs / CsT
+		if (stages) {
 #pragma unroll
-			for (int e = 0; e < 8; ++e)
-				CsT[(d8 + e) * LDT + jj] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
+			for (int k = 0; k < 4; ++k)
+				*(u32x4_t *)(Cs + (4 * kg + k) * LDC + d8) = w[k];
+			uint16_t *const to = CsT + d8 * LDT + 8 * (kg & 3) + 4 * (kg >> 2);
+#pragma unroll
+			for (int e = 0; e < 8; ++e) {
+				const uint32_t sel = e & 1 ? 0x07060302u : 0x05040100u; // the pair's upper or lower halves
+				*(uint2 *)(to + e * LDT) = uint2{__builtin_amdgcn_perm(w[1][e >> 1], w[0][e >> 1], sel),
+				                                 __builtin_amdgcn_perm(w[3][e >> 1], w[2][e >> 1], sel)};
+			}
 		}
 		__syncthreads();
+		load_tile(kt + ATM_KT);
 		f32x4a_t sacc[2] = {f32x4a_t{0.0f, 0.0f, 0.0f, 0.0f}, f32x4a_t{0.0f, 0.0f, 0.0f, 0.0f}};
 #pragma unroll
-		for (int jt = 0; jt < 2; ++jt)
+		for (int sst = 0; sst < KS; ++sst)
 #pragma unroll
-			for (int sst = 0; sst < KS; ++sst) {
-				const bf16x8_t kb =
+			for (int jt = 0; jt < 2; ++jt) {
+				const bf16x8_t ka =
 				    __builtin_bit_cast(bf16x8_t, *(const u32x4_t *)(Cs + (16 * jt + lr) * LDC + 32 * sst + 8 * lq));
-				sacc[jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qh[sst], kb, sacc[jt], 0, 0, 0);
-				sacc[jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ql[sst], kb, sacc[jt], 0, 0, 0);
+				sacc[jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, qh[sst], sacc[jt], 0, 0, 0);
+				sacc[jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka, ql[sst], sacc[jt], 0, 0, 0);
 			}
-		float al[4];
+		float sv[8], mt = -FLT_MAX;
 #pragma unroll
-		for (int g = 0; g < 4; ++g) {
-			const bool v0 = kt + lr <= lim[g], v1 = kt + 16 + lr <= lim[g];
-			const float s0 = v0 ? sacc[0][g] : -FLT_MAX, s1 = v1 ? sacc[1][g] : -FLT_MAX;
-			const float mnew = fmaxf(mrun[g], row16_max(fmaxf(s0, s1)));
-			const float p0 = v0 ? expf(s0 - mnew) : 0.0f, p1 = v1 ? expf(s1 - mnew) : 0.0f;
-			al[g] = expf(mrun[g] - mnew);
-			lrun[g] = lrun[g] * al[g] + row16_sum(p0 + p1);
-			mrun[g] = mnew;
-			const int row = 4 * lq + g;
-			const uint16_t h0 = f2bf(p0), h1 = f2bf(p1);
-			Ps[wave][0][row * LDP + lr] = h0;
-			Ps[wave][0][row * LDP + 16 + lr] = h1;
-			Ps[wave][1][row * LDP + lr] = f2bf(p0 - bf2f(h0));
-			Ps[wave][1][row * LDP + 16 + lr] = f2bf(p1 - bf2f(h1));
+		for (int i = 0; i < 8; ++i) {
+			const int j = kt + 16 * (i >> 2) + 4 * lq + (i & 3);
+			sv[i] = j <= lim ? sacc[i >> 2][i & 3] : -FLT_MAX;
+			mt = fmaxf(mt, sv[i]);
 		}
+		mt = fmaxf(mt, __shfl_xor(mt, 16));
+		mt = fmaxf(mt, __shfl_xor(mt, 32));
+		const float mnew = fmaxf(mrun, mt);
+		const float al = expf(mrun - mnew);
+		mrun = mnew;
+		lrun *= al;
+		u32x4_t ph = {0, 0, 0, 0}, pl = {0, 0, 0, 0};
 #pragma unroll
-		for (int n = 0; n < NT; ++n)
+		for (int i = 0; i < 8; ++i) {
+			const int j = kt + 16 * (i >> 2) + 4 * lq + (i & 3);
+			const float p = j <= lim ? expf(sv[i] - mnew) : 0.0f;
+			lrun += p;
+			const uint16_t h16 = f2bf(p);
+			ph[i >> 1] |= (uint32_t)h16 << (16 * (i & 1));
+			pl[i >> 1] |= (uint32_t)f2bf(p - bf2f(h16)) << (16 * (i & 1));
+		}
+		if (__any(al != 1.0f)) {
 #pragma unroll
-			for (int g = 0; g < 4; ++g)
-				oacc[n][g] *= al[g];
-		__syncthreads(); // the wave's weights are in LDS
-		const bf16x8_t ph = __builtin_bit_cast(bf16x8_t, *(const u32x4_t *)(&Ps[wave][0][lr * LDP + 8 * lq]));
-		const bf16x8_t pl = __builtin_bit_cast(bf16x8_t, *(const u32x4_t *)(&Ps[wave][1][lr * LDP + 8 * lq]));
+			for (int n = 0; n < NT; ++n)
+#pragma unroll
+				for (int g = 0; g < 4; ++g)
+					oacc[n][g] *= al;
+		}
+		const bf16x8_t pbh = __builtin_bit_cast(bf16x8_t, ph), pbl = __builtin_bit_cast(bf16x8_t, pl);
 #pragma unroll
 		for (int n = 0; n < NT; ++n) {
-			const bf16x8_t cb = __builtin_bit_cast(bf16x8_t, *(const u32x4_t *)(CsT + (16 * n + lr) * LDT + 8 * lq));
-			oacc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ph, cb, oacc[n], 0, 0, 0);
-			oacc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pl, cb, oacc[n], 0, 0, 0);
+			const bf16x8_t ca = __builtin_bit_cast(bf16x8_t, *(const u32x4_t *)(CsT + (16 * n + lr) * LDT + 8 * lq));
+			oacc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ca, pbh, oacc[n], 0, 0, 0);
+			oacc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ca, pbl, oacc[n], 0, 0, 0);
 		}
 	}
+	lrun += __shfl_xor(lrun, 16);
+	lrun += __shfl_xor(lrun, 32);
+	if (row >= NR)
+		return;
+	const float inv = 1.0f / lrun;
 #pragma unroll
-	for (int g = 0; g < 4; ++g) {
-		const int r = r0 + wave * 16 + 4 * lq + g;
-		if (r >= NR)
-			continue;
-		const float inv = 1.0f / lrun[g];
+	for (int n = 0; n < NT; ++n) {
+		const int d = 16 * n + 4 * lq;
+		float *out = Ctx + (size_t)row * rank + d;
+		if (rank % 4 == 0 && d < rank) {
+			*(float4_t *)out = float4_t{oacc[n][0] * inv, oacc[n][1] * inv, oacc[n][2] * inv, oacc[n][3] * inv};
+		} else {
 #pragma unroll
-		for (int n = 0; n < NT; ++n) {
-			const int d = 16 * n + lr;
-			if (d < rank)
-				Ctx[(size_t)r * rank + d] = oacc[n][g] * inv;
+			for (int g = 0; g < 4; ++g)
+				if (d + g < rank)
+					out[g] = oacc[n][g] * inv;
 		}
 	}
 }
