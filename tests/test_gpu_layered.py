@@ -209,6 +209,29 @@ def test_latent_portions_bf16(rt, rank):
         model.close()
 
 
+@pytest.mark.parametrize("experts, top, ff, n", [(4, 1, 64, 300), (16, 4, 128, 515), (64, 6, 192, 260), (3, 3, 64, 257), (5, 2, 448, 700)])
+def test_expert_groups_bf16(rt, experts, top, ff, n):
+    """Experts' rows as groups of the large tiles: experts without tokens, with part of a tile and with several."""
+    from yalm_amd import models as M
+
+    cfg = C.config([("rglru", C.rglru(width=64, blocks=2, conv=2),
+                     C.moe(ff=ff, experts=experts, top=top, groups=1, keep=1, shared=None if experts == 3 else (64, 0.75)))],
+                   width=192, vocab=97)
+    model, dec, w = build(rt, cfg, M.BF16, seed=4, max_tokens=800)
+    try:
+        tok = C.tokens(cfg, n, 7)
+        got = dec.step(tok, list(range(n)))
+        frac = 1.0 if top == experts else 0.95  # near ties of the router, as in the tests above
+        assert close_enough(got, R.forward(cfg, w, tok), "bf16", frac)
+        # the same rows in portions of few tokens, the experts by rows: rounding only
+        dec.reset()
+        few = run_portions(dec, tok, [32] * (n // 32))
+        assert close_enough(got, few, "bf16", frac)
+    finally:
+        dec.close()
+        model.close()
+
+
 @pytest.mark.parametrize("n", [9, 16, 17, 32, 33, 64, 65, 130, 255])
 def test_few_row_products_bf16(rt, n):
     """Products of 9 to 255 rows on the prefill unit: streamed in one or several K slices, large tiles in slices."""

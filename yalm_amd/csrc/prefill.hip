@@ -247,7 +247,7 @@ int launch_g8p(const PfForms &f, const uint16_t *A, int lda, int M, int K, int k
 	const int ncu = (int)device_cu_count();
 	const int grid = f.persist && nwg > ncu && !two && !pf::epi_partial<EPI>::value ? ncu : nwg;
 	hipLaunchKernelGGL(kern, dim3(grid), dim3(pf::G_THREADS), lds, st, A, lda, M, K, kb, bm, N, epi, c0,
-	                   two ? c_split : N, two ? K2 : K, nkc);
+	                   two ? c_split : N, two ? K2 : K, nkc, pf::GrpNone{});
 	HIPCHK(hipGetLastError());
 	return YALM_OK;
 }
@@ -1016,6 +1016,61 @@ int pf_gemm_glu_bf16(const uint16_t *A, int lda, int M, int K, const uint16_t *W
 	if (bn == 128)
 		return launch_g16_t<pf::E16GluB, pf::BRowsGlu<64>, 128, 4>(f, A, lda, M, K, K, bm, 2 * hidden, e, st);
 	return YALM_ERR_UNSUPPORTED;
+}
+
+// Products of groups of rows (routed experts): result row r of group g's list is A row r / a_div against the group's
+// matrices, w_bs elements after the group's before it. `rows`: an upper bound of the lists' entries together.
+// Width 256 or 128 by the time the expected tiles take (a group's last row tile half full), as plan_split counts it.
+template <class EPI, class BMAP256, class BMAP128>
+static int launch_groups(const uint16_t *A, int lda, int rows, int K, const BMAP256 &b256, const BMAP128 &b128, int N,
+                         bool whole256, const EPI &epi, const pf::GrpRows &g, hipStream_t st) {
+	const int ncu = (int)device_cu_count(), tm = rows / pf::G_BM + (g.n + 1) / 2;
+	auto cost = [&](int w, int bn) {
+		return (float)((tm * ((N + bn - 1) / bn) + ncu - 1) / ncu) * (K / pf::BK * T8P_KT[w] + T8P_TILE + T8P_EPI);
+	};
+	auto go = [&](auto kern, const auto &bm, size_t lds, int n, bool &attr) {
+		if (!attr) {
+			HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+			attr = true;
+		}
+		hipLaunchKernelGGL(kern, dim3(ncu), dim3(pf::G_THREADS), lds, st, A, lda, 0, K, K, bm, n, epi, 0, n, K, 1 << 24, g);
+		HIPCHK(hipGetLastError());
+		return (int)YALM_OK;
+	};
+	static bool a256 = false, a128 = false;
+	if (whole256 && cost(2, 256) <= cost(0, 128))
+		return go(pf::gemm8p_kernel<EPI, BMAP256, 2, 2, pf::GrpRows>, b256, pf::gemm8p_lds<2, 2>(), (N + 255) / 256 * 256, a256);
+	return go(pf::gemm8p_kernel<EPI, BMAP128, 1, 1, pf::GrpRows>, b128, pf::gemm8p_lds<1, 1>(), (N + 127) / 128 * 128, a128);
+}
+static bool groups_ok(const uint16_t *A, int lda, int rows, int K, const void *W, const void *W2, const pf::GrpRows &g) {
+	return rows > 0 && K % pf::BK == 0 && lda % 8 == 0 && ((size_t)A | (size_t)W | (size_t)W2) % 16 == 0 && g.w_bs % 8 == 0 &&
+	       g.n >= 1 && g.n <= 64 && (size_t)rows * lda < (size_t)1 << 32;
+}
+// The gated pair of the groups: C [rows][ldc] bf16 (mode / limit: E16GluB)
+int pf_groups_glu_bf16(const uint16_t *A, int lda, int rows, int K, const uint16_t *Wg, const uint16_t *Wu, int hidden,
+                       size_t w_bs, uint16_t *C, int ldc, int mode, float limit, const int *lists, int lists_bs,
+                       const int *counts, int n, int a_div, hipStream_t st) {
+	const pf::GrpRows g{lists, counts, n, lists_bs, a_div, w_bs};
+	if (!groups_ok(A, lda, rows, K, Wg, Wu, g) || hidden % 64 != 0)
+		return YALM_ERR_UNSUPPORTED;
+	pf::E16GluBT<true> e;
+	e.c = C;
+	e.ldc = ldc;
+	e.mode = mode;
+	e.limit = limit;
+	return launch_groups(A, lda, rows, K, pf::BRowsGlu<64>{Wg, Wu}, pf::BRowsGlu<32>{Wg, Wu}, 2 * hidden, hidden % 128 == 0, e, g, st);
+}
+// ... one matrix each, N rows: C [rows][ldc] f32
+int pf_groups_bf16(const uint16_t *A, int lda, int rows, int K, const uint16_t *W, int N, size_t w_bs, float *C, int ldc,
+                   const int *lists, int lists_bs, const int *counts, int n, int a_div, hipStream_t st) {
+	const pf::GrpRows g{lists, counts, n, lists_bs, a_div, w_bs};
+	if (!groups_ok(A, lda, rows, K, W, W, g))
+		return YALM_ERR_UNSUPPORTED;
+	pf::E16StoreRows e;
+	e.c = C;
+	e.ldc = ldc;
+	e.N = N;
+	return launch_groups(A, lda, rows, K, pf::BRowsRagged{W, N}, pf::BRowsRagged{W, N}, N, true, e, g, st);
 }
 
 extern "C" int yalm_gemm_f16(float *c, const uint16_t *a, const uint16_t *w, int M, int N, int K) {

@@ -206,13 +206,16 @@ struct E16StoreF32B {
 // FJ / 2, up columns j + FJ / 2 of the same hidden units), C f32: mode 1 gelu_tanh(g) u;
 // mode 2 g' sigmoid(1.702 g') (u' + 1) with g' = min(g, limit), u' = clamp(u, +-limit);
 // mode 3 g sigmoid(g) u.
-struct E16GluB {
+// ROWS: a group's rows (GrpRows): row m of the tile is result row rows[m], stored as bf16, the next product's operand.
+template <bool ROWS>
+struct E16GluBT {
 	static constexpr bool NEEDS_LDS = false;
 	static constexpr bool BF16 = true;
 	float *red = nullptr;
-	float *c;
+	std::conditional_t<ROWS, uint16_t, float> *c;
 	int ldc, M, mode;
 	float limit;
+	const int *rows = nullptr;
 	template <int MODE, int FI, int FJ>
 	__device__ __forceinline__ void apply_t(f32x4_t (&acc)[FI][FJ], int m0, int n0, int lane) const {
 #pragma unroll
@@ -222,6 +225,7 @@ struct E16GluB {
 				const int m = m0 + 16 * i + crow16(r, lane);
 				if (m >= M)
 					continue;
+				auto *const to = c + (size_t)(ROWS ? rows[m] : m) * ldc + n0 + (lane & 15);
 #pragma unroll
 				for (int j = 0; j < FJ / 2; ++j) {
 					const float g = acc[i][j][r], u = acc[i][j + FJ / 2][r];
@@ -234,7 +238,10 @@ struct E16GluB {
 						const float gc = fminf(g, limit), uc = fminf(fmaxf(u, -limit), limit);
 						v = sig_mul(gc, 1.702f * gc) * (uc + 1.0f);
 					}
-					c[(size_t)m * ldc + n0 + 16 * j + (lane & 15)] = v;
+					if constexpr (ROWS)
+						to[16 * j] = __builtin_bit_cast(uint16_t, (__bf16)v);
+					else
+						to[16 * j] = v;
 				}
 			}
 	}
@@ -246,6 +253,35 @@ struct E16GluB {
 			apply_t<3>(acc, m0, n0, lane);
 		else
 			apply_t<2>(acc, m0, n0, lane);
+	}
+};
+using E16GluB = E16GluBT<false>;
+
+// A group's rows (GrpRows), f32: row m of the tile is result row rows[m]
+struct E16StoreRows {
+	static constexpr bool NEEDS_LDS = false;
+	static constexpr bool BF16 = true;
+	float *red = nullptr;
+	float *c;
+	int ldc, M, N;
+	const int *rows = nullptr;
+	template <int FI, int FJ>
+	__device__ __forceinline__ void apply(f32x4_t (&acc)[FI][FJ], int m0, int n0, int lane, int, int) const {
+#pragma unroll
+		for (int i = 0; i < FI; ++i)
+#pragma unroll
+			for (int r = 0; r < 4; ++r) {
+				const int m = m0 + 16 * i + crow16(r, lane);
+				if (m >= M)
+					continue;
+				float *const to = c + (size_t)rows[m] * ldc;
+#pragma unroll
+				for (int j = 0; j < FJ; ++j) {
+					const int n = n0 + 16 * j + (lane & 15);
+					if (n < N)
+						to[n] = acc[i][j][r];
+				}
+			}
 	}
 };
 
@@ -705,10 +741,25 @@ struct epi_partial : std::false_type {};
 template <class EPI>
 struct epi_partial<EPI, std::void_t<decltype(EPI::PARTIAL)>> : std::bool_constant<EPI::PARTIAL> {};
 
-template <class EPI, class BMAP, int FJ0 = 2, int FJ1 = 2>
+// Groups (GrpRows; routed experts): group g is the rows of its list, A row rows[m] / a_div against the weights w_bs
+// further on per group, its row count known on the device only. The row tiles of the groups follow one another; a wave
+// holds the tiles' running sum, group g's in lane g (at most 64 groups), and a tile finds its group by ballot. The LDS-DMA
+// takes an address per lane, so the rows are gathered by it. The launch is persistent: one workgroup per CU.
+struct GrpNone {
+	static constexpr bool ON = false;
+};
+struct GrpRows {
+	static constexpr bool ON = true;
+	const int *rows, *counts; // group g's list at rows + g rows_bs, counts[g] entries
+	int n, rows_bs, a_div;
+	size_t w_bs; // weights per group (elements)
+};
+
+template <class EPI, class BMAP, int FJ0 = 2, int FJ1 = 2, class GRP = GrpNone>
 __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__restrict__ A, int lda, int M, int K,
                                                              int kb, BMAP bm, int N, EPI epi, int c0, int c_split,
-                                                             int K2, int nkc) {
+                                                             int K2, int nkc, GRP grp) {
+	static_assert(!GRP::ON || !epi_partial<EPI>::value, "groups: whole K");
 	constexpr int FI = 8, FJ = FJ0 + FJ1, TM = 128, TN = 16 * FJ, BN = 4 * TN;
 	using elt = bmap_elt<BMAP>;
 	constexpr int EB = sizeof(elt); // bytes per weight
@@ -730,7 +781,18 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
 	const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 	const int wr = wave >> 2, wc = wave & 3;
 
-	const int tiles_m = (M + G_BM - 1) / G_BM, tiles_n = N / BN;
+	int tiles_m = (M + G_BM - 1) / G_BM, cnt = 0, upto = 0; // groups: lane g's rows and row tiles up to and with group g
+	if constexpr (GRP::ON) {
+		cnt = lane < grp.n ? grp.counts[lane] : 0;
+		upto = (cnt + G_BM - 1) / G_BM;
+	#pragma unroll
+		for (int d = 1; d < 64; d <<= 1) {
+			const int below = __shfl_up(upto, d);
+			upto += lane >= d ? below : 0;
+		}
+		tiles_m = __builtin_amdgcn_readlane(upto, 63);
+	}
+	const int tiles_n = N / BN;
 	const int tn_split = c_split / BN; // column tiles with depth K
 	const int ks1 = epi_partial<EPI>::value ? (K / G_BK + nkc - 1) / nkc : 1;
 	const int ks2 = epi_partial<EPI>::value ? (K2 / G_BK + nkc - 1) / nkc : 1;
@@ -758,7 +820,16 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
 		const int tm = wg % tiles_m, tn = wg / tiles_m + (deep ? tn_split : 0);
 		const int Kt = deep ? K2 : K;
 		const int kt0 = ks * nkc; // first K tile of the slice
-		const int row0 = tm * G_BM;
+		int row0 = tm * G_BM;
+		const int *list = nullptr;
+		size_t woff = 0;
+		if constexpr (GRP::ON) {
+			const int g = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)__ballot(upto > tm)) - 1);
+			M = __builtin_amdgcn_readlane(cnt, g);
+			row0 = (tm - __builtin_amdgcn_readlane(upto, g) + (M + G_BM - 1) / G_BM) * G_BM;
+			list = grp.rows + (size_t)g * grp.rows_bs;
+			woff = g * grp.w_bs;
+		}
 		const int colB = c0 + tn * (BN / BMAP::COLS_PER_TILE_DIV); // c0: first column of this launch
 
 		// staging sources: instruction i of a half-tile covers its rows lr = (NI wave + i) * 8
@@ -771,8 +842,13 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
 			const int lr = (2 * wave + i) * 8 + (lane >> 3);
 			const int sw = 8 * ((lane & 7) ^ (lr & 7));
 			const int ra = lr < 64 ? lr : lr + 64; // Am0 tile row; Am1 = + 64
-			aoff[0][i] = (uint32_t)min(row0 + ra, M - 1) * lda + sw;
-			aoff[1][i] = (uint32_t)min(row0 + ra + 64, M - 1) * lda + sw;
+			if constexpr (GRP::ON) {
+				aoff[0][i] = (uint32_t)(list[min(row0 + ra, M - 1)] / grp.a_div) * lda + sw;
+				aoff[1][i] = (uint32_t)(list[min(row0 + ra + 64, M - 1)] / grp.a_div) * lda + sw;
+			} else {
+				aoff[0][i] = (uint32_t)min(row0 + ra, M - 1) * lda + sw;
+				aoff[1][i] = (uint32_t)min(row0 + ra + 64, M - 1) * lda + sw;
+			}
 		}
 		// (E5M2: 16 rows of 64 bytes per instruction, source chunk (lane & 3) ^ ((lr >> 2) & 3), g8frag)
 		const int w0 = HALF0 ? wave & 3 : wave, w1 = HALF1 ? wave & 3 : wave;
@@ -781,12 +857,12 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
 	#pragma unroll
 		for (int i = 0; i < NB0; ++i) {
 			const int lr = brow(NB0 * w0 + i);
-			bp[0][i] = bm.row(colB, (lr / (16 * FJ0)) * TN + lr % (16 * FJ0), kb) + bsw(lr);
+			bp[0][i] = bm.row(colB, (lr / (16 * FJ0)) * TN + lr % (16 * FJ0), kb) + woff + bsw(lr);
 		}
 	#pragma unroll
 		for (int i = 0; i < NB1; ++i) {
 			const int lr = brow(NB1 * w1 + i);
-			bp[1][i] = bm.row(colB, (lr / (16 * FJ1)) * TN + 16 * FJ0 + lr % (16 * FJ1), kb) + bsw(lr);
+			bp[1][i] = bm.row(colB, (lr / (16 * FJ1)) * TN + 16 * FJ0 + lr % (16 * FJ1), kb) + woff + bsw(lr);
 		}
 		// half-tile h (0 Am0, 1 Am1, 2 Bn0, 3 Bn1) of K tile kt into buffer buf
 		auto stage = [&](int buf, int h, int kt) {
@@ -979,6 +1055,10 @@ __global__ __launch_bounds__(G_THREADS, 1) void gemm8p_kernel(const uint16_t *__
 			e.red = (float *)smem;
 		if constexpr (epi_partial<EPI>::value)
 			e.part += (size_t)ks * e.kstride;
+		if constexpr (GRP::ON) {
+			e.M = M;
+			e.rows = list;
+		}
 		const int n0 = BMAP::COLS_PER_TILE_DIV == 1 ? colB + wc * TN : colB + wc * (TN / 2);
 		e.template apply<FI, FJ>(acc, row0 + wr * TM, n0, lane, wc, 4);
 	}

@@ -31,6 +31,11 @@ int pf_gemm_bf16(const uint16_t *A, int lda, int M, int K, const uint16_t *W, in
 int pf_gemm_glu_bf16(const uint16_t *A, int lda, int M, int K, const uint16_t *Wg, const uint16_t *Wu, int hidden,
                      float *C, int ldc, int mode, float limit, float *part, size_t part_floats, hipStream_t st)
     __attribute__((weak));
+int pf_groups_glu_bf16(const uint16_t *A, int lda, int rows, int K, const uint16_t *Wg, const uint16_t *Wu, int hidden,
+                       size_t w_bs, uint16_t *C, int ldc, int mode, float limit, const int *lists, int lists_bs,
+                       const int *counts, int n, int a_div, hipStream_t st) __attribute__((weak));
+int pf_groups_bf16(const uint16_t *A, int lda, int rows, int K, const uint16_t *W, int N, size_t w_bs, float *C, int ldc,
+                   const int *lists, int lists_bs, const int *counts, int n, int a_div, hipStream_t st) __attribute__((weak));
 
 struct yalm_seq_s {
 	yalm_seq_config c{};
@@ -834,6 +839,13 @@ static int gemm_t(Seq *q, const GemmArgs &a, int batches, int max_m) {
 	return YALM_OK;
 }
 // f32w: the matrices are f32 whatever the model's weight type (the recurrence's gates)
+static int to_bf16(Seq *q, const float *A, int lda, int M, int K) { // A's rows into q->a16
+	const size_t n8 = (size_t)M * (K / 8);
+	seq_to_bf16_kernel<<<(unsigned)std::min<size_t>((n8 + SEQ_THREADS - 1) / SEQ_THREADS, 4096), SEQ_THREADS, 0, q->stream>>>(
+	    A, lda, M, K, q->a16);
+	HIPCHK(hipGetLastError());
+	return YALM_OK;
+}
 static int gemm(Seq *q, const GemmArgs &a, int batches = 1, int max_m = -1, bool f32w = false) {
 	if (max_m < 0)
 		max_m = a.M;
@@ -846,10 +858,7 @@ static int gemm(Seq *q, const GemmArgs &a, int batches = 1, int max_m = -1, bool
 	const int act1 = a.epi == EPI_GELU ? 1 : (a.epi == EPI_RELU2 ? 2 : (a.epi == EPI_GELU_ERF ? 3 : 0)); // the large-tile door's activation
 	if (q->a16 && batches == 1 && max_m > GEMV_MAX_M && !a.rows && !a.row_scale && !a.gate && !a.w_sel && a.z_split == 0 && a.ldw == a.K &&
 	    a.K % 64 == 0 && (pair ? a.N % 64 == 0 : (single && a.N >= 128))) {
-		const size_t n8 = (size_t)a.M * (a.K / 8);
-		seq_to_bf16_kernel<<<(unsigned)std::min<size_t>((n8 + SEQ_THREADS - 1) / SEQ_THREADS, 4096), SEQ_THREADS, 0,
-		                     q->stream>>>(a.A, a.lda, a.M, a.K, q->a16);
-		HIPCHK(hipGetLastError());
+		TRY(to_bf16(q, a.A, a.lda, a.M, a.K));
 		const int rc =
 		    pair ? pf_gemm_glu_bf16(q->a16, a.K, a.M, a.K, (const uint16_t *)a.W, (const uint16_t *)a.W2, a.N, a.C, a.ldc,
 		                            a.epi == EPI_GLU_GELU ? 1 : (a.epi == EPI_GLU_CLAMP ? 2 : 3), a.limit, q->gpart,
@@ -1611,6 +1620,21 @@ static bool post_routes(const Seq *q, const yalm_seq_layer &l) {
 	return q->c.block_kind == YALM_BLOCK_POST && l.ff_kind == YALM_FF_MOE && l.router_kind >= YALM_ROUTER_SOFTMAX_NORMED &&
 	       route_lds(q, l);
 }
+// The experts that every token passes through. The combine of the routed experts' rows (B[1]) and theirs (B[3]) happens
+// in the closing norm's launch (add_norm, par_close).
+static int ff_shared(Seq *q, int li, int n) {
+	const yalm_seq_layer &l = q->L[li];
+	const yalm_seq_config &c = q->c;
+	if (l.shared_ff <= 0)
+		return YALM_OK;
+	const bool glu = l.w_gate != nullptr;
+	GemmArgs a = plain(q->In, c.width, glu ? l.ws_gate : l.ws_up, c.width, q->B[2], l.shared_ff, n, l.shared_ff, c.width);
+	a.W2 = glu ? l.ws_up : nullptr;
+	a.epi = glu ? glu_epi(l, EPI_GLU_CLAMP) : plain_epi(l);
+	a.limit = l.shared_limit;
+	TRY(gemm(q, a));
+	return gemm(q, plain(q->B[2], l.shared_ff, l.ws_down, l.shared_ff, q->B[3], c.width, n, c.width, l.shared_ff));
+}
 static int ff_moe(Seq *q, int li, int n, const PostNorm *pn = nullptr) {
 	const yalm_seq_layer &l = q->L[li];
 	const yalm_seq_config &c = q->c;
@@ -1680,6 +1704,27 @@ static int ff_moe(Seq *q, int li, int n, const PostNorm *pn = nullptr) {
 		seq_moe_lists_kernel<<<cdiv(slots, SEQ_THREADS), SEQ_THREADS, 2 * E * sizeof(int), q->stream>>>(q->idx, slots, q->counts, q->lists,
 		                                                                              q->cap, E);
 		HIPCHK(hipGetLastError());
+		// both products on the prefill unit's large tiles, the experts' rows as groups and the hidden rows between them bf16, as
+		// the products round them anyway. 2048 tokens, 16 experts of 896 x 2048, four a token: 267 + 134 us on 128-row tiles
+		// (seq_gemm_bf16_kernel), 105 + 78 so. Few rows an expert: a tile's time does not fall with them, that of seq_rows_kernel
+		// does, and with the width. Both products, rows against groups: width 2048, 64 tokens 87 : 64 us, 32 tokens 61 : 63;
+		// width 1024, the whole portion, 64 tokens 743 : 785 us, 128 tokens 940 : 945, 256 tokens 1150 : 1103.
+		const bool many = n > ROWS_MAX_M || (n > GEMV_MAX_M && (long)slots * c.width >= (long)E * 32768);
+		if (many && glu && q->a16 && !l.expert_in_weighted && (epi == EPI_GLU_GELU || epi == EPI_GLU_CLAMP || epi == EPI_GLU_SILU) && E <= 64 &&
+		    ff % 64 == 0 && c.width % 64 == 0) {
+			TRY(to_bf16(q, q->In, c.width, n, c.width));
+			uint16_t *h16 = (uint16_t *)hx;
+			int rc = pf_groups_glu_bf16(q->a16, c.width, slots, c.width, (const uint16_t *)l.w_gate, (const uint16_t *)l.w_up, ff,
+			                            (size_t)ff * c.width, h16, ff, epi == EPI_GLU_GELU ? 1 : (epi == EPI_GLU_CLAMP ? 2 : 3), l.limit,
+			                            q->lists, q->cap, q->counts, E, top, q->stream);
+			if (rc == YALM_OK)
+				rc = pf_groups_bf16(h16, ff, slots, ff, (const uint16_t *)l.w_down, c.width, (size_t)c.width * ff, yx, c.width, q->lists,
+				                    q->cap, q->counts, E, 1, q->stream);
+			if (rc == YALM_OK)
+				return ff_shared(q, li, n);
+			if (rc != YALM_ERR_UNSUPPORTED)
+				return rc;
+		}
 		GemmArgs a = plain(q->In, c.width, glu ? l.w_gate : l.w_up, c.width, hx, ff, n, ff, c.width);
 		a.W2 = glu ? l.w_up : nullptr;
 		a.w_bs = (long)ff * c.width;
@@ -1698,15 +1743,7 @@ static int ff_moe(Seq *q, int li, int n, const PostNorm *pn = nullptr) {
 		b.counts = q->counts;
 		TRY(gemm(q, b, E, n));
 	}
-	if (l.shared_ff > 0) {
-		GemmArgs a = plain(q->In, c.width, glu ? l.ws_gate : l.ws_up, c.width, hs, l.shared_ff, n, l.shared_ff, c.width);
-		a.W2 = glu ? l.ws_up : nullptr;
-		a.epi = epi;
-		a.limit = l.shared_limit;
-		TRY(gemm(q, a));
-		TRY(gemm(q, plain(hs, l.shared_ff, l.ws_down, l.shared_ff, ys, c.width, n, c.width, l.shared_ff)));
-	}
-	return YALM_OK; // the combine of yx (B[1]) and ys (B[3]) happens in the closing norm's launch (add_norm, par_close)
+	return ff_shared(q, li, n);
 }
 
 // The weights of the experts' combine; none where they have been applied to the experts' inputs.
