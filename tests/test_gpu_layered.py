@@ -232,6 +232,21 @@ def test_expert_groups_bf16(rt, experts, top, ff, n):
         model.close()
 
 
+@pytest.mark.parametrize("sizes", [[31, 32, 33], [64, 65], [9, 97, 63], [200]], ids=["around", "two", "mixed", "long"])
+def test_rglru_chunks(rt, sizes):
+    """The recurrence of portions in chunks of 32 tokens: whole, short and single chunks, from carried states."""
+    from yalm_amd import models as M
+
+    cfg = C.config([("rglru", C.rglru(width=272, blocks=17, conv=3), None)], width=64, vocab=101)
+    model, dec, w = build(rt, cfg, M.F32, seed=2)
+    try:
+        tok = C.tokens(cfg, sum(sizes), 3)
+        assert close_enough(run_portions(dec, tok, sizes), R.forward(cfg, w, tok), "f32")
+    finally:
+        dec.close()
+        model.close()
+
+
 @pytest.mark.parametrize("n", [9, 16, 17, 32, 33, 64, 65, 130, 255])
 def test_few_row_products_bf16(rt, n):
     """Products of 9 to 255 rows on the prefill unit: streamed in one or several K slices, large tiles in slices."""

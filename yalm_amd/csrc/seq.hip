@@ -1018,9 +1018,9 @@ static int mixer_rglru(Seq *q, int li, int n) {
 		seq_rglru_scan_kernel<<<cdiv(W, SEQ_THREADS), SEQ_THREADS, 0, q->stream>>>(r, ig, u, W, q->Z, 2 * W, l.lam,
 		                                                                           q->S[li], so, n);
 	} else {
-		seq_rglru_coef_kernel<<<dim3(cdiv(W, SEQ_THREADS), n), SEQ_THREADS, 0, q->stream>>>(r, ig, u, W, q->Z, 2 * W, l.lam,
-		                                                                                 n);
-		seq_rglru_walk_kernel<<<cdiv(W, SEQ_THREADS), SEQ_THREADS, 0, q->stream>>>(r, ig, u, W, q->S[li], so, n);
+		const dim3 g(cdiv(W, SEQ_THREADS), cdiv(n, RG_CHUNK));
+		seq_rglru_chunk_kernel<<<g, SEQ_THREADS, 0, q->stream>>>(r, ig, u, W, q->Z, 2 * W, l.lam, q->S[li], n);
+		seq_rglru_join_kernel<<<g, SEQ_THREADS, 0, q->stream>>>(r, ig, u, W, q->S[li], so, n);
 	}
 	HIPCHK(hipGetLastError());
 	return gemm(q, plain(so, W, l.w_o, W, q->Yout, c.width, n, c.width, W));
