@@ -324,6 +324,24 @@ def test_first_tokens(rt, n):
         model.close()
 
 
+@pytest.mark.parametrize("at", [14, 270, 1016], ids=["first", "window", "tiles"])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_decode_tiles(rt, at, dtype):
+    """Single tokens across edges of the 16-key tiles, past the end of a window, and from 16-key tiles to 64-key ones
+    (1024 keys); value rows of one and of several groups of 4 entries a thread."""
+    cfg = C.config([("attention", C.window(heads=4, kv_heads=2, dim=24, vdim=40, size=4000), None),
+                    ("attention_2", C.chunk(heads=6, kv_heads=1, dim=20, vdim=198, size=2000, rot_dims=4), None),
+                    ("attention", C.window(heads=2, kv_heads=2, dim=32, vdim=33, size=272), None)], width=64, vocab=101)
+    model, dec, w = build(rt, cfg, wdt_of(dtype), seed=6, max_tokens=1100)
+    try:
+        tok = C.tokens(cfg, at + 20, 9)
+        got = run_portions(dec, tok, [at] + [1] * 20)
+        assert rel_err(got[-20:], R.forward(cfg, w, tok)[-20:]).max() < tol(dtype)
+    finally:
+        dec.close()
+        model.close()
+
+
 @pytest.mark.parametrize("cfg", [C.ODD, C.MIXED], ids=["odd", "mixed"])
 def test_long_decoding(rt, cfg):
     """200 single tokens: every window and chunk of the model passes over decoded tokens

@@ -202,6 +202,10 @@ static bool latent_direct(const yalm_seq_layer &l) {
 static int delta_lpc(int K) {
 	return K <= 32 ? 8 : 16;
 }
+// The most keys that a short portion's tokens see
+static int attn_span(const yalm_seq_config &c, const yalm_seq_layer &l) {
+	return l.mask_kind == YALM_MASK_CAUSAL ? c.max_tokens : std::min(c.max_tokens, l.mask_size + GEMV_MAX_M);
+}
 static int delta_blocks(int K, int cols) {
 	return cdiv(cols, SEQ_THREADS / delta_lpc(K));
 }
@@ -617,14 +621,13 @@ static int create_seq(const yalm_seq_config *config, const yalm_seq_weights *w, 
 			}
 		q->att_splits = std::max(1, std::min(64, cdiv(c.max_tokens, ATS_KT)));
 		size_t part = (size_t)(4 * ATT_BR + GEMV_MAX_M * max_h) * q->att_splits * (att_rank4(max_rank) + 4);
-		// attn: the keys a single token can see, split so that a workgroup walks one tile (up to 64 splits)
+		// attn: the keys a single token can see, split so that a workgroup walks one 16-key tile (up to 64 splits)
 		q->attn_splits.assign(q->L.size(), 1);
 		for (int i = 0; i < (int)q->L.size(); ++i) {
 			const yalm_seq_layer &l = q->L[i];
 			if (l.mixer != YALM_MIX_ATTN && !latent_direct(l))
 				continue;
-			const int span = l.mask_kind == YALM_MASK_CAUSAL ? c.max_tokens : std::min(c.max_tokens, l.mask_size + GEMV_MAX_M);
-			q->attn_splits[i] = std::max(1, std::min(64, cdiv(span, SA_KT)));
+			q->attn_splits[i] = std::max(1, std::min(64, cdiv(attn_span(c, l), SD_KT)));
 			const int vd = l.mixer == YALM_MIX_ATTN ? l.vdim : std::max(l.kv_rank, l.vdim); // the attention's value size
 			part = std::max(part, (size_t)GEMV_MAX_M * l.heads * q->attn_splits[i] * (att_rank4(vd) + 4));
 		}
@@ -1305,8 +1308,9 @@ static int attn_core_t(Seq *q, int li, int n, const AttnArgs &a, const float *Q,
 	// many heads over few key/value heads: blocks of heads per workgroup, at most 16 heads each
 	// and small enough that key splits x key/value heads x blocks fill half the chip
 	int hb = rep;
+	const int tiles = std::max(1, std::min(64, cdiv(attn_span(q->c, q->L[li]), SA_KT)));
 	if (!talk)
-		while (hb > 1 && (hb > 16 || (rep >= 8 && (long)q->attn_splits[li] * a.G * cdiv(rep, hb) < 128)))
+		while (hb > 1 && (hb > 16 || (rep >= 8 && (long)tiles * a.G * cdiv(rep, hb) < 128)))
 			hb = (hb + 1) / 2;
 	const int hz = cdiv(rep, hb);
 	const size_t dec_lds = sa_decode_lds_bytes(hb, DK, talk ? a.H * a.D : 0, a.H);
@@ -1345,7 +1349,7 @@ static int attn_core_t(Seq *q, int li, int n, const AttnArgs &a, const float *Q,
 	while (TQ > 1 && (size_t)TQ * Hb * Gb * D4 * sizeof(float) > 64 * 1024)
 		--TQ;
 	const int R = TQ * Hb;
-	const int S = n <= GEMV_MAX_M ? q->attn_splits[li] : 1;
+	const int S = n <= GEMV_MAX_M ? tiles : 1;
 	const dim3 g(cdiv(n, TQ), S, a.G);
 	const size_t lds = sa_lds_bytes(R, Gb, a.D, a.V);
 	if (lds > 160 * 1024 - 64) {

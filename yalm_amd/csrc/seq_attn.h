@@ -634,12 +634,14 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_attn_kernel(const float *__re
 // split (gridDim.x = S) of the heads of one key/value head (gridDim.y = G; with score mixing
 // their mixed queries meet the whole key row), or of a block of hblk of them (hblk > 0, gridDim.z
 // blocks: many heads over one key/value head, where key splits alone are too few workgroups to
-// fill the chip); a lane owns a key and reads its cache row itself, 16 bytes at a time,
-// eight loads in flight; wave w takes a quarter of the key entries against every head's
-// queries (LDS broadcasts) and leaves partial scores in LDS; wave w then adds them up and
-// normalises heads w, w + 4, ...; then every thread sums NA4 groups of 4 value entries of one
-// head straight from the value rows. Partial results per split as in
-// seq_attn_kernel (S == 1 writes Ctx).
+// fill the chip), and walks it in tiles of KT keys: 64, or 16 where a split is no more than that (a token at up to 1024
+// keys). A lane owns a key and one of 256 / KT slices of its entries: it reads them itself, 16 bytes at a time, eight
+// loads in flight, against every head's queries (LDS broadcasts); the slices' partial scores meet in LDS; wave w adds
+// them up and normalises heads w, w + 4, ...; then every thread sums NA4 groups of 4 value entries of one head straight
+// from the value rows (16-key tiles: all rows in flight at once, and before the scores where a thread has one group).
+// Partial results per split as in seq_attn_kernel (S == 1 writes Ctx). All of it is latency: 800 keys, 8 heads of 256 over 2
+// took 13.5 us in 64-key tiles on 26 workgroups, 9.0 us in 16-key ones on 98.
+#define SD_KT 16
 template <class CT, int NA4>
 __global__ __launch_bounds__(SEQ_THREADS) void seq_attn_decode_kernel(const float *__restrict__ Q,
                                                                       const CT *__restrict__ Kc,
@@ -660,8 +662,8 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_attn_decode_kernel(const floa
 	const int DK = talk ? G * D : D, KL = a.KL, VL = a.VL, kcol = talk ? 0 : blockIdx.y * D;
 	const int DK8 = (DK + 7) & ~7, V4n = (V + 3) >> 2;
 	float *qs = lds;               // [Hb][DK8]
-	float *ps = qs + Hb * DK8;     // [Hb][SA_KT] softmax weights
-	float *pw = ps + Hb * SA_KT;   // [NW][Hb][SA_KT] the waves' partial scores
+	float *ps = qs + Hb * DK8;     // [Hb][KT] softmax weights
+	float *pw = ps + Hb * SA_KT;   // [NW][Hb][KT] the waves' partial scores
 	float *mrun = pw + NW * Hb * SA_KT; // [Hb]
 	float *lrun = mrun + Hb, *alpha = lrun + Hb;
 	const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -669,9 +671,12 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_attn_decode_kernel(const floa
 	const int pos = st->pos;
 	const int klo = attn_first_key(a.mask_kind, a.mask_size, pos);
 	int k_begin = klo, k_end = pos + 1;
+	const int nkeys = pos - klo + 1;
+	int chunk = (((nkeys + S - 1) / S) + SD_KT - 1) & ~(SD_KT - 1);
+	const bool few = chunk <= SD_KT;
 	if (S > 1) {
-		const int nkeys = pos - klo + 1;
-		const int chunk = (((nkeys + S - 1) / S) + SA_KT - 1) & ~(SA_KT - 1);
+		if (!few)
+			chunk = (chunk + SA_KT - 1) & ~(SA_KT - 1);
 		k_begin = klo + split * chunk;
 		k_end = min(pos + 1, k_begin + chunk);
 	}
@@ -710,151 +715,199 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_attn_decode_kernel(const floa
 		acc[x] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 	const bool kvec = DK % EPL == 0 && kcol % EPL == 0 && KL % EPL == 0 && (size_t)Kc % 16 == 0;
 	const bool vvec = V % 4 == 0 && VL % 4 == 0 && (size_t)Vc % 16 == 0;
-	const int DKw = (((DK + NW - 1) / NW) + EPL - 1) / EPL * EPL; // key entries per wave
-	const int dlo = min(wave * DKw, DK), dhi = min(DK, dlo + DKw);
-	__syncthreads();
-	for (int kt = k_begin; kt < k_end; kt += SA_KT) {
-		const int j = kt + lane;
-		const bool live = j < k_end;
-		const CT *krow = Kc + (size_t)(live ? j : k_end - 1) * KL + kcol;
-		// ---- partial scores: wave w takes its slice of the key entries, every head (HP per pass)
-		for (int hp0 = 0; hp0 < Hb; hp0 += HP) {
-			const int nh = min(HP, Hb - hp0);
-			float s[HP];
+	auto walk = [&](auto tile_keys) {
+		constexpr int KT = decltype(tile_keys)::value, NSL = NW * 64 / KT;
+		const int key = lane % KT, slice = wave * (64 / KT) + lane / KT;
+		const int DKw = (((DK + NSL - 1) / NSL) + EPL - 1) / EPL * EPL; // key entries per slice
+		const int dlo = min(slice * DKw, DK), dhi = min(DK, dlo + DKw);
+		for (int kt = k_begin; kt < k_end; kt += KT) {
+			const int j = kt + key;
+			const bool live = j < k_end;
+			const CT *krow = Kc + (size_t)(live ? j : k_end - 1) * KL + kcol;
+			// 4 value entries of a tile's rows (past the end: the last row again, its weight is 0)
+			constexpr bool EARLY = KT == SD_KT && NA4 == 1;
+			using vraw_t = std::conditional_t<sizeof(CT) == 2, uint2, float4_t>;
+			vraw_t vraw[KT == SD_KT ? KT : 1];
+			auto load_values = [&](int u) {
+				const CT *vp = Vc + ((h0 + u / V4n) / rep) * V + 4 * (u % V4n);
 #pragma unroll
-			for (int x = 0; x < HP; ++x)
-				s[x] = 0.0f;
-			if (kvec) {
-				constexpr int U = 8; // loads in flight
-				for (int d0 = dlo; d0 < dhi; d0 += U * EPL) {
-					u32x4_t w[U];
+				for (int jj = 0; jj < (KT == SD_KT ? KT : 1); ++jj)
+					vraw[jj] = *(const vraw_t *)(vp + (size_t)min(kt + jj, k_end - 1) * VL);
+			};
+			if (EARLY && vvec && tid < Hb * V4n)
+				load_values(tid);
+			// ---- partial scores: a lane takes its slice of its key's entries, every head (HP per pass)
+			for (int hp0 = 0; hp0 < Hb; hp0 += HP) {
+				const int nh = min(HP, Hb - hp0);
+				float s[HP];
 #pragma unroll
-					for (int u = 0; u < U; ++u)
-						w[u] = d0 + u * EPL < dhi ? load16(krow + d0 + u * EPL) : u32x4_t{0, 0, 0, 0};
+				for (int x = 0; x < HP; ++x)
+					s[x] = 0.0f;
+				if (kvec) {
+					constexpr int U = 8; // loads in flight
+					for (int d0 = dlo; d0 < dhi; d0 += U * EPL) {
+						u32x4_t w[U];
 #pragma unroll
-					for (int u = 0; u < U; ++u) {
-						const int d = d0 + u * EPL;
-						if (d >= dhi)
-							break;
-						float kf[EPL];
-						if constexpr (sizeof(CT) == 2)
-							WBF16::unpack(w[u], kf);
-						else
-							WF32::unpack(w[u], kf);
+						for (int u = 0; u < U; ++u)
+							w[u] = d0 + u * EPL < dhi ? load16(krow + d0 + u * EPL) : u32x4_t{0, 0, 0, 0};
 #pragma unroll
-						for (int x = 0; x < HP; ++x) {
-							if (x >= nh)
+						for (int u = 0; u < U; ++u) {
+							const int d = d0 + u * EPL;
+							if (d >= dhi)
 								break;
-							const float *qp = qs + (hp0 + x) * DK8 + d;
+							float kf[EPL];
+							if constexpr (sizeof(CT) == 2)
+								WBF16::unpack(w[u], kf);
+							else
+								WF32::unpack(w[u], kf);
 #pragma unroll
-							for (int e = 0; e < EPL; e += 4) {
-								const float4_t qv = *(const float4_t *)(qp + e);
-								s[x] = fmaf(qv[0], kf[e], s[x]);
-								s[x] = fmaf(qv[1], kf[e + 1], s[x]);
-								s[x] = fmaf(qv[2], kf[e + 2], s[x]);
-								s[x] = fmaf(qv[3], kf[e + 3], s[x]);
+							for (int x = 0; x < HP; ++x) {
+								if (x >= nh)
+									break;
+								const float *qp = qs + (hp0 + x) * DK8 + d;
+#pragma unroll
+								for (int e = 0; e < EPL; e += 4) {
+									const float4_t qv = *(const float4_t *)(qp + e);
+									s[x] = fmaf(qv[0], kf[e], s[x]);
+									s[x] = fmaf(qv[1], kf[e + 1], s[x]);
+									s[x] = fmaf(qv[2], kf[e + 2], s[x]);
+									s[x] = fmaf(qv[3], kf[e + 3], s[x]);
+								}
 							}
 						}
 					}
-				}
-			} else {
-				for (int d = dlo; d < dhi; ++d) {
-					float kv;
-					if constexpr (sizeof(CT) == 2)
-						kv = bf2f(krow[d]);
-					else
-						kv = krow[d];
-#pragma unroll
-					for (int x = 0; x < HP; ++x)
-						if (x < nh)
-							s[x] = fmaf(qs[(hp0 + x) * DK8 + d], kv, s[x]);
-				}
-			}
-#pragma unroll
-			for (int x = 0; x < HP; ++x)
-				if (x < nh)
-					pw[(wave * Hb + hp0 + x) * SA_KT + lane] = s[x];
-		}
-		__syncthreads();
-		// ---- running softmax, a wave per head
-		for (int r = wave; r < Hb; r += NW) {
-			float sv = 0.0f;
-#pragma unroll
-			for (int w = 0; w < NW; ++w)
-				sv += pw[(w * Hb + r) * SA_KT + lane];
-			sv = live ? attn_cap(sv, a.softcap) + attn_rel_bias(a, h0 + r, pos - j) : -FLT_MAX;
-			const float mold = mrun[r], lold = lrun[r];
-			const float mnew = fmaxf(mold, wave_max(sv));
-			const float p = live ? expf(sv - mnew) : 0.0f;
-			const float al = expf(mold - mnew);
-			const float l = lold * al + wave_sum(p);
-			ps[r * SA_KT + lane] = p;
-			if (lane == 0) {
-				mrun[r] = mnew;
-				lrun[r] = l;
-				alpha[r] = al;
-			}
-		}
-		__syncthreads();
-		// ---- weighted sums of the values
-		const int nk = min(SA_KT, k_end - kt);
-#pragma unroll
-		for (int x = 0; x < NA4; ++x) {
-			const int u = tid + x * SEQ_THREADS;
-			if (u >= Hb * V4n)
-				continue;
-			const int r = u / V4n, d4 = u % V4n;
-			const CT *vp = Vc + (size_t)kt * VL + ((h0 + r) / rep) * V + 4 * d4;
-			const float al = alpha[r];
-			float4_t v = acc[x];
-			v[0] *= al;
-			v[1] *= al;
-			v[2] *= al;
-			v[3] *= al;
-			const float *pr = ps + r * SA_KT;
-			if (vvec) {
-#pragma unroll 16
-				for (int jj = 0; jj < nk; ++jj) {
-					float c4[4];
-					if constexpr (sizeof(CT) == 2) {
-						const uint2 raw = *(const uint2 *)(vp + (size_t)jj * VL);
-						c4[0] = __builtin_bit_cast(float, raw.x << 16);
-						c4[1] = __builtin_bit_cast(float, raw.x & 0xffff0000u);
-						c4[2] = __builtin_bit_cast(float, raw.y << 16);
-						c4[3] = __builtin_bit_cast(float, raw.y & 0xffff0000u);
-					} else {
-						const float4_t raw = *(const float4_t *)(vp + (size_t)jj * VL);
-						c4[0] = raw[0];
-						c4[1] = raw[1];
-						c4[2] = raw[2];
-						c4[3] = raw[3];
-					}
-					const float p = pr[jj];
-					v[0] = fmaf(p, c4[0], v[0]);
-					v[1] = fmaf(p, c4[1], v[1]);
-					v[2] = fmaf(p, c4[2], v[2]);
-					v[3] = fmaf(p, c4[3], v[3]);
-				}
-			} else {
-				for (int jj = 0; jj < nk; ++jj) {
-					const float p = pr[jj];
-#pragma unroll
-					for (int e = 0; e < 4; ++e) {
-						if (4 * d4 + e >= V)
-							break;
-						float c;
+				} else {
+					for (int d = dlo; d < dhi; ++d) {
+						float kv;
 						if constexpr (sizeof(CT) == 2)
-							c = bf2f(vp[(size_t)jj * VL + e]);
+							kv = bf2f(krow[d]);
 						else
-							c = vp[(size_t)jj * VL + e];
-						v[e] = fmaf(p, c, v[e]);
+							kv = krow[d];
+#pragma unroll
+						for (int x = 0; x < HP; ++x)
+							if (x < nh)
+								s[x] = fmaf(qs[(hp0 + x) * DK8 + d], kv, s[x]);
 					}
 				}
+#pragma unroll
+				for (int x = 0; x < HP; ++x)
+					if (x < nh) {
+#pragma unroll
+						for (int d = KT; d < 64; d <<= 1)
+							s[x] += __shfl_xor(s[x], d);
+						if (lane < KT)
+							pw[(wave * Hb + hp0 + x) * KT + lane] = s[x];
+					}
 			}
-			acc[x] = v;
+			__syncthreads();
+			// ---- running softmax, a wave per head
+			for (int r = wave; r < Hb; r += NW) {
+				float sv = 0.0f;
+#pragma unroll
+				for (int w = 0; w < NW; ++w)
+					sv += pw[(w * Hb + r) * KT + key];
+				const bool mine = live && lane < KT;
+				sv = mine ? attn_cap(sv, a.softcap) + attn_rel_bias(a, h0 + r, pos - j) : -FLT_MAX;
+				const float mold = mrun[r], lold = lrun[r];
+				const float mnew = fmaxf(mold, wave_max(sv));
+				const float p = mine ? expf(sv - mnew) : 0.0f;
+				const float al = expf(mold - mnew);
+				const float l = lold * al + wave_sum(p);
+				if (lane < KT)
+					ps[r * KT + lane] = p;
+				if (lane == 0) {
+					mrun[r] = mnew;
+					lrun[r] = l;
+					alpha[r] = al;
+				}
+			}
+			__syncthreads();
+			// ---- weighted sums of the values
+			const int nk = min(KT, k_end - kt);
+#pragma unroll
+			for (int x = 0; x < NA4; ++x) {
+				const int u = tid + x * SEQ_THREADS;
+				if (u >= Hb * V4n)
+					continue;
+				const int r = u / V4n, d4 = u % V4n;
+				const CT *vp = Vc + (size_t)kt * VL + ((h0 + r) / rep) * V + 4 * d4;
+				const float al = alpha[r];
+				float4_t v = acc[x];
+				v[0] *= al;
+				v[1] *= al;
+				v[2] *= al;
+				v[3] *= al;
+				const float *pr = ps + r * KT;
+				if (KT == SD_KT && vvec) {
+					if (!EARLY)
+						load_values(u);
+#pragma unroll
+					for (int jj = 0; jj < (KT == SD_KT ? KT : 1); ++jj) {
+						const float p = pr[jj];
+						float c4[4];
+						if constexpr (sizeof(CT) == 2) {
+							c4[0] = __builtin_bit_cast(float, vraw[jj].x << 16);
+							c4[1] = __builtin_bit_cast(float, vraw[jj].x & 0xffff0000u);
+							c4[2] = __builtin_bit_cast(float, vraw[jj].y << 16);
+							c4[3] = __builtin_bit_cast(float, vraw[jj].y & 0xffff0000u);
+						} else {
+#pragma unroll
+							for (int e = 0; e < 4; ++e)
+								c4[e] = vraw[jj][e];
+						}
+#pragma unroll
+						for (int e = 0; e < 4; ++e)
+							v[e] = fmaf(p, c4[e], v[e]);
+					}
+				} else if (vvec) {
+#pragma unroll 16
+					for (int jj = 0; jj < nk; ++jj) {
+						float c4[4];
+						if constexpr (sizeof(CT) == 2) {
+							const uint2 raw = *(const uint2 *)(vp + (size_t)jj * VL);
+							c4[0] = __builtin_bit_cast(float, raw.x << 16);
+							c4[1] = __builtin_bit_cast(float, raw.x & 0xffff0000u);
+							c4[2] = __builtin_bit_cast(float, raw.y << 16);
+							c4[3] = __builtin_bit_cast(float, raw.y & 0xffff0000u);
+						} else {
+							const float4_t raw = *(const float4_t *)(vp + (size_t)jj * VL);
+							c4[0] = raw[0];
+							c4[1] = raw[1];
+							c4[2] = raw[2];
+							c4[3] = raw[3];
+						}
+						const float p = pr[jj];
+						v[0] = fmaf(p, c4[0], v[0]);
+						v[1] = fmaf(p, c4[1], v[1]);
+						v[2] = fmaf(p, c4[2], v[2]);
+						v[3] = fmaf(p, c4[3], v[3]);
+					}
+				} else {
+					for (int jj = 0; jj < nk; ++jj) {
+						const float p = pr[jj];
+#pragma unroll
+						for (int e = 0; e < 4; ++e) {
+							if (4 * d4 + e >= V)
+								break;
+							float c;
+							if constexpr (sizeof(CT) == 2)
+								c = bf2f(vp[(size_t)jj * VL + e]);
+							else
+								c = vp[(size_t)jj * VL + e];
+							v[e] = fmaf(p, c, v[e]);
+						}
+					}
+				}
+				acc[x] = v;
+			}
+			__syncthreads(); // ps and alpha are rewritten by the next tile
 		}
-		__syncthreads(); // ps and alpha are rewritten by the next tile
-	}
+	};
+	__syncthreads();
+	if (few)
+		walk(std::integral_constant<int, SD_KT>{});
+	else
+		walk(std::integral_constant<int, SA_KT>{});
 	__syncthreads();
 	const int stride = 4 * V4n + 4;
 #pragma unroll

@@ -2976,15 +2976,17 @@ static inline size_t ats_lds_bytes(int rank) {
 // Ctx[r] = sum_s e^(m_s - M) acc_s / sum_s e^(m_s - M) l_s over the key splits of row r
 // (times gate[r] if given; gate_e: times sigmoid of the row's own gate logits, row r = token
 // r / H, head r % H, logits at gate_e[token * ldg + head * rank + d]).
-// One workgroup per row: every wave works the splits' weights out for itself (lane s holds
-// split s, S <= 64), then the waves share the row's entries.
+// One workgroup per row: every wave works the splits' weights out for itself (lane s holds split s, S <= 64) and adds up
+// every fourth split with a weight, 4 entries a lane (the splits that saw keys come first); then the waves' sums meet.
 __global__ __launch_bounds__(SEQ_THREADS) void seq_latent_merge_kernel(const float *__restrict__ part, int S, int rank,
                                                               float *__restrict__ Ctx,
                                                               const float *__restrict__ gate = nullptr,
                                                               const float *__restrict__ gate_e = nullptr, int ldg = 0,
                                                               int H = 1) {
+	constexpr int NW = SEQ_THREADS / 64;
 	__shared__ float wsm_all[SEQ_THREADS];
-	const int r = blockIdx.x, rank4 = att_rank4(rank), stride = rank4 + 4, lane = threadIdx.x & 63;
+	__shared__ __attribute__((aligned(16))) float red[NW][256];
+	const int r = blockIdx.x, rank4 = att_rank4(rank), stride = rank4 + 4, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 	float *wsm = wsm_all + (threadIdx.x & ~63); // this wave's copy
 	const float *pp = part + (size_t)r * S * stride;
 	const float m = lane < S ? pp[(size_t)lane * stride + rank4] : -FLT_MAX;
@@ -2993,15 +2995,36 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_latent_merge_kernel(const flo
 	const float w = expf(m - M);
 	const float inv = (gate ? gate[r] : 1.0f) / wave_sum(w * l);
 	wsm[lane] = w * inv;
+	const int act = 64 - __clzll((long long)__ballot(l != 0.0f)); // past the last split with a sum
 	__syncthreads();
-	for (int d = threadIdx.x; d < rank; d += SEQ_THREADS) {
-		float v = 0.0f;
-#pragma unroll 8
-		for (int s = 0; s < S; ++s)
-			v = fmaf(wsm[s], pp[(size_t)s * stride + d], v);
-		if (gate_e)
-			v *= sq_sigmoid(gate_e[(size_t)(r / H) * ldg + (size_t)(r % H) * rank + d]);
-		Ctx[(size_t)r * rank + d] = v;
+	for (int d0 = 0; d0 < rank; d0 += 256) {
+		const int d = d0 + 4 * lane;
+		float4_t v = {0.0f, 0.0f, 0.0f, 0.0f};
+		if (d < rank4) {
+			for (int s0 = wave; s0 < act; s0 += 8 * NW) { // eight rows in flight (past the end: the last one, weight 0)
+				float4_t x[8];
+#pragma unroll
+				for (int u = 0; u < 8; ++u)
+					x[u] = *(const float4_t *)(pp + (size_t)min(s0 + u * NW, act - 1) * stride + d);
+#pragma unroll
+				for (int u = 0; u < 8; ++u)
+					v += x[u] * (s0 + u * NW < act ? wsm[s0 + u * NW] : 0.0f);
+			}
+		}
+		if (d0 > 0)
+			__syncthreads();
+		*(float4_t *)&red[wave][4 * lane] = v;
+		__syncthreads();
+		const int e = d0 + threadIdx.x;
+		if (e < rank) {
+			float o = 0.0f;
+#pragma unroll
+			for (int k = 0; k < NW; ++k)
+				o += red[k][threadIdx.x];
+			if (gate_e)
+				o *= sq_sigmoid(gate_e[(size_t)(r / H) * ldg + (size_t)(r % H) * rank + e]);
+			Ctx[(size_t)r * rank + e] = o;
+		}
 	}
 }
 
