@@ -175,7 +175,7 @@ const char *yalm_kernel_name(yalm_decoder d, int kernel_id);
 /* 1 if this decoder's launch path runs attention and the Wo projection (+ the
  * residual add) as ONE launch (attn_wo.h: the Wo weight stream overlaps the
  * attention; replaces attn + fused_matmul_add_residuals, infer.cu:338-524, 270):
- * head_dim 128, fp16 / fp8 weights with 1, 2, 4 or 8 KB (per-rank) Wo rows, and
+ * head_dim 128, fp16 / fp8 weights with 1, 2, 4, 6 or 8 KB (per-rank) Wo rows, and
  * not YALM_LAUNCH_SEPARATE_ATTN_WO. 0 = two separate launches. The split-KV
  * attention output is handed to the Wo workgroups as {value, epoch} granules. */
 int yalm_decoder_attn_wo(yalm_decoder d);

@@ -31,6 +31,9 @@ CASES = [
     ("fp8-xs1-g4", BASE.with_(n_heads=32, n_kv_heads=8, weight_dtype=M.F8E5M2)),
     ("fp8-xs2-g2", BASE.with_(n_heads=64, n_kv_heads=32, weight_dtype=M.F8E5M2)),
     ("f16-q_dim=dim", BASE.with_(dim=2048)),
+    ("f16-xs3-g3", BASE.with_(n_heads=24, n_kv_heads=8)),
+    ("f16-xs3-g8", BASE.with_(n_heads=24, n_kv_heads=3)),
+    ("fp8-xs3-g2", BASE.with_(n_heads=48, n_kv_heads=24, weight_dtype=M.F8E5M2)),
 ]
 
 

@@ -32,13 +32,16 @@
 // forward stopped part-way) stays correct. Every spin is bounded and reports in
 // *err.
 //
-// Geometry: Wo rows are q_dim * BYTES = KB KiB (KB in {1, 2, 4, 8}: 4 and 8 on one GPU
+// Geometry: Wo rows are q_dim * BYTES = KB KiB (KB in {1, 2, 4, 6, 8}: 4, 6 and 8 on one GPU
 // at Mistral / Llama shapes, 2 and 1 for the per-rank Wo of tensor parallelism); Wo
 // workgroup j owns rows [j * AWO_RPW, j * AWO_RPW + AWO_RPW) and thread t loads 16-byte
 // pieces i * 256 + t of that contiguous slice (LPT = AWO_RPW * KB / 4 loads). KB >= 4: a
 // thread's pieces cover every row of the slice, KB / 4 column pieces each; KB < 4: a
 // 4-KiB load instruction covers RPL = 4 / KB rows, so a thread covers every RPL-th row
-// at ONE column piece (256 / RPL threads per row).
+// at ONE column piece (256 / RPL threads per row). KB = 6 (Llama-3.2-3B's 24 heads in fp16): three load
+// instructions cover two rows, the middle one the end of the first (waves 0, 1) and the start of the second (waves 2,
+// 3), so a thread has three column pieces (awo_piece), one per load of a triple. Before, such rows ran as two launches:
+// attention 6.5 + Wo 6.7 us a layer, 10.9 as one.
 //
 // Outputs (round 5): x[row] = x + Wo v on one GPU; under tensor parallelism over RCCL
 // the partial (+ x on rank 0) goes to out = xs for the all-reduce; over IPC each row is
@@ -118,13 +121,22 @@ __device__ __forceinline__ void awo_ld8_sc1(u32x4_t (&v)[8], const void *const (
 // stale tag) slower again: fp8 kv 17 7.40 -> 8.49 us, kv 100 8.86 -> 11.68
 // (profiles/r4k_decode_ab.txt). False if the bounded spin gave up (deadline,
 // s_memrealtime).
-// XS pieces of EPL columns each: piece k of this thread starts at column
-// (piece0 + 256 k) * EPL; wpiece0 = piece0 of the wave's lane 0 (the sentinel heads).
-template <int EPL, int XS>
-__device__ __forceinline__ bool awo_gather_gran(float (&xs)[XS][EPL], const unsigned long long *gran, int piece0,
-                                                int wpiece0, unsigned tag, unsigned long long deadline) {
+// XS pieces of EPL columns each: piece k of thread t starts at column awo_piece<KB>(k, t) * EPL (the sentinel heads:
+// those of the wave's lane 0 and the 63 pieces after it).
+template <int KB>
+__device__ __forceinline__ int awo_piece(int k, int t) {
+	if constexpr (KB == 6) // (k * 256 + t) mod the 384 pieces of a row
+		return k == 0 ? t : (k == 1 ? (t < 128 ? t + 256 : t - 128) : t + 128);
+	else if constexpr (KB >= 4)
+		return k * ATTN_THREADS + t;
+	else
+		return t % (ATTN_THREADS * KB / 4);
+}
+template <int EPL, int XS, int KB>
+__device__ __forceinline__ bool awo_gather_gran(float (&xs)[XS][EPL], const unsigned long long *gran, unsigned tag,
+                                                unsigned long long deadline) {
 	constexpr int LPP = EPL / 2;   // 16-byte loads per piece
-	constexpr int NL = XS * LPP;   // 4, 8 or 16
+	constexpr int NL = XS * LPP;   // 4 to 24
 	constexpr int NB = (NL + 7) / 8;
 	constexpr int D = 128;
 	constexpr int HPP = 64 * EPL / D; // heads per piece (4 or 8)
@@ -134,7 +146,7 @@ __device__ __forceinline__ bool awo_gather_gran(float (&xs)[XS][EPL], const unsi
 	{
 		const int l = lane < XS * HPP ? lane : 0;
 		const int k = l / HPP;
-		const int h = (k * ATTN_THREADS + wpiece0) * EPL / D + l % HPP;
+		const int h = awo_piece<KB>(k, threadIdx.x & ~63) * EPL / D + l % HPP;
 		sent = gran + (size_t)h * D + (D - 1);
 	}
 	asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the slice has landed
@@ -155,7 +167,7 @@ __device__ __forceinline__ bool awo_gather_gran(float (&xs)[XS][EPL], const unsi
 		for (int i = 0; i < 8; ++i) {
 			const int l = bt * 8 + (i < NL - bt * 8 ? i : 0); // pad a short batch with a repeat
 			const int k = l / LPP, e = (l % LPP) * 2;
-			a[i] = gran + (size_t)(k * ATTN_THREADS + piece0) * EPL + e;
+			a[i] = gran + (size_t)awo_piece<KB>(k, threadIdx.x) * EPL + e;
 		}
 		u32x4_t v[8];
 		for (;;) {
@@ -191,12 +203,12 @@ __global__ __launch_bounds__(ATTN_THREADS) void attn_wo_kernel(const float *__re
                                                                const StepState *__restrict__ step, AttnWoArgs p) {
 	constexpr int D = 128;
 	constexpr int EPL = WT::EPL;
-	constexpr int XS = KB >= 4 ? KB / 4 : 1;   // column pieces per thread
-	constexpr int RPL = KB >= 4 ? 1 : 4 / KB;  // rows per 4-KiB load instruction
+	constexpr int XS = KB == 6 ? 3 : (KB >= 4 ? KB / 4 : 1); // column pieces per thread
+	constexpr int RPL = KB >= 4 ? 1 : 4 / KB;  // rows per 4-KiB load instruction (KB <= 4)
 	constexpr int TPR = ATTN_THREADS / RPL;    // threads per row (KB < 4)
 	constexpr int LPT = AWO_RPW * KB / 4;      // 16-byte loads per thread
 	static_assert(ATTN_THREADS == 256 && ATTN_WAVES == 4, "4-wave workgroups: one 4-row reduction per wave");
-	static_assert(KB == 1 || KB == 2 || KB == 4 || KB == 8, "Wo rows of 1, 2, 4 or 8 KiB");
+	static_assert(KB == 1 || KB == 2 || KB == 4 || KB == 6 || KB == 8, "Wo rows of 1, 2, 4, 6 or 8 KiB");
 	const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 	const int G = p.n_heads / p.n_kv;
 	const int units = p.n_kv * (p.S + G - 1); // attention workgroups (head units + split units)
@@ -268,8 +280,7 @@ __global__ __launch_bounds__(ATTN_THREADS) void attn_wo_kernel(const float *__re
 	// only for the heads its columns cover), then dot them into every resident row.
 	const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
 	float xs[XS][EPL];
-	const int piece0 = KB >= 4 ? tid : tid % TPR, wpiece0 = KB >= 4 ? 64 * wave : (64 * wave) % TPR;
-	if (!awo_gather_gran<EPL, XS>(xs, p.gran, piece0, wpiece0, epoch, t0 + AWO_TIMEOUT) && lane == 0)
+	if (!awo_gather_gran<EPL, XS, KB>(xs, p.gran, epoch, t0 + AWO_TIMEOUT) && lane == 0)
 		__hip_atomic_fetch_or(p.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 	if (tr)
 		t_poll = __builtin_amdgcn_s_memrealtime(), c_poll = __builtin_amdgcn_s_memtime();
@@ -278,9 +289,15 @@ __global__ __launch_bounds__(ATTN_THREADS) void attn_wo_kernel(const float *__re
 #pragma unroll
 		for (int r = 0; r < AWO_RPW; ++r) {
 			a0[r] = a1[r] = 0.0f;
+			if constexpr (KB == 6) { // rows r, r + 1: loads 3 r / 2, + 1 (this wave's half), + 2
+				dot16_mix<WT>(a0[r], a1[r], wr[r / 2 * 3 + 2 * (r & 1)], xs[2 * (r & 1)]);
+				if ((wave < 2) == !(r & 1))
+					dot16_mix<WT>(a0[r], a1[r], wr[r / 2 * 3 + 1], xs[1]);
+			} else {
 #pragma unroll
-			for (int k = 0; k < XS; ++k)
-				dot16_mix<WT>(a0[r], a1[r], wr[r * XS + k], xs[k]);
+				for (int k = 0; k < XS; ++k)
+					dot16_mix<WT>(a0[r], a1[r], wr[r * XS + k], xs[k]);
+			}
 		}
 		// ---- resident rows . slice; 4-row transposed wave reductions; fixed-order workgroup sum
 #pragma unroll

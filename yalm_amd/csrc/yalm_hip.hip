@@ -280,7 +280,7 @@ static const void *attn_wo_fn_g(int G) {
 }
 template <class WT>
 static const void *attn_wo_fn_kb(int G, int KB) {
-	return KB == 1 ? attn_wo_fn_g<WT, 1>(G) : KB == 2 ? attn_wo_fn_g<WT, 2>(G) : KB == 4 ? attn_wo_fn_g<WT, 4>(G)
+	return KB == 1 ? attn_wo_fn_g<WT, 1>(G) : KB == 2 ? attn_wo_fn_g<WT, 2>(G) : KB == 4 ? attn_wo_fn_g<WT, 4>(G) : KB == 6 ? attn_wo_fn_g<WT, 6>(G)
 	                                                                            : attn_wo_fn_g<WT, 8>(G);
 }
 static const void *attn_wo_pick(int dtype, int G, int KB) {
@@ -288,7 +288,7 @@ static const void *attn_wo_pick(int dtype, int G, int KB) {
 }
 // The fused launch's plan for a (per-rank) config: 1 with the key splits S and the grid,
 // or 0 = separate attention and Wo launches. Fused needs head_dim 128, G <= 8, fp16 / fp8
-// Wo rows of 1, 2, 4 or 8 KiB (one GPU: 4 / 8; a tensor-parallel rank's Wo slice: 1 / 2 too),
+// Wo rows of 1, 2, 4, 6 or 8 KiB (one GPU: 4 / 6 / 8; a tensor-parallel rank's Wo slice: 1 / 2 too),
 // and the whole grid (attention, one merger per query head, Wo)
 // within the co-resident workgroup slots: a workgroup past them is dispatched only when
 // an earlier one exits, and at short contexts every attention workgroup without keys
@@ -308,7 +308,7 @@ extern "C" int yalm_attn_wo_plan(const yalm_config *cp, int slots, int *splits, 
 	if (G < 1 || G > 8 || (c.weight_dtype != YALM_F16 && c.weight_dtype != YALM_F8E5M2))
 		return 0;
 	const int rb = c.n_heads * c.head_dim * (c.weight_dtype == YALM_F16 ? 2 : 1);
-	if ((rb != 1024 && rb != 2048 && rb != 4096 && rb != 8192) || c.dim < AWO_RPW)
+	if ((rb != 1024 && rb != 2048 && rb != 4096 && rb != 6144 && rb != 8192) || c.dim < AWO_RPW)
 		return 0;
 	const int nchunks = (c.max_seq_len + attn_chunk<128>() - 1) / attn_chunk<128>();
 	const int n_wo = (c.dim + AWO_RPW - 1) / AWO_RPW;
@@ -467,6 +467,9 @@ static int launch_attn_wo(yalm_decoder_s *d, const yalm_block_weights &w, int la
 			break;
 		case 4096:
 			launch_attn_wo_g<WT, 4>(d, w, p, G);
+			break;
+		case 6144:
+			launch_attn_wo_g<WT, 6>(d, w, p, G);
 			break;
 		default:
 			launch_attn_wo_g<WT, 8>(d, w, p, G);
