@@ -908,13 +908,16 @@ static int attn_t(Seq *q, const float *Qa, const void *cache, int rank, int H, i
 	const int na = cdiv(att_rank4(rank), 64);
 	// few rows (single tokens, short portions): the visible keys are split over workgroups
 	if (few) {
-		const dim3 gs(cdiv(NR, ATT_BR), q->att_splits);
-#define ATS_LAUNCH(NA)                                                                                                 \
-	seq_latent_split_kernel<CT, NA><<<gs, SEQ_THREADS, ats_lds_bytes(rank), q->stream>>>(Qa, (const CT *)cache, rank, H, NR, \
-	                                                                                    scale, q->st, q->att_part)
-		if (na <= 1) ATS_LAUNCH(1);
-		else if (na <= 2) ATS_LAUNCH(2);
-		else ATS_LAUNCH(4);
+		// a single token's rows in blocks of 4 unless blocks of 16 cover the chip by themselves
+		const int br = NR > 4 * ATT_BR ? ATT_BR : 4, nb = cdiv(br * (att_rank4(rank) / 4), SEQ_THREADS);
+		const dim3 gs(cdiv(NR, br), q->att_splits);
+#define ATS_LAUNCH(NA, BR)                                                                                             \
+	seq_latent_split_kernel<CT, NA, BR><<<gs, SEQ_THREADS, ats_lds_bytes(rank, BR), q->stream>>>(                      \
+	    Qa, (const CT *)cache, rank, H, NR, scale, q->st, q->att_part)
+		if (br == 4) ATS_LAUNCH(1, 4);
+		else if (nb <= 1) ATS_LAUNCH(1, ATT_BR);
+		else if (nb <= 2) ATS_LAUNCH(2, ATT_BR);
+		else ATS_LAUNCH(4, ATT_BR);
 #undef ATS_LAUNCH
 		seq_latent_merge_kernel<<<NR, SEQ_THREADS, 0, q->stream>>>(q->att_part, q->att_splits, rank, ctx);
 		HIPCHK(hipGetLastError());

@@ -2846,26 +2846,31 @@ static inline size_t att_lds_bytes(int rank) {
 	const int r4 = att_rank4(rank);
 	return sizeof(float) * ((size_t)ATT_BR * r4 + (size_t)ATT_KT * (r4 + 4) + ATT_BR * ATT_KT + 2 * ATT_BR);
 }
-// Single tokens and short portions: the same, the visible keys split over gridDim.y workgroups per ATT_BR rows, in tiles
+// Single tokens and short portions: the same, the visible keys split over gridDim.y workgroups per BR rows, in tiles
 // of ATS_KT keys: 16 rows x 16 keys, a score per thread, so a token at a short context is a handful of workgroups of one tile
 // each (64-key tiles, a workgroup of 16 rows walking them alone: 34 us at 86 keys, LDS reads of one CU). A split leaves
 // (sums, running maximum, running sum) per row in `part` for seq_latent_merge_kernel; one without keys leaves (0, -max, 0).
+// BR rows a workgroup: 16, or 4 where the row blocks and splits would be few workgroups (a row's wave then shares its entries
+// out over 4 lanes per key, and a thread has a quarter of the sums): 16 rows at 86 keys, 6 workgroups of 16 rows 12.7 us, 24
+// of 4 rows 7.0.
 #define ATS_KT 16
-template <class CT, int NA4>
+template <class CT, int NA4, int BR>
 __global__ __launch_bounds__(SEQ_THREADS) void seq_latent_split_kernel(const float *__restrict__ Qa,
                                                                        const CT *__restrict__ cache, int rank, int H, int NR,
                                                                        float scale, const StepState *__restrict__ st,
                                                                        float *__restrict__ part) {
 	extern __shared__ __attribute__((aligned(16))) float lds[];
 	const int rank4 = att_rank4(rank), ldc = rank4 + 4, q4n = rank4 >> 2;
-	float *qs = lds;                     // [ATT_BR][rank4 + 4]
-	float *cs = qs + ATT_BR * ldc;       // [ATS_KT][rank4 + 4]
-	float *ps = cs + ATS_KT * ldc;       // [ATT_BR][ATS_KT]
-	float *alpha = ps + ATT_BR * ATS_KT; // [ATT_BR]
-	const int tid = threadIdx.x, row = tid >> 4, key = tid & 15;
-	const int r0 = blockIdx.x * ATT_BR, S = gridDim.y, split = blockIdx.y;
+	float *qs = lds;                     // [BR][rank4 + 4]
+	float *cs = qs + BR * ldc;       // [ATS_KT][rank4 + 4]
+	float *ps = cs + ATS_KT * ldc;   // [BR][ATS_KT]
+	float *alpha = ps + BR * ATS_KT; // [BR]
+	constexpr int SL = SEQ_THREADS / (BR * ATS_KT); // lanes per (row, key), the key's lanes 16 apart in a wave
+	static_assert(SL == 1 || SL == 4, "a row is 16 lanes or a wave");
+	const int tid = threadIdx.x, row = tid / (ATS_KT * SL), key = tid & 15, sl = SL == 1 ? 0 : (tid >> 4) & 3;
+	const int r0 = blockIdx.x * BR, S = gridDim.y, split = blockIdx.y;
 	const int pos0 = st->pos;
-	const int nkeys = pos0 + (min(r0 + ATT_BR, NR) - 1) / H + 1; // keys visible to the workgroup's last row
+	const int nkeys = pos0 + (min(r0 + BR, NR) - 1) / H + 1; // keys visible to the workgroup's last row
 	const int chunk = (((nkeys + S - 1) / S) + ATS_KT - 1) & ~(ATS_KT - 1);
 	const int k_begin = split * chunk, k_end = min(nkeys, k_begin + chunk);
 	const int lim = r0 + row < NR ? min(pos0 + (r0 + row) / H, k_end - 1) : -1;
@@ -2875,7 +2880,7 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_latent_split_kernel(const flo
 		acc[a] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
 	float mrun = -FLT_MAX, lrun = 0.0f;
 	if (k_begin < k_end)
-		for (int i = tid; i < ATT_BR * rank4; i += SEQ_THREADS) {
+		for (int i = tid; i < BR * rank4; i += SEQ_THREADS) {
 			const int r = i / rank4, d = i % rank4;
 			qs[r * ldc + d] = (r0 + r < NR && d < rank) ? Qa[(size_t)(r0 + r) * rank + d] * scale : 0.0f;
 		}
@@ -2917,28 +2922,34 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_latent_split_kernel(const flo
 			float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 			const float4_t *cj = (const float4_t *)(cs + key * ldc), *qj = (const float4_t *)(qs + row * ldc);
 #pragma unroll 8
-			for (int d = 0; d < q4n; ++d) {
+			for (int d = sl; d < q4n; d += SL) {
 				const float4_t c = cj[d], qv = qj[d];
 #pragma unroll
 				for (int e = 0; e < 4; ++e)
 					s[e] = fmaf(qv[e], c[e], s[e]);
 			}
 			const bool vis = kt + key <= lim;
-			const float sv = vis ? (s[0] + s[1]) + (s[2] + s[3]) : -FLT_MAX;
+			float dot = (s[0] + s[1]) + (s[2] + s[3]);
+			if constexpr (SL > 1) {
+				dot += __shfl_xor(dot, 16);
+				dot += __shfl_xor(dot, 32);
+			}
+			const float sv = vis ? dot : -FLT_MAX;
 			const float mnew = fmaxf(mrun, row16_max(sv));
 			const float p = vis ? expf(sv - mnew) : 0.0f;
 			const float al = expf(mrun - mnew); // 1 while nothing is visible yet, 0 at the first key
 			lrun = lrun * al + row16_sum(p);
 			mrun = mnew;
-			ps[row * ATS_KT + key] = p;
-			if (key == 0)
+			if (sl == 0)
+				ps[row * ATS_KT + key] = p;
+			if (key == 0 && sl == 0)
 				alpha[row] = al;
 		}
 		__syncthreads();
 #pragma unroll
 		for (int a = 0; a < NA4; ++a) {
 			const int u = tid + a * SEQ_THREADS;
-			if (u < ATT_BR * q4n) {
+			if (u < BR * q4n) {
 				const int r = u / q4n, d4 = u % q4n;
 				float4_t v = acc[a] * alpha[r];
 				const float4_t *pr = (const float4_t *)(ps + r * ATS_KT);
@@ -2958,7 +2969,7 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_latent_split_kernel(const flo
 		}
 	}
 	const int stride = rank4 + 4;
-	if (key == 0 && r0 + row < NR) {
+	if (key == 0 && sl == 0 && r0 + row < NR) {
 		float *pp = part + ((size_t)(r0 + row) * S + split) * stride;
 		pp[rank4] = mrun;
 		pp[rank4 + 1] = lrun;
@@ -2966,12 +2977,12 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_latent_split_kernel(const flo
 #pragma unroll
 	for (int a = 0; a < NA4; ++a) {
 		const int u = tid + a * SEQ_THREADS;
-		if (u < ATT_BR * q4n && r0 + u / q4n < NR)
+		if (u < BR * q4n && r0 + u / q4n < NR)
 			*(float4_t *)(part + ((size_t)(r0 + u / q4n) * S + split) * stride + 4 * (u % q4n)) = acc[a];
 	}
 }
-static inline size_t ats_lds_bytes(int rank) {
-	return sizeof(float) * ((size_t)(ATT_BR + ATS_KT) * (att_rank4(rank) + 4) + ATT_BR * ATS_KT + ATT_BR);
+static inline size_t ats_lds_bytes(int rank, int br) {
+	return sizeof(float) * ((size_t)(br + ATS_KT) * (att_rank4(rank) + 4) + br * ATS_KT + br);
 }
 // Ctx[r] = sum_s e^(m_s - M) acc_s / sum_s e^(m_s - M) l_s over the key splits of row r
 // (times gate[r] if given; gate_e: times sigmoid of the row's own gate logits, row r = token
