@@ -624,7 +624,7 @@ int enqueue_prefill(yalm_decoder_s *d, int T, int pos0, bool want_lp, const int 
 	const int half = c.head_dim / 2;
 	pf::rope_table_kernel<<<(T * half + 255) / 256, 256, 0, st>>>(d->inv_freq, half, T, pos0, b.rope);
 	HIPCHK(hipGetLastError());
-	// fp8: every GEMM reads the E5M2 bytes (gemm8p_kernel, skinny_gemm_lds_kernel) with the slices and K order of
+	// fp8: every GEMM reads the E5M2 bytes (gemm8p_kernel, stream_gemm_kernel) with the slices and K order of
 	// the f16 twin, so the results are its bit for bit; forms that name other kernels run on f16 copies
 	const bool raw8 = fp8 && f.p8 && f.skl && f.g16[PG_QKV] < 0 && f.g16[PG_WO] < 0 && f.g16[PG_GLU] < 0 && f.g16[PG_W2] < 0;
 	// GEMM widths are the same for every layer
