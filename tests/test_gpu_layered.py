@@ -247,6 +247,24 @@ def test_rglru_chunks(rt, sizes):
         model.close()
 
 
+@pytest.mark.parametrize("taps", [1, 2, 4, 5, 16])
+def test_convolution_blocks(rt, taps):
+    """Convolutions of portions, 8 tokens a thread: windows of 4 and of 16 taps, the stored inputs of earlier portions shorter
+    and longer than a block."""
+    from yalm_amd import models as M
+
+    cfg = C.config([("rglru", C.rglru(width=48, blocks=3, conv=taps), None),
+                    ("delta", C.delta(heads=2, kv_heads=1, dim=16, vdim=16, conv=taps), None)], width=64, vocab=101)
+    model, dec, w = build(rt, cfg, M.F32, seed=2)
+    try:
+        sizes = [9, 15, 16, 17, 1, 24, 31]
+        tok = C.tokens(cfg, sum(sizes), 3)
+        assert close_enough(run_portions(dec, tok, sizes), R.forward(cfg, w, tok), "f32")
+    finally:
+        dec.close()
+        model.close()
+
+
 @pytest.mark.parametrize("n", [9, 16, 17, 32, 33, 64, 65, 130, 255])
 def test_few_row_products_bf16(rt, n):
     """Products of 9 to 255 rows on the prefill unit: streamed in one or several K slices, large tiles in slices."""

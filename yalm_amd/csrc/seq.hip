@@ -980,8 +980,8 @@ static int conv_launch(Seq *q, const float *Z, int ldz, int col0, int C, int tap
 		seq_conv_step_kernel<<<cdiv(C, SEQ_THREADS), SEQ_THREADS, 0, q->stream>>>(Z, ldz, col0, C, taps, w, bias, silu, state,
 		                                                                          out, C, n);
 	} else {
-		seq_conv_kernel<<<dim3(cdiv(C, SEQ_THREADS), n), SEQ_THREADS, 0, q->stream>>>(Z, ldz, col0, C, taps, w, bias, silu,
-		                                                                              state, out, C, n);
+		(taps <= 4 ? seq_conv_kernel<4> : seq_conv_kernel<SEQ_MAX_TAPS>)<<<dim3(cdiv(C, SEQ_THREADS), cdiv(n, CONV_TB)), SEQ_THREADS, 0,
+		                                                                 q->stream>>>(Z, ldz, col0, C, taps, w, bias, silu, state, out, C, n);
 		if (taps > 1)
 			seq_conv_state_kernel<<<cdiv(C, SEQ_THREADS), SEQ_THREADS, 0, q->stream>>>(Z, ldz, col0, C, taps, state, n);
 	}

@@ -1951,22 +1951,41 @@ __global__ __launch_bounds__(SEQ_THREADS) void seq_gemm_bf16_kernel(GemmArgs a) 
 #define SEQ_MAX_TAPS 16
 // out[t][c] = act(bias[c] + sum_j w[c][j] in(t - (taps - 1) + j)), in(tau) = Z[tau][col0 + c] for
 // tau >= 0, else the sequence's stored last inputs state[(taps - 1) + tau][c] (zeros at the start).
+// A thread takes CONV_TB tokens of a channel, their inputs loaded at once and each read once by it (at most TW taps): bytes
+// bound it, 2048 tokens x 4096 channels 64 MB; a token a thread waited for its taps one after another, 44 us, 16 so.
+#define CONV_TB 8
+template <int TW>
 __global__ __launch_bounds__(SEQ_THREADS) void seq_conv_kernel(const float *__restrict__ Z, int ldz, int col0, int C,
                                                                int taps, const float *__restrict__ w,
                                                                const float *__restrict__ bias, int silu,
                                                                const float *__restrict__ state,
                                                                float *__restrict__ out, int ldo, int T) {
 	const int c = blockIdx.x * SEQ_THREADS + threadIdx.x;
-	const int t = blockIdx.y;
+	const int t0 = blockIdx.y * CONV_TB;
 	if (c >= C)
 		return;
-	float acc = bias ? bias[c] : 0.0f;
-	for (int j = 0; j < taps; ++j) {
-		const int tau = t - (taps - 1) + j;
-		const float v = tau >= 0 ? Z[(size_t)tau * ldz + col0 + c] : state[(size_t)(taps - 1 + tau) * C + c];
-		acc = fmaf(w[(size_t)c * taps + j], v, acc);
+	const int skip = TW - taps; // of the window's TW entries
+	float v[CONV_TB + TW - 1], wv[TW];
+#pragma unroll
+	for (int i = 0; i < CONV_TB + TW - 1; ++i) { // input t0 - (TW - 1) + i
+		const int tau = min(t0 - (TW - 1) + i, T - 1);
+		v[i] = i < skip ? 0.0f : tau >= 0 ? Z[(size_t)tau * ldz + col0 + c] : state[(size_t)(taps - 1 + tau) * C + c];
 	}
-	out[(size_t)t * ldo + c] = silu ? sq_silu(acc) : acc;
+#pragma unroll
+	for (int j = 0; j < TW; ++j)
+		wv[j] = j >= skip ? w[(size_t)c * taps + j - skip] : 0.0f;
+	const float b = bias ? bias[c] : 0.0f;
+#pragma unroll
+	for (int k = 0; k < CONV_TB; ++k) {
+		if (t0 + k >= T)
+			break;
+		float acc = b;
+#pragma unroll
+		for (int j = 0; j < TW; ++j)
+			if (j >= skip)
+				acc = fmaf(wv[j], v[k + j], acc);
+		out[(size_t)(t0 + k) * ldo + c] = silu ? sq_silu(acc) : acc;
+	}
 }
 // Short portions (T <= SEQ_CONV_STEP_T): convolution and state shift in one launch, a thread
 // per channel walking the tokens with the last taps - 1 inputs in registers.
