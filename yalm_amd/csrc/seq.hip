@@ -78,6 +78,7 @@ struct yalm_seq_s {
 	int ldz = 0;
 	float *inv_freq = nullptr;
 	uint16_t *a16 = nullptr;     // [cap][bw] bf16 copy of a product's activations (large-tile GEMM operand)
+	const float *a16_of = nullptr; // a16 holds the portion's rows of this buffer (the last seam left them), else null
 	float *gpart = nullptr;      // f32 partials of those products' K slices (at most 32 MB)
 	size_t gpart_floats = 0;
 	int *tok = nullptr, *want = nullptr;
@@ -843,6 +844,9 @@ static int gemm_t(Seq *q, const GemmArgs &a, int batches, int max_m) {
 }
 // f32w: the matrices are f32 whatever the model's weight type (the recurrence's gates)
 static int to_bf16(Seq *q, const float *A, int lda, int M, int K) { // A's rows into q->a16
+	if (A == q->a16_of && lda == q->c.width && K == q->c.width) // M: the portion's rows, all of them
+		return YALM_OK;
+	q->a16_of = nullptr;
 	const size_t n8 = (size_t)M * (K / 8);
 	seq_to_bf16_kernel<<<(unsigned)std::min<size_t>((n8 + SEQ_THREADS - 1) / SEQ_THREADS, 4096), SEQ_THREADS, 0, q->stream>>>(
 	    A, lda, M, K, q->a16);
@@ -1821,11 +1825,15 @@ static int post_close(Seq *q, const float *wb, int n, const yalm_seq_layer *moe)
 // moe: the layer's routed experts feed the norm (their combine happens inside it) instead of Y
 static int add_norm(Seq *q, const float *wb, const float *w_next, int n, const yalm_seq_layer *moe) {
 	const int w = q->c.width;
+	q->a16_of = nullptr;
 	if (w <= 16 * SEQ_THREADS) { // the row in registers
 		const Combine cb = combine_of(q, moe);
+		const bool b16 = q->a16 && n > GEMV_MAX_M && (w_next || !q->c.pre_norm);
+		if (b16)
+			q->a16_of = q->In;
 #define AN_LAUNCH(E, C)                                                                                                \
 	seq_add_norm_reg_kernel<E, C><<<n, SEQ_THREADS, 0, q->stream>>>(q->X, q->Y, wb, q->c.norm_eps, w, w_next, q->Hn, q->nk, \
-	                                                                q->c.residual_scale, cb)
+	                                                                q->c.residual_scale, cb, b16 ? q->a16 : nullptr)
 		if (w <= 4 * SEQ_THREADS) {
 			if (moe) AN_LAUNCH(4, true);
 			else AN_LAUNCH(4, false);
@@ -1863,6 +1871,7 @@ static int enqueue_portion(Seq *q, const int *tokens_dev, int n) {
 		q->In = q->X;
 	settled(q);
 	q->hn_final = false;
+	q->a16_of = nullptr;
 	const bool fold = an_foldable(q, n);
 	// the seam after a sublayer: applied now, or owed to the product that reads the stream next (identity outputs read the
 	// row that the seam rewrites: now)
@@ -2010,6 +2019,7 @@ static int enqueue_portion(Seq *q, const int *tokens_dev, int n) {
 static int enqueue_logits(Seq *q, const int *rows_dev, int n_rows) {
 	const yalm_seq_config &c = q->c;
 	const dim3 ng(n_rows, q->nk == NK_TANH ? cdiv(c.width, SEQ_THREADS) : 1);
+	q->a16_of = nullptr; // Hn's rows become the asked rows' final norms
 	if (!q->hn_final)
 		seq_norm_kernel<float><<<ng, SEQ_THREADS, 0, q->stream>>>(q->X, c.width, q->final_norm, c.norm_eps, c.width,
 		                                                          q->Hn, c.width, rows_dev, q->st, 0, q->nk, c.logit_scale);
