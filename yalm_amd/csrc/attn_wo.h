@@ -121,20 +121,18 @@ __device__ __forceinline__ void awo_ld8_sc1(u32x4_t (&v)[8], const void *const (
 // stale tag) slower again: fp8 kv 17 7.40 -> 8.49 us, kv 100 8.86 -> 11.68
 // (profiles/r4k_decode_ab.txt). False if the bounded spin gave up (deadline,
 // s_memrealtime).
-// XS pieces of EPL columns each: piece k of thread t starts at column awo_piece<KB>(k, t) * EPL (the sentinel heads:
-// those of the wave's lane 0 and the 63 pieces after it).
+// XS pieces of EPL columns each: piece k of this thread starts at column awo_piece<KB>(k, piece0) * EPL; wpiece0 = piece0
+// of the wave's lane 0 (the sentinel heads).
 template <int KB>
-__device__ __forceinline__ int awo_piece(int k, int t) {
-	if constexpr (KB == 6) // (k * 256 + t) mod the 384 pieces of a row
-		return k == 0 ? t : (k == 1 ? (t < 128 ? t + 256 : t - 128) : t + 128);
-	else if constexpr (KB >= 4)
-		return k * ATTN_THREADS + t;
+__device__ __forceinline__ int awo_piece(int k, int piece0) {
+	if constexpr (KB == 6) // (256 k + piece0) mod the 384 pieces of a row
+		return k == 0 ? piece0 : (k == 1 ? (piece0 < 128 ? piece0 + 256 : piece0 - 128) : piece0 + 128);
 	else
-		return t % (ATTN_THREADS * KB / 4);
+		return k * ATTN_THREADS + piece0;
 }
 template <int EPL, int XS, int KB>
-__device__ __forceinline__ bool awo_gather_gran(float (&xs)[XS][EPL], const unsigned long long *gran, unsigned tag,
-                                                unsigned long long deadline) {
+__device__ __forceinline__ bool awo_gather_gran(float (&xs)[XS][EPL], const unsigned long long *gran, int piece0,
+                                                int wpiece0, unsigned tag, unsigned long long deadline) {
 	constexpr int LPP = EPL / 2;   // 16-byte loads per piece
 	constexpr int NL = XS * LPP;   // 4 to 24
 	constexpr int NB = (NL + 7) / 8;
@@ -146,7 +144,7 @@ __device__ __forceinline__ bool awo_gather_gran(float (&xs)[XS][EPL], const unsi
 	{
 		const int l = lane < XS * HPP ? lane : 0;
 		const int k = l / HPP;
-		const int h = awo_piece<KB>(k, threadIdx.x & ~63) * EPL / D + l % HPP;
+		const int h = awo_piece<KB>(k, wpiece0) * EPL / D + l % HPP;
 		sent = gran + (size_t)h * D + (D - 1);
 	}
 	asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the slice has landed
@@ -167,7 +165,7 @@ __device__ __forceinline__ bool awo_gather_gran(float (&xs)[XS][EPL], const unsi
 		for (int i = 0; i < 8; ++i) {
 			const int l = bt * 8 + (i < NL - bt * 8 ? i : 0); // pad a short batch with a repeat
 			const int k = l / LPP, e = (l % LPP) * 2;
-			a[i] = gran + (size_t)awo_piece<KB>(k, threadIdx.x) * EPL + e;
+			a[i] = gran + (size_t)awo_piece<KB>(k, piece0) * EPL + e;
 		}
 		u32x4_t v[8];
 		for (;;) {
@@ -280,7 +278,8 @@ __global__ __launch_bounds__(ATTN_THREADS) void attn_wo_kernel(const float *__re
 	// only for the heads its columns cover), then dot them into every resident row.
 	const unsigned long long t0 = __builtin_amdgcn_s_memrealtime();
 	float xs[XS][EPL];
-	if (!awo_gather_gran<EPL, XS, KB>(xs, p.gran, epoch, t0 + AWO_TIMEOUT) && lane == 0)
+	const int piece0 = KB >= 4 ? tid : tid % TPR, wpiece0 = KB >= 4 ? 64 * wave : (64 * wave) % TPR;
+	if (!awo_gather_gran<EPL, XS, KB>(xs, p.gran, piece0, wpiece0, epoch, t0 + AWO_TIMEOUT) && lane == 0)
 		__hip_atomic_fetch_or(p.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 	if (tr)
 		t_poll = __builtin_amdgcn_s_memrealtime(), c_poll = __builtin_amdgcn_s_memtime();
